@@ -5,14 +5,21 @@
 // replaying every pseudo-legal move); the CPU generator of this repository (chessgen.c, pinned by
 // the published perft counts) is its checker.
 //
-// One wavefront per position.  The position's bitboards (occupancy by colour, the enemy's pieces
-// by kind) are built once per wave on the scalar unit from the 32 words.  Lane l < 32 generates
-// slot l's pseudo-legal targets -- a slider's reach along a line is two subtractions, the other
-// pieces are shift patterns: no loop over squares -- and each target is tested by "replaying" the
-// move on the bitboards (occupancy, captured piece, en-passant victim, castled rook) and asking
-// whether the enemy attacks the king's square -- for castling the start, crossed and landing
-// squares, evaluated on the position after the move, as the checker does.  For that step the
-// position's moves are dealt out evenly over the 64 lanes.
+// Four positions per wavefront, a row of sixteen lanes each: lane s of the row holds slot s of the side to
+// move (its kings stand in slots 15 and 31, its colours in slots 0..15 and 16..31 by the format) and
+// slot s of the other side.  The bitboards every lane needs (own pieces, the enemy's pieces by kind)
+// are OR-reductions over the row.  A slider's reach along a line is two subtractions and the other
+// pieces are shift patterns, so there is no loop over squares.  Legality takes two questions per lane
+// instead of one replay per move:
+//   * every lane asks which enemies attack the king once this lane's piece has left its square: none
+//     -- the piece may go anywhere it reaches; one -- it must capture that one or step between it and
+//     the king; two -- no move of it helps.  This is what replaying each of its moves would answer:
+//     a piece put on a square can only take the enemy there or block a line.
+//   * lanes 0..7 each try one king step, lanes 8..13 the three squares of either castling, on the
+//     position after the move.
+// En passant, where two pieces leave the board's lines at once, is replayed (a loop that hardly ever
+// runs).  Integer work, bound by the vector ALU: one wavefront per position (its boards built on the
+// scalar unit, each of some 31 moves replayed) took 119 us for 65536 positions, this 24 us (0.9 TB/s of its bytes).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -78,145 +85,146 @@ __device__ __forceinline__ u64 king_pattern(u64 s) {
     return (row | row << 8 | row >> 8) ^ s;
 }
 
-// Does `e` attack square sq, given occupancy occ?  Looked at from the square: a rook placed there
-// sees the enemy's orthogonal sliders exactly when they see it, and so for the other kinds.
-__device__ __forceinline__ bool attacked(const Enemy& e, u64 occ, int sq) {
+// The pieces of `e` that attack square sq, given occupancy occ.  Looked at from the square: a rook placed
+// there sees the enemy's orthogonal sliders exactly when they see it, and so for the other kinds.
+__device__ __forceinline__ u64 attackers(const Enemy& e, u64 occ, int sq) {
     const u64 s = bit(sq);
     // a white pawn on (r-1, c+-1) attacks (r, c); a black one from (r+1, c+-1)
     const u64 pawn_from = e.black ? (((s << 7) & NOT_H) | ((s << 9) & NOT_A)) : (((s >> 7) & NOT_A) | ((s >> 9) & NOT_H));
-    const u64 hit = (pawn_from & e.pawns) | (knight_pattern(s) & e.knights) | (king_pattern(s) & e.king) |
-                    (rook_attacks(occ, sq) & e.orth) | (bishop_attacks(occ, sq) & e.diag);
-    return hit != 0;
+    return (pawn_from & e.pawns) | (knight_pattern(s) & e.knights) | (king_pattern(s) & e.king) |
+           (rook_attacks(occ, sq) & e.orth) | (bishop_attacks(occ, sq) & e.diag);
+}
+
+// the squares strictly between a and x (one bit each) if they share a line, else none
+__device__ __forceinline__ u64 between(int a, u64 x) {
+    const Lines l = lines_through(a);
+    const u64 line = (l.rank & x) ? l.rank : (l.file & x) ? l.file : (l.diag & x) ? l.diag : (l.anti & x) ? l.anti : 0;
+    const u64 s = bit(a), hi = x > s ? x : s, lo = x > s ? s : x;
+    return line & (hi - 1) & ~(lo | (lo - 1));
+}
+
+// OR over the sixteen lanes of a row, in every lane
+template <int CTRL>
+__device__ __forceinline__ unsigned or_ror(unsigned v) {
+    return v | (unsigned)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, false);
+}
+__device__ __forceinline__ u64 row_or(u64 v) {
+    unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
+    lo = or_ror<0x128>(lo); hi = or_ror<0x128>(hi);    // row_ror:8, 4, 2, 1
+    lo = or_ror<0x124>(lo); hi = or_ror<0x124>(hi);
+    lo = or_ror<0x122>(lo); hi = or_ror<0x122>(hi);
+    lo = or_ror<0x121>(lo); hi = or_ror<0x121>(hi);
+    return ((u64)hi << 32) | lo;
 }
 
 __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, const int16_t* control, int n,
                                                       u64* mask, uint8_t* in_check) {
-    const int lane = threadIdx.x & 63;
-    // the position and the side to move are the same for the whole wave: said so, the bitboard
-    // construction below runs on the scalar unit
-    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-    if (b >= n) return;                                 // no workgroup barrier below
-    const int slot = lane & 31, part = lane >> 5;
-    const unsigned w = boards[(size_t)b * 32 + slot];
-    const bool black = __builtin_amdgcn_readfirstlane((int)control[b]) < 0;
+    const int lane = threadIdx.x & 63, slot = lane & 15;
+    const int b_ = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 4);
+    const bool here = b_ < n;
+    const int b = here ? b_ : n - 1;                    // a row past the end repeats the last position and stores nothing
+    const bool black = control[b] < 0;
+    const uint16_t* const bw = boards + (size_t)b * 32;
+    const unsigned w = bw[(black ? 16 : 0) + slot], v = bw[(black ? 0 : 16) + slot];
+    const unsigned kw = bw[black ? 31 : 15], ke = bw[black ? 15 : 31];
 
-    // bitboards, computed by every lane from the words of all 32 slots
-    u64 own = 0, opp = 0, ep_pawns = 0;
-    Enemy e = {0, 0, 0, 0, 0, !black};
-    bool rook_short = false, rook_long = false;         // an unmoved own rook on its corner
-    const unsigned row = black ? 56u : 0u;
-    const unsigned rookw = (black ? COLOR : 0u) | (ROOK << 6);
-#pragma unroll
-    for (int s = 0; s < 32; s++) {
-        const unsigned v = (unsigned)__builtin_amdgcn_readlane((int)w, s);   // wave-uniform: the loop runs on the scalar unit
-        rook_short |= v == (rookw | (row + 7));
-        rook_long |= v == (rookw | row);
-        if (v & CAPTURED) continue;
-        const u64 sb = bit(v & 63);
-        const int t = (v >> 6) & 7;
-        if (((v >> 10) & 1) == (unsigned)black) {
-            own |= sb;
-        } else {
-            opp |= sb;
-            if (t == PAWN) { e.pawns |= sb; if (v & SPECIAL) ep_pawns |= sb; }
-            else if (t == KNIGHT) e.knights |= sb;
-            else if (t == KING) e.king |= sb;
-            if (t == BISHOP || t == QUEEN) e.diag |= sb;
-            if (t == ROOK || t == QUEEN) e.orth |= sb;
-        }
-    }
+    // bitboards, the same in every lane of the row
+    const bool mine = !(w & CAPTURED) && ((w >> 10) & 1) == (unsigned)black;
+    const bool theirs = !(v & CAPTURED) && ((v >> 10) & 1) != (unsigned)black;
+    const int sq = w & 63, t = (w >> 6) & 7, te = (v >> 6) & 7;
+    const u64 fb = bit(sq), vb = theirs ? bit(v & 63) : 0;
+    const u64 own = row_or(mine ? fb : 0);
+    Enemy e;
+    e.black = !black;
+    e.pawns = row_or(te == PAWN ? vb : 0);
+    const u64 ep_pawns = row_or(te == PAWN && (v & SPECIAL) ? vb : 0);
+    e.knights = row_or(te == KNIGHT ? vb : 0);
+    e.diag = row_or(te == BISHOP || te == QUEEN ? vb : 0);
+    e.orth = row_or(te == ROOK || te == QUEEN ? vb : 0);
+    e.king = (ke & CAPTURED) ? 0 : bit(ke & 63);
+    const u64 opp = e.pawns | e.knights | e.diag | e.orth | e.king;
     const u64 occ = own | opp;
-    const int ksq = (black ? __builtin_amdgcn_readlane((int)w, 31) : __builtin_amdgcn_readlane((int)w, 15)) & 63;
-    if (lane == 0 && in_check) in_check[b] = attacked(e, occ, ksq) ? 1 : 0;
+    const int ksq = kw & 63;
+    // an unmoved own rook on its corner
+    const int rowbits = lane & 48;
+    const unsigned home = black ? 56u : 0u, rookw = (black ? COLOR : 0u) | (ROOK << 6);
+    const bool rook_short = (__ballot(w == (rookw | (home + 7))) >> rowbits) & 0xffff;
+    const bool rook_long = (__ballot(w == (rookw | home)) >> rowbits) & 0xffff;
 
-    // pseudo-legal targets of this slot
-    u64 ps = 0;
-    const bool mine = !(w & CAPTURED) && (((w >> 10) & 1) == (unsigned)black);
-    const int sq = w & 63, r = sq >> 3, c = sq & 7, t = (w >> 6) & 7;
+    // ---- what attacks the king once this lane's piece has left its square (the king's own lane: the check) ----
+    const u64 att = attackers(e, occ & ~fb, ksq);
+    u64 allowed = ~0ull;
+    if (att) allowed = (att & (att - 1)) ? 0 : att | between(ksq, att);
+    // a slot without a piece of ours has no moves; the king's lane reports the check
+    if (slot == 15 && in_check && here) in_check[b] = att ? 1 : 0;
+
+    // ---- this lane's king step or castling square ----
+    const u64 kb = bit(ksq);
+    unsigned safe;
+    {
+        const int k9 = slot + (slot >= 4), dr = k9 / 3 - 1, dc = k9 % 3 - 1;
+        const bool step = slot < 8;
+        const int r = (ksq >> 3) + dr, c = (ksq & 7) + dc;
+        const bool kingside = slot < 11;
+        const bool unmoved = !(kw & (CAPTURED | SPECIAL));
+        int at = step ? r * 8 + c : kingside ? ksq + (slot - 8) : ksq - (slot - 11);
+        bool may = step ? (unsigned)r < 8u && (unsigned)c < 8u
+                        : unmoved && (kingside ? rook_short && !(occ & (bit(home + 5) | bit(home + 6)))
+                                               : slot < 14 && rook_long && !(occ & (bit(home + 1) | bit(home + 2) | bit(home + 3))));
+        at &= 63;
+        const u64 tb = step ? bit(at) : bit(home + (kingside ? 6 : 2));
+        if (step) may = may && !(own & tb);
+        u64 occ2 = (occ & ~kb) | tb;
+        if (!step) occ2 = (occ2 & ~bit(home + (kingside ? 7 : 0))) | bit(home + (kingside ? 5 : 3));
+        Enemy e2 = e;
+        e2.pawns &= ~tb; e2.knights &= ~tb; e2.diag &= ~tb; e2.orth &= ~tb;
+        const bool ok = may && attackers(e2, occ2, at) == 0;
+        safe = (unsigned)(__ballot(ok) >> rowbits) & 0xffffu;
+    }
+
+    // ---- the squares this lane's piece reaches ----
+    u64 legal = 0, ep = 0;
     if (mine) {
         if (t == PAWN) {
-            const int dir = black ? -1 : 1, r1 = r + dir;
-            if (r1 >= 0 && r1 < 8) {
-                if (!(occ & bit(r1 * 8 + c))) {
-                    ps |= bit(r1 * 8 + c);
-                    const int r2 = r + 2 * dir;
-                    if (r == (black ? 6 : 1) && !(occ & bit(r2 * 8 + c))) ps |= bit(r2 * 8 + c);
-                }
-#pragma unroll
-                for (int dc = -1; dc <= 1; dc += 2) {
-                    const int cc = c + dc;
-                    if (cc < 0 || cc > 7) continue;
-                    if (opp & bit(r1 * 8 + cc)) ps |= bit(r1 * 8 + cc);
-                    // en passant: an enemy pawn that just double-pushed stands beside us on our fifth rank
-                    if (r == (black ? 3 : 4) && (ep_pawns & bit(r * 8 + cc))) ps |= bit(r1 * 8 + cc);
-                }
+            const int r = sq >> 3;
+            const u64 one = (black ? fb >> 8 : fb << 8) & ~occ;
+            const u64 two = r == (black ? 6 : 1) ? (black ? one >> 8 : one << 8) & ~occ : 0;
+            // the two squares ahead to either side, and the enemy pawns beside us that just double-pushed
+            const u64 west = (fb >> 1) & NOT_H, east = (fb << 1) & NOT_A;
+            const u64 sides = west | east;
+            const u64 ahead = black ? sides >> 8 : sides << 8;
+            legal = (one | two | (ahead & opp)) & allowed;
+            if (r == (black ? 3 : 4)) {
+                const u64 beside = sides & ep_pawns;
+                ep = (black ? beside >> 8 : beside << 8) & ~opp;
             }
         } else if (t == KNIGHT) {
-            ps = knight_pattern(bit(sq)) & ~own;
+            legal = knight_pattern(fb) & ~own & allowed;
         } else if (t == KING) {
-            ps = king_pattern(bit(sq)) & ~own;
-            if (!(w & SPECIAL)) {
-                if (rook_short && !(occ & (bit(row + 5) | bit(row + 6)))) ps |= bit(row + 6);
-                if (rook_long && !(occ & (bit(row + 1) | bit(row + 2) | bit(row + 3)))) ps |= bit(row + 2);
-            }
+            const u64 around = (safe & 7u) | ((safe & 8u) << 5) | ((safe & 16u) << 6) | ((u64)(safe & 0xE0u) << 11);
+            legal = ksq >= 9 ? around << (ksq - 9) : around >> (9 - ksq);
+            if (((safe >> 8) & 7u) == 7u) legal |= bit(home + 6);
+            if (((safe >> 11) & 7u) == 7u) legal |= bit(home + 2);
         } else if (t == BISHOP || t == ROOK || t == QUEEN) {
-            if (t != BISHOP) ps |= rook_attacks(occ, sq);
-            if (t != ROOK) ps |= bishop_attacks(occ, sq);
-            ps &= ~own;
+            u64 reach = 0;
+            if (t != BISHOP) reach |= rook_attacks(occ, sq);
+            if (t != ROOK) reach |= bishop_attacks(occ, sq);
+            legal = reach & ~own & allowed;
         }
     }
-
-    // legality: the position's pseudo-legal moves are dealt out evenly over the 64 lanes (move k of
-    // the slot-major list goes to lane k % 64); each is replayed on the bitboards
-    __shared__ u64 legal[4][32];
-    u64* const mine_out = legal[threadIdx.x >> 6];
-    if (lane < 32) mine_out[lane] = 0;
-    const int cnt = part == 0 ? __popcll(ps) : 0;
-    int first = cnt;                                                // exclusive prefix over slots
-#pragma unroll
-    for (int d = 1; d < 32; d <<= 1) {
-        const int o = __shfl_up(first, d);
-        if (lane >= d) first += o;
-    }
-    first -= cnt;
-    const int total = __shfl(first + cnt, 31);
-    for (int base = 0; base < total; base += 64) {
-        const int k = base + lane;
-        int s = 0;                                                  // the slot whose range holds move k
-#pragma unroll
-        for (int j = 1; j < 32; j++) s = (__shfl(first, j) <= k) ? j : s;
-        const unsigned ws = (unsigned)__shfl((int)w, s);
-        u64 todo = ((u64)(unsigned)__shfl((int)(unsigned)(ps >> 32), s) << 32) | (unsigned)__shfl((int)(unsigned)ps, s);
-        const int skip = k - __shfl(first, s);                      // every lane takes part in the exchanges above
-        if (k >= total) continue;
-        for (int j = skip; j > 0; j--) todo &= todo - 1;
-        const int tsq = __builtin_ctzll(todo);
-        const int from = ws & 63, ts = (ws >> 6) & 7;
-        const u64 tb = bit(tsq), fb = bit(from);
-        u64 occ2 = (occ & ~fb) | tb;
+    while (__any(ep != 0)) {   // en passant: replayed, the victim is behind the target
+        const u64 tb = ep & (0 - ep), victim = black ? tb << 8 : tb >> 8;
         Enemy e2 = e;
-        u64 gone = tb;                                              // a piece standing on the target is captured
-        if (ts == PAWN && !(opp & tb) && (tsq & 7) != (from & 7)) { // en passant: the victim is behind the target
-            const u64 vb = bit(black ? tsq + 8 : tsq - 8);
-            gone |= vb;
-            occ2 &= ~vb;
-        }
+        const u64 gone = tb | victim;
         e2.pawns &= ~gone; e2.knights &= ~gone; e2.diag &= ~gone; e2.orth &= ~gone;
-        bool ok;
-        if (ts == KING && (tsq - from == 2 || tsq - from == -2)) {
-            // the rook jumps too; start, crossed and landing squares must all be safe afterwards
-            const int rfrom = (int)row + (tsq > from ? 7 : 0), rto = (int)row + (tsq > from ? 5 : 3);
-            occ2 = (occ2 & ~bit(rfrom)) | bit(rto);
-            const int lo = tsq < from ? tsq : from;
-            ok = !attacked(e2, occ2, lo) && !attacked(e2, occ2, lo + 1) && !attacked(e2, occ2, lo + 2);
-        } else {
-            ok = !attacked(e2, occ2, ts == KING ? tsq : ksq);
-        }
-        if (ok) atomicOr(&mine_out[s], tb);
+        if (ep && attackers(e2, ((occ & ~fb) | tb) & ~victim, ksq) == 0) legal |= tb;
+        ep &= ep - 1;
     }
-    // same wave, LDS operations complete in order: the words are final
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (lane < 32) mask[(size_t)b * 32 + lane] = mine_out[lane];
+    if (here) {
+        u64* const mw = mask + (size_t)b * 32;
+        mw[(black ? 16 : 0) + slot] = legal;
+        mw[(black ? 0 : 16) + slot] = 0;
+    }
 }
 
 }  // namespace
@@ -231,8 +239,11 @@ extern "C" int bf_movegen(const uint16_t* boards, const int16_t* control, int64_
     if (!boards || !control || !mask) return fail(BF_ERR_ARGUMENT, "boards/control/mask must not be NULL");
     if (((uintptr_t)boards & 1) || ((uintptr_t)control & 1) || ((uintptr_t)mask & 7))
         return fail(BF_ERR_ARGUMENT, "boards and control must be 2-byte and mask 8-byte aligned");
-    hipLaunchKernelGGL(movegen_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, (hipStream_t)stream, boards, control,
-                       (int)n, reinterpret_cast<u64*>(mask), in_check);
+    // four positions per wavefront: workgroups of one wavefront while that spreads a small launch over more
+    // compute units (256 of them hold 1024 positions), of four beyond
+    const int waves = n <= 4096 ? 1 : 4;
+    hipLaunchKernelGGL(movegen_kernel, dim3((unsigned)((n + 4 * waves - 1) / (4 * waves))), dim3(64 * waves), 0, (hipStream_t)stream,
+                       boards, control, (int)n, reinterpret_cast<u64*>(mask), in_check);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         char msg[256];
