@@ -174,6 +174,140 @@ void encoder_forward(torch::Tensor y, torch::Tensor weights, torch::Tensor param
     TORCH_CHECK(rc == BF_OK, "bf_model_forward failed (", rc, "): ", bf_last_error());
 }
 
+// ---- the calls either side of the evaluator ----------------------------------------------------------
+// These launches take 5 to 10 us on the device, so at a search's sizes the host's share decides: checks,
+// allocation and launch in one native call (about 4 us; through ctypes, with the guard and the stream
+// looked up in Python, 10 us for movegen and 36 us for expand_edges, six zero-filling launches of
+// which the kernel then overwrote).
+
+#define BF_VALUE_CHECK(cond, ...) \
+    do {                          \
+        if (!(cond)) throw py::value_error(c10::str(__VA_ARGS__)); \
+    } while (0)
+
+bool shape_is(const torch::Tensor& t, std::initializer_list<int64_t> want) { return t.sizes() == at::IntArrayRef(want); }
+
+void* stream_of(const c10::Device& dev) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream(); }
+
+// hip_impl.movegen: (mask [n, 32] int64, in_check [n] bool)
+std::pair<torch::Tensor, torch::Tensor> movegen(const torch::Tensor& boards, const torch::Tensor& control,
+                                                const c10::optional<std::pair<torch::Tensor, torch::Tensor>>& out) {
+    const int64_t n = boards.dim() ? boards.size(0) : 0;
+    BF_VALUE_CHECK(shape_is(boards, {n, BF_TOKENS}) && boards.scalar_type() == torch::kShort && shape_is(control, {n}) &&
+                       control.scalar_type() == torch::kShort, "boards must be [n,32] int16 and control [n] int16");
+    BF_VALUE_CHECK(boards.is_cuda() && control.is_cuda(), "boards and control must be on the GPU");
+    BF_VALUE_CHECK(boards.is_contiguous() && control.is_contiguous(), "boards and control must be contiguous");
+    const c10::Device dev = boards.device();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
+    const auto opts = boards.options();
+    const torch::Tensor mask = out ? out->first : at::empty({n, BF_TOKENS}, opts.dtype(torch::kLong));
+    const torch::Tensor chk = out ? out->second : at::empty({n}, opts.dtype(torch::kBool));
+    BF_VALUE_CHECK(shape_is(mask, {n, BF_TOKENS}) && mask.scalar_type() == torch::kLong && shape_is(chk, {n}) && chk.scalar_type() == torch::kBool,
+                   "`out` was made for another n");
+    const int rc = bf_movegen(static_cast<const uint16_t*>(boards.data_ptr()), static_cast<const int16_t*>(control.data_ptr()), n,
+                              static_cast<uint64_t*>(mask.data_ptr()), static_cast<uint8_t*>(chk.data_ptr()), stream_of(dev));
+    TORCH_CHECK(rc == BF_OK, "bf_movegen failed (", rc, "): ", bf_last_error());
+    return {mask, chk};
+}
+
+typedef c10::optional<std::pair<torch::Tensor, torch::Tensor>> OptLeaves;
+
+void check_leaves(const torch::Tensor& index, const torch::Tensor& count, int64_t n, const c10::Device& dev) {
+    BF_VALUE_CHECK(index.scalar_type() == torch::kInt && count.scalar_type() == torch::kInt && index.dim() == 1 && index.size(0) >= n &&
+                       count.numel() == 1 && index.device() == dev && count.device() == dev && index.is_contiguous(),
+                   "leaves must be (index [", n, "] int32, count [1] int32) on ", dev.str());
+}
+
+// hip_impl.compact_leaves: (leaf_index [n] int32, leaf_count [1] int32)
+std::pair<torch::Tensor, torch::Tensor> compact_leaves(const torch::Tensor& flags_, const OptLeaves& out) {
+    BF_VALUE_CHECK(flags_.dim() == 1 && (flags_.scalar_type() == torch::kByte || flags_.scalar_type() == torch::kBool) && flags_.is_cuda(),
+                   "flags must be [n] uint8 or bool on the GPU");
+    const int64_t n = flags_.size(0);
+    const torch::Tensor flags = flags_.contiguous();
+    const c10::Device dev = flags.device();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
+    const auto opts = flags.options().dtype(torch::kInt);
+    const torch::Tensor index = out ? out->first : at::zeros({n}, opts), count = out ? out->second : at::zeros({1}, opts);
+    check_leaves(index, count, n, dev);
+    const int rc = bf_compact_leaves(static_cast<const uint8_t*>(flags.data_ptr()), n, static_cast<int32_t*>(index.data_ptr()),
+                                     static_cast<int32_t*>(count.data_ptr()), stream_of(dev));
+    TORCH_CHECK(rc == BF_OK, "bf_compact_leaves failed (", rc, "): ", bf_last_error());
+    return {index, count};
+}
+
+// hip_impl.expand_edges: the dict of edge tensors
+py::dict expand_edges(const torch::Tensor& policy_, const torch::Tensor& promo_, const torch::Tensor& value_, const torch::Tensor& mask_,
+                      const torch::Tensor& boards_, const torch::Tensor& control_, int64_t max_edges, const OptTensor& active_,
+                      const c10::optional<py::dict>& out, const OptLeaves& leaves) {
+    const int64_t n = policy_.dim() ? policy_.size(0) : 0;
+    const auto lt = policy_.scalar_type();
+    BF_VALUE_CHECK(shape_is(policy_, {n, BF_TOKENS, BF_POLICY}) && shape_is(promo_, {n, BF_TOKENS, BF_PROMO}) && lt == promo_.scalar_type() &&
+                       (lt == torch::kHalf || lt == torch::kFloat), "policy must be [n,32,64] and promo [n,32,4], both fp16 or both fp32");
+    BF_VALUE_CHECK(shape_is(value_, {n}) && value_.scalar_type() == torch::kFloat, "value must be [", n, "] float32");
+    BF_VALUE_CHECK(shape_is(mask_, {n, BF_TOKENS}) && mask_.scalar_type() == torch::kLong && shape_is(boards_, {n, BF_TOKENS}) &&
+                       boards_.scalar_type() == torch::kShort && shape_is(control_, {n}) && control_.scalar_type() == torch::kShort,
+                   "mask must be [n,32] int64, boards [n,32] int16, control [n] int16");
+    BF_VALUE_CHECK(max_edges >= 1 && max_edges <= 255, "max_edges must be in [1, 255] (edge indices are uint8 in the search)");
+    BF_VALUE_CHECK(policy_.is_cuda() && promo_.is_cuda() && value_.is_cuda() && mask_.is_cuda() && boards_.is_cuda() && control_.is_cuda() &&
+                       (!active_ || active_->is_cuda()), "all inputs must be on the GPU");
+    const c10::Device dev = policy_.device();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
+    py::dict res;
+    if (out) {
+        res = *out;
+        BF_VALUE_CHECK(shape_is(py::cast<torch::Tensor>(res["edge_move"]), {n, max_edges}), "`out` was made for another n or max_edges");
+    } else {
+        // every row is written unless positions are skipped: only then do the buffers start at zero
+        const bool partial = active_.has_value() || leaves.has_value();
+        const auto make = [&](at::IntArrayRef size, at::ScalarType t) {
+            const auto o = policy_.options().dtype(t);
+            return partial ? at::zeros(size, o) : at::empty(size, o);
+        };
+        res["edge_move"] = make({n, max_edges}, torch::kShort);
+        res["edge_prior"] = make({n, max_edges}, torch::kHalf);
+        res["n_edges"] = make({n}, torch::kInt);
+        res["count"] = make({n}, torch::kInt);
+        res["dropped"] = make({n}, torch::kFloat);
+        res["node_value"] = make({n}, torch::kHalf);
+    }
+    const auto ptr = [&](const char* key) { return py::cast<torch::Tensor>(res[key]).data_ptr(); };
+    // temporaries made here were allocated on the current stream, where the launch is queued: their memory
+    // is handed out again only to work that this stream runs after the kernel
+    const torch::Tensor policy = policy_.contiguous(), promo = promo_.contiguous(), value = value_.contiguous(),
+                        mask = mask_.contiguous(), boards = boards_.contiguous(), control = control_.contiguous();
+    bf_expand_args a{};
+    a.policy = policy.data_ptr();
+    a.promo = promo.data_ptr();
+    a.value = static_cast<const float*>(value.data_ptr());
+    a.mask = static_cast<const uint64_t*>(mask.data_ptr());
+    a.boards = static_cast<const uint16_t*>(boards.data_ptr());
+    a.control = static_cast<const int16_t*>(control.data_ptr());
+    torch::Tensor act;
+    if (active_) {
+        act = active_->scalar_type() == torch::kBool ? active_->contiguous() : active_->to(torch::kByte).contiguous();
+        BF_VALUE_CHECK(shape_is(act, {n}), "active must be [", n, "]");
+        a.active = static_cast<const uint8_t*>(act.data_ptr());
+    }
+    if (leaves) {
+        BF_VALUE_CHECK(!active_, "a compacted leaf list replaces the active flags: pass one of them");
+        check_leaves(leaves->first, leaves->second, n, dev);
+        a.leaf_index = static_cast<const int32_t*>(leaves->first.data_ptr());
+        a.leaf_count = static_cast<const int32_t*>(leaves->second.data_ptr());
+    }
+    a.n = n;
+    a.max_edges = (int32_t)max_edges;
+    a.logits_fp32 = lt == torch::kFloat;
+    a.edge_move = static_cast<int16_t*>(ptr("edge_move"));
+    a.edge_prior = ptr("edge_prior");
+    a.n_edges = static_cast<int32_t*>(ptr("n_edges"));
+    a.count = static_cast<int32_t*>(ptr("count"));
+    a.dropped = static_cast<float*>(ptr("dropped"));
+    a.node_value = ptr("node_value");
+    const int rc = bf_expand(&a, stream_of(dev));
+    TORCH_CHECK(rc == BF_OK, "bf_expand failed (", rc, "): ", bf_last_error());
+    return res;
+}
+
 // Cycles per phase summed over the wavefronts of one launch of the profiling build (see
 // bf_profile_phases); returns an int64 tensor on the device, already written when it is read.
 torch::Tensor profile_phases(torch::Tensor boards, torch::Tensor control, torch::Tensor rep, torch::Tensor weights,
@@ -203,6 +337,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("encoder_forward", &encoder_forward, "the encoder stack alone, in place on y", py::arg("y"), py::arg("weights"),
           py::arg("params"), py::arg("alive"), py::arg("d_model"), py::arg("n_layers"), py::arg("n_heads"), py::arg("d_ff"),
           py::arg("eps"), py::arg("quant") = 0, py::arg("kernel") = 0, py::arg("n_value") = 1, py::arg("workspace") = py::none());
+    m.def("movegen", &movegen, "legal-move words and check flags", py::arg("boards"), py::arg("control"), py::arg("out") = py::none());
+    m.def("compact_leaves", &compact_leaves, "leaf flags to an ordered list and its length", py::arg("flags"), py::arg("out") = py::none());
+    m.def("expand_edges", &expand_edges, "edges of search nodes from logits and legal-move words", py::arg("policy"), py::arg("promo"),
+          py::arg("value"), py::arg("mask"), py::arg("boards"), py::arg("control"), py::arg("max_edges") = 96,
+          py::arg("active") = py::none(), py::arg("out") = py::none(), py::arg("leaves") = py::none());
     m.def("profile_phases", &profile_phases, "cycles per phase of one profiled launch", py::arg("boards"),
           py::arg("control"), py::arg("rep"), py::arg("weights"), py::arg("params"), py::arg("policy"), py::arg("promo"),
           py::arg("value"), py::arg("d_model"), py::arg("n_layers"), py::arg("n_heads"), py::arg("d_ff"), py::arg("eps"),

@@ -170,6 +170,18 @@ def extension_available() -> bool:
     return os.path.exists(_build.TORCH_EXT) and "BROKEFISH_HIP_LIB" not in os.environ
 
 
+_native_ext = False     # not looked up yet
+
+
+def _native():
+    """The extension module where it is the default binding (it then carries the whole of a call's host
+    work), else None: the same checks and the same C-ABI call through ctypes."""
+    global _native_ext
+    if _native_ext is False:
+        _native_ext = load_extension() if extension_available() else None
+    return _native_ext
+
+
 def int8_q_max():
     """(s8, u8) quantisation maxima compiled into the library."""
     a, b = C.c_double(), C.c_double()
@@ -217,6 +229,9 @@ def movegen(boards, control, out=None):
     """Legal-move words on the device (the reference's ``env.movegen``, docs/reference/spec.md:152-172):
     ``boards [n,32]`` int16, ``control [n]`` int16 on the GPU -> ``(mask [n,32] int64, in_check [n] bool)``.
     ``out`` reuses a pair returned earlier.  Asynchronous on the current stream."""
+    ext = _native()
+    if ext is not None:
+        return ext.movegen(boards, control, out)
     n = boards.shape[0]
     if boards.shape != (n, T) or boards.dtype is not torch.int16 or control.shape != (n,) or control.dtype is not torch.int16:
         raise ValueError("boards must be [n,32] int16 and control [n] int16")
@@ -273,6 +288,9 @@ def compact_leaves(flags, out=None):
     count" of the reference's design retrospective (docs/journal/2026-08-09-kernel-design-
     retrospective.md:140-154).  ``forward_full(..., leaves=)`` and ``expand_edges(..., leaves=)``
     take the pair; nothing returns to the host.  ``out`` reuses a pair returned earlier."""
+    ext = _native()
+    if ext is not None:
+        return ext.compact_leaves(flags, out)
     if flags.dim() != 1 or flags.dtype not in (torch.uint8, torch.bool) or not flags.is_cuda:
         raise ValueError("flags must be [n] uint8 or bool on the GPU")
     n = flags.shape[0]
@@ -301,6 +319,9 @@ def expand_edges(policy, promo, value, mask, boards, control, max_edges: int = 9
     (value+1)/2.  ``active`` ([n] bool/uint8) leaves the rows where it is 0 untouched, and so does
     ``leaves`` (the pair :func:`compact_leaves` returns) for positions not in the list; ``out``
     reuses a dict returned earlier.  The launch is asynchronous on the current stream."""
+    ext = _native()
+    if ext is not None:
+        return ext.expand_edges(policy, promo, value, mask, boards, control, max_edges, active, out, leaves)
     n = policy.shape[0]
     if policy.shape != (n, T, N_POLICY) or promo.shape != (n, T, N_PROMO) or policy.dtype != promo.dtype or \
             policy.dtype not in (torch.float16, torch.float32):
