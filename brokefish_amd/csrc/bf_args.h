@@ -124,6 +124,8 @@ struct KArgs {
 
 // Text returned by bf_last_error() on this thread (set by every translation unit of the library).
 void set_error(const char* msg);
+// Whether the current device is one this library's kernels are compiled for (sets the error text if not).
+bool device_is_gfx950();
 
 // One launcher per separately compiled kernel variant (production, debug taps, phase
 // profile); each sets the dynamic-LDS limit once and launches on `stream`.

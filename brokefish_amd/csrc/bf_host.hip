@@ -214,7 +214,7 @@ constexpr int DUO_ROUND = 512;   // positions the two-position kernel holds at o
 
 // Whether the current device is an MI355X-class part (gfx950), looked up once per device; the
 // kernels are compiled for that architecture only.
-static bool device_is_gfx950() {
+bool bf::device_is_gfx950() {
     static std::atomic<unsigned long long> known{0}, good{0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
@@ -255,7 +255,7 @@ static bf::KArgs slice(const bf::KArgs& k, int first, int count) {
 static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream_t stream) {
     const int grid = (k.n + bf::WAVES - 1) / bf::WAVES;
     hipError_t e;
-    if (!device_is_gfx950()) return BF_ERR_DEVICE;
+    if (!bf::device_is_gfx950()) return BF_ERR_DEVICE;
     // The two-position kernel runs in rounds of 512 positions (256 compute units x 2), and a round
     // costs the same whether it is full or not.  When the library chose the kernel itself and the
     // last round would hold at most 256 positions, those go to the one-position form in a second

@@ -110,6 +110,14 @@ def load_library():
         L.bf_board_wstream_bytes.argtypes = [C.POINTER(_Shape)]
         L.bf_board_fparams_floats.restype = C.c_size_t
         L.bf_board_fparams_floats.argtypes = [C.POINTER(_Shape)]
+        L.bf_pack_scratch_floats.restype = C.c_size_t
+        L.bf_pack_scratch_floats.argtypes = [C.POINTER(_Shape)]
+        L.bf_pack_board.restype = C.c_int
+        L.bf_pack_board.argtypes = [C.POINTER(_Shape), C.c_int] + [C.c_void_p] * 6
+        L.bf_fingerprint_partials.restype = C.c_int64
+        L.bf_fingerprint_partials.argtypes = [C.c_void_p, C.c_int]
+        L.bf_fingerprint.restype = C.c_int
+        L.bf_fingerprint.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]
         L.bf_expand.restype = C.c_int
         L.bf_expand.argtypes = [C.POINTER(_ExpandArgs), C.c_void_p]
         L.bf_movegen.restype = C.c_int
@@ -584,6 +592,65 @@ def pack_network_board(sd: Dict[str, torch.Tensor], n_layers: int, d: int, f: in
     return wstream, fparams
 
 
+def pack_board_on_device(net, stack, shape: _Shape, fp8: bool, device):
+    """:func:`pack_network_board` on the GPU (``bf_pack_board``): the parameters of ``net`` (or, with
+    ``net`` None, of the bare encoder ``stack``: inert tables, identity final norm, zero heads, never
+    read back) -> (board_wstream, board_fparams) on ``device``, the same bytes.  Parameters that
+    already lie there in fp32 are read in place.  The blobs are complete when this returns, so that
+    any stream may use them."""
+    d, f, n_value = shape.d_model, shape.d_ff, shape.n_value
+
+    def take(p, *want):
+        t = p.detach().to(device=device, dtype=torch.float32).contiguous()
+        if tuple(t.shape) != want:
+            raise ValueError(f"a parameter is {tuple(t.shape)}, the network shape wants {want}")
+        return t if t.data_ptr() % 16 == 0 else t.clone()
+    lib = load_library()
+    with torch.cuda.device(device), torch.no_grad():
+        keep = []
+        for lay in stack.layers:
+            at = lay.self_attn
+            keep += [take(lay.norm1.weight, d), take(lay.norm1.bias, d), take(at.in_proj_weight, 3 * d, d), take(at.in_proj_bias, 3 * d),
+                     take(at.out_proj.weight, d, d), take(at.out_proj.bias, d), take(lay.norm2.weight, d), take(lay.norm2.bias, d),
+                     take(lay.linear1.weight, f, d), take(lay.linear1.bias, f), take(lay.linear2.weight, d, f), take(lay.linear2.bias, d)]
+        n_layer_ptrs = len(keep)
+        tables = (("emb_square", 64), ("emb_type_special", 12), ("emb_color_turn", 4), ("emb_clock", 101), ("emb_rep", 3))
+        heads = (("policy", N_POLICY), ("promo", N_PROMO), ("value", n_value))
+        if net is not None:
+            keep += [take(getattr(net, name).weight, rows, d) for name, rows in tables]
+            keep += [take(net.norm_f.weight, d), take(net.norm_f.bias, d)]
+            keep += [take(getattr(net, name).weight, rows, d) for name, rows in heads]
+        else:
+            zero = torch.zeros(101, d, device=device)
+            keep += [zero] * 5 + [torch.ones(d, device=device), zero] + [zero] * 3
+        ptrs = (C.c_void_p * len(keep))(*[t.data_ptr() for t in keep])
+        wstream = torch.empty(lib.bf_board_wstream_bytes(C.byref(shape)), dtype=torch.uint8, device=device)
+        fparams = torch.empty(lib.bf_board_fparams_floats(C.byref(shape)), dtype=torch.float32, device=device)
+        scratch = torch.empty(lib.bf_pack_scratch_floats(C.byref(shape)), dtype=torch.float32, device=device)
+        stream = torch.cuda.current_stream(device)
+        rc = lib.bf_pack_board(C.byref(shape), 1 if fp8 else 0, ptrs, C.byref(ptrs, n_layer_ptrs * C.sizeof(C.c_void_p)),
+                               wstream.data_ptr(), fparams.data_ptr(), scratch.data_ptr(), C.c_void_p(stream.cuda_stream))
+        if rc:
+            raise RuntimeError(f"bf_pack_board failed ({rc}): {lib.bf_last_error().decode()}")
+        stream.synchronize()
+    return wstream, fparams
+
+
+def fingerprint_on_device(params):
+    """The weight fingerprint (``bf_fingerprint``) of fp32 tensors that lie contiguously on one GPU."""
+    lib = load_library()
+    n = len(params)
+    numel = (C.c_int64 * n)(*[p.numel() for p in params])
+    ptrs = (C.c_void_p * n)(*[p.data_ptr() for p in params])
+    dev = params[0].device
+    with torch.cuda.device(dev):
+        buf = torch.empty(lib.bf_fingerprint_partials(numel, n) + 1, dtype=torch.float64, device=dev)
+        rc = lib.bf_fingerprint(ptrs, numel, n, buf.data_ptr() + 8, buf.data_ptr(), C.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
+    if rc:
+        raise RuntimeError(f"bf_fingerprint failed ({rc}): {lib.bf_last_error().decode()}")
+    return float(buf[0])
+
+
 # --------------------------------------------------------------------------- #
 # the evaluator object
 # --------------------------------------------------------------------------- #
@@ -686,15 +753,6 @@ class FusedEncoder:
             raise RuntimeError("no GPU visible: the evaluator has no CPU path")
         self.device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
         self._shape = _Shape(self.d_model, self.n_layers, self.n_heads, self.d_ff, self.n_value, self.eps)
-        if net is not None:
-            sd = {k: v.detach() for k, v in net.state_dict().items()}
-        else:   # bare stack: inert tables, identity final norm, zero heads (never read back)
-            d = self.d_model
-            sd = {"encoder." + k: v.detach() for k, v in source.state_dict().items()}
-            for name, rows in (("emb_square", 64), ("emb_type_special", 12), ("emb_color_turn", 4),
-                               ("emb_clock", 101), ("emb_rep", 3), ("policy", 64), ("promo", 4), ("value", 1)):
-                sd[name + ".weight"] = torch.zeros(rows, d)
-            sd["norm_f.weight"], sd["norm_f.bias"] = torch.ones(d), torch.zeros(d)
         # Two packings of the same weights (see include/brokefish_hip.h): the one-position-per-
         # workgroup kernels (TWIN / OCTO / BOARD, what kernel="auto" runs) read the board blobs; the
         # four-positions-per-workgroup kernel is packed, and its workspace allocated, only when it
@@ -702,6 +760,15 @@ class FusedEncoder:
         self.kernel = kernel
         self.wstream = self.fparams = self.board_wstream = self.board_fparams = None
         if kernel == "quad":
+            if net is not None:
+                sd = {k: v.detach() for k, v in net.state_dict().items()}
+            else:   # bare stack: inert tables, identity final norm, zero heads (never read back)
+                d = self.d_model
+                sd = {"encoder." + k: v.detach() for k, v in source.state_dict().items()}
+                for name, rows in (("emb_square", 64), ("emb_type_special", 12), ("emb_color_turn", 4),
+                                   ("emb_clock", 101), ("emb_rep", 3), ("policy", 64), ("promo", 4), ("value", 1)):
+                    sd[name + ".weight"] = torch.zeros(rows, d)
+                sd["norm_f.weight"], sd["norm_f.bias"] = torch.ones(d), torch.zeros(d)
             wstream, fparams = pack_network(sd, self.n_layers, self.d_model, self.d_ff, self.n_value,
                                             fmt="e4m3" if self.fp8 else "int8")
             if wstream.size != self._lib.bf_wstream_bytes(C.byref(self._shape)) or \
@@ -710,13 +777,8 @@ class FusedEncoder:
             self.wstream = torch.from_numpy(wstream).to(self.device)
             self.fparams = torch.from_numpy(fparams).to(self.device)
         else:
-            wstream, fparams = pack_network_board(sd, self.n_layers, self.d_model, self.d_ff, self.n_value,
-                                                  fmt="e4m3" if self.fp8 else "int8")
-            if wstream.size != self._lib.bf_board_wstream_bytes(C.byref(self._shape)) or \
-                    fparams.size != self._lib.bf_board_fparams_floats(C.byref(self._shape)):
-                raise RuntimeError("packed blob sizes disagree with the library's layout (board kernel)")
-            self.board_wstream = torch.from_numpy(wstream).to(self.device)
-            self.board_fparams = torch.from_numpy(fparams).to(self.device)
+            self.board_wstream, self.board_fparams = pack_board_on_device(net, net.encoder if net is not None else source,
+                                                                          self._shape, self.fp8, self.device)
         self._buffered_full = 0
         self._backbone = None
         self._profile, self._profile_waves, self._profile_kept = None, 0, None

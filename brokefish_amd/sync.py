@@ -20,9 +20,17 @@ from . import encoder_impl
 @torch.no_grad()
 def weight_fingerprint(net) -> float:
     """One float that changes if any parameter does, or if the same values are permuted: an
-    index-weighted float64 sum over the parameters in name order (brokefish/train/sync.py:34-49)."""
+    index-weighted float64 sum over the parameters in name order (brokefish/train/sync.py:34-49).
+    Parameters on a GPU (fp32, as a trainer holds them) are summed there, two launches and one wait
+    for the whole network; the order of the sum differs from the CPU's, so a value is compared with
+    one taken on the same device."""
+    named = sorted(net.named_parameters(), key=lambda kv: kv[0])
+    if named and all(p.dtype is torch.float32 and p.is_cuda and p.device == named[0][1].device and p.is_contiguous()
+                     and p.numel() for _, p in named):
+        from .hip_impl import fingerprint_on_device
+        return fingerprint_on_device([p for _, p in named])
     acc = 0.0
-    for i, (_, p) in enumerate(sorted(net.named_parameters(), key=lambda kv: kv[0])):
+    for i, (_, p) in enumerate(named):
         f = p.detach().reshape(-1).double()
         idx = torch.arange(1, f.numel() + 1, device=f.device, dtype=torch.float64)
         acc += float(((i + 1) * f * (idx % 9973.0 + 1.0)).sum())

@@ -107,6 +107,33 @@ size_t bf_workspace_bytes(const bf_shape* s, int64_t n);
 size_t bf_board_wstream_bytes(const bf_shape* s);
 size_t bf_board_fparams_floats(const bf_shape* s);
 
+/* Packing of a network that lies in fp32 on the device into the BOARD / TWIN / OCTO / DUO blobs
+ * (board_wstream: bf_board_wstream_bytes, board_fparams: bf_board_fparams_floats), quantised and laid
+ * out on the device.  Names and shapes are those of the reference's modules (reference
+ * brokefish/nn/model.py:276-361: weights [out, in] row-major, in_proj stacks Q, K, V); all pointers are
+ * 16-byte aligned DEVICE memory, `layers` itself is a host array of n_layers entries, `scratch` holds
+ * bf_pack_scratch_floats(shape) floats.  Replaces the host-side packer of the reference
+ * (brokefish/nn/cuda_impl.py:119-531, class FusedEncoder).  Asynchronous on `stream`. */
+typedef struct {
+    const float *norm1_w, *norm1_b, *in_proj_w, *in_proj_b, *out_proj_w, *out_proj_b;
+    const float *norm2_w, *norm2_b, *linear1_w, *linear1_b, *linear2_w, *linear2_b;
+} bf_layer_weights;
+typedef struct {
+    const float *emb_square, *emb_type_special, *emb_color_turn, *emb_clock, *emb_rep;
+    const float *norm_f_w, *norm_f_b, *policy, *promo, *value;
+} bf_global_weights;
+size_t bf_pack_scratch_floats(const bf_shape* s);
+int bf_pack_board(const bf_shape* s, int quant, const bf_layer_weights* layers, const bf_global_weights* g,
+                  uint8_t* board_wstream, float* board_fparams, float* scratch, void* stream);
+
+/* The weight fingerprint of the reference's training loop (reference brokefish/train/sync.py:34-49): the
+ * float64 sum over parameters i of (i + 1) * sum_j f_j * (j % 9973 + 1), j from 1, written to *out (DEVICE
+ * memory).  params / numel are host arrays of n fp32 DEVICE arrays and their lengths; `partials` is
+ * DEVICE memory of bf_fingerprint_partials(numel, n) doubles.  The order of the sums is fixed: the same
+ * weights give the same bits.  Asynchronous on `stream`. */
+int64_t bf_fingerprint_partials(const int64_t* numel, int n);
+int bf_fingerprint(const float* const* params, const int64_t* numel, int n, double* partials, double* out, void* stream);
+
 /* Optional debug outputs ("taps") and teacher forcing.  All pointers may be NULL.
  * B = boards in the call, L = layers run, kc = K / 256.
  * Replaces the reference's debug_stage / forward_stage mechanism
