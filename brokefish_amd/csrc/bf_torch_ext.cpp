@@ -8,8 +8,11 @@
 
 // PyTorch on ROCm presents its devices under the type name "cuda": these are the guard and stream
 // classes of that arrangement
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+
+#include <pybind11/stl.h>
 
 #include <string>
 #include <vector>
@@ -189,6 +192,11 @@ bool shape_is(const torch::Tensor& t, std::initializer_list<int64_t> want) { ret
 
 void* stream_of(const c10::Device& dev) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream(); }
 
+// a new tensor straight from the caching allocator (at::empty takes the dispatcher's way there)
+torch::Tensor fresh(at::IntArrayRef size, at::ScalarType type, const c10::Device& dev) {
+    return at::detail::empty_cuda(size, type, dev, c10::nullopt);
+}
+
 // hip_impl.movegen: (mask [n, 32] int64, in_check [n] bool)
 std::pair<torch::Tensor, torch::Tensor> movegen(const torch::Tensor& boards, const torch::Tensor& control,
                                                 const c10::optional<std::pair<torch::Tensor, torch::Tensor>>& out) {
@@ -199,9 +207,8 @@ std::pair<torch::Tensor, torch::Tensor> movegen(const torch::Tensor& boards, con
     BF_VALUE_CHECK(boards.is_contiguous() && control.is_contiguous(), "boards and control must be contiguous");
     const c10::Device dev = boards.device();
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
-    const auto opts = boards.options();
-    const torch::Tensor mask = out ? out->first : at::empty({n, BF_TOKENS}, opts.dtype(torch::kLong));
-    const torch::Tensor chk = out ? out->second : at::empty({n}, opts.dtype(torch::kBool));
+    const torch::Tensor mask = out ? out->first : fresh({n, BF_TOKENS}, torch::kLong, dev);
+    const torch::Tensor chk = out ? out->second : fresh({n}, torch::kBool, dev);
     BF_VALUE_CHECK(shape_is(mask, {n, BF_TOKENS}) && mask.scalar_type() == torch::kLong && shape_is(chk, {n}) && chk.scalar_type() == torch::kBool,
                    "`out` was made for another n");
     const int rc = bf_movegen(static_cast<const uint16_t*>(boards.data_ptr()), static_cast<const int16_t*>(control.data_ptr()), n,
@@ -260,8 +267,7 @@ py::dict expand_edges(const torch::Tensor& policy_, const torch::Tensor& promo_,
         // every row is written unless positions are skipped: only then do the buffers start at zero
         const bool partial = active_.has_value() || leaves.has_value();
         const auto make = [&](at::IntArrayRef size, at::ScalarType t) {
-            const auto o = policy_.options().dtype(t);
-            return partial ? at::zeros(size, o) : at::empty(size, o);
+            return partial ? at::zeros(size, policy_.options().dtype(t)) : fresh(size, t, dev);
         };
         res["edge_move"] = make({n, max_edges}, torch::kShort);
         res["edge_prior"] = make({n, max_edges}, torch::kHalf);
@@ -308,6 +314,73 @@ py::dict expand_edges(const torch::Tensor& policy_, const torch::Tensor& promo_,
     return res;
 }
 
+// ---- packing and the fingerprint ---------------------------------------------------------------------
+// `params` are the network's parameters in the order of bf_layer_weights, layer by layer, and of
+// bf_global_weights; those that are not fp32, contiguous, aligned and on `device` are copied there first.
+// The blobs are complete when this returns, so that any stream may use them.
+std::pair<torch::Tensor, torch::Tensor> pack_board(const std::vector<torch::Tensor>& params, int64_t d_model, int64_t n_layers,
+                                                   int64_t d_ff, int64_t n_value, double eps, bool fp8, int64_t device) {
+    const bf_shape shape{(int32_t)d_model, (int32_t)n_layers, (int32_t)(d_model / 32), (int32_t)d_ff, (int32_t)n_value, (float)eps};
+    const int64_t d = d_model, f = d_ff, nl = 12 * n_layers;
+    BF_VALUE_CHECK((int64_t)params.size() == nl + 10, "pack_board takes ", nl + 10, " parameters, got ", params.size());
+    const int64_t layer[12][2] = {{d, 0}, {d, 0}, {3 * d, d}, {3 * d, 0}, {d, d}, {d, 0}, {d, 0}, {d, 0}, {f, d}, {f, 0}, {d, f}, {d, 0}};
+    const int64_t global[10][2] = {{64, d}, {12, d}, {4, d}, {101, d}, {3, d}, {d, 0}, {d, 0}, {BF_POLICY, d}, {BF_PROMO, d}, {n_value, d}};
+    const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)device);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
+    at::NoGradGuard no_grad;
+    std::vector<torch::Tensor> keep;
+    std::vector<const float*> ptrs;
+    ptrs.reserve(params.size());
+    for (size_t i = 0; i < params.size(); i++) {
+        const int64_t* want = (int64_t)i < nl ? layer[i % 12] : global[i - nl];
+        torch::Tensor t = params[i];
+        BF_VALUE_CHECK(want[1] ? shape_is(t, {want[0], want[1]}) : shape_is(t, {want[0]}), "a parameter is ", t.sizes(),
+                       ", the network shape wants ", want[0], want[1] ? " rows of " : " elements", want[1] ? std::to_string(want[1]) : "");
+        if (t.scalar_type() != torch::kFloat || t.device() != dev || !t.is_contiguous() || ((uintptr_t)t.data_ptr() & 15)) {
+            t = t.detach().to(at::TensorOptions().device(dev).dtype(torch::kFloat)).contiguous();
+            if ((uintptr_t)t.data_ptr() & 15) t = t.clone();
+            keep.push_back(t);
+        }
+        ptrs.push_back(static_cast<const float*>(t.data_ptr()));
+    }
+    const auto opts = at::TensorOptions().device(dev);
+    const torch::Tensor ws = at::empty({(int64_t)bf_board_wstream_bytes(&shape)}, opts.dtype(torch::kByte)),
+                        fp = at::empty({(int64_t)bf_board_fparams_floats(&shape)}, opts.dtype(torch::kFloat)),
+                        scratch = at::empty({(int64_t)bf_pack_scratch_floats(&shape)}, opts.dtype(torch::kFloat));
+    const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
+    const int rc = bf_pack_board(&shape, fp8 ? BF_QUANT_E4M3 : BF_QUANT_INT8, reinterpret_cast<const bf_layer_weights*>(ptrs.data()),
+                                 reinterpret_cast<const bf_global_weights*>(ptrs.data() + nl), static_cast<uint8_t*>(ws.data_ptr()),
+                                 static_cast<float*>(fp.data_ptr()), static_cast<float*>(scratch.data_ptr()), stream.stream());
+    TORCH_CHECK(rc == BF_OK, "bf_pack_board failed (", rc, "): ", bf_last_error());
+    {
+        py::gil_scoped_release no_gil;
+        stream.synchronize();
+    }
+    return {ws, fp};
+}
+
+// sync.weight_fingerprint of parameters in name order; None where they are not all fp32, contiguous and on one GPU
+c10::optional<double> fingerprint(const std::vector<torch::Tensor>& params) {
+    std::vector<const float*> ptrs;
+    std::vector<int64_t> numel;
+    for (const torch::Tensor& t : params) {
+        if (!t.is_cuda() || t.device() != params[0].device() || t.scalar_type() != torch::kFloat || !t.is_contiguous() || !t.numel())
+            return c10::nullopt;
+        ptrs.push_back(static_cast<const float*>(t.data_ptr()));
+        numel.push_back(t.numel());
+    }
+    if (params.empty()) return c10::nullopt;
+    const c10::Device dev = params[0].device();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
+    const int n = (int)params.size();
+    const torch::Tensor buf = at::empty({bf_fingerprint_partials(numel.data(), n) + 1}, at::TensorOptions().device(dev).dtype(torch::kDouble));
+    double* const out = static_cast<double*>(buf.data_ptr());
+    const int rc = bf_fingerprint(ptrs.data(), numel.data(), n, out + 1, out, stream_of(dev));
+    TORCH_CHECK(rc == BF_OK, "bf_fingerprint failed (", rc, "): ", bf_last_error());
+    py::gil_scoped_release no_gil;
+    return buf[0].item<double>();
+}
+
 // Cycles per phase summed over the wavefronts of one launch of the profiling build (see
 // bf_profile_phases); returns an int64 tensor on the device, already written when it is read.
 torch::Tensor profile_phases(torch::Tensor boards, torch::Tensor control, torch::Tensor rep, torch::Tensor weights,
@@ -342,6 +415,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("expand_edges", &expand_edges, "edges of search nodes from logits and legal-move words", py::arg("policy"), py::arg("promo"),
           py::arg("value"), py::arg("mask"), py::arg("boards"), py::arg("control"), py::arg("max_edges") = 96,
           py::arg("active") = py::none(), py::arg("out") = py::none(), py::arg("leaves") = py::none());
+    m.def("pack_board", &pack_board, "a network's parameters into the board blobs", py::arg("params"), py::arg("d_model"), py::arg("n_layers"),
+          py::arg("d_ff"), py::arg("n_value"), py::arg("eps"), py::arg("fp8"), py::arg("device"));
+    m.def("fingerprint", &fingerprint, "index-weighted float64 sum over parameters on one GPU, or None", py::arg("params"));
     m.def("profile_phases", &profile_phases, "cycles per phase of one profiled launch", py::arg("boards"),
           py::arg("control"), py::arg("rep"), py::arg("weights"), py::arg("params"), py::arg("policy"), py::arg("promo"),
           py::arg("value"), py::arg("d_model"), py::arg("n_layers"), py::arg("n_heads"), py::arg("d_ff"), py::arg("eps"),

@@ -598,31 +598,35 @@ def pack_board_on_device(net, stack, shape: _Shape, fp8: bool, device):
     read back) -> (board_wstream, board_fparams) on ``device``, the same bytes.  Parameters that
     already lie there in fp32 are read in place.  The blobs are complete when this returns, so that
     any stream may use them."""
-    d, f, n_value = shape.d_model, shape.d_ff, shape.n_value
-
-    def take(p, *want):
-        t = p.detach().to(device=device, dtype=torch.float32).contiguous()
-        if tuple(t.shape) != want:
-            raise ValueError(f"a parameter is {tuple(t.shape)}, the network shape wants {want}")
-        return t if t.data_ptr() % 16 == 0 else t.clone()
+    d, f, n_value, device = shape.d_model, shape.d_ff, shape.n_value, torch.device(device)
+    params = []
+    for lay in stack.layers:
+        at = lay.self_attn
+        n1, n2, op, l1, l2 = lay.norm1, lay.norm2, at.out_proj, lay.linear1, lay.linear2
+        params += [n1.weight, n1.bias, at.in_proj_weight, at.in_proj_bias, op.weight, op.bias,
+                   n2.weight, n2.bias, l1.weight, l1.bias, l2.weight, l2.bias]
+    n_layer_ptrs = len(params)
+    rows = (64, 12, 4, 101, 3, None, None, N_POLICY, N_PROMO, n_value)
+    if net is not None:
+        params += [m.weight for m in (net.emb_square, net.emb_type_special, net.emb_color_turn, net.emb_clock, net.emb_rep)]
+        params += [net.norm_f.weight, net.norm_f.bias, net.policy.weight, net.promo.weight, net.value.weight]
+    else:
+        params += [torch.zeros(*(d,) if r is None else (r, d), device=device) for r in rows]
+        params[n_layer_ptrs + 5].fill_(1.0)
+    ext = _native()
+    if ext is not None:
+        index = torch.cuda.current_device() if device.index is None else device.index
+        return ext.pack_board(params, d, shape.n_layers, f, n_value, shape.eps, fp8, index)
+    want = [(d,), (d,), (3 * d, d), (3 * d,), (d, d), (d,), (d,), (d,), (f, d), (f,), (d, f), (d,)] * shape.n_layers
+    want += [(d,) if r is None else (r, d) for r in rows]
     lib = load_library()
     with torch.cuda.device(device), torch.no_grad():
         keep = []
-        for lay in stack.layers:
-            at = lay.self_attn
-            keep += [take(lay.norm1.weight, d), take(lay.norm1.bias, d), take(at.in_proj_weight, 3 * d, d), take(at.in_proj_bias, 3 * d),
-                     take(at.out_proj.weight, d, d), take(at.out_proj.bias, d), take(lay.norm2.weight, d), take(lay.norm2.bias, d),
-                     take(lay.linear1.weight, f, d), take(lay.linear1.bias, f), take(lay.linear2.weight, d, f), take(lay.linear2.bias, d)]
-        n_layer_ptrs = len(keep)
-        tables = (("emb_square", 64), ("emb_type_special", 12), ("emb_color_turn", 4), ("emb_clock", 101), ("emb_rep", 3))
-        heads = (("policy", N_POLICY), ("promo", N_PROMO), ("value", n_value))
-        if net is not None:
-            keep += [take(getattr(net, name).weight, rows, d) for name, rows in tables]
-            keep += [take(net.norm_f.weight, d), take(net.norm_f.bias, d)]
-            keep += [take(getattr(net, name).weight, rows, d) for name, rows in heads]
-        else:
-            zero = torch.zeros(101, d, device=device)
-            keep += [zero] * 5 + [torch.ones(d, device=device), zero] + [zero] * 3
+        for p, w in zip(params, want):
+            t = p.detach().to(device=device, dtype=torch.float32).contiguous()
+            if tuple(t.shape) != w:
+                raise ValueError(f"a parameter is {tuple(t.shape)}, the network shape wants {w}")
+            keep.append(t if t.data_ptr() % 16 == 0 else t.clone())
         ptrs = (C.c_void_p * len(keep))(*[t.data_ptr() for t in keep])
         wstream = torch.empty(lib.bf_board_wstream_bytes(C.byref(shape)), dtype=torch.uint8, device=device)
         fparams = torch.empty(lib.bf_board_fparams_floats(C.byref(shape)), dtype=torch.float32, device=device)
@@ -637,18 +641,10 @@ def pack_board_on_device(net, stack, shape: _Shape, fp8: bool, device):
 
 
 def fingerprint_on_device(params):
-    """The weight fingerprint (``bf_fingerprint``) of fp32 tensors that lie contiguously on one GPU."""
-    lib = load_library()
-    n = len(params)
-    numel = (C.c_int64 * n)(*[p.numel() for p in params])
-    ptrs = (C.c_void_p * n)(*[p.data_ptr() for p in params])
-    dev = params[0].device
-    with torch.cuda.device(dev):
-        buf = torch.empty(lib.bf_fingerprint_partials(numel, n) + 1, dtype=torch.float64, device=dev)
-        rc = lib.bf_fingerprint(ptrs, numel, n, buf.data_ptr() + 8, buf.data_ptr(), C.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
-    if rc:
-        raise RuntimeError(f"bf_fingerprint failed ({rc}): {lib.bf_last_error().decode()}")
-    return float(buf[0])
+    """The weight fingerprint (``bf_fingerprint``) of tensors in name order, or None where they are not
+    all fp32, contiguous and on one GPU (or the extension module is not there)."""
+    ext = _native()
+    return ext.fingerprint(params) if ext is not None else None
 
 
 # --------------------------------------------------------------------------- #

@@ -25,10 +25,11 @@ def weight_fingerprint(net) -> float:
     for the whole network; the order of the sum differs from the CPU's, so a value is compared with
     one taken on the same device."""
     named = sorted(net.named_parameters(), key=lambda kv: kv[0])
-    if named and all(p.dtype is torch.float32 and p.is_cuda and p.device == named[0][1].device and p.is_contiguous()
-                     and p.numel() for _, p in named):
+    if named and named[0][1].is_cuda:
         from .hip_impl import fingerprint_on_device
-        return fingerprint_on_device([p for _, p in named])
+        got = fingerprint_on_device([p for _, p in named])
+        if got is not None:
+            return got
     acc = 0.0
     for i, (_, p) in enumerate(named):
         f = p.detach().reshape(-1).double()
