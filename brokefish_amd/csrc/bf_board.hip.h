@@ -420,7 +420,7 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
         }
         const float v = xsum(tiles_sum(ts), 1);
         const float var = (v + partner(v, g)) * (1.0f / D);
-        const float rstd = 1.0f / __builtin_sqrtf(var + a.eps);
+        const float rstd = recip_sqrt(var + a.eps);
 #pragma unroll
         for (int i = 0; i < TWW; i++)
 #pragma unroll
@@ -455,13 +455,13 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
             sa[c] = m > 0.0f ? (FP8 ? m * 0.125f : div127(m)) : 1.0f;
         }
         const float so = KC == 1 ? sa[0] : (q < WPC ? sa[0] : sa[KC - 1]);
-        const float inv = 1.0f / so;
+        const Quot by = quot_by(so);
 #pragma unroll
         for (int i = 0; i < TWW; i++) {
             v4i w;
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                w[j] = (int)quant4<FP8>(y[i][4 * j], y[i][4 * j + 1], y[i][4 * j + 2], y[i][4 * j + 3], so, inv);
+                w[j] = (int)quant4<FP8>(y[i][4 * j], y[i][4 * j + 1], y[i][4 * j + 2], y[i][4 * j + 3], by);
             *reinterpret_cast<v4i*>(act + (TW * q + t0 + i) * FRAG + lane * 16) = w;
             if (TAPS && tap)
 #pragma unroll
@@ -719,7 +719,7 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
                 p[r] = exp_neg(p[r] - mx);
                 lsum = lsum + p[r];
             }
-            const float rl = 1.0f / (lsum + partner(lsum, g));
+            const float rl = recip(lsum + partner(lsum, g));
             v16f oa = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
             for (int r = 0; r < 16; r++) oa = BF_F32MMA(vf[r], p[r] * rl, oa);
@@ -843,15 +843,15 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
                     sh[2 * st + c] = m > 0.0f ? (FP8 ? m * 0.125f : div255(m)) : 1.0f;
                 }
                 const float s8 = q < 2 ? sh[2 * st] : sh[2 * st + 1];
-                const float inv = 1.0f / s8;
+                const Quot by = quot_by(s8);
 #pragma unroll
                 for (int i = 0; i < HT; i++) {
                     v4i w;
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         unsigned u;
-                        if constexpr (FP8) u = quant4<true>(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], s8, inv);
-                        else u = quant4_relu_u8(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], s8, inv);
+                        if constexpr (FP8) u = quant4<true>(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], by);
+                        else u = quant4_relu_u8(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], by);
                         if (TAPS && a.taps.qa_ff2)
                             *reinterpret_cast<unsigned*>(a.taps.qa_ff2 + (bl * T + t) * F + 512 * st + 128 * q + 32 * (h0 + i) + 8 * j + 4 * g) = u;
                         w[j] = (int)(FP8 ? u : (u ^ 0x80808080u));
@@ -995,15 +995,15 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
                         sh[c] = m > 0.0f ? (FP8 ? m * 0.125f : div255(m)) : 1.0f;
                     }
                     const float s8 = q < 2 ? sh[0] : sh[1];
-                    const float inv = 1.0f / s8;
+                    const Quot by = quot_by(s8);
 #pragma unroll
                     for (int i = 0; i < HT; i++) {
                         v4i w;
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
                             unsigned u;
-                            if constexpr (FP8) u = quant4<true>(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], s8, inv);
-                            else u = quant4_relu_u8(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], s8, inv);
+                            if constexpr (FP8) u = quant4<true>(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], by);
+                            else u = quant4_relu_u8(hf[i][4 * j], hf[i][4 * j + 1], hf[i][4 * j + 2], hf[i][4 * j + 3], by);
                             if (TAPS && a.taps.qa_ff2)
                                 *reinterpret_cast<unsigned*>(a.taps.qa_ff2 + (bl * T + t) * F + 512 * st + 128 * q + 32 * (h0 + i) + 8 * j + 4 * g) = u;
                             w[j] = (int)(FP8 ? u : (u ^ 0x80808080u));

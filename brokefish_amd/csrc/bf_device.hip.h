@@ -33,7 +33,10 @@ __device__ __forceinline__ float partner(float v, int g) {
 // exp(x) for x <= 0; same operation sequence as the CPU checker's bfo_exp_neg
 __device__ __forceinline__ float exp_neg(float x) {
     const float t = x * 1.44269504088896341f;
-    const float n = __builtin_rintf(t);
+    // rint(t) by adding 1.5 * 2^23: the sum's low bits are the integer, ready to be shifted into the
+    // exponent (an addition and a subtraction issue faster than a rounding and a conversion)
+    const float tm = t + 12582912.0f;
+    const float n = tm - 12582912.0f;
     float r = __builtin_fmaf(n, -0.693359375f, x);
     r = __builtin_fmaf(n, 2.12194440e-4f, r);
     const float z = r * r;
@@ -45,7 +48,7 @@ __device__ __forceinline__ float exp_neg(float x) {
     p = __builtin_fmaf(p, r, 5.0000001201e-1f);
     float y = __builtin_fmaf(p, z, r);
     y = y + 1.0f;
-    const float s = __int_as_float(__float_as_int(y) + (((int)n) << 23));
+    const float s = __int_as_float((int)((unsigned)__float_as_int(y) + ((unsigned)__float_as_int(tm) << 23)));
     return (x >= -87.0f) ? s : 0.0f;
 }
 
@@ -151,25 +154,45 @@ __device__ __forceinline__ float div255(float m) {
     return __builtin_fmaf(__builtin_fmaf(-q, 255.0f, m), c, q);
 }
 
+// 1 / x, correctly rounded: the hardware's reciprocal and one Newton step (equal to IEEE division for
+// every mantissa and every exponent whose reciprocal is a normal number, checked on the device
+// exhaustively; the compiler's division takes 11 instructions, four times as many).
+__device__ __forceinline__ float recip(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+// 1 / sqrt(x) as a correctly rounded square root and a correctly rounded reciprocal of it (the square root
+// from the hardware's reciprocal root and one residual: exact for 2^-67 <= x < 2^53, checked likewise).
+__device__ __forceinline__ float recip_sqrt(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s0 = x * y;
+    return recip(__builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0));
+}
+
+// The reciprocal of an activation scale in two floats, hi = fl(1 / sa) and lo the rest of it, so that
+// fma(v, hi, v * lo) rounds v / sa where it matters in two instructions instead of three: it falls on the
+// same side of every half-integer up to 255.5 (every midpoint of two e4m3 values) as the correctly
+// rounded quotient, ties included.  The product's own error is 2^-48 of the quotient, so only pairs
+// whose quotient lies that close to the edge of a tie's rounding interval could differ; there are
+// 7564 such pairs of significands within sixteen times that distance, and all agree
+// (tests/test_quotient.py enumerates them; the last term of lo is what two of them need).
+struct Quot { float hi, lo; };
+__device__ __forceinline__ Quot quot_by(float sa) {
+    const float hi = recip(sa);
+    const float rem = __builtin_fmaf(-sa, hi, 1.0f);
+    return {hi, __builtin_fmaf(rem, hi, (rem * hi) * (0.5f * rem))};
+}
+__device__ __forceinline__ float quot(float v, const Quot& d) { return __builtin_fmaf(v, d.hi, v * d.lo); }
+
 // ---- row operations -------------------------------------------------------------------
 
-// four quotients v / sa (correctly rounded) -> one packed dword.
-// int8: round to nearest even, low bytes gathered.  e4m3: clamp to the format's range and
-// convert with the hardware's round-to-nearest-even OCP e4m3 conversion.
+// four quotients v / sa -> one packed dword.
+// int8: round to nearest even, low bytes gathered.  e4m3: the hardware's round-to-nearest-even OCP
+// e4m3 conversion; the row scale keeps |v / sa| at 8, far from where the conversion would overflow.
 template <bool FP8>
-__device__ __forceinline__ unsigned quant4(float v0, float v1, float v2, float v3, float sa, float inv) {
-    float qf[4];
-    const float v[4] = {v0, v1, v2, v3};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        // correctly rounded v / sa from the reciprocal and two fused corrections
-        const float q0 = v[i] * inv;
-        const float rem = __builtin_fmaf(-q0, sa, v[i]);
-        qf[i] = __builtin_fmaf(rem, inv, q0);
-    }
+__device__ __forceinline__ unsigned quant4(float v0, float v1, float v2, float v3, const Quot& by) {
+    const float qf[4] = {quot(v0, by), quot(v1, by), quot(v2, by), quot(v3, by)};
     if constexpr (FP8) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) qf[i] = __builtin_fminf(__builtin_fmaxf(qf[i], -448.0f), 448.0f);
         int w = __builtin_amdgcn_cvt_pk_fp8_f32(qf[0], qf[1], 0, false);
         w = __builtin_amdgcn_cvt_pk_fp8_f32(qf[2], qf[3], w, true);
         return (unsigned)w;
@@ -188,19 +211,15 @@ __device__ __forceinline__ unsigned quant4(float v0, float v1, float v2, float v
 }
 
 // The unsigned int8 quantiser of the feed-forward hidden row with the ReLU folded in: four
-// correctly rounded quotients v / sa, converted with v_cvt_pk_u8_f32 -- round to nearest even,
+// quotients v / sa, converted with v_cvt_pk_u8_f32 -- round to nearest even,
 // saturating to [0, 255], so a negative input gives 0 exactly as max(v, 0) would (held against
 // rint + clamp on the host, every tie k + 0.5 included, by tests/test_quantiser_gpu.py) -- each
 // conversion writing its own byte of the dword.
-__device__ __forceinline__ unsigned quant4_relu_u8(float v0, float v1, float v2, float v3, float sa, float inv) {
+__device__ __forceinline__ unsigned quant4_relu_u8(float v0, float v1, float v2, float v3, const Quot& by) {
     const float v[4] = {v0, v1, v2, v3};
     unsigned w = 0;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float q0 = v[i] * inv;
-        const float rem = __builtin_fmaf(-q0, sa, v[i]);
-        w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(rem, inv, q0), i, w);
-    }
+    for (int i = 0; i < 4; i++) w = __builtin_amdgcn_cvt_pk_u8_f32(quot(v[i], by), i, w);
     return w;
 }
 
@@ -215,12 +234,12 @@ __device__ __forceinline__ void quant_s8(const float (&y)[NTILES][16], int g, v4
         for (int r = 0; r < 16; r++) am = __builtin_fmaxf(am, __builtin_fabsf(y[n][r]));
     am = __builtin_fmaxf(am, partner(am, g));
     sa = am > 0.0f ? (FP8 ? am * 0.125f : div127(am)) : 1.0f;
-    const float inv = 1.0f / sa;
+    const Quot by = quot_by(sa);
 #pragma unroll
     for (int n = 0; n < NTILES; n++)
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            q[n][j] = (int)quant4<FP8>(y[n][4 * j], y[n][4 * j + 1], y[n][4 * j + 2], y[n][4 * j + 3], sa, inv);
+            q[n][j] = (int)quant4<FP8>(y[n][4 * j], y[n][4 * j + 1], y[n][4 * j + 2], y[n][4 * j + 3], by);
 }
 
 }  // namespace bf

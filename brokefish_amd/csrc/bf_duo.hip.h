@@ -277,7 +277,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
         for (int p = 0; p < NP; p++) {
             const float var = (v[p] + partner(v[p], g)) * (1.0f / D);
-            rstd[p] = 1.0f / __builtin_sqrtf(var + a.eps);
+            rstd[p] = recip_sqrt(var + a.eps);
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -311,11 +311,11 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             m = __builtin_fmaxf(m, partner(m, g));
             sa[p] = m > 0.0f ? (FP8 ? m * 0.125f : div127(m)) : 1.0f;
             if (publish_scales && wave == 0 && g == 0) tok[p * 32 + t] = sa[p];
-            const float inv = 1.0f / sa[p];
+            const Quot by = quot_by(sa[p]);
             v4i w;
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                w[j] = (int)quant4<FP8>(y[p][4 * j], y[p][4 * j + 1], y[p][4 * j + 2], y[p][4 * j + 3], sa[p], inv);
+                w[j] = (int)quant4<FP8>(y[p][4 * j], y[p][4 * j + 1], y[p][4 * j + 2], y[p][4 * j + 3], by);
             if constexpr (FP8) {
                 const v2l wl = __builtin_bit_cast(v2l, w);
 #pragma unroll
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                     pr[r] = exp_neg(pr[r] - mx);
                     lsum = lsum + pr[r];
                 }
-                const float rl = 1.0f / (lsum + partner(lsum, g));
+                const float rl = recip(lsum + partner(lsum, g));
                 v16f oa = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
                 for (int r = 0; r < 16; r++) oa = BF_F32MMA(vf[p][r], pr[r] * rl, oa);
@@ -715,15 +715,15 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                     sh[p][2 * st + c] = m > 0.0f ? (FP8 ? m * 0.125f : div255(m)) : 1.0f;
                 }
                 const float s8 = q < 2 ? sh[p][2 * st] : sh[p][2 * st + 1];
-                const float inv = 1.0f / s8;
+                const Quot by = quot_by(s8);
 #pragma unroll
                 for (int i = 0; i < HT; i++) {
                     v4i w;
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         unsigned u;
-                        if constexpr (FP8) u = quant4<true>(hf[p][i][4 * j], hf[p][i][4 * j + 1], hf[p][i][4 * j + 2], hf[p][i][4 * j + 3], s8, inv);
-                        else u = quant4_relu_u8(hf[p][i][4 * j], hf[p][i][4 * j + 1], hf[p][i][4 * j + 2], hf[p][i][4 * j + 3], s8, inv);
+                        if constexpr (FP8) u = quant4<true>(hf[p][i][4 * j], hf[p][i][4 * j + 1], hf[p][i][4 * j + 2], hf[p][i][4 * j + 3], by);
+                        else u = quant4_relu_u8(hf[p][i][4 * j], hf[p][i][4 * j + 1], hf[p][i][4 * j + 2], hf[p][i][4 * j + 3], by);
                         if (TAPS && a.taps.qa_ff2 && live[p])
                             *reinterpret_cast<unsigned*>(a.taps.qa_ff2 + (bl[p] * T + t) * F + 512 * st + 128 * q + 32 * (HT * sub + i) + 8 * j + 4 * g) = u;
                         w[j] = (int)(FP8 ? u : (u ^ 0x80808080u));

@@ -111,7 +111,7 @@ __device__ __forceinline__ void layernorm(const float (&x)[NT][16], const float*
     }
     const float v = ((sg[0] + sg[1]) + sg[2]) + sg[3];
     const float var = (v + partner(v, g)) * (1.0f / D);
-    const float rstd = 1.0f / __builtin_sqrtf(var + eps);
+    const float rstd = recip_sqrt(var + eps);
 #pragma unroll
     for (int n = 0; n < NT; n++)
 #pragma unroll
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(THREADS, 1) void eval_kernel(const KArgs a) {
                 p[r] = exp_neg(p[r] - mx);
                 lsum = lsum + p[r];
             }
-            const float rl = 1.0f / (lsum + partner(lsum, g));
+            const float rl = recip(lsum + partner(lsum, g));
             v16f oa = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
             for (int r = 0; r < 16; r++) oa = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[r], p[r] * rl, oa, 0, 0, 0);
@@ -454,14 +454,14 @@ __global__ __launch_bounds__(THREADS, 1) void eval_kernel(const KArgs a) {
                     // e4m3: the ordinary signed quantiser (the values are non-negative).
                     am = __builtin_fmaxf(am, partner(am, g));
                     const float s8 = am > 0.0f ? am / (FP8 ? 8.0f : 255.0f) : 1.0f;
-                    const float inv = 1.0f / s8;
+                    const Quot by = quot_by(s8);
                     sh[c] = s8;
 #pragma unroll
                     for (int s2 = 0; s2 < 8; s2++)
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
                             const unsigned w = quant4<FP8>(hf[s2][4 * j], hf[s2][4 * j + 1], hf[s2][4 * j + 2],
-                                                           hf[s2][4 * j + 3], s8, inv);
+                                                           hf[s2][4 * j + 3], by);
                             if (TAPS && a.taps.qa_ff2 && valid)
                                 *reinterpret_cast<unsigned*>(a.taps.qa_ff2 + (bl * T + t) * F + 256 * c + 32 * s2 + 8 * j + 4 * g) = w;
                             hq[c][s2][j] = (int)(FP8 ? w : (w ^ 0x80808080u));

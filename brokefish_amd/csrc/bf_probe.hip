@@ -179,12 +179,16 @@ template <int MODE>
 __global__ void quant_probe(const float* x, float scale, long n4, unsigned* out) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n4) return;
-    const float4 v = reinterpret_cast<const float4*>(x)[i];
-    const float inv = 1.0f / scale;
+    float4 v = reinterpret_cast<const float4*>(x)[i];
+    const bf::Quot by = bf::quot_by(scale);
     unsigned w;
-    if constexpr (MODE == BF_PROBE_S8) w = bf::quant4<false>(v.x, v.y, v.z, v.w, scale, inv);
-    else if constexpr (MODE == BF_PROBE_U8_RELU) w = bf::quant4_relu_u8(v.x, v.y, v.z, v.w, scale, inv);
-    else w = bf::quant4<true>(v.x, v.y, v.z, v.w, scale, inv);
+    if constexpr (MODE == BF_PROBE_S8) w = bf::quant4<false>(v.x, v.y, v.z, v.w, by);
+    else if constexpr (MODE == BF_PROBE_U8_RELU) w = bf::quant4_relu_u8(v.x, v.y, v.z, v.w, by);
+    else {   // any value may be asked for here: clamped to the format's range first, as the header says
+        const float top = 448.0f * scale;
+        auto clamp = [&](float f) { return __builtin_fminf(__builtin_fmaxf(f, -top), top); };
+        w = bf::quant4<true>(clamp(v.x), clamp(v.y), clamp(v.z), clamp(v.w), by);
+    }
     out[i] = w;
 }
 
