@@ -9,15 +9,18 @@
 // count, the mass dropped by the truncation and the value mapped from [-1,1] to [0,1].
 // Restates reference docs/reference/search.md:616-636 and brokefish/search/torch_impl.py:962-1033.
 //
-// One wavefront per position: lane l owns half a mask word (slot l/2, squares 32*(l%2) ..+31), so
-// lane order is canonical order and an edge's index is a prefix sum over lanes.  A position has
-// some 30 legal moves over its 64 half-words, so the lanes first lay the candidates out in LDS
-// in canonical order (a lane walks only the set bits of its half-word, its logits staged in LDS)
-// and then take one to four candidates each: softmax, truncation and the stores are lane-parallel
-// over candidates, counts and ranks come from ballots.  The truncation threshold (the E-th largest
-// log-prior) is found by bisection on the ordered bit pattern of the float.  A mask with more
-// candidates than the layout holds (256; no legal position has them) is handled without it, every
-// pass walking the lanes' set bits again.
+// Two positions per wavefront, 32 lanes each: lane s of a half owns the mask word of slot s, so lane order
+// is canonical order and a slot's first edge index is a prefix sum over the half.  Candidates (some 31
+// per position) are then taken one per lane, 32 a round: a lane finds the slot its candidate belongs to
+// by a running maximum over the slots' first indices and the square as the k-th set bit of that
+// slot's word -- no loop over bits -- and fetches its one logit straight from the policy row (the loop,
+// with the logits it might need staged in LDS, remains for wavefronts in which a pawn promotes).
+// Reductions run over DPP and lane swaps, ranks and counts over ballots; the edges are put together in
+// LDS and leave as whole 16-byte pieces.  The truncation threshold (the E-th largest log-prior) is
+// found by bisection on the ordered bit pattern of the float.  A position with more than 128 candidates
+// (a constructed one, or an arbitrary mask) takes the whole wavefront, every pass walking the bits again.
+// Bound by instruction issue and, from some 16384 positions on, by HBM; one position per wavefront with
+// staged logits took 48 us for 65536 positions (E = 96), this 23 us (4 TB/s of its bytes).
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -27,9 +30,6 @@
 #include "bf_args.h"
 
 namespace {
-
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int PAWN = 0;          // reference docs/reference/spec.md:47
 constexpr int PROMO_SHIFT = 11;  // brokefish/search/torch_impl.py:61-62
@@ -45,6 +45,7 @@ struct KExpand {
     const int* leaf_index;        // optional compacted list: slot j expands position leaf_index[j] for j < *leaf_count
     const int* leaf_count;
     int n, E, logits_fp32;
+    int whole_rows;               // a row of edges is whole 16-byte pieces, and few enough to be put together in LDS
     int16_t* edge_move;
     _Float16* edge_prior;
     int* n_edges;
@@ -83,11 +84,6 @@ __device__ __forceinline__ unsigned ordered(float f) {
     const unsigned u = __float_as_uint(f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
-
-// lanes below this one whose bit is set in a ballot
-__device__ __forceinline__ int lanes_below(unsigned long long ballot) {
-    return __builtin_amdgcn_mbcnt_hi((unsigned)(ballot >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)ballot, 0));
-}
 // what one lane of this wave wrote to LDS is read by another: LDS operations of a wave are carried
 // out in program order, the fences keep the compiler from changing that order
 __device__ __forceinline__ void wave_lds_sync() {
@@ -96,77 +92,113 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int EXPAND_WAVES = 4;       // positions per workgroup
-constexpr int CAND_CAP = 256;         // candidates a wave lays out in LDS (no legal chess position has more)
-
-// FP32: the logits come as float32 (parity runs) instead of fp16 (the search contract); the staged
-// rows are then twice as large, which costs resident wavefronts, so the two are separate kernels.
-template <bool FP32>
-__global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand a) {
-    constexpr int ROW_STRIDE = (FP32 ? 128 : 64) + 16;   // bytes per lane of staged logits + a pad that spreads the banks
-    __shared__ __attribute__((aligned(16))) char row_lds[EXPAND_WAVES][64 * ROW_STRIDE];
-    __shared__ float cand_l[EXPAND_WAVES][CAND_CAP];
-    __shared__ int16_t cand_c[EXPAND_WAVES][CAND_CAP];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int b = blockIdx.x * EXPAND_WAVES + wv;
-    if (b >= a.n) return;                       // no workgroup barrier below: a wave may leave
-    if (a.leaf_index) {
-        if (b >= *a.leaf_count) return;
-        b = __builtin_amdgcn_readfirstlane(a.leaf_index[b]);
-        if ((unsigned)b >= (unsigned)a.n) return;   // not a position of this launch
+// ---- operations within a half (32 lanes) of the wavefront ---------------------------------------------
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ int dpp0(int v) {   // 0 where no lane supplies a value
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, true);
+}
+constexpr int ROW_SHR = 0x110, ROW_ROR = 0x120, ROW_BCAST15 = 0x142;
+// inclusive scans: within a row of sixteen, then the first row's last lane into the second row
+__device__ __forceinline__ int half_scan_add(int v) {
+    v += dpp0<ROW_SHR + 1>(v);
+    v += dpp0<ROW_SHR + 2>(v);
+    v += dpp0<ROW_SHR + 4>(v);
+    v += dpp0<ROW_SHR + 8>(v);
+    v += dpp0<ROW_BCAST15, 0xa>(v);
+    return v;
+}
+__device__ __forceinline__ int half_scan_max(int v) {   // of values >= 0
+    v = max(v, dpp0<ROW_SHR + 1>(v));
+    v = max(v, dpp0<ROW_SHR + 2>(v));
+    v = max(v, dpp0<ROW_SHR + 4>(v));
+    v = max(v, dpp0<ROW_SHR + 8>(v));
+    v = max(v, dpp0<ROW_BCAST15, 0xa>(v));
+    return v;
+}
+template <typename OP>
+__device__ __forceinline__ float half_reduce(float v, OP op) {   // the result in every lane of the half
+    v = op(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ROW_ROR + 8, 0xf, 0xf, false)));
+    v = op(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ROW_ROR + 4, 0xf, 0xf, false)));
+    v = op(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ROW_ROR + 2, 0xf, 0xf, false)));
+    v = op(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ROW_ROR + 1, 0xf, 0xf, false)));
+    const int i = __float_as_int(v);
+    const auto r = __builtin_amdgcn_permlane16_swap(i, i, false, false);
+    return op(__int_as_float(r[0]), __int_as_float(r[1]));
+}
+__device__ __forceinline__ float half_max(float v) { return half_reduce(v, [](float x, float y) { return fmaxf(x, y); }); }
+__device__ __forceinline__ float half_sum(float v) { return half_reduce(v, [](float x, float y) { return x + y; }); }
+// lanes of this half below this one whose bit is set in a ballot
+__device__ __forceinline__ int half_below(unsigned long long ballot, int half) {
+    return half ? __builtin_amdgcn_mbcnt_hi((unsigned)(ballot >> 32), 0) : __builtin_amdgcn_mbcnt_lo((unsigned)ballot, 0);
+}
+// position of the k-th (from 0) set bit of a 64-bit word
+__device__ __forceinline__ int kth_bit(unsigned lo, unsigned hi, int k) {
+    int c = __popc(lo);
+    const bool up = k >= c;
+    unsigned x = up ? hi : lo;
+    int at = up ? 32 : 0;
+    k -= up ? c : 0;
+#pragma unroll
+    for (int w = 16; w >= 1; w >>= 1) {
+        c = __popc(x & ((1u << w) - 1u));
+        const bool t = k >= c;
+        k -= t ? c : 0;
+        x = t ? x >> w : x;
+        at += t ? w : 0;
     }
-    if (a.active && !a.active[b]) return;
-    const int p = lane >> 1, half = lane & 1;
+    return at;
+}
 
+constexpr int EXPAND_WAVES = 4;       // wavefronts per workgroup
+constexpr int ROUNDS = 4;             // candidates of a position in the two-position form: 32 per round
+constexpr int CAND_CAP = 32 * ROUNDS;
+
+template <bool FP32>
+__device__ __forceinline__ float logit(const void* p, size_t i) {
+    return FP32 ? ((const float*)p)[i] : (float)((const _Float16*)p)[i];
+}
+// log_softmax of a slot's four promotion logits
+template <bool FP32>
+__device__ __forceinline__ void promotion_logs(const void* promo, size_t slot, float (&lp)[4]) {
+    float x[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = logit<FP32>(promo, slot * 4 + k);
+    const float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+    const float s = ((__expf(x[0] - mx) + __expf(x[1] - mx)) + __expf(x[2] - mx)) + __expf(x[3] - mx);
+    const float ls = __logf(s);
+#pragma unroll
+    for (int k = 0; k < 4; k++) lp[k] = (x[k] - mx) - ls;
+}
+__device__ __forceinline__ void write_counts(const KExpand& a, int b, int n_edges, int total, bool trunc, float s_all, float s_keep) {
+    a.n_edges[b] = n_edges;
+    if (a.count) a.count[b] = total;
+    if (a.dropped) a.dropped[b] = trunc ? (s_all - s_keep) / s_all : 0.0f;
+    if (a.node_value) a.node_value[b] = (_Float16)((a.value[b] + 1.0f) / 2.0f);
+}
+
+// One position on the whole wavefront, any number of candidates: lane l owns half a mask word (slot l / 2,
+// squares 32 * (l % 2) .. + 31), nothing is stored per candidate, every pass walks the lane's bits again.
+template <bool FP32>
+__device__ void expand_many(const KExpand& a, int b, int lane) {
+    const int p = lane >> 1, half = lane & 1;
     const unsigned word = a.boards[(size_t)b * 32 + p];
     const int ctrl = a.control[b];
     const bool pawn = ((word >> 11) & 1u) == 0 && ((word >> 6) & 7u) == PAWN;
     const uint64_t m64 = a.mask[(size_t)b * 32 + p];
     const unsigned mh = half ? (unsigned)(m64 >> 32) : (unsigned)m64;
-    // last rank of the side to move: rank 7 (squares 56..63) for white, rank 0 for black
     const unsigned last = ctrl < 0 ? (half == 0 ? 0xFFu : 0u) : (half == 1 ? 0xFF000000u : 0u);
     const unsigned pr = pawn ? (mh & last) : 0u;
-
-    const int cnt = __popc(mh) + 3 * __popc(pr);
-    const int before = wave_exclusive(cnt, lane);
-    const int total = __shfl(before + cnt, 63);
-
-    // A lane that has moves stages its 32 policy logits in LDS, where the walks below pick the
-    // ones its mask names (a lane without a move, which is most of them, loads nothing).
-    char* const myrow = row_lds[wv] + lane * ROW_STRIDE;
-    if (mh) {
-        if constexpr (FP32) {
-            const float* row = (const float*)a.policy + ((size_t)b * 32 + p) * 64 + 32 * half;
-#pragma unroll
-            for (int j = 0; j < 8; j++) *reinterpret_cast<v4f*>(myrow + 16 * j) = *reinterpret_cast<const v4f*>(row + 4 * j);
-        } else {
-            const _Float16* row = (const _Float16*)a.policy + ((size_t)b * 32 + p) * 64 + 32 * half;
-#pragma unroll
-            for (int j = 0; j < 4; j++) *reinterpret_cast<v8h*>(myrow + 16 * j) = *reinterpret_cast<const v8h*>(row + 8 * j);
-        }
-    }
-    // its slot's promotion log-probabilities, where a pawn reaches the last rank
+    const int total = wave_sum((int)(__popc(mh) + 3 * __popc(pr)));
     float lp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (pr) {
-        float x[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            x[k] = FP32 ? ((const float*)a.promo)[((size_t)b * 32 + p) * 4 + k]
-                        : (float)((const _Float16*)a.promo)[((size_t)b * 32 + p) * 4 + k];
-        const float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-        const float s = ((__expf(x[0] - mx) + __expf(x[1] - mx)) + __expf(x[2] - mx)) + __expf(x[3] - mx);
-        const float ls = __logf(s);
-#pragma unroll
-        for (int k = 0; k < 4; k++) lp[k] = (x[k] - mx) - ls;
-    }
+    if (pr) promotion_logs<FP32>(a.promo, (size_t)b * 32 + p, lp);
     // visit this lane's candidates in canonical order: f(log-prior, move code)
     auto each = [&](auto&& f) {
         unsigned m = mh;
         while (m) {
             const int i = __builtin_ctz(m);
             m &= m - 1;
-            const float l = FP32 ? reinterpret_cast<const float*>(myrow)[i] : (float)reinterpret_cast<const _Float16*>(myrow)[i];
             const int mv = p * 64 + 32 * half + i;
+            const float l = logit<FP32>(a.policy, (size_t)b * 2048 + mv);
             if ((pr >> i) & 1u) {
 #pragma unroll
                 for (int k = 0; k < 4; k++) f(l + lp[k], mv | (k << PROMO_SHIFT));
@@ -178,168 +210,271 @@ __global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand
     int16_t* const em = a.edge_move + (size_t)b * a.E;
     _Float16* const ep = a.edge_prior + (size_t)b * a.E;
     const bool trunc = total > a.E;
-    int n_edges;
-    float s_all, s_keep;
-
-    if (total <= CAND_CAP) {
-        // ---- the candidates laid out in LDS in canonical order, then one to four per lane ----------
-        float* const cl = cand_l[wv];
-        int16_t* const cc = cand_c[wv];
-        {
-            int j = before;
-            each([&](float l, int code) {
-                cl[j] = l;
-                cc[j] = (int16_t)code;
-                j++;
-            });
-        }
-        wave_lds_sync();
-        constexpr int R = CAND_CAP / 64;
-        float l[R], e[R];
-        int code[R];
-        bool has[R];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int idx = lane + 64 * r;
-            has[r] = idx < total;
-            l[r] = has[r] ? cl[idx] : -INFINITY;
-            code[r] = has[r] ? cc[idx] : 0;
-            mx = fmaxf(mx, l[r]);
-        }
-        mx = wave_max(mx);
-        float sa = 0.0f;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            e[r] = has[r] ? __expf(l[r] - mx) : 0.0f;
-            sa += e[r];
-        }
-        s_all = wave_sum(sa);
-        if (!trunc) {
-            // everything survives, in place
-            n_edges = total;
-            s_keep = s_all;
-            const float inv = 1.0f / s_keep;
-#pragma unroll
-            for (int r = 0; r < R; r++)
-                if (has[r]) {
-                    em[lane + 64 * r] = (int16_t)code[r];
-                    ep[lane + 64 * r] = (_Float16)(e[r] * inv);
-                }
-        } else {
-            // T = ordered pattern of the E-th largest log-prior, `need` ties at T survive
-            unsigned o[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) o[r] = has[r] ? ordered(l[r]) : 0u;
-            unsigned T = 0;
+    float mx = -INFINITY;
+    each([&](float l, int) { mx = fmaxf(mx, l); });
+    mx = wave_max(mx);
+    unsigned T = 0;   // ordered pattern of the E-th largest log-prior, `need` ties at T survive
+    int need = 0, tie_before = 0;
+    if (trunc) {
 #pragma clang loop unroll(disable)
-            for (int bit = 31; bit >= 0; bit--) {
-                const unsigned cand = T | (1u << bit);
-                int c = 0;
-#pragma unroll
-                for (int r = 0; r < R; r++) c += __popcll(__ballot(has[r] && o[r] >= cand));
-                if (c >= a.E) T = cand;
-            }
-            int gt = 0;
-#pragma unroll
-            for (int r = 0; r < R; r++) gt += __popcll(__ballot(has[r] && o[r] > T));
-            const int need = a.E - gt;
-            int ties = 0, kept_before = 0;
-            float sk = 0.0f;
-            bool keep[R];
-            int pos[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const bool eq = has[r] && o[r] == T;
-                const unsigned long long eqb = __ballot(eq);
-                keep[r] = has[r] && (o[r] > T || (eq && ties + lanes_below(eqb) < need));
-                ties += __popcll(eqb);
-                const unsigned long long kb = __ballot(keep[r]);
-                pos[r] = kept_before + lanes_below(kb);
-                kept_before += __popcll(kb);
-                sk += keep[r] ? e[r] : 0.0f;
-            }
-            n_edges = kept_before;
-            s_keep = wave_sum(sk);
-            const float inv = 1.0f / s_keep;
-#pragma unroll
-            for (int r = 0; r < R; r++)
-                if (keep[r]) {
-                    em[pos[r]] = (int16_t)code[r];
-                    ep[pos[r]] = (_Float16)(e[r] * inv);
-                }
+        for (int bit = 31; bit >= 0; bit--) {
+            const unsigned cand = T | (1u << bit);
+            int c = 0;
+            each([&](float l, int) { c += ordered(l) >= cand; });
+            if (wave_sum(c) >= a.E) T = cand;
         }
-    } else {
-        // ---- more candidates than the layout holds (no legal position: an arbitrary mask): nothing
-        // is stored per candidate, every pass walks the lane's squares again ---------------------------
-        float mx = -INFINITY;
-        each([&](float l, int) { mx = fmaxf(mx, l); });
-        mx = wave_max(mx);
-        unsigned T = 0;
-        int need = 0, tie_before = 0;
-        if (trunc) {
-#pragma clang loop unroll(disable)
-            for (int bit = 31; bit >= 0; bit--) {
-                const unsigned cand = T | (1u << bit);
-                int c = 0;
-                each([&](float l, int) { c += ordered(l) >= cand; });
-                if (wave_sum(c) >= a.E) T = cand;
-            }
-            int gt = 0, eq = 0;
-            each([&](float l, int) {
-                const unsigned o = ordered(l);
-                gt += o > T;
-                eq += o == T;
-            });
-            need = a.E - wave_sum(gt);
-            tie_before = wave_exclusive(eq, lane);
-        }
-        // one pass: kept count of this lane, softmax denominators over all and over the survivors
-        int kept = 0, tie = tie_before;
-        float sa = 0.0f, sk = 0.0f;
+        int gt = 0, eq = 0;
         each([&](float l, int) {
-            const float e = __expf(l - mx);
-            sa += e;
-            bool keep = true;
-            if (trunc) {
-                const unsigned o = ordered(l);
-                keep = o > T || (o == T && tie < need);
-                tie += o == T;
-            }
-            if (keep) { kept++; sk += e; }
+            const unsigned o = ordered(l);
+            gt += o > T;
+            eq += o == T;
         });
-        s_all = wave_sum(sa);
-        s_keep = wave_sum(sk);
-        int pos = wave_exclusive(kept, lane);
-        n_edges = __shfl(pos + kept, 63);
-        // write the survivors in canonical order
-        const float inv = 1.0f / s_keep;
-        tie = tie_before;
-        each([&](float l, int code) {
-            bool keep = true;
-            if (trunc) {
-                const unsigned o = ordered(l);
-                keep = o > T || (o == T && tie < need);
-                tie += o == T;
-            }
-            if (keep) {
-                em[pos] = (int16_t)code;
-                ep[pos] = (_Float16)(__expf(l - mx) * inv);
-                pos++;
-            }
-        });
+        need = a.E - wave_sum(gt);
+        tie_before = wave_exclusive(eq, lane);
     }
-    // unused edge slots read as no edge
-    for (int i = n_edges + lane; i < a.E; i += 64) {
+    // one pass: kept count of this lane, softmax denominators over all and over the survivors
+    int kept = 0, tie = tie_before;
+    float sa = 0.0f, sk = 0.0f;
+    each([&](float l, int) {
+        const float e = __expf(l - mx);
+        sa += e;
+        bool keep = true;
+        if (trunc) {
+            const unsigned o = ordered(l);
+            keep = o > T || (o == T && tie < need);
+            tie += o == T;
+        }
+        if (keep) { kept++; sk += e; }
+    });
+    const float s_all = wave_sum(sa), s_keep = wave_sum(sk);
+    int pos = wave_exclusive(kept, lane);
+    const int n_edges = __shfl(pos + kept, 63);
+    // write the survivors in canonical order
+    const float inv = 1.0f / s_keep;
+    tie = tie_before;
+    each([&](float l, int code) {
+        bool keep = true;
+        if (trunc) {
+            const unsigned o = ordered(l);
+            keep = o > T || (o == T && tie < need);
+            tie += o == T;
+        }
+        if (keep) {
+            em[pos] = (int16_t)code;
+            ep[pos] = (_Float16)(__expf(l - mx) * inv);
+            pos++;
+        }
+    });
+    for (int i = n_edges + lane; i < a.E; i += 64) {   // unused edge slots read as no edge
         em[i] = 0;
         ep[i] = (_Float16)0.0f;
     }
-    if (lane == 0) {
-        a.n_edges[b] = n_edges;
-        if (a.count) a.count[b] = total;
-        if (a.dropped) a.dropped[b] = trunc ? (s_all - s_keep) / s_all : 0.0f;
-        if (a.node_value) a.node_value[b] = (_Float16)((a.value[b] + 1.0f) / 2.0f);
+    if (lane == 0) write_counts(a, b, n_edges, total, trunc, s_all, s_keep);
+}
+
+template <bool FP32>
+__global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand a) {
+    __shared__ __attribute__((aligned(16))) int16_t code_lds[EXPAND_WAVES][2][CAND_CAP];
+    __shared__ __attribute__((aligned(16))) _Float16 prior_lds[EXPAND_WAVES][2][CAND_CAP];
+    __shared__ float add_lds[EXPAND_WAVES][2][CAND_CAP];      // promotion log-probability of a candidate
+    __shared__ unsigned owner_lds[EXPAND_WAVES][2][CAND_CAP / 4];   // one byte per candidate
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, s = lane & 31, half = lane >> 5;
+    const int j = 2 * (blockIdx.x * EXPAND_WAVES + wv) + half;
+    // the half's position; a half without one has no candidates and stores nothing
+    int b = j;
+    bool ok = j < a.n;
+    if (a.leaf_index) {
+        ok = ok && j < *a.leaf_count;
+        b = ok ? a.leaf_index[j] : 0;
+        ok = ok && (unsigned)b < (unsigned)a.n;
     }
+    if (ok && a.active) ok = a.active[b] != 0;
+    if (!ok) b = 0;
+    if (__ballot(ok) == 0) return;                       // no workgroup barrier below: a wave may leave
+
+    const unsigned word = a.boards[(size_t)b * 32 + s];
+    const int ctrl = a.control[b];
+    const uint64_t m64 = ok ? a.mask[(size_t)b * 32 + s] : 0;
+    const bool pawn = ((word >> 11) & 1u) == 0 && ((word >> 6) & 7u) == PAWN;
+    // last rank of the side to move: rank 7 (squares 56..63) for white, rank 0 for black
+    const uint64_t pr = pawn ? m64 & (ctrl < 0 ? 0xFFull : 0xFFull << 56) : 0;
+    const int cnt = __popcll(m64) + 3 * __popcll(pr);
+    const int inc = half_scan_add(cnt), before = inc - cnt;
+    const int total0 = __builtin_amdgcn_readlane(inc, 31), total1 = __builtin_amdgcn_readlane(inc, 63);
+    const int total = half ? total1 : total0, most = max(total0, total1);
+    if (most > CAND_CAP) {
+        const int b0 = __builtin_amdgcn_readlane(b, 0), b1 = __builtin_amdgcn_readlane(b, 32);
+        const unsigned long long oks = __ballot(ok);
+        if (oks & 1) expand_many<FP32>(a, b0, lane);
+        if (oks >> 32) expand_many<FP32>(a, b1, lane);
+        return;
+    }
+    const int rounds = (most + 31) >> 5;
+    int16_t* const cc = code_lds[wv][half];
+    float* const add = add_lds[wv][half];
+    const size_t row = (size_t)b * 2048;
+    float l[ROUNDS], e[ROUNDS];
+    int code[ROUNDS];
+    bool has[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        has[r] = 32 * r + s < total;
+        l[r] = -INFINITY;
+        code[r] = 0;
+    }
+    if (__ballot(pr != 0) == 0) {
+        // the slot a candidate belongs to: the last one whose first index is not beyond it
+        unsigned char* const owner = reinterpret_cast<unsigned char*>(owner_lds[wv][half]);
+        owner_lds[wv][half][s] = 0;
+        wave_lds_sync();
+        if (cnt) owner[before] = (unsigned char)s;
+        wave_lds_sync();
+        int carry0 = 0, carry1 = 0;
+        const int mlo = (int)(unsigned)m64, mhi = (int)(unsigned)(m64 >> 32);
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++)
+            if (r < rounds) {
+                const int own = max(half_scan_max(owner[32 * r + s]), half ? carry1 : carry0);
+                carry0 = __builtin_amdgcn_readlane(own, 31);
+                carry1 = __builtin_amdgcn_readlane(own, 63);
+                const int src = 4 * (32 * half + own);
+                const int k = 32 * r + s - __builtin_amdgcn_ds_bpermute(src, before);
+                const unsigned lo = (unsigned)__builtin_amdgcn_ds_bpermute(src, mlo), hi = (unsigned)__builtin_amdgcn_ds_bpermute(src, mhi);
+                if (has[r]) {
+                    code[r] = own * 64 + kth_bit(lo, hi, k);
+                    l[r] = logit<FP32>(a.policy, row + code[r]);
+                }
+            }
+    } else {
+        float lp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (pr) promotion_logs<FP32>(a.promo, (size_t)b * 32 + s, lp);
+        int i = before;
+        for (uint64_t m = m64; m; m &= m - 1) {
+            const int sq = __builtin_ctzll(m), mv = s * 64 + sq;
+            if ((pr >> sq) & 1) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    cc[i + k] = (int16_t)(mv | (k << PROMO_SHIFT));
+                    add[i + k] = lp[k];
+                }
+                i += 4;
+            } else {
+                cc[i] = (int16_t)mv;
+                add[i++] = 0.0f;
+            }
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++)
+            if (has[r]) {
+                code[r] = cc[32 * r + s];
+                l[r] = logit<FP32>(a.policy, row + (code[r] & 2047)) + add[32 * r + s];
+            }
+        wave_lds_sync();
+    }
+    float mx = l[0];
+#pragma unroll
+    for (int r = 1; r < ROUNDS; r++) mx = fmaxf(mx, l[r]);
+    mx = half_max(mx);
+    float sa = 0.0f;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        e[r] = 0.0f;
+        if (r < rounds) e[r] = has[r] ? __expf(l[r] - mx) : 0.0f;
+        sa += e[r];
+    }
+    const float s_all = half_sum(sa);
+    const bool trunc = total > a.E;
+    int n_edges = total;
+    float s_keep = s_all;
+    int pos[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) pos[r] = 32 * r + s;
+    if (most > a.E) {
+        // T = ordered pattern of the E-th largest log-prior of each half (0: everything is kept)
+        unsigned o[ROUNDS];
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) o[r] = has[r] ? ordered(l[r]) : 0u;
+        // -- or any pattern that exactly E of its candidates reach, which ends the search for that half early
+        unsigned T0 = 0, T1 = 0;
+        bool found0 = total0 <= a.E, found1 = total1 <= a.E;
+#pragma clang loop unroll(disable)
+        for (int bit = 31; bit >= 0 && !(found0 && found1); bit--) {
+            const unsigned cand = (half ? T1 : T0) | (1u << bit);
+            int c0 = 0, c1 = 0;
+#pragma unroll
+            for (int r = 0; r < ROUNDS; r++)
+                if (r < rounds) {
+                    const unsigned long long v = __ballot(o[r] >= cand);
+                    c0 += __popc((unsigned)v);
+                    c1 += __popc((unsigned)(v >> 32));
+                }
+            if (!found0 && c0 >= a.E) T0 |= 1u << bit;
+            if (!found1 && c1 >= a.E) T1 |= 1u << bit;
+            found0 |= c0 == a.E;
+            found1 |= c1 == a.E;
+        }
+        const unsigned T = half ? T1 : T0;
+        int gt = 0;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            const unsigned long long v = __ballot(o[r] > T);
+            gt += __popc(half ? (unsigned)(v >> 32) : (unsigned)v);
+        }
+        const int need = a.E - gt;
+        int ties = 0, kept = 0;
+        float sk = 0.0f;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            const bool eq = has[r] && o[r] == T;
+            const unsigned long long eqb = __ballot(eq);
+            has[r] = has[r] && (o[r] > T || (eq && ties + half_below(eqb, half) < need));
+            ties += __popc(half ? (unsigned)(eqb >> 32) : (unsigned)eqb);
+            const unsigned long long kb = __ballot(has[r]);
+            pos[r] = kept + half_below(kb, half);
+            kept += __popc(half ? (unsigned)(kb >> 32) : (unsigned)kb);
+            sk += has[r] ? e[r] : 0.0f;
+        }
+        n_edges = kept;
+        s_keep = half_sum(sk);
+    }
+    const float inv = 1.0f / s_keep;
+    int16_t* const em = a.edge_move + (size_t)b * a.E;
+    _Float16* const ep = a.edge_prior + (size_t)b * a.E;
+    if (a.whole_rows) {
+        // rows of whole 16-byte pieces: put together in LDS, unused slots (no edge) included
+        _Float16* const pp = prior_lds[wv][half];
+        typedef int v4i __attribute__((ext_vector_type(4)));
+        if (s < CAND_CAP / 8) {
+            reinterpret_cast<v4i*>(cc)[s] = v4i{0, 0, 0, 0};
+            reinterpret_cast<v4i*>(pp)[s] = v4i{0, 0, 0, 0};
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++)
+            if (r < rounds && has[r]) {
+                cc[pos[r]] = (int16_t)code[r];
+                pp[pos[r]] = (_Float16)(e[r] * inv);
+            }
+        wave_lds_sync();
+        if (ok && s < a.E / 8) {
+            reinterpret_cast<v4i*>(em)[s] = reinterpret_cast<const v4i*>(cc)[s];
+            reinterpret_cast<v4i*>(ep)[s] = reinterpret_cast<const v4i*>(pp)[s];
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++)
+            if (has[r]) {
+                em[pos[r]] = (int16_t)code[r];
+                ep[pos[r]] = (_Float16)(e[r] * inv);
+            }
+        if (ok)
+            for (int i = n_edges + s; i < a.E; i += 32) {
+                em[i] = 0;
+                ep[i] = (_Float16)0.0f;
+            }
+    }
+    if (ok && s == 0) write_counts(a, b, n_edges, total, trunc, s_all, s_keep);
 }
 
 }  // namespace
@@ -413,7 +548,8 @@ extern "C" int bf_expand(const bf_expand_args* a, void* stream) {
     k.edge_move = a->edge_move; k.edge_prior = reinterpret_cast<_Float16*>(a->edge_prior);
     k.n_edges = a->n_edges; k.count = a->count; k.dropped = a->dropped;
     k.node_value = reinterpret_cast<_Float16*>(a->node_value);
-    const dim3 grid((k.n + EXPAND_WAVES - 1) / EXPAND_WAVES), block(64 * EXPAND_WAVES);
+    k.whole_rows = k.E % 8 == 0 && k.E <= CAND_CAP && (((uintptr_t)k.edge_move | (uintptr_t)k.edge_prior) & 15) == 0;
+    const dim3 grid((k.n + 2 * EXPAND_WAVES - 1) / (2 * EXPAND_WAVES)), block(64 * EXPAND_WAVES);
     if (k.logits_fp32) hipLaunchKernelGGL(expand_kernel<true>, grid, block, 0, (hipStream_t)stream, k);
     else hipLaunchKernelGGL(expand_kernel<false>, grid, block, 0, (hipStream_t)stream, k);
     const hipError_t e = hipGetLastError();

@@ -1,0 +1,49 @@
+"""Edge rows in their different forms (whole 16-byte pieces, odd lengths, longer than the LDS row) and the
+leaf compaction at the edges of its workgroups."""
+import pytest
+import torch
+
+from brokefish_amd import positions
+from brokefish_amd.hip_impl import compact_leaves, expand_edges
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 515])
+@pytest.mark.parametrize("edges", [1, 8, 31, 32, 95, 128, 136, 255])
+def test_edge_rows_do_not_depend_on_their_form(n, edges):
+    b, c, r, m = (t.cuda() for t in positions.random_positions(n, plies=150, seed=n, stamp_queen=True))
+    g = torch.Generator(device="cuda").manual_seed(n)
+    logits = [torch.randn(n, 32, k, generator=g, device="cuda").half() for k in (64, 4)]
+    value = torch.rand(n, generator=g, device="cuda")
+    got = expand_edges(*logits, value, m, b, c, edges)
+    full = expand_edges(*logits, value, m, b, c, 254)            # nothing truncated, rows stored edge by edge
+    assert torch.equal(got["count"], full["count"]) and torch.equal(got["n_edges"], full["count"].clamp(max=edges))
+    assert torch.equal(got["node_value"], full["node_value"])
+    logp = full["edge_prior"].float()
+    for i in range(min(n, 64)):
+        k = int(full["count"][i])
+        mine, prior = got["edge_move"][i].tolist(), got["edge_prior"][i].float()
+        if k <= edges:
+            assert mine[:k] == full["edge_move"][i, :k].tolist() and torch.equal(got["edge_prior"][i, :k], full["edge_prior"][i, :k])
+            assert float(got["dropped"][i]) == 0.0 and not any(mine[k:]) and not prior[k:].any()
+        else:
+            at = [full["edge_move"][i, :k].tolist().index(x) for x in mine]
+            assert at == sorted(at)                              # survivors in canonical order
+            cut = logp[i, :k].sort(descending=True).values[edges - 1]
+            assert float(logp[i, at].min()) >= float(cut) * (1 - 2e-3)
+            assert abs(float(prior.sum()) - 1) < 5e-3
+            assert abs(float(got["dropped"][i]) - (1 - float(logp[i, at].sum()) / float(logp[i, :k].sum()))) < 5e-3
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 16383, 16384, 16385, 49999])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_compaction_at_the_edges_of_its_workgroups(n, shift):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    for share in (0.0, 0.4, 1.0):
+        raw = torch.randint(1, 256, (n + shift,), generator=g, device="cuda").to(torch.uint8)
+        raw[torch.rand(n + shift, generator=g, device="cuda") >= share] = 0
+        flags = raw[shift:]                                      # shift 1: not aligned to sixteen bytes
+        index, count = compact_leaves(flags)
+        want = flags.nonzero().flatten().int()
+        assert int(count) == want.numel() and torch.equal(index[:want.numel()], want) and not index[want.numel():].any()
