@@ -99,6 +99,10 @@ constexpr int N_PHASES = 12;
 // phase slots of the optional cycle profile
 enum { PH_EMBED, PH_LN1, PH_QKV, PH_ATTN, PH_OUT, PH_LN2, PH_FF1, PH_FF2, PH_HEADS, PH_STORE, PH_SYNC, PH_TOTAL };
 
+// What a kernel is compiled for: evaluation; the debug taps; the encoder stack alone (residual stream in and
+// out through the tap table, no board words, no heads, nothing else tapped)
+enum { MODE_EVAL = 0, MODE_TAPS = 1, MODE_ENC = 2 };
+
 struct KArgs {
     const uint16_t* boards;
     const int16_t* control;
@@ -159,6 +163,12 @@ hipError_t launch_duo256(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_taps(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_fp8(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_fp8_taps(const KArgs& k, hipStream_t stream);
+// the encoder-only builds of the kernels AUTO chooses from
+hipError_t launch_duo256_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_solo256_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_twin256_fp8_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_octo256_fp8_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_octo512_enc(const KArgs& k, hipStream_t stream);
 // the builds that carry the phase profile
 hipError_t launch_twin256_prof(const KArgs& k, hipStream_t stream);
 hipError_t launch_octo512_prof(const KArgs& k, hipStream_t stream);

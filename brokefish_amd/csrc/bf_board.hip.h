@@ -228,8 +228,9 @@ constexpr bool block_at_covers_layer() {
     return true;
 }
 
-template <int DM, bool TAPS, bool TWIN, bool FP8, bool OCTO = false, bool PROF = false>
+template <int DM, int MODE, bool TWIN, bool FP8, bool OCTO = false, bool PROF = false>
 __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TWIN_OCC : 1) void board_kernel(const KArgs a) {
+    constexpr bool TAPS = MODE == MODE_TAPS, ENC = MODE == MODE_ENC;
     typedef Cfg<DM, TWIN, OCTO> C;
     typedef typename Acc<FP8>::type acc_t;
     static_assert(!FP8 || DM == 256, "e4m3: one k-chunk per matmul of the width (fp32 sums over the chunks of ffn2 only)");
@@ -513,16 +514,16 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
     // An encoder-only launch (tap table with `alive`): the residual stream comes in through x_in, the
     // token mask through `alive`, the stream after the last layer goes out through resid_last, and
     // there are no board words and no heads.
-    const bool enc_only = TAPS && a.taps.alive != nullptr;
+    const bool enc_only = ENC || (TAPS && a.taps.alive != nullptr);
     const unsigned word = enc_only ? (a.taps.alive[(size_t)b * T + t] ? 0u : 0x800u) : a.boards[(size_t)b * T + t];
     const int ctrl = enc_only ? 1 : a.control[b];
     const unsigned alive = (unsigned)__ballot(((word >> 11) & 1) == 0 && g == 0);
-    if (TAPS && a.taps.x_in) {
+    if (ENC || (TAPS && a.taps.x_in)) {
 #pragma unroll
         for (int i = 0; i < TWW; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const v4f v = ldg4(a.taps.x_in + ((size_t)b * T + t) * D + 32 * (TW * q + t0 + i) + 8 * j + 4 * g);
+                const v4f v = stream_in(a.taps, ((size_t)b * T + t) * D + 32 * (TW * q + t0 + i) + 8 * j + 4 * g);
 #pragma unroll
                 for (int k = 0; k < 4; k++) x[i][4 * j + k] = v[k];
             }
@@ -1116,6 +1117,15 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
                 for (int r = 0; r < 16; r++)
                     a.taps.resid[(bl * T + t) * D + 32 * (TW * q + t0 + i) + ch(r, g)] = x[i][r];
     }
+    if constexpr (ENC) {
+#pragma unroll
+        for (int i = 0; i < TWW; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                stream_out(a.taps, ((size_t)b * T + t) * D + 32 * (TW * q + t0 + i) + 8 * j + 4 * g,
+                           v4f{x[i][4 * j], x[i][4 * j + 1], x[i][4 * j + 2], x[i][4 * j + 3]});
+        return;
+    }
     if (TAPS && a.taps.resid_last)
 #pragma unroll
         for (int i = 0; i < TWW; i++)
@@ -1334,7 +1344,7 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
 #undef BF_PHASE
 }
 
-template <int DM, bool TAPS, bool TWIN, bool FP8 = false, bool OCTO = false, bool PROF = false>
+template <int DM, int MODE, bool TWIN, bool FP8 = false, bool OCTO = false, bool PROF = false>
 hipError_t launch_board(const KArgs& k, hipStream_t stream) {
     // more than 64 KiB of dynamic LDS has to be requested once per kernel and device (one bit
     // per device ordinal; a device beyond the mask asks every time)
@@ -1344,12 +1354,12 @@ hipError_t launch_board(const KArgs& k, hipStream_t stream) {
     if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
     const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
     if (!(lds_set.load(std::memory_order_relaxed) & bit)) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&board_kernel<DM, TAPS, TWIN, FP8, OCTO, PROF>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&board_kernel<DM, MODE, TWIN, FP8, OCTO, PROF>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (e != hipSuccess) return e;
         lds_set.fetch_or(bit, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((board_kernel<DM, TAPS, TWIN, FP8, OCTO, PROF>), dim3(k.n), dim3(OCTO ? 2 * THREADS : THREADS), lds_bytes, stream, k);
+    hipLaunchKernelGGL((board_kernel<DM, MODE, TWIN, FP8, OCTO, PROF>), dim3(k.n), dim3(OCTO ? 2 * THREADS : THREADS), lds_bytes, stream, k);
     return hipGetLastError();
 }
 

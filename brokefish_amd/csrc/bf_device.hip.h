@@ -84,6 +84,19 @@ __device__ __forceinline__ void load_tile16i(const float* p, int g, v4i (&b)[4])
     for (int j = 0; j < 4; j++) b[j] = ldg4i(p + 8 * j + 4 * g);
 }
 
+// four floats of the residual stream an encoder-only launch takes in and gives back: fp32, or fp16 converted on
+// the way (a caller in half precision needs no pass of its own before and after)
+__device__ __forceinline__ v4f stream_in(const bf_taps& t, size_t at) {
+    if (!t.x_in_h) return ldg4(t.x_in + at);
+    const v4h h = *reinterpret_cast<const v4h*>(static_cast<const _Float16*>(t.x_in_h) + at);
+    return v4f{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
+}
+__device__ __forceinline__ void stream_out(const bf_taps& t, size_t at, const v4f& v) {
+    if (t.resid_last_h)
+        *reinterpret_cast<v4h*>(static_cast<_Float16*>(t.resid_last_h) + at) = v4h{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+    else *reinterpret_cast<v4f*>(t.resid_last + at) = v;
+}
+
 // Eight e4m3 bytes (byte j of `bytes` = this lane's k index j) as eight fp16 values.  Exact:
 // every e4m3 value, subnormals included, is an fp16 value.
 __device__ __forceinline__ v8h e4m3x8_as_f16(long bytes) {

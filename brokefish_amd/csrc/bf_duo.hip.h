@@ -77,8 +77,9 @@ __device__ __forceinline__ v16f f16_step(const v8h& w, const v8h& act, const v16
 template <bool SWAP>
 __device__ __forceinline__ v16i f16_step(const v8h&, const v8h&, const v16i& acc) { return acc; }
 
-template <bool TAPS, bool FP8, bool PROF = false, int NPOS = 2>
+template <int MODE, bool FP8, bool PROF = false, int NPOS = 2>
 __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
+    constexpr bool TAPS = MODE == MODE_TAPS, ENC = MODE == MODE_ENC;
     typedef Cfg<FP8, NPOS> C;
     static_assert(NPOS == 2 || (NPOS == 1 && !FP8), "one position per workgroup: the int8 format");
     typedef typename Acc<FP8>::type acc_t;
@@ -349,7 +350,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     // An encoder-only launch (tap table with `alive`): the residual stream comes in through x_in, the
     // token mask through `alive`, the stream after the last layer goes out through resid_last, and
     // there are no board words and no heads.
-    const bool enc_only = TAPS && a.taps.alive != nullptr;
+    const bool enc_only = ENC || (TAPS && a.taps.alive != nullptr);
     // ---- embedding (this wave's tile, both positions) ----------------------------------------------
     float x[NP][16];
     unsigned alive[NP];
@@ -360,10 +361,10 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         const unsigned word = enc_only ? (a.taps.alive[(size_t)b * T + t] ? 0u : 0x800u) : a.boards[(size_t)b * T + t];
         ctrl[p] = enc_only ? 1 : a.control[b];
         alive[p] = (unsigned)__ballot(((word >> 11) & 1) == 0 && g == 0);
-        if (TAPS && a.taps.x_in) {
+        if (ENC || (TAPS && a.taps.x_in)) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const v4f v = ldg4(a.taps.x_in + ((size_t)b * T + t) * D + 32 * tile + 8 * j + 4 * g);
+                const v4f v = stream_in(a.taps, ((size_t)b * T + t) * D + 32 * tile + 8 * j + 4 * g);
 #pragma unroll
                 for (int k = 0; k < 4; k++) x[p][4 * j + k] = v[k];
             }
@@ -818,6 +819,16 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                     for (int r = 0; r < 16; r++)
                         a.taps.resid[(bl[p] * T + t) * D + 32 * tile + ch(r, g)] = x[p][r];
     }
+    if constexpr (ENC) {
+#pragma unroll
+        for (int p = 0; p < NP; p++)
+            if (live[p])
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    stream_out(a.taps, ((size_t)bp[p] * T + t) * D + 32 * tile + 8 * j + 4 * g,
+                               v4f{x[p][4 * j], x[p][4 * j + 1], x[p][4 * j + 2], x[p][4 * j + 3]});
+        return;
+    }
     if (TAPS && a.taps.resid_last)
 #pragma unroll
         for (int p = 0; p < NP; p++)
@@ -1016,7 +1027,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #undef BF_PHASE
 }
 
-template <bool TAPS, bool FP8 = false, bool PROF = false, int NPOS = 2>
+template <int MODE, bool FP8 = false, bool PROF = false, int NPOS = 2>
 hipError_t launch_duo(const KArgs& k, hipStream_t stream) {
     // more than 64 KiB of dynamic LDS has to be requested once per kernel and device
     static std::atomic<unsigned long long> lds_set{0};
@@ -1025,12 +1036,12 @@ hipError_t launch_duo(const KArgs& k, hipStream_t stream) {
     if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
     const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
     if (!(lds_set.load(std::memory_order_relaxed) & bit)) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_kernel<TAPS, FP8, PROF, NPOS>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_kernel<MODE, FP8, PROF, NPOS>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (e != hipSuccess) return e;
         lds_set.fetch_or(bit, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((duo_kernel<TAPS, FP8, PROF, NPOS>), dim3((k.n + NPOS - 1) / NPOS), dim3(512), lds_bytes, stream, k);
+    hipLaunchKernelGGL((duo_kernel<MODE, FP8, PROF, NPOS>), dim3((k.n + NPOS - 1) / NPOS), dim3(512), lds_bytes, stream, k);
     return hipGetLastError();
 }
 

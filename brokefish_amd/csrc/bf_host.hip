@@ -145,6 +145,17 @@ static int choose_kernel(const bf_eval_args* a) {
 
 extern "C" int bf_kernel_choice(const bf_eval_args* args) { return choose_kernel(args); }
 
+// Whether the encoder-only build of kernel `kind` serves this launch: nothing but the stream is tapped, and the
+// kernel is one of those AUTO chooses from (the others run their taps build, whose every phase tests for taps).
+static bool enc_build(const bf_eval_args* a, int kind) {
+    const bf_taps* t = a->taps;
+    if (!t || !t->alive || t->embed || t->qa_qkv || t->acc_qkv || t->qa_out || t->acc_out || t->qa_ff1 || t->acc_ff1 || t->qa_ff2 ||
+        t->acc_ff2 || t->resid || t->normed)
+        return false;
+    if (a->shape.d_model == 512) return kind == BF_KERNEL_OCTO;
+    return a->quant == BF_QUANT_INT8 ? kind == BF_KERNEL_OCTO || kind == BF_KERNEL_DUO : kind == BF_KERNEL_OCTO || kind == BF_KERNEL_TWIN;
+}
+
 static int check_args(const bf_eval_args* a, bf::KArgs* k, int* kind) {
     *kind = choose_kernel(a);
     if (*kind < 0) return *kind;
@@ -152,10 +163,13 @@ static int check_args(const bf_eval_args* a, bf::KArgs* k, int* kind) {
     if (a->n < 1 || a->n > (1ll << 28)) return fail(BF_ERR_ARGUMENT, "n must be in [1, 2^28]");
     // encoder-only launch: residual stream in and out through the tap table, no board words, no heads
     const bool enc_only = a->taps && a->taps->alive;
+    if (a->taps && (a->taps->x_in_h || a->taps->resid_last_h) && !enc_build(a, *kind))
+        return fail(BF_ERR_UNSUPPORTED, "x_in_h / resid_last_h: encoder-only launches of the kernel AUTO chooses, without other taps");
     if (enc_only) {
-        if (!a->taps->x_in || !a->taps->resid_last)
+        if (!(a->taps->x_in || a->taps->x_in_h) || !(a->taps->resid_last || a->taps->resid_last_h))
             return fail(BF_ERR_ARGUMENT, "an encoder-only launch (taps.alive) needs taps.x_in and taps.resid_last");
-        if ((uintptr_t)a->taps->resid_last & 15) return fail(BF_ERR_ARGUMENT, "resid_last must be 16-byte aligned");
+        if (((uintptr_t)a->taps->resid_last & 15) || (((uintptr_t)a->taps->x_in_h | (uintptr_t)a->taps->resid_last_h) & 7))
+            return fail(BF_ERR_ARGUMENT, "resid_last must be 16-byte aligned, x_in_h and resid_last_h 8-byte aligned");
         if (a->leaf_index || a->leaf_count || a->active)
             return fail(BF_ERR_ARGUMENT, "an encoder-only launch takes neither active flags nor a leaf list");
     } else {
@@ -240,6 +254,15 @@ static bf::KArgs slice(const bf::KArgs& k, int first, int count) {
     bf::KArgs s = k;
     const size_t f = (size_t)first, logit = k.out_fp32 ? 4 : 2;
     s.n = count;
+    if (k.taps.alive) {   // encoder-only: the stream and the token mask are the arrays
+        const size_t at = f * BF_TOKENS * bf::D;
+        s.taps.alive += f * BF_TOKENS;
+        if (s.taps.x_in) s.taps.x_in += at;
+        if (s.taps.resid_last) s.taps.resid_last += at;
+        if (s.taps.x_in_h) s.taps.x_in_h = static_cast<const uint16_t*>(s.taps.x_in_h) + at;
+        if (s.taps.resid_last_h) s.taps.resid_last_h = static_cast<uint16_t*>(s.taps.resid_last_h) + at;
+        return s;
+    }
     s.boards += f * BF_TOKENS;
     s.control += f;
     s.rep += f;
@@ -256,23 +279,28 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
     const int grid = (k.n + bf::WAVES - 1) / bf::WAVES;
     hipError_t e;
     if (!bf::device_is_gfx950()) return BF_ERR_DEVICE;
+    const bool enc = !k.profile && enc_build(a, kind);
     // The two-position kernel runs in rounds of 512 positions (256 compute units x 2), and a round
     // costs the same whether it is full or not.  When the library chose the kernel itself and the
     // last round would hold at most 256 positions, those go to the one-position form in a second
     // launch on the same stream, whose single round is a third shorter (640 positions: 0.33 ms
     // instead of 0.39).  Not with a leaf list (its length is on the device), taps or the profile.
-    if (kind == BF_KERNEL_DUO && a->kernel == BF_KERNEL_AUTO && a->quant == BF_QUANT_INT8 && !a->taps && !k.profile &&
+    if (kind == BF_KERNEL_DUO && a->kernel == BF_KERNEL_AUTO && a->quant == BF_QUANT_INT8 && (!a->taps || enc) && !k.profile &&
         !k.leaf_index && k.n > DUO_ROUND && k.n % DUO_ROUND != 0 && k.n % DUO_ROUND <= DUO_ROUND / 2) {
         const int head = k.n - k.n % DUO_ROUND;
-        e = bf::launch_duo256(slice(k, 0, head), stream);
-        if (e == hipSuccess) e = bf::launch_solo256(slice(k, head, k.n - head), stream);
+        e = (enc ? bf::launch_duo256_enc : bf::launch_duo256)(slice(k, 0, head), stream);
+        if (e == hipSuccess) e = (enc ? bf::launch_solo256_enc : bf::launch_solo256)(slice(k, head, k.n - head), stream);
         if (e != hipSuccess) {
             snprintf(g_err, sizeof(g_err), "kernel launch failed: %s", hipGetErrorString(e));
             return BF_ERR_LAUNCH;
         }
         return BF_OK;
     }
-    if (kind == BF_KERNEL_OCTO) {
+    if (enc) {
+        if (a->shape.d_model == 512) e = bf::launch_octo512_enc(k, stream);
+        else if (a->quant == BF_QUANT_E4M3) e = (kind == BF_KERNEL_OCTO ? bf::launch_octo256_fp8_enc : bf::launch_twin256_fp8_enc)(k, stream);
+        else e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_enc : bf::launch_duo256_enc)(k, stream);
+    } else if (kind == BF_KERNEL_OCTO) {
         // eight wavefronts per position: the 512-wide network and the e4m3 format on the board kernel's
         // eight-wavefront form; the 256-wide int8 network on the two-position kernel's one-position
         // form, which issues each product under the previous one's epilogue

@@ -46,12 +46,12 @@ _TAP_PTRS = ["embed", "qa_qkv", "acc_qkv", "qa_out", "acc_out", "qa_ff1", "acc_f
              "qa_ff2", "acc_ff2", "resid", "normed", "resid_last"]
 
 
-ABI_VERSION = 6     # BF_ABI_VERSION of include/brokefish_hip.h that the structs below mirror
+ABI_VERSION = 7     # BF_ABI_VERSION of include/brokefish_hip.h that the structs below mirror
 
 
 class _Taps(C.Structure):
     _fields_ = ([("x_in", C.c_void_p), ("layer_begin", C.c_int32), ("layer_end", C.c_int32)]
-                + [(n, C.c_void_p) for n in _TAP_PTRS] + [("alive", C.c_void_p)])
+                + [(n, C.c_void_p) for n in _TAP_PTRS] + [("alive", C.c_void_p), ("x_in_h", C.c_void_p), ("resid_last_h", C.c_void_p)])
 
 
 class _ExpandArgs(C.Structure):
@@ -918,32 +918,38 @@ class FusedEncoder:
             raise ValueError(f"out must be {tuple(x.shape)} on {x.device}")
         # An encoder-only launch (reference csrc/encoder.cu:1752-1764): the residual stream goes in
         # and comes out through the tap table, the token mask replaces the board words, no heads
-        # run.  What is needed beyond x, alive and out is kept between calls, so a repeated call
-        # with out= given (fp32, contiguous) allocates nothing.
+        # run.  The kernels kernel="auto" chooses from take and return fp16 as well as fp32; for the
+        # others and for other types the conversion is a pass of its own, over buffers that are kept
+        # between calls.  A repeated call with out= given (contiguous, of a type the kernel
+        # writes) allocates nothing.
         bb = self._backbone
         if bb is None or bb["cap"] < n:
             bb = self._backbone = {"cap": n, "ones": torch.ones(n, T, dtype=torch.int8, device=self.device),
                                    "x": None, "y": None}
         alive8 = bb["ones"][:n] if alive is None else alive.contiguous()      # bool or int8: one byte, non-zero = live
-        if x.dtype is torch.float32 and x.is_contiguous():
-            x32 = x
+        native = (torch.float32, torch.float16) if self.kernel == "auto" else (torch.float32,)
+        if x.dtype in native and x.is_contiguous() and x.data_ptr() % 16 == 0:
+            xk = x
         else:
             if bb["x"] is None or bb["x"].shape[0] < n:
                 bb["x"] = torch.empty(bb["cap"], T, d, dtype=torch.float32, device=self.device)
-            x32 = bb["x"][:n]
-            x32.copy_(x)
-        direct = out is not None and out.dtype is torch.float32 and out.is_contiguous()
-        if direct:
-            y32 = out
+            xk = bb["x"][:n]
+            xk.copy_(x)
+        if out is None and x.dtype in native:
+            yk = result = torch.empty(n, T, d, dtype=x.dtype, device=x.device)
+        elif out is not None and out.dtype in native and out.is_contiguous() and out.data_ptr() % 16 == 0:
+            yk = result = out
         else:
             if bb["y"] is None or bb["y"].shape[0] < n:
                 bb["y"] = torch.empty(bb["cap"], T, d, dtype=torch.float32, device=self.device)
-            y32 = bb["y"][:n]
+            yk, result = bb["y"][:n], None
         for name, t_ in (("x", x), ("alive", alive), ("out", out)):
             if t_ is not None and t_.device != self.device:
                 raise ValueError(f"{name} is on {t_.device}, the evaluator's weights are on {self.device}")
         taps = _Taps()
-        taps.x_in, taps.resid_last, taps.alive = x32.data_ptr(), y32.data_ptr(), alive8.data_ptr()
+        taps.alive = alive8.data_ptr()
+        setattr(taps, "x_in" if xk.dtype is torch.float32 else "x_in_h", xk.data_ptr())
+        setattr(taps, "resid_last" if yk.dtype is torch.float32 else "resid_last_h", yk.data_ptr())
         taps.layer_begin, taps.layer_end = 0, self.n_layers
         a = _Args()
         a.n, a.shape = n, self._shape
@@ -958,12 +964,12 @@ class FusedEncoder:
         a.kernel, a.quant, a.value_mode = self.KERNELS[self.kernel], (1 if self.fp8 else 0), self.vmode
         a.taps = C.pointer(taps)      # the library copies the table at launch
         self._call(a)
-        if direct:
-            return out
+        if result is not None:
+            return result
         if out is not None:
-            out.copy_(y32)
+            out.copy_(yk)
             return out
-        return y32.to(x.dtype, copy=True)
+        return yk.to(x.dtype, copy=True)
 
     __call__ = forward
 

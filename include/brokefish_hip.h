@@ -161,6 +161,8 @@ typedef struct {
                          * mask of attention keys comes from here, no board words are read and no
                          * heads run -- boards, control, rep, mask, policy, promo and value of
                          * bf_eval_args are ignored and may be NULL */
+    const void* x_in_h;  /* encoder-only launches of AUTO, with no other tap: the stream in fp16 instead of */
+    void* resid_last_h;  /* x_in, and the result in fp16 instead of resid_last (8-byte aligned)             */
 } bf_taps;
 
 typedef struct {
@@ -232,7 +234,7 @@ typedef struct {
  * BF_ABI_TAG before its first call and refuses a library it was not built for (a shorter
  * bf_eval_args would make the library read pointers from beyond the caller's struct).  No
  * counterpart in the reference, whose module and kernels are one compilation. */
-#define BF_ABI_VERSION 6
+#define BF_ABI_VERSION 7
 #define BF_ABI_TAG (((uint64_t)BF_ABI_VERSION << 32) | (uint64_t)sizeof(bf_eval_args))
 uint64_t bf_abi_tag(void);
 
