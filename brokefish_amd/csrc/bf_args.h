@@ -99,6 +99,12 @@ constexpr int N_PHASES = 12;
 // phase slots of the optional cycle profile
 enum { PH_EMBED, PH_LN1, PH_QKV, PH_ATTN, PH_OUT, PH_LN2, PH_FF1, PH_FF2, PH_HEADS, PH_STORE, PH_SYNC, PH_TOTAL };
 
+// Positions the two-position kernel holds at once on 256 compute units: a round, which costs the same full or not.
+constexpr int DUO_ROUND = 512;
+// How many of cnt positions are left to the one-position form: a last round of at most half the positions, which
+// that form does in two thirds of the time.
+__host__ __device__ constexpr int round_rest(int cnt) { return cnt % DUO_ROUND <= DUO_ROUND / 2 ? cnt % DUO_ROUND : 0; }
+
 // What a kernel is compiled for: evaluation; the debug taps; the encoder stack alone (residual stream in and
 // out through the tap table, no board words, no heads, nothing else tapped)
 enum { MODE_EVAL = 0, MODE_TAPS = 1, MODE_ENC = 2 };
@@ -111,6 +117,10 @@ struct KArgs {
     const uint8_t* active;        // optional [n]: positions with 0 are skipped, their outputs untouched
     const int* leaf_index;        // optional compacted list: slot j of the launch evaluates position leaf_index[j] ...
     const int* leaf_count;        // ... for j < *leaf_count; slots past the count do nothing
+    // A leaf list shared by two launches, the two-position kernel in front and its one-position form behind:
+    // the former takes whole rounds, the latter what round_rest() leaves.
+    int list_split;
+    int grid;                     // workgroups of the one-position form, 0: one per position
     int n;
     const uint8_t* wstream;
     const float* fparams;

@@ -108,12 +108,19 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     int bp[NP];
     bool live[NP];
     {
-        const int cnt = a.leaf_index ? *a.leaf_count : a.n;
+        int cnt = a.n, first = NP * (int)blockIdx.x;
+        if (a.leaf_index) {
+            cnt = *a.leaf_count;
+            if (a.list_split) {
+                if (NP == 1) first += cnt - round_rest(cnt);
+                else cnt -= round_rest(cnt);
+            }
+        }
         bool any = false;
         int some = 0;
 #pragma unroll
         for (int p = 0; p < NP; p++) {
-            const int j = NP * (int)blockIdx.x + p;
+            const int j = first + p;
             int b = j;
             bool ok = j < cnt;
             if (a.leaf_index) {
@@ -1041,7 +1048,7 @@ hipError_t launch_duo(const KArgs& k, hipStream_t stream) {
         if (e != hipSuccess) return e;
         lds_set.fetch_or(bit, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((duo_kernel<MODE, FP8, PROF, NPOS>), dim3((k.n + NPOS - 1) / NPOS), dim3(512), lds_bytes, stream, k);
+    hipLaunchKernelGGL((duo_kernel<MODE, FP8, PROF, NPOS>), dim3(k.grid ? k.grid : (k.n + NPOS - 1) / NPOS), dim3(512), lds_bytes, stream, k);
     return hipGetLastError();
 }
 

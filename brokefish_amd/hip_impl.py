@@ -776,6 +776,8 @@ class FusedEncoder:
             self.board_wstream, self.board_fparams = pack_board_on_device(net, net.encoder if net is not None else source,
                                                                           self._shape, self.fp8, self.device)
         self._buffered_full = 0
+        # launches of more positions than this run the two-position kernel (int8, kernel="auto", 256 wide)
+        self._pair_above = int(self._lib.bf_board_max_n()) if kernel == "auto" and self.int8 and not wide else 1 << 62
         self._backbone = None
         self._profile, self._profile_waves, self._profile_kept = None, 0, None
         self.best_move = None
@@ -804,6 +806,9 @@ class FusedEncoder:
             self.promo_out = torch.empty(n, T, N_PROMO, device=self.device, dtype=self.out_dtype)
             self.value_out = torch.empty(n, device=self.device, dtype=torch.float32)
             self.best_out = torch.empty(n, device=self.device, dtype=torch.int32)
+            if n > self._pair_above:      # the list that active flags are compacted into
+                self._leaf_list = (torch.empty(n, device=self.device, dtype=torch.int32),
+                                   torch.empty(1, device=self.device, dtype=torch.int32))
             nbytes = self._lib.bf_workspace_bytes(C.byref(self._shape), n) if self.wstream is not None else 0
             self.workspace = torch.empty(nbytes, device=self.device, dtype=torch.uint8)
             self._buffered_full = n
@@ -997,6 +1002,11 @@ class FusedEncoder:
             if active is not None:
                 raise ValueError("a compacted leaf list replaces the active flags: pass one of them")
             leaves = _check_leaves(leaves, n, self.device)
+        elif active is not None and n > self._pair_above and self._profile is None and active.device == self.device:
+            # the two-position kernel pairs neighbours, so scattered flags would leave half-empty pairs in
+            # every round: compacted (3 to 5 us), 1000 flags of which a third are set take one round
+            # instead of two
+            leaves, active = compact_leaves(active, out=self._leaf_list), None
         if self._profile is not None:
             # set_profile(True): the launch goes through the phase-accounting build, which adds
             # into the counters that read_profile returns
