@@ -132,6 +132,7 @@ struct KArgs {
     int vmode;                    // value head: 0 king row, 1 pooled (mean of the normalised live tokens), 2 prenorm
     float eps;
     float* xpark;                 // workspace: 32 KiB per board slot, residual stream parked during the FFN
+    uint8_t* team_ws;             // exchange buffers of the team form (several workgroups per position)
     unsigned long long* profile;  // [N_PHASES] cycle sums over waves, profile builds only
     bf_taps taps;
 };
@@ -195,5 +196,15 @@ hipError_t launch_prof_fp8(const KArgs& k, int grid, hipStream_t stream);
 hipError_t launch_solo256(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_taps(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_prof(const KArgs& k, hipStream_t stream);
+// several workgroups per position: launches of at most team_positions() positions (0: not on this device; `look`
+// allows the one look at the device, which synchronises), with team_slot_bytes() of workspace for each
+hipError_t launch_team256(const KArgs& k, hipStream_t stream);
+hipError_t launch_team256_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_team256_fp8(const KArgs& k, hipStream_t stream);
+hipError_t launch_team256_fp8_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_team512(const KArgs& k, hipStream_t stream);
+hipError_t launch_team512_enc(const KArgs& k, hipStream_t stream);
+size_t team_slot_bytes(int d_model);
+int team_positions(int d_model, bool look);
 
 }  // namespace bf

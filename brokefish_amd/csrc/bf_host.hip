@@ -80,6 +80,11 @@ extern "C" size_t bf_workspace_bytes(const bf_shape* s, int64_t n) {
     return slots * bf::T * bf::D * sizeof(float);
 }
 
+extern "C" size_t bf_team_workspace_bytes(const bf_shape* s) {
+    if (!board_shape_ok(s)) return 0;
+    return bf::team_positions(s->d_model, true) * bf::team_slot_bytes(s->d_model);
+}
+
 extern "C" size_t bf_layer_stride_floats(const bf_shape* s) {
     if (!shape_ok(s)) return 0;
     return bf::PARAM_FLOATS;
@@ -191,6 +196,7 @@ static int check_args(const bf_eval_args* a, bf::KArgs* k, int* kind) {
     if (a->leaf_index && a->active) return fail(BF_ERR_ARGUMENT, "a compacted leaf list replaces the active flags: pass one of them");
     if (((uintptr_t)a->leaf_index & 3) || ((uintptr_t)a->leaf_count & 3))
         return fail(BF_ERR_ARGUMENT, "leaf_index / leaf_count must be 4-byte aligned");
+    if ((uintptr_t)a->team_workspace & 255) return fail(BF_ERR_ARGUMENT, "team_workspace must be 256-byte aligned");
     if (a->value_mode < BF_VALUE_KING || a->value_mode > BF_VALUE_PRENORM)
         return fail(BF_ERR_ARGUMENT, "value_mode must be BF_VALUE_KING, BF_VALUE_POOLED or BF_VALUE_PRENORM");
     if (a->value_mode != BF_VALUE_KING && !board)
@@ -205,6 +211,7 @@ static int check_args(const bf_eval_args* a, bf::KArgs* k, int* kind) {
     k->policy = a->policy; k->promo = a->promo; k->value = a->value; k->best = a->best_move;
     k->out_fp32 = a->out_fp32 ? 1 : 0;
     k->xpark = static_cast<float*>(a->workspace);
+    k->team_ws = static_cast<uint8_t*>(a->team_workspace);
     k->n_layers = a->shape.n_layers; k->n_value = a->shape.n_value; k->eps = a->shape.eps;
     k->vmode = a->value_mode;
     k->l0 = 0; k->l1 = a->shape.n_layers;
@@ -248,12 +255,12 @@ bool bf::device_is_gfx950() {
 }
 
 // the arguments of a launch over positions [first, first + count) of the caller's arrays
-static bf::KArgs slice(const bf::KArgs& k, int first, int count) {
+static bf::KArgs slice(const bf::KArgs& k, int d_model, int first, int count) {
     bf::KArgs s = k;
     const size_t f = (size_t)first, logit = k.out_fp32 ? 4 : 2;
     s.n = count;
     if (k.taps.alive) {   // encoder-only: the stream and the token mask are the arrays
-        const size_t at = f * BF_TOKENS * bf::D;
+        const size_t at = f * BF_TOKENS * d_model;
         s.taps.alive += f * BF_TOKENS;
         if (s.taps.x_in) s.taps.x_in += at;
         if (s.taps.resid_last) s.taps.resid_last += at;
@@ -273,11 +280,43 @@ static bf::KArgs slice(const bf::KArgs& k, int first, int count) {
     return s;
 }
 
+// Positions a team launch of this call may hold: 0 unless AUTO chose, a workspace came along and nothing but the
+// stream is tapped.
+static int team_limit(const bf_eval_args* a, const bf::KArgs& k, bool enc) {
+    if (a->kernel != BF_KERNEL_AUTO || !k.team_ws || k.profile || (a->taps && !enc)) return 0;
+    const size_t fits = a->team_workspace_bytes / bf::team_slot_bytes(a->shape.d_model);
+    const int most = bf::team_positions(a->shape.d_model, false);
+    return fits < (size_t)most ? (int)fits : most;
+}
+
+static hipError_t launch_team(const bf_eval_args* a, const bf::KArgs& k, bool enc, hipStream_t stream) {
+    if (a->shape.d_model == 512) return (enc ? bf::launch_team512_enc : bf::launch_team512)(k, stream);
+    if (a->quant == BF_QUANT_E4M3) return (enc ? bf::launch_team256_fp8_enc : bf::launch_team256_fp8)(k, stream);
+    return (enc ? bf::launch_team256_enc : bf::launch_team256)(k, stream);
+}
+
 static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream_t stream) {
     const int grid = (k.n + bf::WAVES - 1) / bf::WAVES;
     hipError_t e;
     if (!bf::device_is_gfx950()) return BF_ERR_DEVICE;
     const bool enc = !k.profile && enc_build(a, kind);
+    // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
+    // position 124 -> 90 us, e4m3 155 -> 106; 512 wide 750 -> 346 us), and so does what is left of the 512-wide
+    // network's rounds of 256 positions if it is no more.
+    const int team = team_limit(a, k, enc);
+    if (kind == BF_KERNEL_OCTO && team > 0) {
+        const int left = k.n <= team ? k.n : a->shape.d_model == 512 && !k.leaf_index ? k.n % (int)kBoardMaxN : 0;
+        if (left && left <= team) {
+            e = hipSuccess;
+            if (left < k.n) e = (enc ? bf::launch_octo512_enc : bf::launch_octo512)(slice(k, a->shape.d_model, 0, k.n - left), stream);
+            if (e == hipSuccess) e = launch_team(a, left == k.n ? k : slice(k, a->shape.d_model, k.n - left, left), enc, stream);
+            if (e != hipSuccess) {
+                snprintf(g_err, sizeof(g_err), "kernel launch failed: %s", hipGetErrorString(e));
+                return BF_ERR_LAUNCH;
+            }
+            return BF_OK;
+        }
+    }
     // When the library chose the two-position kernel itself, a last round of at most 256 positions goes to the
     // one-position form in a second launch on the same stream (640 positions: 0.33 ms instead of 0.39).  With
     // a leaf list the count is on the device: both forms are launched and each takes its share of the list
@@ -291,11 +330,12 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
                 front.list_split = back.list_split = 1;
                 back.grid = rest;
             } else {
-                front = slice(k, 0, k.n - rest);
-                back = slice(k, k.n - rest, rest);
+                front = slice(k, bf::D, 0, k.n - rest);
+                back = slice(k, bf::D, k.n - rest, rest);
             }
             e = (enc ? bf::launch_duo256_enc : bf::launch_duo256)(front, stream);
-            if (e == hipSuccess) e = (enc ? bf::launch_solo256_enc : bf::launch_solo256)(back, stream);
+            if (e == hipSuccess)
+                e = !k.leaf_index && rest <= team ? launch_team(a, back, enc, stream) : (enc ? bf::launch_solo256_enc : bf::launch_solo256)(back, stream);
             if (e != hipSuccess) {
                 snprintf(g_err, sizeof(g_err), "kernel launch failed: %s", hipGetErrorString(e));
                 return BF_ERR_LAUNCH;

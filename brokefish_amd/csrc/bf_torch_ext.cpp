@@ -39,7 +39,7 @@ Checked check(const torch::Tensor& boards, const torch::Tensor& control, const t
               int64_t n_heads, int64_t d_ff, double eps, int64_t quant, int64_t kernel, int64_t n_value,
               int64_t vmode, const OptTensor& mask_, const OptTensor& best_move_, const OptTensor& active_,
               const OptTensor& workspace_, const OptTensor& leaf_index_ = c10::nullopt,
-              const OptTensor& leaf_count_ = c10::nullopt) {
+              const OptTensor& leaf_count_ = c10::nullopt, const OptTensor& team_workspace_ = c10::nullopt) {
     const torch::Tensor mask = get(mask_), best_move = get(best_move_), active = get(active_), workspace = get(workspace_);
     const torch::Tensor leaf_index = get(leaf_index_), leaf_count = get(leaf_count_);
     TORCH_CHECK(boards.is_cuda() && boards.scalar_type() == torch::kShort && boards.is_contiguous() &&
@@ -113,6 +113,12 @@ Checked check(const torch::Tensor& boards, const torch::Tensor& control, const t
     a.value_mode = (int32_t)vmode;
     a.leaf_index = static_cast<const int32_t*>(ptr_or_null(leaf_index));
     a.leaf_count = static_cast<const int32_t*>(ptr_or_null(leaf_count));
+    const torch::Tensor team = get(team_workspace_);
+    if (!absent(team)) {
+        TORCH_CHECK(on_dev(team) && team.scalar_type() == torch::kByte, "team_workspace must be uint8 on the boards' device");
+        a.team_workspace = team.data_ptr();
+        a.team_workspace_bytes = (size_t)team.numel();
+    }
     return c;
 }
 
@@ -120,9 +126,9 @@ void model_forward(torch::Tensor boards, torch::Tensor control, torch::Tensor re
                    torch::Tensor params, torch::Tensor policy, torch::Tensor promo, torch::Tensor value,
                    int64_t d_model, int64_t n_layers, int64_t n_heads, int64_t d_ff, double eps, int64_t quant,
                    int64_t kernel, int64_t n_value, int64_t vmode, OptTensor mask, OptTensor best_move,
-                   OptTensor active, OptTensor workspace, OptTensor leaf_index, OptTensor leaf_count) {
+                   OptTensor active, OptTensor workspace, OptTensor leaf_index, OptTensor leaf_count, OptTensor team_workspace) {
     const Checked c = check(boards, control, rep, weights, params, policy, promo, value, d_model, n_layers, n_heads,
-                            d_ff, eps, quant, kernel, n_value, vmode, mask, best_move, active, workspace, leaf_index, leaf_count);
+                            d_ff, eps, quant, kernel, n_value, vmode, mask, best_move, active, workspace, leaf_index, leaf_count, team_workspace);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(c.device);     // the launch goes to the tensors' device
     const int rc = bf_model_forward(&c.a, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(c.device.index()).stream());
     TORCH_CHECK(rc == BF_OK, "bf_model_forward failed (", rc, "): ", bf_last_error());
@@ -406,7 +412,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("d_model"), py::arg("n_layers"), py::arg("n_heads"), py::arg("d_ff"), py::arg("eps"),
           py::arg("quant") = 0, py::arg("kernel") = 0, py::arg("n_value") = 1, py::arg("vmode") = 0,
           py::arg("mask") = py::none(), py::arg("best_move") = py::none(), py::arg("active") = py::none(),
-          py::arg("workspace") = py::none(), py::arg("leaf_index") = py::none(), py::arg("leaf_count") = py::none());
+          py::arg("workspace") = py::none(), py::arg("leaf_index") = py::none(), py::arg("leaf_count") = py::none(),
+          py::arg("team_workspace") = py::none());
     m.def("encoder_forward", &encoder_forward, "the encoder stack alone, in place on y", py::arg("y"), py::arg("weights"),
           py::arg("params"), py::arg("alive"), py::arg("d_model"), py::arg("n_layers"), py::arg("n_heads"), py::arg("d_ff"),
           py::arg("eps"), py::arg("quant") = 0, py::arg("kernel") = 0, py::arg("n_value") = 1, py::arg("workspace") = py::none());

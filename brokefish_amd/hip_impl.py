@@ -46,7 +46,7 @@ _TAP_PTRS = ["embed", "qa_qkv", "acc_qkv", "qa_out", "acc_out", "qa_ff1", "acc_f
              "qa_ff2", "acc_ff2", "resid", "normed", "resid_last"]
 
 
-ABI_VERSION = 7     # BF_ABI_VERSION of include/brokefish_hip.h that the structs below mirror
+ABI_VERSION = 8     # BF_ABI_VERSION of include/brokefish_hip.h that the structs below mirror
 
 
 class _Taps(C.Structure):
@@ -70,7 +70,8 @@ class _Args(C.Structure):
                 ("best_move", C.c_void_p), ("out_fp32", C.c_int32), ("quant", C.c_int32),
                 ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t), ("taps", C.POINTER(_Taps)),
                 ("board_wstream", C.c_void_p), ("board_fparams", C.c_void_p), ("active", C.c_void_p),
-                ("kernel", C.c_int32), ("value_mode", C.c_int32), ("leaf_index", C.c_void_p), ("leaf_count", C.c_void_p)]
+                ("kernel", C.c_int32), ("value_mode", C.c_int32), ("leaf_index", C.c_void_p), ("leaf_count", C.c_void_p),
+                ("team_workspace", C.c_void_p), ("team_workspace_bytes", C.c_size_t)]
 
 
 _lib = None
@@ -109,6 +110,8 @@ def load_library():
         L.bf_board_wstream_bytes.restype = C.c_size_t
         L.bf_board_wstream_bytes.argtypes = [C.POINTER(_Shape)]
         L.bf_board_fparams_floats.restype = C.c_size_t
+        L.bf_team_workspace_bytes.restype = C.c_size_t
+        L.bf_team_workspace_bytes.argtypes = [C.POINTER(_Shape)]
         L.bf_board_fparams_floats.argtypes = [C.POINTER(_Shape)]
         L.bf_pack_scratch_floats.restype = C.c_size_t
         L.bf_pack_scratch_floats.argtypes = [C.POINTER(_Shape)]
@@ -778,6 +781,11 @@ class FusedEncoder:
         self._buffered_full = 0
         # launches of more positions than this run the two-position kernel (int8, kernel="auto", 256 wide)
         self._pair_above = int(self._lib.bf_board_max_n()) if kernel == "auto" and self.int8 and not wide else 1 << 62
+        # exchange memory of the form that spreads a position over several compute units: one per stream,
+        # as launches on different streams may overlap
+        with torch.cuda.device(self.device):
+            self._team_bytes = int(self._lib.bf_team_workspace_bytes(C.byref(self._shape))) if kernel == "auto" else 0
+        self._team = {}
         self._backbone = None
         self._profile, self._profile_waves, self._profile_kept = None, 0, None
         self.best_move = None
@@ -861,7 +869,35 @@ class FusedEncoder:
         if need:
             a.workspace, a.workspace_bytes = self.workspace.data_ptr(), self.workspace.numel()
         a.taps = C.pointer(taps) if taps is not None else None
+        self._lend_team(a)
         return a
+
+    def _lend_team(self, a: _Args) -> None:
+        ws = self._team_workspace(a.n)
+        if ws is not None:
+            a.team_workspace, a.team_workspace_bytes, a._keep = ws.data_ptr(), ws.numel(), ws
+
+    TEAM_STREAMS = 16      # streams whose exchange memory is kept (13 MB each, 512 wide 21)
+
+    def _team_workspace(self, n: int):
+        """The exchange memory for a launch of ``n`` positions on the current stream, or None where no
+        part of such a launch uses it (at most 64 positions, or what is left of rounds of 512; 512 wide:
+        32, or what is left of rounds of 256)."""
+        if not self._team_bytes:
+            return None
+        wide = self.d_model != self.D
+        left = n % 256 if wide else n if self.fp8 else n % 512
+        if not 0 < left <= (32 if wide else 64):
+            return None
+        if torch.cuda.is_current_stream_capturing():      # a graph has its own, cleared by each replay
+            return torch.zeros(self._team_bytes, dtype=torch.uint8, device=self.device)
+        key = torch.cuda.current_stream(self.device).cuda_stream
+        ws = self._team.get(key)
+        if ws is None:
+            if len(self._team) >= self.TEAM_STREAMS:
+                self._team.pop(next(iter(self._team)))
+            ws = self._team.setdefault(key, torch.zeros(self._team_bytes, dtype=torch.uint8, device=self.device))
+        return ws
 
     def kernel_choice(self, n: int) -> str:
         """Which kernel a call with ``n`` positions runs ("quad", "board", "twin", "octo" or "duo")."""
@@ -968,6 +1004,7 @@ class FusedEncoder:
             a.board_wstream, a.board_fparams = self.board_wstream.data_ptr(), self.board_fparams.data_ptr()
         a.kernel, a.quant, a.value_mode = self.KERNELS[self.kernel], (1 if self.fp8 else 0), self.vmode
         a.taps = C.pointer(taps)      # the library copies the table at launch
+        self._lend_team(a)
         self._call(a)
         if result is not None:
             return result
@@ -1035,7 +1072,8 @@ class FusedEncoder:
                 self.KERNELS[self.kernel], self.n_value, self.vmode,
                 mask if mask is not None else none, self.best_out if mask is not None else none,
                 active if active is not None else none, self.workspace if quad else none,
-                leaves[0] if leaves is not None else none, leaves[1] if leaves is not None else none)
+                leaves[0] if leaves is not None else none, leaves[1] if leaves is not None else none,
+                self._team_workspace(n))
         else:
             self._call(self._args(boards, control, rep, mask, self.policy_out, self.promo_out,
                                   self.value_out, self.best_out, active=active, leaves=leaves))

@@ -107,6 +107,11 @@ size_t bf_workspace_bytes(const bf_shape* s, int64_t n);
 size_t bf_board_wstream_bytes(const bf_shape* s);
 size_t bf_board_fparams_floats(const bf_shape* s);
 
+/* Size of team_workspace of bf_eval_args: the largest launch of that form on the current device, 0 where the
+ * device (or its partitioning) or the shape does not carry it.  The first call on a device looks how its
+ * workgroups are placed (one small launch and a synchronisation); the form runs only after such a call. */
+size_t bf_team_workspace_bytes(const bf_shape* s);
+
 /* Packing of a network that lies in fp32 on the device into the BOARD / TWIN / OCTO / DUO blobs
  * (board_wstream: bf_board_wstream_bytes, board_fparams: bf_board_fparams_floats), quantised and laid
  * out on the device.  Names and shapes are those of the reference's modules (reference
@@ -226,6 +231,13 @@ typedef struct {
      * list stay untouched.  Both or neither. */
     const int32_t* leaf_index;
     const int32_t* leaf_count;
+    /* optional: DEVICE memory of team_workspace_bytes (bf_team_workspace_bytes(shape) serves every launch; 256-byte
+     * aligned) through which the workgroups of one position exchange what they computed.  With it AUTO gives the
+     * smallest launches, and a short last round, to a form that spreads a position over several compute
+     * units; the results are the same bits.  Zero before its first use and then left alone by the caller;
+     * launches that may overlap need workspaces of their own. */
+    void* team_workspace;
+    size_t team_workspace_bytes;
 } bf_eval_args;
 
 /* Binary interface of this header.  BF_ABI_VERSION is raised whenever a struct or a signature of
@@ -234,7 +246,7 @@ typedef struct {
  * BF_ABI_TAG before its first call and refuses a library it was not built for (a shorter
  * bf_eval_args would make the library read pointers from beyond the caller's struct).  No
  * counterpart in the reference, whose module and kernels are one compilation. */
-#define BF_ABI_VERSION 7
+#define BF_ABI_VERSION 8
 #define BF_ABI_TAG (((uint64_t)BF_ABI_VERSION << 32) | (uint64_t)sizeof(bf_eval_args))
 uint64_t bf_abi_tag(void);
 
