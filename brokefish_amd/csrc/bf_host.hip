@@ -301,15 +301,16 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
     if (!bf::device_is_gfx950()) return BF_ERR_DEVICE;
     const bool enc = !k.profile && enc_build(a, kind);
     // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
-    // position 124 -> 90 us, e4m3 155 -> 106; 512 wide 750 -> 346 us), and so does what is left of the 512-wide
-    // network's rounds of 256 positions if it is no more.
+    // position 124 -> 84 us, e4m3 155 -> 96; 512 wide 750 -> 275 us), and so does what is left of the 512-wide
+    // network's rounds of 256 positions (727 us each) where two team launches (328 us each) hold it.
     const int team = team_limit(a, k, enc);
     if (kind == BF_KERNEL_OCTO && team > 0) {
-        const int left = k.n <= team ? k.n : a->shape.d_model == 512 && !k.leaf_index ? k.n % (int)kBoardMaxN : 0;
-        if (left && left <= team) {
+        const int left = k.n <= team ? k.n : a->shape.d_model == 512 && !k.leaf_index ? k.n % (int)kBoardMaxN : 0;   // a list's length is on the device
+        if (left && left <= (a->shape.d_model == 512 ? 2 : 1) * team) {
             e = hipSuccess;
             if (left < k.n) e = (enc ? bf::launch_octo512_enc : bf::launch_octo512)(slice(k, a->shape.d_model, 0, k.n - left), stream);
-            if (e == hipSuccess) e = launch_team(a, left == k.n ? k : slice(k, a->shape.d_model, k.n - left, left), enc, stream);
+            for (int at = k.n - left; at < k.n && e == hipSuccess; at += team)
+                e = launch_team(a, left <= team && left == k.n ? k : slice(k, a->shape.d_model, at, k.n - at < team ? k.n - at : team), enc, stream);
             if (e != hipSuccess) {
                 snprintf(g_err, sizeof(g_err), "kernel launch failed: %s", hipGetErrorString(e));
                 return BF_ERR_LAUNCH;

@@ -12,28 +12,40 @@
 //   - member m computes the 256 hidden channels of k-chunk m, which are one quantiser group of their own, and
 //     that chunk's part of the second matmul for the whole width; the int32 (e4m3: fp32) partial accumulators
 //     and the chunk's scales go to everybody (exchange B), who sums them in chunk order.
-// So a layer has two exchanges, its weights are read once per team except the output projection's, and a wavefront
-// never has more than one tile (width 512: two) in a matmul.  Measured: one position 124 -> 90 us, 64 positions
-// 120 -> 95, e4m3 155 -> 106; width 512, 16 layers: one position 750 -> 346 us, 32 positions 727 -> 381.  The arithmetic is that of the other kernels,
-// operation for operation: the results are bit-identical to theirs.
+// So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
+// tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
+// except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
+// 124 -> 84 us, e4m3 155 -> 96, width 512 with 16 layers 750 -> 275; 64 positions 120 -> 88, e4m3 155 -> 100; 32 of the
+// wide network 727 -> 328.  The arithmetic is that of the other kernels, operation for operation: the results are
+// bit-identical to theirs.
+//
+// Rows and tiles.  For everything per row (LayerNorm, quantisers, residual sums) a wavefront owns the rows of four
+// tokens, a lane a 16-value chain of one of them, so a row's sums and maxima are a few cross-lane instructions.  With
+// the accumulator layout's split (a wavefront a tile, all tokens), as the other kernels have it, each of these was an
+// exchange through LDS: thirteen barriers a layer instead of seven, 90 us instead of 84.  The matmuls take the
+// quantised rows from LDS; their results come back as rows through LDS (output projection) or on the way through
+// the L2, where pieces are laid out so that four tokens, 64 bytes, stay together on either side.
+//
+// What bounds it now: a layer is some 20 k clocks at width 256, of which the waits for other members are 1.5 k; the unit's
+// path to the L2 moves 400 KB in it (6.3 k clocks, most of it under something else), two LayerNorms, three
+// quantisers and the epilogues are some 7 k of vector work, attention 2.8 k.
 //
 // An exchange: a wavefront stores its piece, waits until the L2 has it (vmcnt), and stores a flag; the wavefronts that
-// need the piece poll the flag past their L1 (sc1) and then load the piece past it (dword flags; polling tags inside
-// the data itself was slower, every poll is 16 KiB).  Members sit behind one L2
-// because workgroups go to the XCDs in turn (blockIdx % 8; bf_team_setup looks at the device before the form is
-// used).  Measured on its own: 3.0 k clocks from store to data with 4 x 32 KiB exchanged.  Flags count layers over
-// all launches of a workspace (each member keeps the count, a multiple it adds at its end), so nothing is
-// cleared between launches.  Waiting is bounded: a wavefront that has waited some seconds gives up, publishes nothing
-// any more and makes its part of the stream NaN.  Members of a team are consecutive workgroups of their XCD and
-// are dispatched in order, so at most NWG - 1 workgroups of a launch per XCD ever wait for a unit to come free.
+// need the piece poll the flags past their L1 (sc1) and then load the piece past it (polling tags inside the data
+// itself was slower: every poll is 16 KiB).  Members sit behind one L2 because workgroups go to the XCDs in turn
+// (blockIdx % 8; bf_team_workspace_bytes looks at the device before the form is used).  Flags count layers over all
+// launches of a workspace (each member keeps the count), so nothing is cleared between launches.  Waiting is
+// bounded: a wavefront that has waited some seconds gives up, publishes nothing any more and makes its rows NaN.
+// Members of a team are consecutive workgroups of their XCD and are dispatched in order, so at most NWG - 1
+// workgroups of a launch per XCD ever wait for a unit to come free.
 //
-// No exchange buffer is written twice in a layer, and one set per team is enough: a member writes A or B of
-// layer l + 1 only after barriers that follow its wavefronts' loads of B of layer l from all members, and every
-// wavefront loads A of a layer before it stores its B.
+// One set of exchange buffers per team is enough: a member writes A, B or C of layer l + 1 only after barriers that
+// follow all its wavefronts' loads of the last exchange of layer l from all members, and every wavefront loads A of a
+// layer before it stores its B.
 //
-// LDS map: [xch: 3 slots x 8 waves x 64 floats] [act: the quantised row of the width] [hid: the quantised chunk]
-// [tok: activation scales of the row that feeds QKV] [qkv: Q, K, V of two heads, 24 KiB] [par: a layer's side
-// parameters, twice].  During the heads the normalised stream (fp32) overlays qkv / par.
+// LDS map: [xch: 8 waves x 64 floats] [act: the quantised rows of the width] [hid: the quantised chunk] [tok: the
+// activation scales of act's rows] [par: a layer's side parameters, twice] [ex: Q, K, V of two heads; the output
+// projection's tiles; the normalised stream (fp32) of the heads].
 #pragma once
 
 #include "bf_board.hip.h"
@@ -55,35 +67,48 @@ template <int DM>
 struct Cfg : Layout<DM> {
     typedef Layout<DM> L;
     static constexpr int NWG = L::KCF, NW = 8;      // members of a team; wavefronts of a member
-    static constexpr int TWW = L::NT / NW;          // tiles of the width a wavefront owns
-    static constexpr int NHW = L::NT / NWG;         // heads of a member
-    static_assert(NHW == 2, "two heads per member");
-    static constexpr int XS = NW * 64;
+    static constexpr int TWW = L::NT / NW;          // tiles of a matmul over the width a wavefront computes
+    static constexpr int NP = TWW;                  // tiles of a row a lane holds, of the four rows a wavefront owns
+    static_assert(L::NT / NWG == 2, "two heads per member");
+    // side parameters of a quarter in LDS: part A, the head of part B, this member's row of 128 * sum(w), its step of the hidden biases
+    static constexpr int P_B = L::A_FLOATS, P_WSUM = P_B + L::B_LDS_FLOATS, P_BFF1 = P_WSUM + L::CW, P_FLOATS = P_BFF1 + 128;
     static constexpr int XCH_OFF = 0;
-    static constexpr int ACT_OFF = XCH_OFF + 3 * XS * 4;
+    static constexpr int ACT_OFF = XCH_OFF + NW * 64 * 4;
     static constexpr int HID_OFF = ACT_OFF + L::NT * FRAG;
     static constexpr int TOK_OFF = HID_OFF + 8 * FRAG;
-    static constexpr int QKV_OFF = TOK_OFF + FRAG;
-    static constexpr int PAR_OFF = QKV_OFF + NHW * 3 * 4 * FRAG;
-    static constexpr int PAR_BYTES = 4 * L::PW_FLOATS * 4;
-    static constexpr int USED_BYTES = PAR_OFF + 2 * PAR_BYTES;
+    static constexpr int PAR_OFF = TOK_OFF + FRAG;
+    static constexpr int PAR_BYTES = 4 * P_FLOATS * 4;
+    static constexpr int EX_OFF = PAR_OFF + 2 * PAR_BYTES;
+    static constexpr int EX_TILE = 4 * FRAG + 64;   // a tile in accumulator layout; the padding spreads the tiles of a row over the banks
+    static constexpr int EX_BYTES = L::NT * EX_TILE > 24 * FRAG ? L::NT * EX_TILE : 24 * FRAG;
+    static constexpr int USED_BYTES = EX_OFF + EX_BYTES;
     // more than half a compute unit's LDS: never two workgroups on one unit while another is empty
     static constexpr int LDS_BYTES = USED_BYTES < 81 * 1024 ? 81 * 1024 : USED_BYTES;
     static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
-    static_assert(QKV_OFF + L::NT * 4 * FRAG <= LDS_BYTES, "normalised stream overlay");
-    // a team's part of the workspace, bytes
-    static constexpr int FLAG_A = 64, FLAG_B = 128;           // dwords: first flag of exchange A, of exchange B
-    static constexpr int WS_A = 4096;                         // [tile][quad 4][64 lanes] 16 bytes
-    static constexpr int WS_B = WS_A + L::NT * 4 * FRAG;      // [member][wave][4 TWW quads + scale][64 lanes] 16 bytes
-    static constexpr int B_PIECE = (4 * TWW + 1) * FRAG;
-    static constexpr int WS_BYTES = WS_B + NWG * NW * B_PIECE;
-    static_assert(NWG <= FLAG_A && FLAG_A + 2 * L::NT <= FLAG_B && (FLAG_B + NWG * NW) * 4 <= WS_A, "flags");
+    // a team's part of the workspace, bytes.  A stream-shaped piece is [owner wave][quad 4][NP][64 lanes] 16 bytes.
+    static constexpr int FLAG_A = 64, FLAG_B = 128;           // dwords: first flag of exchange A [query half][tile], of exchange B [member][wave]
+    static constexpr int ROWS = L::NT * 4 * FRAG;             // a stream-shaped piece; an owner wave's part; a quad of that
+    static constexpr int ROWS_W = ROWS / NW, ROWS_Q = ROWS_W / 4;
+    static constexpr int WS_A = 4096, WS_B = WS_A + ROWS, WS_S = WS_B + NWG * ROWS;   // [member]: accumulators; scales [member][token]
+    // more than four members: exchange B in two steps, each member sums the accumulators of two tiles and gives the sums to all
+    static constexpr bool TWO_STEPS = NWG > 4;
+    static constexpr int FLAG_C = FLAG_B + NWG * NW, WS_C = WS_S + NWG * 128;   // the second step: [member][wave]; stream-shaped
+    static constexpr int WS_BYTES = (WS_C + (TWO_STEPS ? ROWS : 0) + 4095) / 4096 * 4096;
+    static_assert(NWG <= FLAG_A && FLAG_A + 2 * L::NT <= FLAG_B && (FLAG_C + NWG * NW) * 4 <= WS_A, "flags");
+    static_assert(!TWO_STEPS || NWG * TWW == L::NT, "a member's tiles are those of one wavefront");
 };
 
 constexpr int SPIN_LIMIT = 1 << 23;   // polls of some 600 clocks: about two seconds
 constexpr int SC1 = 16;               // cache policy of a load that goes past the L1
 
-// the other of lanes l and l ^ 16, and both in row order
+// a value from another lane of the row of 16 (data-parallel primitive); lanes past the row read 0
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int SHL = 0x100, SHR = 0x110, ROR = 0x120;   // shift to lower lanes, to higher ones, rotate
+
+// the values of lanes l and l ^ 16 in row order
 __device__ __forceinline__ v2u rows_of(float v) {
     const unsigned u = (unsigned)__float_as_int(v);
     const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
@@ -96,7 +121,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     typedef Cfg<DM> C;
     typedef typename Acc<FP8>::type acc_t;
     constexpr int D = C::D, NT = C::NT, TW = C::TW, CW = C::CW, KC = C::KC, KCF = C::KCF, NWG = C::NWG, TWW = C::TWW;
-    constexpr int BPW = C::BPW, HB = C::HB, XS = C::XS;
+    constexpr int BPW = C::BPW, HB = C::HB, NP = C::NP;
     constexpr int BASE = 4 * KC * TW, SSTR = 4 * KC + 2 * TW;   // a quarter's stream: first feed-forward block of a layer, blocks of a step
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -124,14 +149,20 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     uint8_t* const act = lds + C::ACT_OFF;
     uint8_t* const hid = lds + C::HID_OFF;
     float* const tok = reinterpret_cast<float*>(lds + C::TOK_OFF);
-    float* const qkv = reinterpret_cast<float*>(lds + C::QKV_OFF);
+    uint8_t* const ex = lds + C::EX_OFF;
+    float* const qkv = reinterpret_cast<float*>(ex);
     const float* const gp = a.fparams + (size_t)4 * a.n_layers * C::PW_FLOATS;
-    auto par = [&](int l, int quarter) { return reinterpret_cast<const float*>(lds + C::PAR_OFF + (l & 1) * C::PAR_BYTES) + quarter * C::PW_FLOATS; };
-    auto fetch_par = [&](int l) {   // a quarter's part A by its first wave, part B by its second
+    const int fq = 2 * (m & 1) + (wave >> 2), fh = wave & 3, fst = m >> 1;   // hidden tile 8 m + wave: its quarter, number there, step
+    auto par = [&](int l, int quarter) { return reinterpret_cast<const float*>(lds + C::PAR_OFF + (l & 1) * C::PAR_BYTES) + quarter * C::P_FLOATS; };
+    auto fetch_par = [&](int l) {   // a quarter's part A by its first wave, the rest by its second
         const float* src = a.fparams + ((size_t)q * a.n_layers + l) * C::PW_FLOATS;
         float* dst = const_cast<float*>(par(l, q));
-        if (wave & 1) dma(src + C::A_FLOATS, dst + C::A_FLOATS, C::B_FLOATS, lane);
-        else dma(src, dst, C::A_FLOATS, lane);
+        if (wave & 1) {
+            src += C::A_FLOATS;
+            dma(src, dst + C::P_B, C::B_LDS_FLOATS, lane);
+            dma(src + C::B_WSUM + m * CW, dst + C::P_WSUM, CW, lane);
+            dma(src + C::B_BFF1 + 128 * fst, dst + C::P_BFF1, 128, lane);
+        } else dma(src, dst, C::A_FLOATS, lane);
     };
     // block `idx` of layer l in a quarter's stream.  Buffer loads with the block's place in a scalar register: one
     // vector register of addresses for all of them (the stream is far below 4 GiB).
@@ -164,7 +195,6 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
         for (int c = 0; c < KC; c++) load_block(w[c], q, l, 3 * KC * TW + KC * (iq0 + i) + c);
     };
-    const int fq = 2 * (m & 1) + (wave >> 2), fh = wave & 3, fst = m >> 1;   // hidden tile 8 m + wave: its quarter, number there, step
     auto fetch_ff1 = [&](int l) {
 #pragma unroll
         for (int c = 0; c < KC; c++) load_block(SB[c], fq, l, BASE + fst * SSTR + KC * fh + c);
@@ -181,78 +211,90 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     };
     const acc_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
-    // row sums and the quantiser: bf_board.hip.h's, with tiles TWW wave ... owned by a wave in order
-    auto xsum = [&](float part, int sl) -> float {
-        xch[sl * XS + wave * 64 + lane] = part;
-        lds_barrier();
-        const float* p = xch + sl * XS + lane;
-        return (((p[0] + p[64]) + (p[128] + p[192])) + (p[256] + p[320])) + (p[384] + p[448]);
+    // ---- rows: a wavefront owns the rows of tokens 4 wave .. + 3; a lane holds NP tiles of one of them, the half rg of the
+    // accumulator layout.  Four neighbouring lanes are four tokens, which are neighbours in every buffer (64 bytes) ----
+    const int row = 4 * wave + (lane & 3), rk = (lane >> 2) & 7, rg = lane >> 5;   // the token; tiles NP rk ..; the half
+    const int rq = rk >> 1, ri = NP * (rk & 1);                                    // their quarter, the first one's number there
+    // Sum of a row: tiles of a quarter as a tree, the quarters in order, the halves, as bf_args.h has it (v: the sum over the lane's
+    // tiles).  A lane row of 16 holds two quarters: what lies in lanes 4 .. 15 comes to lanes 0 .. 3 and the result goes back.
+    auto rowsum = [&](float v) -> float {
+        v = v + dpp<SHL + 4>(v);
+        const v2u r = rows_of(v);
+        const float lo = __int_as_float(r[0]), hi = __int_as_float(r[1]);
+        float s = ((lo + dpp<SHL + 8>(lo)) + hi) + dpp<SHL + 8>(hi);
+        s = s + partner(s, rg);
+        int u = __float_as_int(s);
+        u = __builtin_amdgcn_update_dpp(u, u, SHR + 4, 0xf, 0x2, false);
+        u = __builtin_amdgcn_update_dpp(u, u, SHR + 8, 0xf, 0xc, false);
+        return __int_as_float(u);
     };
-    auto layernorm = [&](const float (&x)[TWW][16], const float* gamma, const float* beta, float (&y)[TWW][16]) {
-        float ts[TWW];
+    // largest value of a row's 256-wide chunk
+    auto chunkmax = [&](float v) -> float {
+        v = __builtin_fmaxf(v, dpp<ROR + 4>(v));
+        v = __builtin_fmaxf(v, dpp<ROR + 8>(v));
+        v = __builtin_fmaxf(v, partner(v, rg));
+        if constexpr (KC == 1) {
+            const v2u r = rows_of(v);
+            v = __builtin_fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
+        }
+        return v;
+    };
+    // y = LayerNorm(x); gamma / beta: this lane's half of its first tile's parameters
+    auto layernorm = [&](const float (&x)[NP][16], const float* gamma, const float* beta, float (&y)[NP][16]) {
+        float ts[NP];
 #pragma unroll
-        for (int i = 0; i < TWW; i++) {
+        for (int p = 0; p < NP; p++) {
             float acc = 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc = acc + x[i][r];
-            ts[i] = acc;
+            for (int r = 0; r < 16; r++) acc = acc + x[p][r];
+            ts[p] = acc;
         }
-        const float s = xsum(TWW == 1 ? ts[0] : ts[0] + ts[TWW - 1], 0);
-        const float mean = (s + partner(s, g)) * (1.0f / D);
+        const float mean = rowsum(NP == 1 ? ts[0] : ts[0] + ts[NP - 1]) * (1.0f / D);
 #pragma unroll
-        for (int i = 0; i < TWW; i++) {
+        for (int p = 0; p < NP; p++) {
             float acc = 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const float d = x[i][r] - mean;
+                const float d = x[p][r] - mean;
                 acc = __builtin_fmaf(d, d, acc);
             }
-            ts[i] = acc;
+            ts[p] = acc;
         }
-        const float v = xsum(TWW == 1 ? ts[0] : ts[0] + ts[TWW - 1], 1);
-        const float var = (v + partner(v, g)) * (1.0f / D);
-        const float rstd = recip_sqrt(var + a.eps);
+        const float rstd = recip_sqrt(rowsum(NP == 1 ? ts[0] : ts[0] + ts[NP - 1]) * (1.0f / D) + a.eps);
 #pragma unroll
-        for (int i = 0; i < TWW; i++)
+        for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const v4f ga = ldg4(gamma + 32 * i + 8 * j + 4 * g);
-                const v4f be = ldg4(beta + 32 * i + 8 * j + 4 * g);
+                const v4f ga = ldg4(gamma + 32 * p + 8 * j), be = ldg4(beta + 32 * p + 8 * j);
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const float d = x[i][4 * j + k] - mean;
-                    y[i][4 * j + k] = __builtin_fmaf(d * rstd, ga[k], be[k]);
+                    const float d = x[p][4 * j + k] - mean;
+                    y[p][4 * j + k] = __builtin_fmaf(d * rstd, ga[k], be[k]);
                 }
             }
     };
-    auto quant_exchange = [&](const float (&y)[TWW][16], float (&sa)[KC], bool publish_scales) {
+    // quantise a row: its bytes go to the activation buffer as operand fragments, its scale(s) to the token table
+    auto quantise = [&](const float (&y)[NP][16]) {
         float am = 0.0f;
 #pragma unroll
-        for (int i = 0; i < TWW; i++)
+        for (int p = 0; p < NP; p++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) am = __builtin_fmaxf(am, __builtin_fabsf(y[i][r]));
-        xch[2 * XS + wave * 64 + lane] = am;
-        lds_barrier();
+            for (int r = 0; r < 16; r++) am = __builtin_fmaxf(am, __builtin_fabsf(y[p][r]));
+        am = chunkmax(am);
+        const float sa = am > 0.0f ? (FP8 ? am * 0.125f : div127(am)) : 1.0f;
+        if (rg == 0 && rk % (8 / KC) == 0) tok[rk / (8 / KC) * 32 + row] = sa;
+        const Quot by = quot_by(sa);
 #pragma unroll
-        for (int c = 0; c < KC; c++) {
-            float mx = 0.0f;
-#pragma unroll
-            for (int w = 8 / KC * c; w < 8 / KC * (c + 1); w++) mx = __builtin_fmaxf(mx, xch[2 * XS + w * 64 + lane]);
-            mx = __builtin_fmaxf(mx, partner(mx, g));
-            sa[c] = mx > 0.0f ? (FP8 ? mx * 0.125f : div127(mx)) : 1.0f;
-        }
-        if (publish_scales && wave == 0 && g == 0)
-#pragma unroll
-            for (int c = 0; c < KC; c++) tok[c * 32 + t] = sa[c];
-        const Quot by = quot_by(KC == 1 || wave < 4 ? sa[0] : sa[KC - 1]);
-#pragma unroll
-        for (int i = 0; i < TWW; i++) {
+        for (int p = 0; p < NP; p++) {
             v4i w;
 #pragma unroll
-            for (int j = 0; j < 4; j++) w[j] = (int)quant4<FP8>(y[i][4 * j], y[i][4 * j + 1], y[i][4 * j + 2], y[i][4 * j + 3], by);
-            *reinterpret_cast<v4i*>(act + (TWW * wave + i) * FRAG + lane * 16) = w;
+            for (int j = 0; j < 4; j++) w[j] = (int)quant4<FP8>(y[p][4 * j], y[p][4 * j + 1], y[p][4 * j + 2], y[p][4 * j + 3], by);
+            *reinterpret_cast<v4i*>(act + (NP * rk + p) * FRAG + (rg * 32 + row) * 16) = w;
         }
-        lds_barrier();
+    };
+    auto scales = [&](float (&sa)[KC]) {   // of this lane's token, in the accumulator layout
+#pragma unroll
+        for (int c = 0; c < KC; c++) sa[c] = tok[c * 32 + t];
     };
     // wait until `count` flags, `stride` dwords apart, have reached `tag`
     auto wait_flags = [&](int first, int stride, int count, int tag) {
@@ -270,49 +312,52 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         wait_vm<0>();
         if (lane == 0 && !dead) __builtin_amdgcn_raw_buffer_store_b32((unsigned)tag, wsr, 0, at * 4, 0);
     };
-    auto take = [&](int at) -> v4i { return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wsr, lane16, at, SC1)); };
+    // quad j of tile p of this wave's rows from the stream-shaped piece at `at`
+    auto take = [&](int at, int p, int j) -> v4i {
+        return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wsr, lane16, at + wave * C::ROWS_W + j * C::ROWS_Q + p * FRAG, SC1));
+    };
+    // where lane (t, g) of a tile in the accumulator layout has its place in a stream-shaped piece
+    auto piece_at = [&](int tk, int half) { return (tk >> 2) * C::ROWS_W + (half * 32 + (tk & 3)) * 16; };
+    auto tile_at = [&](int tile) { return tile % NP * FRAG + tile / NP * 64; };
 
-    // ---- start: parameters and weights of the first layer --------------------------------------------
-    if (a.l1 > a.l0) {
-        fetch_par(a.l0);
-        fetch_qkv(a.l0);
-        fetch_out(SB, a.l0, 0);
-    }
+    // ---- start: parameters of the first layer; its weights follow the embedding's loads, which return in order ----
+    if (a.l1 > a.l0) fetch_par(a.l0);
 
     // ---- embedding, or the caller's stream -------------------------------------------------------------
-    float x[TWW][16];
-    const unsigned word = ENC ? (a.taps.alive[(size_t)b * T + t] ? 0u : 0x800u) : a.boards[(size_t)b * T + t];
+    float x[NP][16];
+    const unsigned own_word = ENC ? (a.taps.alive[(size_t)b * T + t] ? 0u : 0x800u) : a.boards[(size_t)b * T + t];
+    const unsigned row_word = ENC ? 0u : a.boards[(size_t)b * T + row];
     const int ctrl = ENC ? 1 : a.control[b];
-    const unsigned alive = (unsigned)__ballot(((word >> 11) & 1) == 0 && g == 0);
-    if constexpr (ENC) {
+    int rp = ENC ? 0 : a.rep[b];
+    rp = rp > 2 ? 2 : rp;
+    const unsigned alive = (unsigned)__ballot(((own_word >> 11) & 1) == 0 && g == 0);
 #pragma unroll
-        for (int i = 0; i < TWW; i++)
+    for (int p = 0; p < NP; p++) {
+        const size_t at = ((size_t)b * T + row) * D + 32 * (NP * rk + p) + 4 * rg;
+        if constexpr (ENC) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const v4f v = stream_in(a.taps, ((size_t)b * T + t) * D + 32 * (TWW * wave + i) + 8 * j + 4 * g);
+                const v4f v = stream_in(a.taps, at + 8 * j);
 #pragma unroll
-                for (int k = 0; k < 4; k++) x[i][4 * j + k] = v[k];
+                for (int k = 0; k < 4; k++) x[p][4 * j + k] = v[k];
             }
-    } else {
-        const int stm = ctrl < 0;
-        int clock = (ctrl < 0 ? -ctrl : ctrl) - 1;
-        clock = clock < 0 ? 0 : (clock > 100 ? 100 : clock);
-        int rp = a.rep[b];
-        rp = rp > 2 ? 2 : rp;
-        int ts = ((word >> 6) & 7) * 2 + ((word >> 9) & 1);
-        ts = ts > 11 ? 11 : ts;
-        const int ct = ((word >> 10) & 1) * 2 + stm;
-        const int own = 32 * TWW * wave + 4 * g;
-        const float* e_sq = gp + C::G_SQ + (word & 63) * D + own;
-        const float* e_ts = gp + C::G_TS + ts * D + own;
-        const float* e_ct = gp + C::G_CT + ct * D + own;
-        const float* e_ck = gp + C::G_CLOCK + clock * D + own;
-        const float* e_rp = gp + C::G_REP + rp * D + own;
-#pragma unroll
-        for (int i = 0; i < TWW; i++)
+        } else {
+            const unsigned word = row_word;
+            const int stm = ctrl < 0;
+            int clock = (ctrl < 0 ? -ctrl : ctrl) - 1;
+            clock = clock < 0 ? 0 : (clock > 100 ? 100 : clock);
+            int ts = ((word >> 6) & 7) * 2 + ((word >> 9) & 1);
+            ts = ts > 11 ? 11 : ts;
+            const int ct = ((word >> 10) & 1) * 2 + stm;
+            const int own = 32 * (NP * rk + p) + 4 * rg;
+            const float* e_sq = gp + C::G_SQ + (word & 63) * D + own;
+            const float* e_ts = gp + C::G_TS + ts * D + own;
+            const float* e_ct = gp + C::G_CT + ct * D + own;
+            const float* e_ck = gp + C::G_CLOCK + clock * D + own;
+            const float* e_rp = gp + C::G_REP + rp * D + own;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int c = 32 * i + 8 * j;
+                const int c = 8 * j;
                 const v4f vs = ldg4(e_sq + c), vt = ldg4(e_ts + c), vc = ldg4(e_ct + c);
                 const v4f vk = ldg4(e_ck + c), vr = ldg4(e_rp + c);
 #pragma unroll
@@ -320,25 +365,32 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                     const float per_board = vk[k] + vr[k];
                     float v = vs[k] + vt[k];
                     v = v + vc[k];
-                    x[i][4 * j + k] = v + per_board;
+                    x[p][4 * j + k] = v + per_board;
                 }
             }
+        }
     }
-    wait_vm<0>();   // the parameters have landed (the next barrier shows them to the other waves)
+#pragma unroll
+    for (int p = 0; p < NP; p++) pin16(x[p]);   // has arrived, and with it the parameters, which were asked for before
+    if (a.l1 > a.l0) {
+        fetch_qkv(a.l0);
+        if constexpr (TWW == 1) fetch_out(SB, a.l0, 0);
+    }
+    lds_barrier();
 
     for (int l = a.l0; l < a.l1; l++) {
         const int tag = tag0 + (l - a.l0) + 1;
         const int lnext = l + 1 < a.l1 ? l + 1 : l;   // after the last layer its own weights come once more (and are not used)
-        const float* const pq = par(l, q);                       // this wave's quarter: parts A and B
-        const float* const pB = pq + C::A_FLOATS;
+        const float* const pq = par(l, q);                       // parameters of this wave's matmul tiles
+        const float* const pr = par(l, rq) + 32 * ri + 4 * rg;   // of its rows: this lane's chain
 
         // ---- LayerNorm 1, quantise ---------------------------------------------------------------------
-        float sa[KC];
         {
-            float y[TWW][16];
-            layernorm(x, pq + C::A_LN1G + 32 * iq0, pq + C::A_LN1B + 32 * iq0, y);
-            quant_exchange(y, sa, true);
+            float y[NP][16];
+            layernorm(x, pr + C::A_LN1G, pr + C::A_LN1B, y);
+            quantise(y);
         }
+        lds_barrier();
         if (lnext != l) fetch_par(lnext);   // the other copy's last reads lie before the barriers above
 
         __builtin_amdgcn_sched_barrier(0);
@@ -348,7 +400,8 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             const float* const pA = par(l, hq);
             const float sw = pA[C::A_SW + tq * TW + hi];
             acc_t acc[KC];
-            float v[16];
+            float v[16], sa[KC];
+            scales(sa);
             if (tq < 2) {
 #pragma unroll
                 for (int c = 0; c < KC; c++) acc[c] = product(std::false_type(), SA[c], act + 8 * c * FRAG, zero);
@@ -379,7 +432,10 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                     *reinterpret_cast<v4f*>(to + ((g * 2 + odd) * 2 + iq) * 128) = v4f{v[8 * iq + odd], v[8 * iq + 2 + odd], v[8 * iq + 4 + odd], v[8 * iq + 6 + odd]};
         }
         if constexpr (TWW == 1) fetch_ff2(l);
-        else fetch_out(SA, l, 1);
+        else {
+            fetch_out(SB, l, 0);
+            fetch_out(SA, l, 1);
+        }
         lds_barrier();
 
         __builtin_amdgcn_sched_barrier(0);
@@ -445,24 +501,26 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
             for (int u = 0; u < 2; u++)
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, oa[u]), wsr,
-                                                       (G >> 1) * FRAG + ((G & 1) * 32 + c16) * 16, C::WS_A + (tile * 4 + 2 * u) * FRAG + qb * 256, 0);
-            raise_flag(C::FLAG_A + tile * 2 + qb, tag);
+                                                       piece_at(c16, G & 1) + (G >> 1) * C::ROWS_Q, C::WS_A + 4 * qb * C::ROWS_W + 2 * u * C::ROWS_Q + tile_at(tile), 0);
+            raise_flag(C::FLAG_A + qb * NT + tile, tag);
         }
 
         // ---- exchange A, output projection + residual --------------------------------------------------
         {
-            float o[TWW][16];
-            wait_flags(C::FLAG_A + TWW * wave * 2, 1, 2 * TWW, tag);
+            float o[NP][16];
+            wait_flags(C::FLAG_A + (wave >> 2) * NT, 1, NT, tag);
 #pragma unroll
-            for (int i = 0; i < TWW; i++)
+            for (int p = 0; p < NP; p++)
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const v4f v = __builtin_bit_cast(v4f, take(C::WS_A + ((TWW * wave + i) * 4 + j) * FRAG));
+                    const v4f v = __builtin_bit_cast(v4f, take(C::WS_A, p, j));
 #pragma unroll
-                    for (int k = 0; k < 4; k++) o[i][4 * j + k] = v[k];
+                    for (int k = 0; k < 4; k++) o[p][4 * j + k] = v[k];
                 }
+            quantise(o);
+            lds_barrier();
             float so[KC];
-            quant_exchange(o, so, false);
+            scales(so);
 #pragma unroll
             for (int i = 0; i < TWW; i++) {
                 acc_t acc[KC];
@@ -473,29 +531,45 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 load_tile16(pq + C::A_BOUT + 32 * (iq0 + i), g, bo);
                 const float sw = pq[C::A_SW + 3 * TW + iq0 + i];
 #pragma unroll
-                for (int r = 0; r < 16; r++) x[i][r] = x[i][r] + (chunk_sum<KC, false>(acc, r, so) * sw + bo[r / 4][r % 4]);
-                pin16(x[i]);
+                for (int j = 0; j < 4; j++) {
+                    v4f v;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) v[k] = chunk_sum<KC, false>(acc, 4 * j + k, so) * sw + bo[j][k];
+                    *reinterpret_cast<v4f*>(ex + (TWW * wave + i) * C::EX_TILE + j * FRAG + lane16) = v;
+                }
             }
-            if constexpr (TWW > 1) fetch_ff2(l);
+            lds_barrier();
+#pragma unroll
+            for (int p = 0; p < NP; p++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const v4f v = *reinterpret_cast<const v4f*>(ex + (NP * rk + p) * C::EX_TILE + j * FRAG + (rg * 32 + row) * 16);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) x[p][4 * j + k] = x[p][4 * j + k] + v[k];
+                }
         }
 
         __builtin_amdgcn_sched_barrier(0);
         // ---- LayerNorm 2, quantise, this member's chunk of the hidden row ---------------------------------
         {
-            float y[TWW][16];
-            layernorm(x, pB + C::B_LN2G + 32 * iq0, pB + C::B_LN2B + 32 * iq0, y);
-            quant_exchange(y, sa, false);
+            float y[NP][16];
+            layernorm(x, pr + C::P_B + C::B_LN2G, pr + C::P_B + C::B_LN2B, y);
+            quantise(y);
         }
+        lds_barrier();
         __builtin_amdgcn_sched_barrier(0);
         float sh;
+        if constexpr (TWW > 1) fetch_ff2(l);
         {
-            const float* const pF = par(l, fq) + C::A_FLOATS;
+            const float* const pF = par(l, fq);
             acc_t acc[KC];
+            float sa[KC];
+            scales(sa);
 #pragma unroll
             for (int c = 0; c < KC; c++) acc[c] = product(std::false_type(), SB[c], act + 8 * c * FRAG, zero);
             v4f b1[4];
-            load_tile16(pF + C::B_BFF1 + 128 * fst + 32 * fh, g, b1);
-            const float sw1 = pF[C::B_SW + 4 * fst + fh];
+            load_tile16(pF + C::P_BFF1 + 32 * fh, g, b1);
+            const float sw1 = pF[C::P_B + C::B_SW + 4 * fst + fh];
             float hf[16], am = 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -526,79 +600,113 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         // ---- second matmul over this member's chunk, exchange B ------------------------------------------
         {
-            acc_t own[TWW];
-            const int mine = C::WS_B + (m * 8 + wave) * C::B_PIECE;
 #pragma unroll
             for (int i = 0; i < TWW; i++) {
-                acc_t init = zero;
+                acc_t acc = zero;
                 if constexpr (!FP8) {   // 128 * sum(w): the offset of the unsigned bytes stored as q - 128
                     v4i w0[4];
-                    load_tile16i(pB + C::B_WSUM + m * CW + 32 * (iq0 + i), g, w0);
+                    load_tile16i(pq + C::P_WSUM + 32 * (iq0 + i), g, w0);
 #pragma unroll
-                    for (int r = 0; r < 16; r++) init[r] = w0[r / 4][r % 4];
+                    for (int r = 0; r < 16; r++) acc[r] = w0[r / 4][r % 4];
                 }
-                own[i] = product(std::false_type(), SA[i], hid, init);
+                acc = product(std::false_type(), SA[i], hid, acc);
 #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    __builtin_amdgcn_raw_buffer_store_b128(v4i{accbits(own[i], 4 * j), accbits(own[i], 4 * j + 1), accbits(own[i], 4 * j + 2), accbits(own[i], 4 * j + 3)},
-                                                           wsr, lane16, mine + (4 * i + j) * FRAG, 0);
+                for (int j = 0; j < 4; j++) {
+                    const v4i v = {accbits(acc, 4 * j), accbits(acc, 4 * j + 1), accbits(acc, 4 * j + 2), accbits(acc, 4 * j + 3)};
+                    const int tile = TWW * wave + i;
+                    if constexpr (C::TWO_STEPS) __builtin_amdgcn_raw_buffer_store_b128(v, wsr, lane16, C::WS_B + m * C::ROWS + (tile * 4 + j) * FRAG, 0);
+                    else __builtin_amdgcn_raw_buffer_store_b128(v, wsr, piece_at(t, g), C::WS_B + m * C::ROWS + j * C::ROWS_Q + tile_at(tile), 0);
+                }
             }
-            __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(sh), wsr, lane * 4, mine + 4 * TWW * FRAG, 0);
+            if (wave == 0 && g == 0) __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(sh), wsr, t * 4, C::WS_S + m * 128, 0);
             raise_flag(C::FLAG_B + m * 8 + wave, tag);
-            wait_flags(C::FLAG_B + wave, 8, NWG, tag);
-            float shc[NWG];
+            if constexpr (C::TWO_STEPS) {
+                // wave (i, j): quad j of tile TWW m + i
+                const int i = wave >> 2, j = wave & 3, tile = TWW * m + i, tq2 = tile / TW, ti = tile % TW;
+                wait_flags(C::FLAG_B + m, 8, NWG, tag);
+                v4i piece[NWG];
+                float shc[NWG];
 #pragma unroll
-            for (int c = 0; c < NWG; c++)
-                shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, lane * 4, C::WS_B + (c * 8 + wave) * C::B_PIECE + 4 * TWW * FRAG, SC1));
+                for (int c = 0; c < NWG; c++) {
+                    piece[c] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wsr, lane16, C::WS_B + c * C::ROWS + (tile * 4 + j) * FRAG, SC1));
+                    shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, t * 4, C::WS_S + c * 128, SC1));
+                }
+                const float* const pc = par(l, tq2) + C::P_B;
+                const v4f b2 = ldg4(pc + C::B_BFF2 + 32 * ti + 8 * j + 4 * g);
+                const float sw = pc[C::B_SW + 16 + ti];
+                v4f upd;
 #pragma unroll
-            for (int i = 0; i < TWW; i++) {
+                for (int k = 0; k < 4; k++) {
+                    double o64 = (double)piece[0][k] * (double)shc[0];
+#pragma unroll
+                    for (int c = 1; c < NWG; c++) o64 = __builtin_fma((double)piece[c][k], (double)shc[c], o64);
+                    upd[k] = (float)o64 * sw + b2[k];
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, upd), wsr, piece_at(t, g), C::WS_C + j * C::ROWS_Q + tile_at(tile), 0);
+                raise_flag(C::FLAG_C + m * 8 + wave, tag);
+                wait_flags(C::FLAG_C, 1, NWG * 8, tag);
+#pragma unroll
+                for (int p = 0; p < NP; p++)
+#pragma unroll
+                    for (int jj = 0; jj < 4; jj++) {
+                        const v4f v = __builtin_bit_cast(v4f, take(C::WS_C, p, jj));
+#pragma unroll
+                        for (int k = 0; k < 4; k++) x[p][4 * jj + k] = x[p][4 * jj + k] + v[k];
+                    }
+            } else {
+                wait_flags(C::FLAG_B, 1, NWG * 8, tag);
+                const float* const prB = par(l, rq) + C::P_B;
+                float shc[NWG];
+#pragma unroll
+                for (int c = 0; c < NWG; c++) shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, row * 4, C::WS_S + c * 128, SC1));
+                v4i piece[NWG][4];
+#pragma unroll
+                for (int c = 0; c < NWG; c++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) piece[c][j] = take(C::WS_B + c * C::ROWS, 0, j);
                 double o64[16];
                 float o32[16];
 #pragma unroll
-                for (int c0 = 0; c0 < NWG; c0 += 4) {   // four members' pieces in flight
-                    __builtin_amdgcn_sched_barrier(0);
-                    v4i piece[4][4];
+                for (int c = 0; c < NWG; c++) {
+                    if constexpr (FP8) {
+                        const float sw2 = prB[C::B_SW + 16 + ri * KCF + c];
 #pragma unroll
-                    for (int u = 0; u < 4; u++)
+                        for (int r = 0; r < 16; r++) {
+                            const float part = (__int_as_float(piece[c][r / 4][r % 4]) * shc[c]) * sw2;
+                            o32[r] = c == 0 ? part : o32[r] + part;
+                        }
+                    } else {
+                        const double sc = (double)shc[c];
 #pragma unroll
-                        for (int j = 0; j < 4; j++) piece[u][j] = take(C::WS_B + ((c0 + u) * 8 + wave) * C::B_PIECE + (4 * i + j) * FRAG);
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int c = c0 + u;
-                        if constexpr (FP8) {
-                            const float sw = pB[C::B_SW + 16 + (iq0 + i) * KCF + c];
-#pragma unroll
-                            for (int r = 0; r < 16; r++) {
-                                const float part = (__int_as_float(piece[u][r / 4][r % 4]) * shc[c]) * sw;
-                                o32[r] = c == 0 ? part : o32[r] + part;
-                            }
-                        } else {
-                            const double sc = (double)shc[c];
-#pragma unroll
-                            for (int r = 0; r < 16; r++) {
-                                const double full = (double)piece[u][r / 4][r % 4];
-                                o64[r] = c == 0 ? full * sc : __builtin_fma(full, sc, o64[r]);
-                            }
+                        for (int r = 0; r < 16; r++) {
+                            const double full = (double)piece[c][r / 4][r % 4];
+                            o64[r] = c == 0 ? full * sc : __builtin_fma(full, sc, o64[r]);
                         }
                     }
                 }
-                v4f b2[4];
-                load_tile16(pB + C::B_BFF2 + 32 * (iq0 + i), g, b2);
-                const float sw = pB[C::B_SW + 16 + iq0 + i];
+                const float sw = prB[C::B_SW + 16 + ri];
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    float upd;
-                    if constexpr (FP8) upd = o32[r] + b2[r / 4][r % 4];
-                    else upd = (float)o64[r] * sw + b2[r / 4][r % 4];
-                    x[i][r] = x[i][r] + upd;
+                for (int j = 0; j < 4; j++) {
+                    const v4f b2 = ldg4(pr + C::P_B + C::B_BFF2 + 8 * j);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const int r = 4 * j + k;
+                        float upd;
+                        if constexpr (FP8) upd = o32[r] + b2[k];
+                        else upd = (float)o64[r] * sw + b2[k];
+                        x[0][r] = x[0][r] + upd;
+                    }
                 }
+            }
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
                 if (dead)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) x[i][r] = __builtin_nanf("");
-                pin16(x[i]);
+                    for (int r = 0; r < 16; r++) x[p][r] = __builtin_nanf("");
+                pin16(x[p]);
             }
             fetch_qkv(lnext);
-            fetch_out(SB, lnext, 0);
+            if constexpr (TWW == 1) fetch_out(SB, lnext, 0);
         }
     }
     if (wave == 0 && lane == 0) flags[m] = tag0 + (a.l1 - a.l0);
@@ -606,11 +714,11 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     if constexpr (ENC) {
         if (m == 0)
 #pragma unroll
-            for (int i = 0; i < TWW; i++)
+            for (int p = 0; p < NP; p++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    stream_out(a.taps, ((size_t)b * T + t) * D + 32 * (TWW * wave + i) + 8 * j + 4 * g,
-                               v4f{x[i][4 * j], x[i][4 * j + 1], x[i][4 * j + 2], x[i][4 * j + 3]});
+                    stream_out(a.taps, ((size_t)b * T + row) * D + 32 * (NP * rk + p) + 4 * rg + 8 * j,
+                               v4f{x[p][4 * j], x[p][4 * j + 1], x[p][4 * j + 2], x[p][4 * j + 3]});
         return;
     }
 
@@ -627,17 +735,20 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         for (int f = 0; f < HEAD_SET; f++)
             hw[f] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane_at + f % 4 * FRAG, at + f / 4 * 4 * FRAG, 0));
     };
-    if (m == 0) load_head(wave >> 2, (wave >> 1) & 1, 0);
-    else if (wave < 2) load_head(2, 0, 0);
-    float hn[TWW][16];
-    layernorm(x, gp + C::G_NFG + 32 * TWW * wave, gp + C::G_NFB + 32 * TWW * wave, hn);
-    float* const hnb = qkv;
-    auto publish = [&](const float (&v)[TWW][16]) {
+    // member 0: wave (ht, rh, th) has rows 16 rh .. of head tile ht for tokens 16 th ..; member 1: waves 0 and 1, tile 2
+    const int ht = m == 0 ? wave >> 2 : 2, rh = m == 0 ? (wave >> 1) & 1 : 0;
+    load_head(ht, rh, 0);
+    float hn[NP][16];
+    const float* const gn = gp + 32 * NP * rk + 4 * rg;
+    layernorm(x, gn + C::G_NFG, gn + C::G_NFB, hn);
+    // as operand fragments (tile, quad)
+    float* const hnb = reinterpret_cast<float*>(ex);
+    auto publish = [&](const float (&v)[NP][16]) {
 #pragma unroll
-        for (int i = 0; i < TWW; i++)
+        for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                *reinterpret_cast<v4f*>(hnb + (((TWW * wave + i) * 4 + j) * 64 + lane) * 4) = v4f{v[i][4 * j], v[i][4 * j + 2], v[i][4 * j + 1], v[i][4 * j + 3]};
+                *reinterpret_cast<v4f*>(ex + (NP * rk + p) * C::EX_TILE + j * FRAG + (rg * 32 + row) * 16) = v4f{v[p][4 * j], v[p][4 * j + 2], v[p][4 * j + 1], v[p][4 * j + 3]};
     };
     publish(hn);
     lds_barrier();
@@ -654,7 +765,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
             for (int f = 0; f < HEAD_SET; f++) {
                 const v4f w = __builtin_bit_cast(v4f, hw[f]);
-                const v2f h = *reinterpret_cast<const v2f*>(hp + (f0 + f) * 256);
+                const v2f h = *reinterpret_cast<const v2f*>(hp + (f0 + f) / 4 * (C::EX_TILE / 4) + (f0 + f) % 4 * 256);
                 acc = __builtin_amdgcn_mfma_f32_16x16x4f32(up ? w[1] : w[0], h[0], acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_16x16x4f32(up ? w[3] : w[2], h[1], acc, 0, 0, 0);
             }
@@ -663,7 +774,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     };
     if (m == 0) {
         // policy: squares 32 ht + 16 rh + 4 G .. of token 16 th + c16, optional legal-move AND and argmax
-        const int ht = wave >> 2, rh = (wave >> 1) & 1, th = wave & 1, tk = 16 * th + c16, sq0 = 32 * ht + 16 * rh + 4 * G;
+        const int th = wave & 1, tk = 16 * th + c16, sq0 = 32 * ht + 16 * rh + 4 * G;
         unsigned long long mw = ~0ull;
         if (a.mask) mw = a.mask[(size_t)b * T + tk];
         const v4f hd = head_product(ht, rh, th);
@@ -691,15 +802,15 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 bi = tk_ ? oi : bi;
             }
             if (lane == 0) {
-                xch[2 * XS + wave * 2] = bv;
-                xch[2 * XS + wave * 2 + 1] = __int_as_float(bi);
+                xch[wave * 2] = bv;
+                xch[wave * 2 + 1] = __int_as_float(bi);
             }
             lds_barrier();
             if (wave == 0 && lane == 0) {
 #pragma unroll
                 for (int w = 1; w < 8; w++) {
-                    const float ov = xch[2 * XS + w * 2];
-                    const int oi = __float_as_int(xch[2 * XS + w * 2 + 1]);
+                    const float ov = xch[w * 2];
+                    const int oi = __float_as_int(xch[w * 2 + 1]);
                     const bool tk_ = better(ov, oi, bv, bi);
                     bv = tk_ ? ov : bv;
                     bi = tk_ ? oi : bi;
@@ -730,29 +841,48 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     // pooled heads: the mean over the live tokens of the normalised stream (1), or the final norm of the mean of the
     // residual stream (2), through the value rows like a token; White's frame, so negated when Black is to move
     if (a.vmode != 0) {
-        float pv[TWW][16];
+        // the mean runs over the tokens of a channel, a butterfly over the lanes of the accumulator layout: there and back
+        if (a.vmode == 2) {
+            lds_barrier();   // every wave has finished reading the normalised stream
+            publish(x);
+            lds_barrier();
+        }
         const bool lv = (alive >> t) & 1u;
         const float cdiv = (float)(__builtin_popcount(alive) > 0 ? __builtin_popcount(alive) : 1);
+        v4f pv[TWW][4];
 #pragma unroll
         for (int i = 0; i < TWW; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                float v = lv ? (a.vmode == 1 ? hn[i][r] : x[i][r]) : 0.0f;
+            for (int j = 0; j < 4; j++) {
+                const v4f s = *reinterpret_cast<const v4f*>(ex + (TWW * wave + i) * C::EX_TILE + j * FRAG + lane16);
 #pragma unroll
-                for (int d = 16; d >= 1; d >>= 1) v = v + __shfl_xor(v, d);
-                pv[i][r] = v / cdiv;
+                for (int k = 0; k < 4; k++) {
+                    float v = lv ? s[k] : 0.0f;
+#pragma unroll
+                    for (int d = 16; d >= 1; d >>= 1) v = v + __shfl_xor(v, d);
+                    pv[i][j][k] = v / cdiv;
+                }
             }
-        if (a.vmode == 2) {
-            float hv[TWW][16];
-            layernorm(pv, gp + C::G_NFG + 32 * TWW * wave, gp + C::G_NFB + 32 * TWW * wave, hv);
-#pragma unroll
-            for (int i = 0; i < TWW; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) pv[i][r] = hv[i][r];
-        }
-        lds_barrier();   // every wave has finished reading the normalised stream
-        publish(pv);
         lds_barrier();
+#pragma unroll
+        for (int i = 0; i < TWW; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) *reinterpret_cast<v4f*>(ex + (TWW * wave + i) * C::EX_TILE + j * FRAG + lane16) = pv[i][j];
+        lds_barrier();
+        if (a.vmode == 2) {
+            float v[NP][16], hv[NP][16];
+#pragma unroll
+            for (int p = 0; p < NP; p++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const v4f s = *reinterpret_cast<const v4f*>(ex + (NP * rk + p) * C::EX_TILE + j * FRAG + (rg * 32 + row) * 16);
+                    v[p][4 * j] = s[0]; v[p][4 * j + 2] = s[1]; v[p][4 * j + 1] = s[2]; v[p][4 * j + 3] = s[3];
+                }
+            layernorm(v, gn + C::G_NFG, gn + C::G_NFB, hv);
+            lds_barrier();
+            publish(hv);
+            lds_barrier();
+        }
         if (wave == 0) {
             if constexpr (8 * HB > HEAD_SET) load_head(2, 0, 0);   // else they are still there
             const v4f hd = head_product(2, 0, 0);

@@ -882,12 +882,12 @@ class FusedEncoder:
     def _team_workspace(self, n: int):
         """The exchange memory for a launch of ``n`` positions on the current stream, or None where no
         part of such a launch uses it (at most 64 positions, or what is left of rounds of 512; 512 wide:
-        32, or what is left of rounds of 256)."""
+        of 256)."""
         if not self._team_bytes:
             return None
         wide = self.d_model != self.D
         left = n % 256 if wide else n if self.fp8 else n % 512
-        if not 0 < left <= (32 if wide else 64):
+        if not 0 < left <= 64:
             return None
         if torch.cuda.is_current_stream_capturing():      # a graph has its own, cleared by each replay
             return torch.zeros(self._team_bytes, dtype=torch.uint8, device=self.device)
