@@ -602,6 +602,12 @@ def pack_board_on_device(net, stack, shape: _Shape, fp8: bool, device):
     already lie there in fp32 are read in place.  The blobs are complete when this returns, so that
     any stream may use them."""
     d, f, n_value, device = shape.d_model, shape.d_ff, shape.n_value, torch.device(device)
+    ext = _native()
+    index = torch.cuda.current_device() if device.index is None else device.index
+    if ext is not None and net is not None:
+        blobs = ext.pack_net(net, d, shape.n_layers, f, n_value, shape.eps, fp8, index)
+        if blobs is not None:
+            return blobs
     params = []
     for lay in stack.layers:
         at = lay.self_attn
@@ -616,9 +622,7 @@ def pack_board_on_device(net, stack, shape: _Shape, fp8: bool, device):
     else:
         params += [torch.zeros(*(d,) if r is None else (r, d), device=device) for r in rows]
         params[n_layer_ptrs + 5].fill_(1.0)
-    ext = _native()
     if ext is not None:
-        index = torch.cuda.current_device() if device.index is None else device.index
         return ext.pack_board(params, d, shape.n_layers, f, n_value, shape.eps, fp8, index)
     want = [(d,), (d,), (3 * d, d), (3 * d,), (d, d), (d,), (d,), (d,), (f, d), (f,), (d, f), (d,)] * shape.n_layers
     want += [(d,) if r is None else (r, d) for r in rows]
@@ -643,11 +647,12 @@ def pack_board_on_device(net, stack, shape: _Shape, fp8: bool, device):
     return wstream, fparams
 
 
-def fingerprint_on_device(params):
-    """The weight fingerprint (``bf_fingerprint``) of tensors in name order, or None where they are not
-    all fp32, contiguous and on one GPU (or the extension module is not there)."""
+def fingerprint_on_device(net):
+    """The weight fingerprint (``bf_fingerprint``) of a module, queued on the current stream (``.value()``
+    waits for it), or None where its parameters are not all fp32, contiguous and on one GPU (or the
+    extension module is not there)."""
     ext = _native()
-    return ext.fingerprint(params) if ext is not None else None
+    return ext.fingerprint(net) if ext is not None else None
 
 
 # --------------------------------------------------------------------------- #

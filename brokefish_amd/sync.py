@@ -17,6 +17,14 @@ import torch
 from . import encoder_impl
 
 
+def _fingerprint_on_device(net):
+    """The fingerprint queued on the GPU that holds the parameters, or None."""
+    if not torch.cuda.is_available():
+        return None
+    from .hip_impl import fingerprint_on_device
+    return fingerprint_on_device(net)
+
+
 @torch.no_grad()
 def weight_fingerprint(net) -> float:
     """One float that changes if any parameter does, or if the same values are permuted: an
@@ -24,14 +32,11 @@ def weight_fingerprint(net) -> float:
     Parameters on a GPU (fp32, as a trainer holds them) are summed there, two launches and one wait
     for the whole network; the order of the sum differs from the CPU's, so a value is compared with
     one taken on the same device."""
-    named = sorted(net.named_parameters(), key=lambda kv: kv[0])
-    if named and named[0][1].is_cuda:
-        from .hip_impl import fingerprint_on_device
-        got = fingerprint_on_device([p for _, p in named])
-        if got is not None:
-            return got
+    got = _fingerprint_on_device(net)
+    if got is not None:
+        return got.value()
     acc = 0.0
-    for i, (_, p) in enumerate(named):
+    for i, (_, p) in enumerate(sorted(net.named_parameters(), key=lambda kv: kv[0])):
         f = p.detach().reshape(-1).double()
         idx = torch.arange(1, f.numel() + 1, device=f.device, dtype=torch.float64)
         acc += float(((i + 1) * f * (idx % 9973.0 + 1.0)).sum())
@@ -58,8 +63,10 @@ class PackedWeights:
             raise ValueError(f"this library provides impl 'hip'; impl is {impl!r}")
         kw = {"fp8": True} if fp8 else {"int8": True}
         kw.update(kwargs)
-        return cls(encoder=encoder_impl(impl)(net, **kw), weight_gen=int(weight_gen),
-                   fingerprint=weight_fingerprint(net))
+        queued = _fingerprint_on_device(net)      # runs in front of the packing: one wait for both
+        encoder = encoder_impl(impl)(net, **kw)
+        return cls(encoder=encoder, weight_gen=int(weight_gen),
+                   fingerprint=queued.value() if queued is not None else weight_fingerprint(net))
 
     def evaluate(self):
         """The evaluator the search wants: ``(boards, control, rep) -> fp16 logits, fp32 value``."""
