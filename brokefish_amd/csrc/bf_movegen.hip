@@ -19,7 +19,9 @@
 //     position after the move.
 // En passant, where two pieces leave the board's lines at once, is replayed (a loop that hardly ever
 // runs).  Integer work, bound by the vector ALU: one wavefront per position (its boards built on the
-// scalar unit, each of some 31 moves replayed) took 119 us for 65536 positions, this 24 us (0.9 TB/s of its bytes).
+// scalar unit, each of some 31 moves replayed) took 119 us for 65536 positions, this 24 us, and with the squares'
+// diagonals, knight's and king's steps looked up (839 instead of 1016 vector instructions a wavefront) 19 us (1.1 TB/s
+// of its bytes).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -54,59 +56,64 @@ __device__ __forceinline__ u64 line_attacks(u64 occ, u64 m, u64 s) {
     const u64 down = __brevll(__brevll(o) - __brevll(s));
     return (up ^ down) & m;
 }
-// the four lines through square sq (the square itself excluded)
-struct Lines { u64 rank, file, diag, anti; };
-__device__ __forceinline__ Lines lines_through(int sq) {
-    const int r = sq >> 3, c = sq & 7;
-    const u64 s = bit(sq);
-    Lines l;
-    l.rank = (0xFFull << (8 * r)) ^ s;
-    l.file = (FILE_A << c) ^ s;
-    const int d = r - c;            // a1-h8 direction: 0x8040201008040201 shifted by whole ranks
-    l.diag = (d >= 0 ? 0x8040201008040201ull << (8 * d) : 0x8040201008040201ull >> (8 * -d)) ^ s;
-    const int e = r + c - 7;        // a8-h1 direction
-    l.anti = (e >= 0 ? 0x0102040810204080ull << (8 * e) : 0x0102040810204080ull >> (8 * -e)) ^ s;
-    return l;
-}
-__device__ __forceinline__ u64 rook_attacks(u64 occ, int sq) {
-    const Lines l = lines_through(sq);
-    return line_attacks(occ, l.rank, bit(sq)) | line_attacks(occ, l.file, bit(sq));
-}
-__device__ __forceinline__ u64 bishop_attacks(u64 occ, int sq) {
-    const Lines l = lines_through(sq);
-    return line_attacks(occ, l.diag, bit(sq)) | line_attacks(occ, l.anti, bit(sq));
-}
 __device__ __forceinline__ u64 knight_pattern(u64 s) {
-    return ((s << 17) & NOT_A) | ((s << 10) & NOT_AB) | ((s >> 6) & NOT_AB) | ((s >> 15) & NOT_A) |
-           ((s << 15) & NOT_H) | ((s << 6) & NOT_GH) | ((s >> 10) & NOT_GH) | ((s >> 17) & NOT_H);
+    const u64 near = ((s >> 1) & NOT_H) | ((s << 1) & NOT_A), far = ((s >> 2) & NOT_GH) | ((s << 2) & NOT_AB);
+    return near << 16 | near >> 16 | far << 8 | far >> 8;
 }
 __device__ __forceinline__ u64 king_pattern(u64 s) {
     const u64 row = s | ((s << 1) & NOT_A) | ((s >> 1) & NOT_H);
     return (row | row << 8 | row >> 8) ^ s;
 }
-
-// The pieces of `e` that attack square sq, given occupancy occ.  Looked at from the square: a rook placed
-// there sees the enemy's orthogonal sliders exactly when they see it, and so for the other kinds.
-__device__ __forceinline__ u64 attackers(const Enemy& e, u64 occ, int sq) {
-    const u64 s = bit(sq);
-    // a white pawn on (r-1, c+-1) attacks (r, c); a black one from (r+1, c+-1)
-    const u64 pawn_from = e.black ? (((s << 7) & NOT_H) | ((s << 9) & NOT_A)) : (((s >> 7) & NOT_A) | ((s >> 9) & NOT_H));
-    return (pawn_from & e.pawns) | (knight_pattern(s) & e.knights) | (king_pattern(s) & e.king) |
-           (rook_attacks(occ, sq) & e.orth) | (bishop_attacks(occ, sq) & e.diag);
+__device__ __forceinline__ u64 diagonal(int sq) {   // a1-h8 direction: 0x8040201008040201 shifted by whole ranks
+    const int d = (sq >> 3) - (sq & 7);
+    return (d >= 0 ? 0x8040201008040201ull << (8 * d) : 0x8040201008040201ull >> (8 * -d)) ^ bit(sq);
+}
+__device__ __forceinline__ u64 antidiagonal(int sq) {   // a8-h1 direction
+    const int e = (sq >> 3) + (sq & 7) - 7;
+    return (e >= 0 ? 0x0102040810204080ull << (8 * e) : 0x0102040810204080ull >> (8 * -e)) ^ bit(sq);
 }
 
-// the squares strictly between a and x (one bit each) if they share a line, else none
-__device__ __forceinline__ u64 between(int a, u64 x) {
-    const Lines l = lines_through(a);
-    const u64 line = (l.rank & x) ? l.rank : (l.file & x) ? l.file : (l.diag & x) ? l.diag : (l.anti & x) ? l.anti : 0;
-    const u64 s = bit(a), hi = x > s ? x : s, lo = x > s ? s : x;
+// What a square decides: its lines (the square itself excluded), the knight's and the king's steps from it.
+struct Square { u64 diag, anti, knight, king, rank, file, s; };
+// Large launches look the first four up: a table of 2 KiB in LDS that the workgroup fills at its start, a field by
+// each of its four wavefronts (a field is 10 to 25 instructions, and a lane asks for three squares).
+template <bool TABLE>
+__device__ __forceinline__ Square square(int sq, const ulonglong2 (*table)[2]) {
+    Square q;
+    q.s = bit(sq);
+    q.rank = (0xFFull << (sq & 56)) ^ q.s;
+    q.file = (FILE_A << (sq & 7)) ^ q.s;
+    if constexpr (TABLE) {
+        const ulonglong2 a = table[sq][0], b = table[sq][1];
+        q.diag = a.x; q.anti = a.y; q.knight = b.x; q.king = b.y;
+    } else {
+        q.diag = diagonal(sq); q.anti = antidiagonal(sq); q.knight = knight_pattern(q.s); q.king = king_pattern(q.s);
+    }
+    return q;
+}
+__device__ __forceinline__ u64 rook_attacks(u64 occ, const Square& q) { return line_attacks(occ, q.rank, q.s) | line_attacks(occ, q.file, q.s); }
+__device__ __forceinline__ u64 bishop_attacks(u64 occ, const Square& q) { return line_attacks(occ, q.diag, q.s) | line_attacks(occ, q.anti, q.s); }
+
+// The pieces of `e` that attack square q, given occupancy occ.  Looked at from the square: a rook placed
+// there sees the enemy's orthogonal sliders exactly when they see it, and so for the other kinds.
+__device__ __forceinline__ u64 attackers(const Enemy& e, u64 occ, const Square& q) {
+    // a white pawn on (r-1, c+-1) attacks (r, c); a black one from (r+1, c+-1): the king's steps on the rank behind
+    const u64 pawn_from = q.king & (e.black ? q.s << 7 | q.s << 9 : q.s >> 7 | q.s >> 9);
+    return (pawn_from & e.pawns) | (q.knight & e.knights) | (q.king & e.king) |
+           (rook_attacks(occ, q) & e.orth) | (bishop_attacks(occ, q) & e.diag);
+}
+
+// the squares strictly between q and x (one bit) if they share a line, else none
+__device__ __forceinline__ u64 between(const Square& q, u64 x) {
+    const u64 line = (q.rank & x) ? q.rank : (q.file & x) ? q.file : (q.diag & x) ? q.diag : (q.anti & x) ? q.anti : 0;
+    const u64 hi = x > q.s ? x : q.s, lo = x > q.s ? q.s : x;
     return line & (hi - 1) & ~(lo | (lo - 1));
 }
 
 // OR over the sixteen lanes of a row, in every lane
 template <int CTRL>
 __device__ __forceinline__ unsigned or_ror(unsigned v) {
-    return v | (unsigned)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, false);
+    return v | (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
 }
 __device__ __forceinline__ u64 row_or(u64 v) {
     unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
@@ -117,8 +124,15 @@ __device__ __forceinline__ u64 row_or(u64 v) {
     return ((u64)hi << 32) | lo;
 }
 
+template <bool TABLE>
 __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, const int16_t* control, int n,
                                                       u64* mask, uint8_t* in_check) {
+    __shared__ ulonglong2 table[TABLE ? 64 : 1][2];
+    if constexpr (TABLE) {   // 256 lanes: a wavefront a field
+        const int sq = threadIdx.x & 63, field = threadIdx.x >> 6;
+        reinterpret_cast<u64*>(table[sq])[field] = field == 0 ? diagonal(sq) : field == 1 ? antidiagonal(sq) : field == 2 ? knight_pattern(bit(sq)) : king_pattern(bit(sq));
+        __syncthreads();
+    }
     const int lane = threadIdx.x & 63, slot = lane & 15;
     const int b_ = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 4);
     const bool here = b_ < n;
@@ -152,14 +166,15 @@ __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, co
     const bool rook_long = (__ballot(w == (rookw | home)) >> rowbits) & 0xffff;
 
     // ---- what attacks the king once this lane's piece has left its square (the king's own lane: the check) ----
-    const u64 att = attackers(e, occ & ~fb, ksq);
+    const Square king = square<TABLE>(ksq, table);
+    const u64 att = attackers(e, occ & ~fb, king);
     u64 allowed = ~0ull;
-    if (att) allowed = (att & (att - 1)) ? 0 : att | between(ksq, att);
+    if (att) allowed = (att & (att - 1)) ? 0 : att | between(king, att);
     // a slot without a piece of ours has no moves; the king's lane reports the check
     if (slot == 15 && in_check && here) in_check[b] = att ? 1 : 0;
 
     // ---- this lane's king step or castling square ----
-    const u64 kb = bit(ksq);
+    const u64 kb = king.s;
     unsigned safe;
     {
         const int k9 = slot + (slot >= 4), dr = k9 / 3 - 1, dc = k9 % 3 - 1;
@@ -178,12 +193,13 @@ __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, co
         if (!step) occ2 = (occ2 & ~bit(home + (kingside ? 7 : 0))) | bit(home + (kingside ? 5 : 3));
         Enemy e2 = e;
         e2.pawns &= ~tb; e2.knights &= ~tb; e2.diag &= ~tb; e2.orth &= ~tb;
-        const bool ok = may && attackers(e2, occ2, at) == 0;
+        const bool ok = may && attackers(e2, occ2, square<TABLE>(at, table)) == 0;
         safe = (unsigned)(__ballot(ok) >> rowbits) & 0xffffu;
     }
 
     // ---- the squares this lane's piece reaches ----
     u64 legal = 0, ep = 0;
+    const Square from = square<TABLE>(sq, table);
     if (mine) {
         if (t == PAWN) {
             const int r = sq >> 3;
@@ -199,7 +215,7 @@ __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, co
                 ep = (black ? beside >> 8 : beside << 8) & ~opp;
             }
         } else if (t == KNIGHT) {
-            legal = knight_pattern(fb) & ~own & allowed;
+            legal = from.knight & ~own & allowed;
         } else if (t == KING) {
             const u64 around = (safe & 7u) | ((safe & 8u) << 5) | ((safe & 16u) << 6) | ((u64)(safe & 0xE0u) << 11);
             legal = ksq >= 9 ? around << (ksq - 9) : around >> (9 - ksq);
@@ -207,8 +223,8 @@ __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, co
             if (((safe >> 11) & 7u) == 7u) legal |= bit(home + 2);
         } else if (t == BISHOP || t == ROOK || t == QUEEN) {
             u64 reach = 0;
-            if (t != BISHOP) reach |= rook_attacks(occ, sq);
-            if (t != ROOK) reach |= bishop_attacks(occ, sq);
+            if (t != BISHOP) reach |= rook_attacks(occ, from);
+            if (t != ROOK) reach |= bishop_attacks(occ, from);
             legal = reach & ~own & allowed;
         }
     }
@@ -217,7 +233,7 @@ __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, co
         Enemy e2 = e;
         const u64 gone = tb | victim;
         e2.pawns &= ~gone; e2.knights &= ~gone; e2.diag &= ~gone; e2.orth &= ~gone;
-        if (ep && attackers(e2, ((occ & ~fb) | tb) & ~victim, ksq) == 0) legal |= tb;
+        if (ep && attackers(e2, ((occ & ~fb) | tb) & ~victim, king) == 0) legal |= tb;
         ep &= ep - 1;
     }
     if (here) {
@@ -242,8 +258,8 @@ extern "C" int bf_movegen(const uint16_t* boards, const int16_t* control, int64_
     // four positions per wavefront: workgroups of one wavefront while that spreads a small launch over more
     // compute units (256 of them hold 1024 positions), of four beyond
     const int waves = n <= 4096 ? 1 : 4;
-    hipLaunchKernelGGL(movegen_kernel, dim3((unsigned)((n + 4 * waves - 1) / (4 * waves))), dim3(64 * waves), 0, (hipStream_t)stream,
-                       boards, control, (int)n, reinterpret_cast<u64*>(mask), in_check);
+    hipLaunchKernelGGL(waves == 1 ? movegen_kernel<false> : movegen_kernel<true>, dim3((unsigned)((n + 4 * waves - 1) / (4 * waves))), dim3(64 * waves), 0,
+                       (hipStream_t)stream, boards, control, (int)n, reinterpret_cast<u64*>(mask), in_check);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         char msg[256];
