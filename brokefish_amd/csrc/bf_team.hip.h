@@ -15,8 +15,8 @@
 // So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
 // tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
 // except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
-// 124 -> 84 us, e4m3 155 -> 96, width 512 with 16 layers 750 -> 275; 64 positions 120 -> 88, e4m3 155 -> 100; 32 of the
-// wide network 727 -> 328.  The arithmetic is that of the other kernels, operation for operation: the results are
+// 124 -> 82 us, e4m3 155 -> 95, width 512 with 16 layers 750 -> 273; 64 positions 120 -> 87, e4m3 155 -> 99; 32 of the
+// wide network 727 -> 327.  The arithmetic is that of the other kernels, operation for operation: the results are
 // bit-identical to theirs.
 //
 // Rows and tiles.  For everything per row (LayerNorm, quantisers, residual sums) a wavefront owns the rows of four
@@ -92,9 +92,10 @@ struct Cfg : Layout<DM> {
     static constexpr int WS_A = 4096, WS_B = WS_A + ROWS, WS_S = WS_B + NWG * ROWS;   // [member]: accumulators; scales [member][token]
     // more than four members: exchange B in two steps, each member sums the accumulators of two tiles and gives the sums to all
     static constexpr bool TWO_STEPS = NWG > 4;
-    static constexpr int FLAG_C = FLAG_B + NWG * NW, WS_C = WS_S + NWG * 128;   // the second step: [member][wave]; stream-shaped
+    static constexpr int FLAG_C = FLAG_B + NWG * NW, FLAG_H = FLAG_C + NWG * NW, WS_H = 3072;   // heads: [policy job]; its best move, 16 bytes
+    static constexpr int WS_C = WS_S + NWG * 128;   // the second step: [member][wave]; stream-shaped
     static constexpr int WS_BYTES = (WS_C + (TWO_STEPS ? ROWS : 0) + 4095) / 4096 * 4096;
-    static_assert(NWG <= FLAG_A && FLAG_A + 2 * L::NT <= FLAG_B && (FLAG_C + NWG * NW) * 4 <= WS_A, "flags");
+    static_assert(NWG <= FLAG_A && FLAG_A + 2 * L::NT <= FLAG_B && (FLAG_H + 8) * 4 <= WS_H && WS_H + 8 * 16 <= WS_A, "flags");
     static_assert(!TWO_STEPS || NWG * TWW == L::NT, "a member's tiles are those of one wavefront");
 };
 
@@ -722,8 +723,11 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         return;
     }
 
-    // ---- final norm and heads: member 0 the policy, member 1 promotion and value -------------------------
-    if (m > 1) return;
+    // ---- final norm and heads ------------------------------------------------------------------------------
+    // Ten products of 16 rows of a head tile with 16 tokens, dealt out over the members' first wavefronts (each takes
+    // a SIMD's matrix pipe and 32 KiB of head tile for itself): 0..7 the policy (tile, rows, tokens), 8 and 9 promotion
+    // and value (the first rows of tile 2).
+    const int job = wave * NWG + m;
     const int G = lane >> 4, c16 = lane & 15;
     // the head tile's fragments, HEAD_SET of them; the first ones now
     constexpr int HEAD_SET = 32;
@@ -735,9 +739,8 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         for (int f = 0; f < HEAD_SET; f++)
             hw[f] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane_at + f % 4 * FRAG, at + f / 4 * 4 * FRAG, 0));
     };
-    // member 0: wave (ht, rh, th) has rows 16 rh .. of head tile ht for tokens 16 th ..; member 1: waves 0 and 1, tile 2
-    const int ht = m == 0 ? wave >> 2 : 2, rh = m == 0 ? (wave >> 1) & 1 : 0;
-    load_head(ht, rh, 0);
+    const int ht = job >> 2, rh = job < 8 ? (job >> 1) & 1 : 0, th = job & 1;   // job < 10: rows 16 rh .. of head tile ht, tokens 16 th ..
+    if (job < 10) load_head(ht, rh, 0);
     float hn[NP][16];
     const float* const gn = gp + 32 * NP * rk + 4 * rg;
     layernorm(x, gn + C::G_NFG, gn + C::G_NFB, hn);
@@ -772,9 +775,9 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         }
         return acc;
     };
-    if (m == 0) {
+    if (job < 8) {
         // policy: squares 32 ht + 16 rh + 4 G .. of token 16 th + c16, optional legal-move AND and argmax
-        const int th = wave & 1, tk = 16 * th + c16, sq0 = 32 * ht + 16 * rh + 4 * G;
+        const int tk = 16 * th + c16, sq0 = 32 * ht + 16 * rh + 4 * G;
         unsigned long long mw = ~0ull;
         if (a.mask) mw = a.mask[(size_t)b * T + tk];
         const v4f hd = head_product(ht, rh, th);
@@ -790,35 +793,38 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         if (a.out_fp32) *reinterpret_cast<v4f*>((float*)a.policy + at) = v4f{v[0], v[1], v[2], v[3]};
         else *reinterpret_cast<v4h*>((_Float16*)a.policy + at) = v4h{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
         if (a.mask && a.best) {
-            auto better = [](float ov, int oi, float bv_, int bi_) {   // larger, lowest index on ties; no move at all is worst
-                return oi != 0x7fffffff && (bi_ == 0x7fffffff || ov > bv_ || (ov == bv_ && oi < bi_));
+            // larger, lowest index on ties; no move at all is worst
+            auto merge = [&](float ov, int oi) {
+                const bool take_ = oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi));
+                bv = take_ ? ov : bv;
+                bi = take_ ? oi : bi;
             };
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) {
-                const float ov = __shfl_xor(bv, d);
-                const int oi = __shfl_xor(bi, d);
-                const bool tk_ = better(ov, oi, bv, bi);
-                bv = tk_ ? ov : bv;
-                bi = tk_ ? oi : bi;
-            }
-            if (lane == 0) {
-                xch[wave * 2] = bv;
-                xch[wave * 2 + 1] = __int_as_float(bi);
-            }
-            lds_barrier();
-            if (wave == 0 && lane == 0) {
-#pragma unroll
-                for (int w = 1; w < 8; w++) {
-                    const float ov = xch[w * 2];
-                    const int oi = __float_as_int(xch[w * 2 + 1]);
-                    const bool tk_ = better(ov, oi, bv, bi);
-                    bv = tk_ ? ov : bv;
-                    bi = tk_ ? oi : bi;
-                }
-                a.best[b] = bi == 0x7fffffff ? -1 : bi;
+            auto over_dpp = [&](auto ctrl) {
+                constexpr int c = decltype(ctrl)::value;
+                merge(dpp<c>(bv), __builtin_amdgcn_update_dpp(0, bi, c, 0xf, 0xf, true));
+            };
+            auto over_lanes_of_row = [&]() {   // xor 1, xor 2, the mirrored eight
+                over_dpp(std::integral_constant<int, 0xb1>());
+                over_dpp(std::integral_constant<int, 0x4e>());
+                over_dpp(std::integral_constant<int, 0x141>());
+            };
+            over_lanes_of_row();
+            over_dpp(std::integral_constant<int, 0x140>());
+            merge(__shfl_xor(bv, 16), __shfl_xor(bi, 16));
+            merge(__shfl_xor(bv, 32), __shfl_xor(bi, 32));
+            // the eight wavefronts' winners meet in member 0
+            const int tag = tag0 + (a.l1 - a.l0);
+            if (lane == 0) __builtin_amdgcn_raw_buffer_store_b64(v2u{(unsigned)__float_as_int(bv), (unsigned)bi}, wsr, 0, C::WS_H + job * 16, 0);
+            raise_flag(C::FLAG_H + job, tag);
+            if (job == 0) {
+                wait_flags(C::FLAG_H, 1, 8, tag);
+                const v2u w = __builtin_amdgcn_raw_buffer_load_b64(wsr, (lane & 7) * 16, C::WS_H, SC1);
+                bv = __int_as_float((int)w[0]);
+                bi = (int)w[1];
+                over_lanes_of_row();
+                if (lane == 0) a.best[b] = bi == 0x7fffffff ? -1 : bi;
             }
         }
-        return;
     }
     auto value_of = [&](const v4f& hd) -> float {
         if (a.n_value == 1) return tanh_dev(hd[0]);
@@ -828,9 +834,9 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         return (e2 - e0) / ((e0 + e1) + e2);
     };
     // rows 0..3 of head tile 2 are the promotion rows (lane row 0), rows 4.. the value rows (lane row 1)
-    if (wave < 2) {
-        const v4f hd = head_product(2, 0, wave);
-        const int tk = 16 * wave + c16;
+    if (job == 8 || job == 9) {
+        const v4f hd = head_product(2, 0, th);
+        const int tk = 16 * th + c16;
         if (G == 0) {
             const size_t at = ((size_t)b * T + tk) * 4;
             if (a.out_fp32) *reinterpret_cast<v4f*>((float*)a.promo + at) = hd;
@@ -840,7 +846,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     }
     // pooled heads: the mean over the live tokens of the normalised stream (1), or the final norm of the mean of the
     // residual stream (2), through the value rows like a token; White's frame, so negated when Black is to move
-    if (a.vmode != 0) {
+    if (a.vmode != 0 && m == 0) {   // by all wavefronts of the member that has job 8
         // the mean runs over the tokens of a channel, a butterfly over the lanes of the accumulator layout: there and back
         if (a.vmode == 2) {
             lds_barrier();   // every wave has finished reading the normalised stream
@@ -883,7 +889,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             publish(hv);
             lds_barrier();
         }
-        if (wave == 0) {
+        if (job == 8) {
             if constexpr (8 * HB > HEAD_SET) load_head(2, 0, 0);   // else they are still there
             const v4f hd = head_product(2, 0, 0);
             if (lane == 16) {
