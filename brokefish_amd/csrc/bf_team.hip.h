@@ -15,8 +15,8 @@
 // So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
 // tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
 // except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
-// 124 -> 82 us, e4m3 155 -> 95, width 512 with 16 layers 750 -> 273; 64 positions 120 -> 87, e4m3 155 -> 99; 32 of the
-// wide network 727 -> 327.  The arithmetic is that of the other kernels, operation for operation: the results are
+// 124 -> 82 us, e4m3 155 -> 96, width 512 with 16 layers 750 -> 271; 64 positions 120 -> 87, e4m3 155 -> 99; 32 of the
+// wide network 727 -> 321.  The arithmetic is that of the other kernels, operation for operation: the results are
 // bit-identical to theirs.
 //
 // Rows and tiles.  For everything per row (LayerNorm, quantisers, residual sums) a wavefront owns the rows of four
@@ -89,14 +89,24 @@ struct Cfg : Layout<DM> {
     static constexpr int FLAG_A = 64, FLAG_B = 128;           // dwords: first flag of exchange A [query half][tile], of exchange B [member][wave]
     static constexpr int ROWS = L::NT * 4 * FRAG;             // a stream-shaped piece; an owner wave's part; a quad of that
     static constexpr int ROWS_W = ROWS / NW, ROWS_Q = ROWS_W / 4;
-    static constexpr int WS_A = 4096, WS_B = WS_A + ROWS, WS_S = WS_B + NWG * ROWS;   // [member]: accumulators; scales [member][token]
     // more than four members: exchange B in two steps, each member sums the accumulators of two tiles and gives the sums to all
     static constexpr bool TWO_STEPS = NWG > 4;
+    static constexpr int WS_A = 4096, WS_B = WS_A + ROWS, WS_S = WS_B + NWG * ROWS;   // [member]: accumulators; scales [member][token]
     static constexpr int FLAG_C = FLAG_B + NWG * NW, FLAG_H = FLAG_C + NWG * NW, WS_H = 3072;   // heads: [policy job]; its best move, 16 bytes
-    static constexpr int WS_C = WS_S + NWG * 128;   // the second step: [member][wave]; stream-shaped
+    static constexpr int WS_C = WS_S + NWG * T * 4;   // the second step: [member][wave]; stream-shaped
     static constexpr int WS_BYTES = (WS_C + (TWO_STEPS ? ROWS : 0) + 4095) / 4096 * 4096;
     static_assert(NWG <= FLAG_A && FLAG_A + 2 * L::NT <= FLAG_B && (FLAG_H + 8) * 4 <= WS_H && WS_H + 8 * 16 <= WS_A, "flags");
     static_assert(!TWO_STEPS || NWG * TWW == L::NT, "a member's tiles are those of one wavefront");
+    // Who waits for whom in exchange B.  A wavefront's flag stands for what that wavefront itself stored and for nothing else, so a
+    // reader may load only what was stored by a wavefront whose flag it waits for (tests/test_team_exchange.py goes through all pairs).
+    // In one step it waits for all wavefronts; in two, member m loads what wavefront m of every member stored, and the scales,
+    // which a member's wavefront 0 stores.
+    static constexpr int FLAGS_B = TWO_STEPS ? 2 * NWG : NWG * NW;
+    static constexpr int flag_b(int member, int wave) { return FLAG_B + member * NW + wave; }
+    static constexpr int awaited_b(int reader, int i) { return TWO_STEPS ? flag_b(i % NWG, i < NWG ? reader : 0) : flag_b(0, i); }   // the i-th of FLAGS_B
+    static constexpr int scales_b(int member) { return WS_S + member * T * 4; }
+    static constexpr int piece_b(int member, int tile, int quad) { return WS_B + member * ROWS + (tile * 4 + quad) * FRAG; }   // in two steps
+    static constexpr int tile_b(int member, int wave) { return TWW * member + (wave >> 2); }   // the tile whose accumulators a wavefront sums, in two steps
 };
 
 constexpr int SPIN_LIMIT = 1 << 23;   // polls of some 600 clocks: about two seconds
@@ -297,11 +307,11 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
         for (int c = 0; c < KC; c++) sa[c] = tok[c * 32 + t];
     };
-    // wait until `count` flags, `stride` dwords apart, have reached `tag`
-    auto wait_flags = [&](int first, int stride, int count, int tag) {
+    // wait until `count` flags have reached `tag`; `at`: this lane's one
+    auto wait_flags = [&](int at, int count, int tag) {
         for (int spins = 0; !dead;) {
             int f = tag;
-            if (lane < count) f = (int)__builtin_amdgcn_raw_buffer_load_b32(wsr, lane * (stride * 4), first * 4, SC1);
+            if (lane < count) f = (int)__builtin_amdgcn_raw_buffer_load_b32(wsr, at * 4, 0, SC1);
             if (__all(f - tag >= 0)) break;
             if (++spins > SPIN_LIMIT) dead = true;
             asm volatile("" ::: "memory");
@@ -509,7 +519,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         // ---- exchange A, output projection + residual --------------------------------------------------
         {
             float o[NP][16];
-            wait_flags(C::FLAG_A + (wave >> 2) * NT, 1, NT, tag);
+            wait_flags(C::FLAG_A + (wave >> 2) * NT + lane, NT, tag);
 #pragma unroll
             for (int p = 0; p < NP; p++)
 #pragma unroll
@@ -615,22 +625,22 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 for (int j = 0; j < 4; j++) {
                     const v4i v = {accbits(acc, 4 * j), accbits(acc, 4 * j + 1), accbits(acc, 4 * j + 2), accbits(acc, 4 * j + 3)};
                     const int tile = TWW * wave + i;
-                    if constexpr (C::TWO_STEPS) __builtin_amdgcn_raw_buffer_store_b128(v, wsr, lane16, C::WS_B + m * C::ROWS + (tile * 4 + j) * FRAG, 0);
+                    if constexpr (C::TWO_STEPS) __builtin_amdgcn_raw_buffer_store_b128(v, wsr, lane16, C::piece_b(m, tile, j), 0);
                     else __builtin_amdgcn_raw_buffer_store_b128(v, wsr, piece_at(t, g), C::WS_B + m * C::ROWS + j * C::ROWS_Q + tile_at(tile), 0);
                 }
             }
-            if (wave == 0 && g == 0) __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(sh), wsr, t * 4, C::WS_S + m * 128, 0);
-            raise_flag(C::FLAG_B + m * 8 + wave, tag);
+            if (wave == 0 && g == 0) __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(sh), wsr, t * 4, C::scales_b(m), 0);
+            raise_flag(C::flag_b(m, wave), tag);
+            wait_flags(C::awaited_b(m, lane), C::FLAGS_B, tag);
             if constexpr (C::TWO_STEPS) {
-                // wave (i, j): quad j of tile TWW m + i
-                const int i = wave >> 2, j = wave & 3, tile = TWW * m + i, tq2 = tile / TW, ti = tile % TW;
-                wait_flags(C::FLAG_B + m, 8, NWG, tag);
+                // wave (i, j): quad j of tile i of this member's
+                const int j = wave & 3, tile = C::tile_b(m, wave), tq2 = tile / TW, ti = tile % TW;
                 v4i piece[NWG];
                 float shc[NWG];
 #pragma unroll
                 for (int c = 0; c < NWG; c++) {
-                    piece[c] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wsr, lane16, C::WS_B + c * C::ROWS + (tile * 4 + j) * FRAG, SC1));
-                    shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, t * 4, C::WS_S + c * 128, SC1));
+                    piece[c] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wsr, lane16, C::piece_b(c, tile, j), SC1));
+                    shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, t * 4, C::scales_b(c), SC1));
                 }
                 const float* const pc = par(l, tq2) + C::P_B;
                 const v4f b2 = ldg4(pc + C::B_BFF2 + 32 * ti + 8 * j + 4 * g);
@@ -645,7 +655,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 }
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, upd), wsr, piece_at(t, g), C::WS_C + j * C::ROWS_Q + tile_at(tile), 0);
                 raise_flag(C::FLAG_C + m * 8 + wave, tag);
-                wait_flags(C::FLAG_C, 1, NWG * 8, tag);
+                wait_flags(C::FLAG_C + lane, NWG * 8, tag);
 #pragma unroll
                 for (int p = 0; p < NP; p++)
 #pragma unroll
@@ -655,11 +665,10 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                         for (int k = 0; k < 4; k++) x[p][4 * jj + k] = x[p][4 * jj + k] + v[k];
                     }
             } else {
-                wait_flags(C::FLAG_B, 1, NWG * 8, tag);
                 const float* const prB = par(l, rq) + C::P_B;
                 float shc[NWG];
 #pragma unroll
-                for (int c = 0; c < NWG; c++) shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, row * 4, C::WS_S + c * 128, SC1));
+                for (int c = 0; c < NWG; c++) shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, row * 4, C::scales_b(c), SC1));
                 v4i piece[NWG][4];
 #pragma unroll
                 for (int c = 0; c < NWG; c++)
@@ -817,7 +826,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             if (lane == 0) __builtin_amdgcn_raw_buffer_store_b64(v2u{(unsigned)__float_as_int(bv), (unsigned)bi}, wsr, 0, C::WS_H + job * 16, 0);
             raise_flag(C::FLAG_H + job, tag);
             if (job == 0) {
-                wait_flags(C::FLAG_H, 1, 8, tag);
+                wait_flags(C::FLAG_H + lane, 8, tag);
                 const v2u w = __builtin_amdgcn_raw_buffer_load_b64(wsr, (lane & 7) * 16, C::WS_H, SC1);
                 bv = __int_as_float((int)w[0]);
                 bi = (int)w[1];
