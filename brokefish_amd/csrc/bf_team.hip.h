@@ -33,7 +33,7 @@
 // An exchange: a wavefront stores its piece, waits until the L2 has it (vmcnt), and stores a flag; the wavefronts that
 // need the piece poll the flags past their L1 (sc1) and then load the piece past it (polling tags inside the data
 // itself was slower: every poll is 16 KiB).  Members sit behind one L2 because workgroups go to the XCDs in turn
-// (blockIdx % 8; bf_team_workspace_bytes looks at the device before the form is used).  Flags count layers over all
+// (blockIdx % 8; bf_team_workspace_bytes looks at the device before the form is used).  Flags count layers, modulo 2^32, over all
 // launches of a workspace (each member keeps the count), so nothing is cleared between launches.  Waiting is
 // bounded: a wavefront that has waited some seconds gives up, publishes nothing any more and makes its rows NaN.
 // Members of a team are consecutive workgroups of their XCD and are dispatched in order, so at most NWG - 1
@@ -109,6 +109,11 @@ struct Cfg : Layout<DM> {
     static constexpr int tile_b(int member, int wave) { return TWW * member + (wave >> 2); }   // the tile whose accumulators a wavefront sums, in two steps
 };
 
+// Tags count modulo 2^32 (2^31 layers are some six hours of launches in a row).  A flag of the exchanges is raised in every layer,
+// so it lags by one launch at most; those of the heads are raised in launches with a best move only and may lag by any number.
+struct Reached { __host__ __device__ constexpr bool operator()(unsigned flag, unsigned tag) const { return (int)(flag - tag) >= 0; } };
+struct Equal { __host__ __device__ constexpr bool operator()(unsigned flag, unsigned tag) const { return flag == tag; } };
+
 constexpr int SPIN_LIMIT = 1 << 23;   // polls of some 600 clocks: about two seconds
 constexpr int SC1 = 16;               // cache policy of a load that goes past the L1
 
@@ -152,8 +157,8 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 
     uint8_t* const ws = a.team_ws + (size_t)slot * C::WS_BYTES;
     const __amdgpu_buffer_rsrc_t wsr = __builtin_amdgcn_make_buffer_rsrc(ws, 0, C::WS_BYTES, 0x00020000);
-    int* const flags = reinterpret_cast<int*>(ws);
-    const int tag0 = __builtin_amdgcn_readfirstlane(flags[m]);   // layers of the launches before this one
+    unsigned* const flags = reinterpret_cast<unsigned*>(ws);
+    const unsigned tag0 = (unsigned)__builtin_amdgcn_readfirstlane((int)flags[m]);   // layers of the launches before this one, modulo 2^32
     bool dead = false;                                           // this wave has given up waiting
 
     float* const xch = reinterpret_cast<float*>(lds + C::XCH_OFF);
@@ -307,21 +312,23 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
         for (int c = 0; c < KC; c++) sa[c] = tok[c * 32 + t];
     };
-    // wait until `count` flags have reached `tag`; `at`: this lane's one
-    auto wait_flags = [&](int at, int count, int tag) {
+    // wait until `met` holds of `count` flags and `tag`; `at`: this lane's flag
+    constexpr Reached reached;
+    constexpr Equal equal;
+    auto wait_flags = [&](int at, int count, unsigned tag, auto met) {
         for (int spins = 0; !dead;) {
-            int f = tag;
-            if (lane < count) f = (int)__builtin_amdgcn_raw_buffer_load_b32(wsr, at * 4, 0, SC1);
-            if (__all(f - tag >= 0)) break;
+            unsigned f = tag;
+            if (lane < count) f = __builtin_amdgcn_raw_buffer_load_b32(wsr, at * 4, 0, SC1);
+            if (__all(met(f, tag))) break;
             if (++spins > SPIN_LIMIT) dead = true;
             asm volatile("" ::: "memory");
         }
         asm volatile("" ::: "memory");
     };
     // this wave's piece is stored: let the L2 have it, then raise the flag
-    auto raise_flag = [&](int at, int tag) {
+    auto raise_flag = [&](int at, unsigned tag) {
         wait_vm<0>();
-        if (lane == 0 && !dead) __builtin_amdgcn_raw_buffer_store_b32((unsigned)tag, wsr, 0, at * 4, 0);
+        if (lane == 0 && !dead) __builtin_amdgcn_raw_buffer_store_b32(tag, wsr, 0, at * 4, 0);
     };
     // quad j of tile p of this wave's rows from the stream-shaped piece at `at`
     auto take = [&](int at, int p, int j) -> v4i {
@@ -390,7 +397,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     lds_barrier();
 
     for (int l = a.l0; l < a.l1; l++) {
-        const int tag = tag0 + (l - a.l0) + 1;
+        const unsigned tag = tag0 + (l - a.l0) + 1;
         const int lnext = l + 1 < a.l1 ? l + 1 : l;   // after the last layer its own weights come once more (and are not used)
         const float* const pq = par(l, q);                       // parameters of this wave's matmul tiles
         const float* const pr = par(l, rq) + 32 * ri + 4 * rg;   // of its rows: this lane's chain
@@ -519,7 +526,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         // ---- exchange A, output projection + residual --------------------------------------------------
         {
             float o[NP][16];
-            wait_flags(C::FLAG_A + (wave >> 2) * NT + lane, NT, tag);
+            wait_flags(C::FLAG_A + (wave >> 2) * NT + lane, NT, tag, reached);
 #pragma unroll
             for (int p = 0; p < NP; p++)
 #pragma unroll
@@ -631,7 +638,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             }
             if (wave == 0 && g == 0) __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(sh), wsr, t * 4, C::scales_b(m), 0);
             raise_flag(C::flag_b(m, wave), tag);
-            wait_flags(C::awaited_b(m, lane), C::FLAGS_B, tag);
+            wait_flags(C::awaited_b(m, lane), C::FLAGS_B, tag, reached);
             if constexpr (C::TWO_STEPS) {
                 // wave (i, j): quad j of tile i of this member's
                 const int j = wave & 3, tile = C::tile_b(m, wave), tq2 = tile / TW, ti = tile % TW;
@@ -655,7 +662,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 }
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, upd), wsr, piece_at(t, g), C::WS_C + j * C::ROWS_Q + tile_at(tile), 0);
                 raise_flag(C::FLAG_C + m * 8 + wave, tag);
-                wait_flags(C::FLAG_C + lane, NWG * 8, tag);
+                wait_flags(C::FLAG_C + lane, NWG * 8, tag, reached);
 #pragma unroll
                 for (int p = 0; p < NP; p++)
 #pragma unroll
@@ -822,11 +829,11 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             merge(__shfl_xor(bv, 16), __shfl_xor(bi, 16));
             merge(__shfl_xor(bv, 32), __shfl_xor(bi, 32));
             // the eight wavefronts' winners meet in member 0
-            const int tag = tag0 + (a.l1 - a.l0);
+            const unsigned tag = tag0 + (a.l1 - a.l0);
             if (lane == 0) __builtin_amdgcn_raw_buffer_store_b64(v2u{(unsigned)__float_as_int(bv), (unsigned)bi}, wsr, 0, C::WS_H + job * 16, 0);
             raise_flag(C::FLAG_H + job, tag);
             if (job == 0) {
-                wait_flags(C::FLAG_H + lane, 8, tag);
+                wait_flags(C::FLAG_H + lane, 8, tag, equal);
                 const v2u w = __builtin_amdgcn_raw_buffer_load_b64(wsr, (lane & 7) * 16, C::WS_H, SC1);
                 bv = __int_as_float((int)w[0]);
                 bi = (int)w[1];

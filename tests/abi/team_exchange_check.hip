@@ -1,5 +1,6 @@
 // Host program of tests/test_team_exchange.py: goes through exchange B of the team form as Cfg lays it out, for both
-// network widths, and prints every load whose bytes were stored by a wavefront that the reader does not wait for.
+// network widths, prints every load whose bytes were stored by a wavefront that the reader does not wait for, and compares
+// flags with tags over the wrap of their count.
 #include <cstdio>
 #include <set>
 #include <utility>
@@ -63,7 +64,24 @@ int check() {
 
 }  // namespace
 
+// A flag of the exchanges waited for in one launch is the count of this launch or of one before it: raised or not must be told
+// apart wherever the count stands, and the heads' flags however many launches they were not raised in.
+int check_counts() {
+    int bad = 0;
+    const unsigned starts[] = {0u, 1u, 0x7ffffff0u, 0x7fffffffu, 0x80000000u, 0xfffffff0u, 0xffffffffu};
+    for (unsigned tag0 : starts)
+        for (unsigned layer = 1; layer <= 64; layer++) {
+            const unsigned tag = tag0 + layer;
+            for (unsigned lag = 1; lag <= layer + 64; lag++) bad += bf::team::Reached()(tag - lag, tag) || bf::team::Equal()(tag - lag, tag);
+            for (unsigned lag = 1u << 20; lag; lag <<= 1) bad += bf::team::Equal()(tag - lag, tag);
+            bad += !bf::team::Reached()(tag, tag) || !bf::team::Equal()(tag, tag);
+        }
+    printf("counts: %d faults\n", bad);
+    return bad;
+}
+
 int main() {
+    if (check_counts()) return 1;
     const int narrow = check<256>(), wide = check<512>();
     return narrow || wide;
 }

@@ -4,15 +4,25 @@ walks the layout functions the kernel is compiled with, for both network widths.
 import os
 import subprocess
 
+import pytest
+
 from brokefish_amd import _build
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def test_every_load_of_the_second_exchange_waits_for_its_store(tmp_path):
-    exe = str(tmp_path / "team_exchange_check")
+@pytest.fixture(scope="module")
+def checked(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("team") / "team_exchange_check")
     subprocess.run([_build.hipcc_path(), "-x", "hip", "--cuda-host-only", "-std=c++17", "-O1", "-Wno-unused-command-line-argument",
                     "-I", _build.INCLUDE, "-I", _build.CSRC, os.path.join(HERE, "abi", "team_exchange_check.hip"), "-o", exe], check=True)
-    run = subprocess.run([exe], capture_output=True, text=True)
-    assert run.returncode == 0, run.stdout
-    assert "width 256" in run.stdout and "width 512" in run.stdout
+    return subprocess.run([exe], capture_output=True, text=True).stdout
+
+
+def test_every_load_of_the_second_exchange_waits_for_its_store(checked):
+    for width in (256, 512):
+        assert any(line.startswith(f"width {width}:") and line.endswith(" 0 faults") for line in checked.splitlines()), checked
+
+
+def test_flags_are_told_from_earlier_ones_where_the_count_wraps(checked):
+    assert "counts: 0 faults" in checked, checked

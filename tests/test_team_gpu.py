@@ -85,3 +85,19 @@ def test_team_launches_in_a_graph_and_on_two_streams():
     torch.cuda.synchronize()
     assert_same(a, want_y)
     assert_same(b, want_x)
+
+
+@pytest.mark.parametrize("shape,start", [("base", 2 ** 31 - 5), ("base", 2 ** 32 - 5), ("wide", 2 ** 31 - 5)])
+def test_the_count_of_layers_wraps(shape, start):
+    team, single = pair(shape)
+    x = batch(9)
+    team.forward_masked(*x)
+    ws, = team._team.values()
+    flags = ws.view(torch.int32).view(64 if shape == "base" else 32, -1)[:, :768]     # the counts and the flags of every position
+    flags.fill_(start if start < 2 ** 31 else start - 2 ** 32)
+    want = [t.clone() for t in single.forward_masked(*x)]
+    for i in range(6):           # two layers each: before, over and behind the wrap
+        if i == 3:               # a launch that raises no flag of the heads
+            assert_same(team.forward_full(*x[:3]), single.forward_full(*x[:3]))
+        else:
+            assert_same(team.forward_masked(*x), want)
