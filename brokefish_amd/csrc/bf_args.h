@@ -133,6 +133,7 @@ struct KArgs {
     float eps;
     float* xpark;                 // workspace: 32 KiB per board slot, residual stream parked during the FFN
     uint8_t* team_ws;             // exchange buffers of the team form (several workgroups per position)
+    int* team_gave_up;            // host memory: becomes 1 when a wavefront of that form gives up waiting
     unsigned long long* profile;  // [N_PHASES] cycle sums over waves, profile builds only
     bf_taps taps;
 };
@@ -206,5 +207,9 @@ hipError_t launch_team512(const KArgs& k, hipStream_t stream);
 hipError_t launch_team512_enc(const KArgs& k, hipStream_t stream);
 size_t team_slot_bytes(int d_model);
 int team_positions(int d_model, bool look);
+// The word of the current device that team launches report a give-up in (team_positions() has found the device fit), and
+// whether one has been reported since this was last asked
+int* team_report_word();
+bool team_gave_up();
 
 }  // namespace bf

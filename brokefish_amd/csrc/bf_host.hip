@@ -85,6 +85,8 @@ extern "C" size_t bf_team_workspace_bytes(const bf_shape* s) {
     return bf::team_positions(s->d_model, true) * bf::team_slot_bytes(s->d_model);
 }
 
+extern "C" int bf_team_gave_up(void) { return bf::team_gave_up() ? 1 : 0; }
+
 extern "C" size_t bf_layer_stride_floats(const bf_shape* s) {
     if (!shape_ok(s)) return 0;
     return bf::PARAM_FLOATS;
@@ -289,7 +291,8 @@ static int team_limit(const bf_eval_args* a, const bf::KArgs& k, bool enc) {
     return fits < (size_t)most ? (int)fits : most;
 }
 
-static hipError_t launch_team(const bf_eval_args* a, const bf::KArgs& k, bool enc, hipStream_t stream) {
+static hipError_t launch_team(const bf_eval_args* a, bf::KArgs k, bool enc, hipStream_t stream) {
+    k.team_gave_up = bf::team_report_word();
     if (a->shape.d_model == 512) return (enc ? bf::launch_team512_enc : bf::launch_team512)(k, stream);
     if (a->quant == BF_QUANT_E4M3) return (enc ? bf::launch_team256_fp8_enc : bf::launch_team256_fp8)(k, stream);
     return (enc ? bf::launch_team256_enc : bf::launch_team256)(k, stream);
@@ -299,6 +302,9 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
     const int grid = (k.n + bf::WAVES - 1) / bf::WAVES;
     hipError_t e;
     if (!bf::device_is_gfx950()) return BF_ERR_DEVICE;
+    if (bf::team_gave_up())
+        return fail(BF_ERR_TEAM, "an earlier launch on this device gave up waiting for compute units held by other launches and its outputs "
+                                 "are NaN (see team_workspace of bf_eval_args); nothing was launched now");
     const bool enc = !k.profile && enc_build(a, kind);
     // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
     // position 124 -> 84 us, e4m3 155 -> 96; 512 wide 750 -> 275 us), and so does what is left of the 512-wide

@@ -35,9 +35,14 @@
 // itself was slower: every poll is 16 KiB).  Members sit behind one L2 because workgroups go to the XCDs in turn
 // (blockIdx % 8; bf_team_workspace_bytes looks at the device before the form is used).  Flags count layers, modulo 2^32, over all
 // launches of a workspace (each member keeps the count), so nothing is cleared between launches.  Waiting is
-// bounded: a wavefront that has waited some seconds gives up, publishes nothing any more and makes its rows NaN.
+// bounded: a wavefront that has waited some seconds gives up.  It publishes nothing any more, so that everybody who needs
+// its pieces gives up too; its member's outputs become NaN, the best move -1, and a word in host memory tells the library,
+// which reports it with the next call (BF_ERR_TEAM).
 // Members of a team are consecutive workgroups of their XCD and are dispatched in order, so at most NWG - 1
-// workgroups of a launch per XCD ever wait for a unit to come free.
+// workgroups of a launch per XCD ever wait for a unit to come free.  With 32 units per XCD that allows ten launches at a
+// time on a device, all processes together (width 512: four); were there more, incomplete teams could hold every unit
+// of an XCD and wait for one another until they give up.  A process stays below that by itself with HIP's four
+// hardware queues; with more than the bound allows (GPU_MAX_HW_QUEUES) the form is not used.
 //
 // One set of exchange buffers per team is enough: a member writes A, B or C of layer l + 1 only after barriers that
 // follow all its wavefronts' loads of the last exchange of layer l from all members, and every wavefront loads A of a
@@ -113,6 +118,9 @@ struct Cfg : Layout<DM> {
 // so it lags by one launch at most; those of the heads are raised in launches with a best move only and may lag by any number.
 struct Reached { __host__ __device__ constexpr bool operator()(unsigned flag, unsigned tag) const { return (int)(flag - tag) >= 0; } };
 struct Equal { __host__ __device__ constexpr bool operator()(unsigned flag, unsigned tag) const { return flag == tag; } };
+
+// Whether launches on `queues` hardware queues at a time, teams of `members`, leave a unit of an XCD to somebody who completes a team
+__host__ __device__ constexpr bool units_suffice(int queues, int members, int units) { return (long long)queues * (members - 1) < units; }
 
 constexpr int SPIN_LIMIT = 1 << 23;   // polls of some 600 clocks: about two seconds
 constexpr int SC1 = 16;               // cache policy of a load that goes past the L1
@@ -320,7 +328,10 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             unsigned f = tag;
             if (lane < count) f = __builtin_amdgcn_raw_buffer_load_b32(wsr, at * 4, 0, SC1);
             if (__all(met(f, tag))) break;
-            if (++spins > SPIN_LIMIT) dead = true;
+            if (++spins > SPIN_LIMIT) {
+                dead = true;
+                if (lane == 0) *a.team_gave_up = 1;
+            }
             asm volatile("" ::: "memory");
         }
         asm volatile("" ::: "memory");
@@ -770,7 +781,10 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 *reinterpret_cast<v4f*>(ex + (NP * rk + p) * C::EX_TILE + j * FRAG + (rg * 32 + row) * 16) = v4f{v[p][4 * j], v[p][4 * j + 2], v[p][4 * j + 1], v[p][4 * j + 3]};
     };
     publish(hn);
+    if (lane == 0) xch[wave * 64] = dead ? 1.0f : 0.0f;   // a wave that has given up stands for its member
     lds_barrier();
+#pragma unroll
+    for (int w = 0; w < 8; w++) dead |= __builtin_amdgcn_readfirstlane(__float_as_int(xch[w * 64])) != 0;
     // (elements 0 and 2 of a register quad lie together, as do 1 and 3.)
     // Rows 16 rh .. of head tile `ht` times tokens 16 th ..: the chain of the 32x32x2 form, two of whose steps (four k) are
     // one step here.  Lane (row or token, k) takes element k / 2 and 2 + k / 2 of the fragment lane of half k % 2.
@@ -791,12 +805,16 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         }
         return acc;
     };
+    auto marked = [&](const v4f& v) -> v4f {
+        const float nan = __builtin_nanf("");
+        return dead ? v4f{nan, nan, nan, nan} : v;
+    };
     if (job < 8) {
         // policy: squares 32 ht + 16 rh + 4 G .. of token 16 th + c16, optional legal-move AND and argmax
         const int tk = 16 * th + c16, sq0 = 32 * ht + 16 * rh + 4 * G;
         unsigned long long mw = ~0ull;
         if (a.mask) mw = a.mask[(size_t)b * T + tk];
-        const v4f hd = head_product(ht, rh, th);
+        const v4f hd = marked(head_product(ht, rh, th));
         float bv = -__builtin_inff(), v[4];
         int bi = 0x7fffffff;
 #pragma unroll
@@ -838,11 +856,12 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 bv = __int_as_float((int)w[0]);
                 bi = (int)w[1];
                 over_lanes_of_row();
-                if (lane == 0) a.best[b] = bi == 0x7fffffff ? -1 : bi;
+                if (lane == 0) a.best[b] = dead || bi == 0x7fffffff ? -1 : bi;
             }
         }
     }
     auto value_of = [&](const v4f& hd) -> float {
+        if (dead) return __builtin_nanf("");   // (the functions below need not hand a NaN on)
         if (a.n_value == 1) return tanh_dev(hd[0]);
         const float r0 = hd[0], r1 = hd[1], r2 = hd[2];   // classes loss, draw, win
         const float mx = __builtin_fmaxf(__builtin_fmaxf(r0, r1), r2);
@@ -851,7 +870,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     };
     // rows 0..3 of head tile 2 are the promotion rows (lane row 0), rows 4.. the value rows (lane row 1)
     if (job == 8 || job == 9) {
-        const v4f hd = head_product(2, 0, th);
+        const v4f hd = marked(head_product(2, 0, th));
         const int tk = 16 * th + c16;
         if (G == 0) {
             const size_t at = ((size_t)b * T + tk) * 4;

@@ -112,6 +112,7 @@ def load_library():
         L.bf_board_fparams_floats.restype = C.c_size_t
         L.bf_team_workspace_bytes.restype = C.c_size_t
         L.bf_team_workspace_bytes.argtypes = [C.POINTER(_Shape)]
+        L.bf_team_gave_up.restype = C.c_int
         L.bf_board_fparams_floats.argtypes = [C.POINTER(_Shape)]
         L.bf_pack_scratch_floats.restype = C.c_size_t
         L.bf_pack_scratch_floats.argtypes = [C.POINTER(_Shape)]

@@ -26,7 +26,8 @@ enum bf_status {
     BF_ERR_ARGUMENT = -1,   /* null / misaligned pointer, bad size or mode */
     BF_ERR_UNSUPPORTED = -2, /* network shape this build has no kernel for */
     BF_ERR_LAUNCH = -3,     /* hipLaunchKernel reported an error */
-    BF_ERR_DEVICE = -4      /* not a gfx950 device */
+    BF_ERR_DEVICE = -4,     /* not a gfx950 device */
+    BF_ERR_TEAM = -5        /* an EARLIER launch gave up waiting, see team_workspace of bf_eval_args */
 };
 
 /* Operand format of the four weight matmuls of every layer.
@@ -109,8 +110,13 @@ size_t bf_board_fparams_floats(const bf_shape* s);
 
 /* Size of team_workspace of bf_eval_args: the largest launch of that form on the current device, 0 where the
  * device (or its partitioning) or the shape does not carry it.  The first call on a device looks how its
- * workgroups are placed (one small launch and a synchronisation); the form runs only after such a call. */
+ * workgroups are placed (one small launch and a synchronisation, and 4 KiB of pinned host memory that the
+ * process keeps); the form runs only after such a call. */
 size_t bf_team_workspace_bytes(const bf_shape* s);
+/* Whether a launch of that form on the current device has given up waiting since this was last asked or
+ * BF_ERR_TEAM was last returned: 1 or 0.  For callers that replay graphs, or want to know once a stream has
+ * been synchronised; every other call that launches the evaluator asks by itself. */
+int bf_team_gave_up(void);
 
 /* Packing of a network that lies in fp32 on the device into the BOARD / TWIN / OCTO / DUO blobs
  * (board_wstream: bf_board_wstream_bytes, board_fparams: bf_board_fparams_floats), quantised and laid
@@ -235,7 +241,15 @@ typedef struct {
      * aligned) through which the workgroups of one position exchange what they computed.  With it AUTO gives the
      * smallest launches, and a short last round, to a form that spreads a position over several compute
      * units; the results are the same bits.  Zero before its first use and then left alone by the caller;
-     * launches that may overlap need workspaces of their own. */
+     * launches that may overlap need workspaces of their own.
+     * At most ten launches of this form may be under way on a device at a time (512 wide: four; a wide one
+     * counts 7 and another one 3 of 31), over all streams and PROCESSES.  A process with HIP's default of four hardware
+     * queues (GPU_MAX_HW_QUEUES; streams of one priority) stays below that by itself, and where GPU_MAX_HW_QUEUES
+     * alone allows more the form is not used; several processes that share a GPU and may exceed it together
+     * pass no team workspace (FusedEncoder: kernel="octo").  Otherwise launches may hold the compute units each
+     * other's workgroups wait for.  After some two seconds such a launch gives up and ends: outputs it could
+     * not compute are NaN, best_move is -1, and the next call that launches the evaluator on this device
+     * launches nothing and returns BF_ERR_TEAM (once). */
     void* team_workspace;
     size_t team_workspace_bytes;
 } bf_eval_args;

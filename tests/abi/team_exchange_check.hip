@@ -80,8 +80,25 @@ int check_counts() {
     return bad;
 }
 
+// The launches of a process must leave a unit of every XCD to somebody who completes a team: in the worst case each of
+// them has all members of a team but one in place.
+int check_units() {
+    int bad = 0;
+    for (int members : {bf::team::Cfg<256>::NWG, bf::team::Cfg<512>::NWG})
+        for (int units = 1; units <= 40; units++)
+            for (int queues = 1; queues <= 32; queues++) {
+                int left = units;
+                for (int i = 0; i < queues; i++) left -= left < members - 1 ? left : members - 1;
+                bad += bf::team::units_suffice(queues, members, units) != (left > 0);
+            }
+    bad += !bf::team::units_suffice(4, bf::team::Cfg<512>::NWG, 32) || bf::team::units_suffice(5, bf::team::Cfg<512>::NWG, 32);
+    bad += !bf::team::units_suffice(10, bf::team::Cfg<256>::NWG, 32) || bf::team::units_suffice(11, bf::team::Cfg<256>::NWG, 32);
+    printf("units: %d faults\n", bad);
+    return bad;
+}
+
 int main() {
-    if (check_counts()) return 1;
+    if (check_counts() || check_units()) return 1;
     const int narrow = check<256>(), wide = check<512>();
     return narrow || wide;
 }

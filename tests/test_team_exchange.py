@@ -26,3 +26,7 @@ def test_every_load_of_the_second_exchange_waits_for_its_store(checked):
 
 def test_flags_are_told_from_earlier_ones_where_the_count_wraps(checked):
     assert "counts: 0 faults" in checked, checked
+
+
+def test_the_form_is_used_only_where_a_process_leaves_units_to_complete_a_team(checked):
+    assert "units: 0 faults" in checked, checked

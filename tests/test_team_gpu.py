@@ -87,6 +87,29 @@ def test_team_launches_in_a_graph_and_on_two_streams():
     assert_same(b, want_x)
 
 
+@pytest.mark.parametrize("shape,head,wdl", [("base", "king", False), ("base", "prenorm", True), ("wide", "king", True)])
+def test_a_launch_that_gives_up_marks_its_outputs_and_is_reported(shape, head, wdl):
+    # member 0 of every position counts ahead of the others: it waits for flags they do not raise in this launch, gives
+    # up at the limit of its waiting, and the others, who need its pieces, do so too: the launch ends
+    team, single = pair(shape, head=head, wdl=wdl)
+    x = batch(3)
+    want = [t.clone() for t in single.forward_masked(*x)]
+    assert_same(team.forward_masked(*x), want)
+    ws, = team._team.values()
+    saved = ws.clone()
+    ws.view(torch.int32).view(64 if shape == "base" else 32, -1)[:, 0] += 1000
+    policy, promo, value, best = team.forward_masked(*x)
+    torch.cuda.synchronize()
+    legal = ((x[3].unsqueeze(-1) >> torch.arange(64, device="cuda")) & 1).bool()
+    assert bool((best == -1).all()) and bool(value.isnan().all()) and bool(promo.isnan().all())
+    assert bool(policy[legal].isnan().all()) and bool((policy[~legal] == float("-inf")).all())
+    ws.copy_(saved)
+    with pytest.raises(RuntimeError, match="gave up"):
+        team.forward_masked(*x)
+    assert_same(team.forward_masked(*x), want)                                 # reported once
+    assert team._lib.bf_team_gave_up() == 0
+
+
 @pytest.mark.parametrize("shape,start", [("base", 2 ** 31 - 5), ("base", 2 ** 32 - 5), ("wide", 2 ** 31 - 5)])
 def test_the_count_of_layers_wraps(shape, start):
     team, single = pair(shape)
