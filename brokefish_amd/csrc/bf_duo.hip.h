@@ -110,7 +110,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     {
         int cnt = a.n, first = NP * (int)blockIdx.x;
         if (a.leaf_index) {
-            cnt = *a.leaf_count;
+            cnt = *a.leaf_count < a.n ? *a.leaf_count : a.n;   // the list has n entries whatever the count says
             if (a.list_split) {
                 if (NP == 1) first += cnt - round_rest(cnt);
                 else cnt -= round_rest(cnt);

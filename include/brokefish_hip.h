@@ -234,7 +234,8 @@ typedef struct {
      * workgroups past the count leave at once, so no host round trip is needed to learn how many
      * leaves a simulation step produced.  Inputs are read and outputs written at the position's own
      * row, as with `active` (which must be NULL when a list is given); rows of positions not in the
-     * list stay untouched.  Both or neither. */
+     * list stay untouched.  Of a count above n the first n entries are taken; entries that are no position of
+     * the launch are passed over.  Both or neither. */
     const int32_t* leaf_index;
     const int32_t* leaf_count;
     /* optional: DEVICE memory of team_workspace_bytes (bf_team_workspace_bytes(shape) serves every launch; 256-byte

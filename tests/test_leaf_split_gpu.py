@@ -35,3 +35,21 @@ def test_live_counts_at_the_edges_of_a_round(made, live):
         for g, w in zip(got, want):
             assert torch.equal(g[on], w[on]), how
             assert bool((g[~on] == 7.0).all()), how            # rows of the others are left as they were
+
+
+@pytest.mark.parametrize("n,kernel", [(1300, "auto"), (1201, "auto"), (601, "duo"), (257, "auto"), (90, "auto"), (33, "auto"), (90, "twin"), (90, "board"), (90, "quad")])
+def test_of_a_count_above_n_the_first_n_entries_are_taken(n, kernel):
+    # a list longer than the launch, and a count that says so: what lies behind the n-th entry is no business of this launch
+    torch.manual_seed(0)
+    net = BrokefishNet(n_layers=1).eval().randomise_layers_(seed=7)
+    model = encoder_impl("hip")(net, int8=True, kernel=kernel)
+    b, c, r, _ = [t.cuda() for t in positions.random_positions(n, plies=80, seed=7)]
+    want = [t.clone() for t in model.forward_full(b, c, r)]
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(n)).int()
+    index = torch.cat([order, torch.zeros(700, dtype=torch.int32)]).cuda()
+    for count in (n, n + 1, n + 300, n + 600):
+        for t in (model.policy_out, model.promo_out, model.value_out):
+            t.fill_(7.0)
+        got = model.forward_full(b, c, r, leaves=(index, torch.tensor([count], dtype=torch.int32, device="cuda")))
+        for g, w in zip(got, want):
+            assert torch.equal(g, w), count
