@@ -17,8 +17,10 @@
 // with the logits it might need staged in LDS, remains for wavefronts in which a pawn promotes).
 // Reductions run over DPP and lane swaps, ranks and counts over ballots; the edges are put together in
 // LDS and leave as whole 16-byte pieces.  The truncation threshold (the E-th largest log-prior) is
-// found by bisection on the ordered bit pattern of the float.  A position with more than 128 candidates
-// (a constructed one, or an arbitrary mask) takes the whole wavefront, every pass walking the bits again.
+// found by bisection on the ordered bit pattern of the float.  More than 128 candidates of a position take a
+// second build of the same code with twice the rounds (5000 positions of 218 moves: 15 us; holding all of them to
+// its size would cost the others 8 %, 20 % where rows truncate), more than 256 (no legal position, an
+// arbitrary mask) the whole wavefront for the one position, every pass walking the bits again (184 us).
 // Bound by instruction issue and, from some 16384 positions on, by HBM; one position per wavefront with
 // staged logits took 48 us for 65536 positions (E = 96), this 23 us (4 TB/s of its bytes).
 #include <hip/hip_runtime.h>
@@ -150,8 +152,17 @@ __device__ __forceinline__ int kth_bit(unsigned lo, unsigned hi, int k) {
 }
 
 constexpr int EXPAND_WAVES = 4;       // wavefronts per workgroup
-constexpr int ROUNDS = 4;             // candidates of a position in the two-position form: 32 per round
-constexpr int CAND_CAP = 32 * ROUNDS;
+// Candidates of a position in the two-position form, 32 per round: a wavefront in which a position has more than the few
+// rounds hold (128; random games have 31, a board of queens up to 218) runs the form of eight rounds.
+constexpr int FEW_ROUNDS = 4, MOST_ROUNDS = 8;
+constexpr int CAND_CAP = 32 * MOST_ROUNDS;
+
+struct Shared {   // a half's part of the LDS
+    int16_t* code;
+    _Float16* prior;
+    float* add;          // promotion log-probability of a candidate
+    unsigned* owner;     // one byte per candidate
+};
 
 template <bool FP32>
 __device__ __forceinline__ float logit(const void* p, size_t i) {
@@ -272,46 +283,15 @@ __device__ void expand_many(const KExpand& a, int b, int lane) {
     if (lane == 0) write_counts(a, b, n_edges, total, trunc, s_all, s_keep);
 }
 
-template <bool FP32>
-__global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand a) {
-    __shared__ __attribute__((aligned(16))) int16_t code_lds[EXPAND_WAVES][2][CAND_CAP];
-    __shared__ __attribute__((aligned(16))) _Float16 prior_lds[EXPAND_WAVES][2][CAND_CAP];
-    __shared__ float add_lds[EXPAND_WAVES][2][CAND_CAP];      // promotion log-probability of a candidate
-    __shared__ unsigned owner_lds[EXPAND_WAVES][2][CAND_CAP / 4];   // one byte per candidate
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, s = lane & 31, half = lane >> 5;
-    const int j = 2 * (blockIdx.x * EXPAND_WAVES + wv) + half;
-    // the half's position; a half without one has no candidates and stores nothing
-    int b = j;
-    bool ok = j < a.n;
-    if (a.leaf_index) {
-        ok = ok && j < *a.leaf_count;
-        b = ok ? a.leaf_index[j] : 0;
-        ok = ok && (unsigned)b < (unsigned)a.n;
-    }
-    if (ok && a.active) ok = a.active[b] != 0;
-    if (!ok) b = 0;
-    if (__ballot(ok) == 0) return;                       // no workgroup barrier below: a wave may leave
-
-    const unsigned word = a.boards[(size_t)b * 32 + s];
-    const int ctrl = a.control[b];
-    const uint64_t m64 = ok ? a.mask[(size_t)b * 32 + s] : 0;
-    const bool pawn = ((word >> 11) & 1u) == 0 && ((word >> 6) & 7u) == PAWN;
-    // last rank of the side to move: rank 7 (squares 56..63) for white, rank 0 for black
-    const uint64_t pr = pawn ? m64 & (ctrl < 0 ? 0xFFull : 0xFFull << 56) : 0;
-    const int cnt = __popcll(m64) + 3 * __popcll(pr);
-    const int inc = half_scan_add(cnt), before = inc - cnt;
-    const int total0 = __builtin_amdgcn_readlane(inc, 31), total1 = __builtin_amdgcn_readlane(inc, 63);
-    const int total = half ? total1 : total0, most = max(total0, total1);
-    if (most > CAND_CAP) {
-        const int b0 = __builtin_amdgcn_readlane(b, 0), b1 = __builtin_amdgcn_readlane(b, 32);
-        const unsigned long long oks = __ballot(ok);
-        if (oks & 1) expand_many<FP32>(a, b0, lane);
-        if (oks >> 32) expand_many<FP32>(a, b1, lane);
-        return;
-    }
+// The candidates of a wavefront's two positions, one half each (lane s of it owns slot s): m64 its legal-move word, pr the
+// squares of it that promote, cnt its candidates and before those of the slots in front; total0 / total1 the two
+// positions' (most: the larger, at most 32 ROUNDS).  A half's result does not depend on the other one.
+template <bool FP32, int ROUNDS>
+__device__ __forceinline__ void expand_pair(const KExpand& a, const Shared& sh, int b, bool ok, int s, int half, uint64_t m64, uint64_t pr, int cnt, int before,
+                                            int total0, int total1, int total, int most) {
     const int rounds = (most + 31) >> 5;
-    int16_t* const cc = code_lds[wv][half];
-    float* const add = add_lds[wv][half];
+    int16_t* const cc = sh.code;
+    float* const add = sh.add;
     const size_t row = (size_t)b * 2048;
     float l[ROUNDS], e[ROUNDS];
     int code[ROUNDS];
@@ -324,8 +304,9 @@ __global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand
     }
     if (__ballot(pr != 0) == 0) {
         // the slot a candidate belongs to: the last one whose first index is not beyond it
-        unsigned char* const owner = reinterpret_cast<unsigned char*>(owner_lds[wv][half]);
-        owner_lds[wv][half][s] = 0;
+        unsigned char* const owner = reinterpret_cast<unsigned char*>(sh.owner);
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r += 4) sh.owner[8 * r + s] = 0;
         wave_lds_sync();
         if (cnt) owner[before] = (unsigned char)s;
         wave_lds_sync();
@@ -443,12 +424,10 @@ __global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand
     _Float16* const ep = a.edge_prior + (size_t)b * a.E;
     if (a.whole_rows) {
         // rows of whole 16-byte pieces: put together in LDS, unused slots (no edge) included
-        _Float16* const pp = prior_lds[wv][half];
+        _Float16* const pp = sh.prior;
         typedef int v4i __attribute__((ext_vector_type(4)));
-        if (s < CAND_CAP / 8) {
-            reinterpret_cast<v4i*>(cc)[s] = v4i{0, 0, 0, 0};
-            reinterpret_cast<v4i*>(pp)[s] = v4i{0, 0, 0, 0};
-        }
+        reinterpret_cast<v4i*>(cc)[s] = v4i{0, 0, 0, 0};
+        reinterpret_cast<v4i*>(pp)[s] = v4i{0, 0, 0, 0};
         wave_lds_sync();
 #pragma unroll
         for (int r = 0; r < ROUNDS; r++)
@@ -475,6 +454,59 @@ __global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand
             }
     }
     if (ok && s == 0) write_counts(a, b, n_edges, total, trunc, s_all, s_keep);
+}
+
+template <bool FP32>
+__global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand a) {
+    __shared__ __attribute__((aligned(16))) int16_t code_lds[EXPAND_WAVES][2][CAND_CAP];
+    __shared__ __attribute__((aligned(16))) _Float16 prior_lds[EXPAND_WAVES][2][CAND_CAP];
+    __shared__ float add_lds[EXPAND_WAVES][2][CAND_CAP];
+    __shared__ unsigned owner_lds[EXPAND_WAVES][2][CAND_CAP / 4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, s = lane & 31, half = lane >> 5;
+    const int j = 2 * (blockIdx.x * EXPAND_WAVES + wv) + half;
+    // the half's position; a half without one has no candidates and stores nothing
+    int b = j;
+    bool ok = j < a.n;
+    if (a.leaf_index) {
+        ok = ok && j < *a.leaf_count;
+        b = ok ? a.leaf_index[j] : 0;
+        ok = ok && (unsigned)b < (unsigned)a.n;
+    }
+    if (ok && a.active) ok = a.active[b] != 0;
+    if (!ok) b = 0;
+    if (__ballot(ok) == 0) return;                       // no workgroup barrier below: a wave may leave
+
+    const unsigned word = a.boards[(size_t)b * 32 + s];
+    const int ctrl = a.control[b];
+    uint64_t m64 = ok ? a.mask[(size_t)b * 32 + s] : 0;
+    const bool pawn = ((word >> 11) & 1u) == 0 && ((word >> 6) & 7u) == PAWN;
+    // last rank of the side to move: rank 7 (squares 56..63) for white, rank 0 for black
+    uint64_t pr = pawn ? m64 & (ctrl < 0 ? 0xFFull : 0xFFull << 56) : 0;
+    int cnt = __popcll(m64) + 3 * __popcll(pr);
+    const int inc = half_scan_add(cnt);
+    int before = inc - cnt;
+    int total0 = __builtin_amdgcn_readlane(inc, 31), total1 = __builtin_amdgcn_readlane(inc, 63);
+    int total = half ? total1 : total0, most = max(total0, total1);
+    if (most > CAND_CAP) {
+        // a position with more goes through the whole wavefront first and leaves an empty half behind; the other
+        // half's goes on as it would beside any neighbour
+        if (total0 > CAND_CAP) expand_many<FP32>(a, __builtin_amdgcn_readlane(b, 0), lane);
+        if (total1 > CAND_CAP) expand_many<FP32>(a, __builtin_amdgcn_readlane(b, 32), lane);
+        const bool many = total > CAND_CAP;
+        ok = ok && !many;
+        if (__ballot(ok) == 0) return;
+        m64 = many ? 0 : m64;
+        pr = many ? 0 : pr;
+        cnt = many ? 0 : cnt;
+        before = many ? 0 : before;
+        total0 = total0 > CAND_CAP ? 0 : total0;
+        total1 = total1 > CAND_CAP ? 0 : total1;
+        total = half ? total1 : total0;
+        most = max(total0, total1);
+    }
+    const Shared sh = {code_lds[wv][half], prior_lds[wv][half], add_lds[wv][half], owner_lds[wv][half]};
+    if (most <= 32 * FEW_ROUNDS) expand_pair<FP32, FEW_ROUNDS>(a, sh, b, ok, s, half, m64, pr, cnt, before, total0, total1, total, most);
+    else expand_pair<FP32, MOST_ROUNDS>(a, sh, b, ok, s, half, m64, pr, cnt, before, total0, total1, total, most);
 }
 
 }  // namespace

@@ -36,6 +36,35 @@ def test_edge_rows_do_not_depend_on_their_form(n, edges):
             assert abs(float(got["dropped"][i]) - (1 - float(logp[i, at].sum()) / float(logp[i, :k].sum()))) < 5e-3
 
 
+def with_candidates(counts, seed):
+    """Positions with legal-move words of so many set bits (arbitrary ones beyond chess), and logits with ties."""
+    n = len(counts)
+    b, c, _, _ = positions.random_positions(n, plies=150, seed=seed, stamp_queen=True)
+    g = torch.Generator().manual_seed(seed)
+    bits = torch.zeros(n, 2048, dtype=torch.int64)
+    for i, k in enumerate(counts):
+        bits[i, torch.randperm(2048, generator=g)[:k]] = 1
+    m = (bits.view(n, 32, 64) << torch.arange(64)).sum(-1)
+    logits = [(torch.randint(-24, 25, (n, 32, k), generator=g) / 8).half() for k in (64, 4)]
+    return [t.cuda() for t in (*logits, torch.rand(n, generator=g), m, b, c)]
+
+
+@pytest.mark.parametrize("edges", [32, 96, 100, 136])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_edges_of_a_position_do_not_depend_on_its_neighbour(edges, fp32):
+    counts = [0, 1, 31, 33, 90, 110, 128, 129, 160, 218, 230, 256, 257, 400]      # promotions add to some of them
+    p, q, v, m, b, c = with_candidates(counts, 3)
+    if fp32:
+        p, q = p.float(), q.float()
+    k = len(counts)
+    alone = [expand_edges(p[i:i + 1], q[i:i + 1], v[i:i + 1], m[i:i + 1], b[i:i + 1], c[i:i + 1], edges) for i in range(k)]
+    at = torch.cartesian_prod(torch.arange(k), torch.arange(k)).flatten().cuda()   # every position beside every other, on either side
+    pairs = expand_edges(p[at], q[at], v[at], m[at], b[at], c[at], edges)
+    for name, got in pairs.items():
+        want = torch.cat([a[name] for a in alone])[at]
+        assert torch.equal(got.view(torch.int16) if got.dtype is torch.float16 else got, want.view(torch.int16) if want.dtype is torch.float16 else want), name
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 16383, 16384, 16385, 49999])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_compaction_at_the_edges_of_its_workgroups(n, shift):
