@@ -81,9 +81,9 @@ __device__ __forceinline__ int wave_exclusive(int v, int lane) {
     }
     return inc - v;
 }
-// bit pattern whose unsigned order is the order of the floats
+// bit pattern whose unsigned order is the order of the floats (-0 + 0 is 0: the two zeros are one value)
 __device__ __forceinline__ unsigned ordered(float f) {
-    const unsigned u = __float_as_uint(f);
+    const unsigned u = __float_as_uint(f + 0.0f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 // what one lane of this wave wrote to LDS is read by another: LDS operations of a wave are carried

@@ -65,6 +65,18 @@ def test_edges_of_a_position_do_not_depend_on_its_neighbour(edges, fp32):
         assert torch.equal(got.view(torch.int16) if got.dtype is torch.float16 else got, want.view(torch.int16) if want.dtype is torch.float16 else want), name
 
 
+@pytest.mark.parametrize("count", [40, 120, 200, 300])
+def test_the_two_zeros_are_one_value_at_the_cut(count):
+    # every log-prior is a zero of either sign: the cut falls among ties, which canonical order decides
+    p, q, v, m, b, c = with_candidates([count] * 8, 5)
+    b |= 0x40                                                   # no pawns (a promotion would split its move's mass)
+    p = torch.where(torch.rand(p.shape, generator=torch.Generator().manual_seed(1)) < 0.5, -0.0, 0.0).half().cuda()
+    got = expand_edges(p, q, v, m, b, c, 32)
+    for i in range(8):
+        bits = ((m[i].unsqueeze(-1) >> torch.arange(64, device="cuda")) & 1).flatten().nonzero().flatten()
+        assert torch.equal(got["edge_move"][i].int(), bits[:32].int()) and torch.equal(got["edge_prior"][i].float(), torch.full((32,), 1 / 32, device="cuda"))
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 16383, 16384, 16385, 49999])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_compaction_at_the_edges_of_its_workgroups(n, shift):
