@@ -85,6 +85,8 @@ extern "C" size_t bf_team_workspace_bytes(const bf_shape* s) {
     return bf::team_positions(s->d_model, true) * bf::team_slot_bytes(s->d_model);
 }
 
+extern "C" size_t bf_team_position_bytes(const bf_shape* s) { return board_shape_ok(s) ? bf::team_slot_bytes(s->d_model) : 0; }
+
 extern "C" int bf_team_gave_up(void) { return bf::team_gave_up() ? 1 : 0; }
 
 extern "C" size_t bf_layer_stride_floats(const bf_shape* s) {

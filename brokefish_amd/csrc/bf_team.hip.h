@@ -96,7 +96,7 @@ struct Cfg : Layout<DM> {
     static constexpr int ROWS_W = ROWS / NW, ROWS_Q = ROWS_W / 4;
     // more than four members: exchange B in two steps, each member sums the accumulators of two tiles and gives the sums to all
     static constexpr bool TWO_STEPS = NWG > 4;
-    static constexpr int WS_A = 4096, WS_B = WS_A + ROWS, WS_S = WS_B + NWG * ROWS;   // [member]: accumulators; scales [member][token]
+    static constexpr int WS_A = BF_TEAM_FLAG_BYTES, WS_B = WS_A + ROWS, WS_S = WS_B + NWG * ROWS;   // [member]: accumulators; scales [member][token]
     static constexpr int FLAG_C = FLAG_B + NWG * NW, FLAG_H = FLAG_C + NWG * NW, WS_H = 3072;   // heads: [policy job]; its best move, 16 bytes
     static constexpr int WS_C = WS_S + NWG * T * 4;   // the second step: [member][wave]; stream-shaped
     static constexpr int WS_BYTES = (WS_C + (TWO_STEPS ? ROWS : 0) + 4095) / 4096 * 4096;

@@ -112,6 +112,8 @@ def load_library():
         L.bf_board_fparams_floats.restype = C.c_size_t
         L.bf_team_workspace_bytes.restype = C.c_size_t
         L.bf_team_workspace_bytes.argtypes = [C.POINTER(_Shape)]
+        L.bf_team_position_bytes.restype = C.c_size_t
+        L.bf_team_position_bytes.argtypes = [C.POINTER(_Shape)]
         L.bf_team_gave_up.restype = C.c_int
         L.bf_board_fparams_floats.argtypes = [C.POINTER(_Shape)]
         L.bf_pack_scratch_floats.restype = C.c_size_t
@@ -883,7 +885,15 @@ class FusedEncoder:
         if ws is not None:
             a.team_workspace, a.team_workspace_bytes, a._keep = ws.data_ptr(), ws.numel(), ws
 
-    TEAM_STREAMS = 16      # streams whose exchange memory is kept (13 MB each, 512 wide 21)
+    TEAM_STREAMS = 16      # streams whose exchange memory is kept (11 MB each, 512 wide 21)
+    TEAM_FLAG_BYTES = 4096 # of a position's part, what has to be zero before its first use (BF_TEAM_FLAG_BYTES)
+
+    def _captured_team_workspace(self, n: int):
+        # a captured launch has its own, of the size it needs (172 KB a position, 512 wide 664), whose flags each replay clears
+        part = int(self._lib.bf_team_position_bytes(C.byref(self._shape)))
+        ws = torch.empty(min(n, self._team_bytes // part), part, dtype=torch.uint8, device=self.device)
+        ws[:, :self.TEAM_FLAG_BYTES].zero_()
+        return ws.view(-1)
 
     def _team_workspace(self, n: int):
         """The exchange memory for a launch of ``n`` positions on the current stream, or None where no
@@ -895,8 +905,8 @@ class FusedEncoder:
         left = n % 256 if wide else n if self.fp8 else n % 512
         if not 0 < left <= 64:
             return None
-        if torch.cuda.is_current_stream_capturing():      # a graph has its own, cleared by each replay
-            return torch.zeros(self._team_bytes, dtype=torch.uint8, device=self.device)
+        if torch.cuda.is_current_stream_capturing():
+            return self._captured_team_workspace(left)
         key = torch.cuda.current_stream(self.device).cuda_stream
         ws = self._team.get(key)
         if ws is None:

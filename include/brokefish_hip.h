@@ -113,6 +113,10 @@ size_t bf_board_fparams_floats(const bf_shape* s);
  * workgroups are placed (one small launch and a synchronisation, and 4 KiB of pinned host memory that the
  * process keeps); the form runs only after such a call. */
 size_t bf_team_workspace_bytes(const bf_shape* s);
+/* Of which a position of a launch takes so much (0 for an unsupported shape): a workspace of fewer serves launches of as
+ * many positions.  Of each part only the first BF_TEAM_FLAG_BYTES have to be zero before its first use. */
+size_t bf_team_position_bytes(const bf_shape* s);
+#define BF_TEAM_FLAG_BYTES 4096
 /* Whether a launch of that form on the current device has given up waiting since this was last asked or
  * BF_ERR_TEAM was last returned: 1 or 0.  For callers that replay graphs, or want to know once a stream has
  * been synchronised; every other call that launches the evaluator asks by itself. */
@@ -241,7 +245,7 @@ typedef struct {
     /* optional: DEVICE memory of team_workspace_bytes (bf_team_workspace_bytes(shape) serves every launch; 256-byte
      * aligned) through which the workgroups of one position exchange what they computed.  With it AUTO gives the
      * smallest launches, and a short last round, to a form that spreads a position over several compute
-     * units; the results are the same bits.  Zero before its first use and then left alone by the caller;
+     * units; the results are the same bits.  Zero before its first use (bf_team_position_bytes) and then left alone by the caller;
      * launches that may overlap need workspaces of their own.
      * At most ten launches of this form may be under way on a device at a time (512 wide: four; a wide one
      * counts 7 and another one 3 of 31), over all streams and PROCESSES.  A process with HIP's default of four hardware

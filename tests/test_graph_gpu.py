@@ -1,8 +1,10 @@
 """The device chain (move generation -> evaluator -> edge expansion) under HIP graph capture.
 
-Small launches are latency-bound (a 64-position evaluation is 0.12 ms of kernel time), so a search
-would capture the chain once and replay it.  None of the three entry points allocates, waits on
-the host or clears memory with a memset node, so the chain can be captured as it is.  Each replay
+Small launches are latency-bound (a 64-position evaluation is 0.09 ms of kernel time), so a search
+would capture the chain once and replay it.  None of the three entry points waits on the host or clears
+memory with a memset node, so the chain can be captured as it is.  What a captured call allocates comes from
+the graph's pool: its outputs where the caller gives none, and the exchange memory of a launch that spreads its
+positions over several compute units, whose flags (4 KB a position) each replay clears.  Each replay
 is checked against the eager chain on the same inputs, with eager work and synchronisations
 between the replays.
 """

@@ -87,6 +87,31 @@ def test_team_launches_in_a_graph_and_on_two_streams():
     assert_same(b, want_x)
 
 
+@pytest.mark.parametrize("shape,n,parts", [("base", 3, 3), ("base", 512 + 9, 9), ("wide", 20, 20), ("wide", 50, 32)])
+def test_a_captured_launch_has_exchange_memory_of_its_size_and_clears_its_flags(shape, n, parts):
+    team, single = pair(shape)
+    x = batch(n)
+    want = [t.clone() for t in single.forward_masked(*x)]
+    team.forward_masked(*x)
+    taken = []
+    make = team._captured_team_workspace
+    team._captured_team_workspace = lambda k: taken.append(make(k)) or taken[-1]
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = team.forward_masked(*x)
+    ws, = taken
+    assert ws.numel() == parts * (team._team_bytes // (64 if shape == "base" else 32))
+    ws = ws.view(parts, -1)
+    for junk in (0, 0x55, 0xff):          # what a replay finds there does not matter, and it clears no more than the flags
+        ws.fill_(junk)
+        g.replay()
+        torch.cuda.synchronize()
+        assert_same(out, want)
+        # the counts start anew (two layers; the wide network's fifty positions are two launches), and nothing else was cleared
+        assert bool((ws.view(torch.int32)[:, 0] <= 4).all()) and bool((ws[:, 2048:3072] == 0).all()) and bool((ws[:, -256:] == junk).all())
+
+
 @pytest.mark.parametrize("shape,head,wdl", [("base", "king", False), ("base", "prenorm", True), ("wide", "king", True)])
 def test_a_launch_that_gives_up_marks_its_outputs_and_is_reported(shape, head, wdl):
     # member 0 of every position counts ahead of the others: it waits for flags they do not raise in this launch, gives
