@@ -167,19 +167,22 @@ __device__ __forceinline__ float div255(float m) {
     return __builtin_fmaf(__builtin_fmaf(-q, 255.0f, m), c, q);
 }
 
-// 1 / x, correctly rounded: the hardware's reciprocal and one Newton step (equal to IEEE division for
-// every mantissa and every exponent whose reciprocal is a normal number, checked on the device
-// exhaustively; the compiler's division takes 11 instructions, four times as many).
+// 1 / x, correctly rounded for 2^-126 <= |x| <= 2^126: the hardware's reciprocal and one Newton step (the compiler's
+// division takes 11 instructions, four times as many).  Beyond: NaN for 0, subnormal and infinite x, 0 for others.
+// Callers: scales (2^-126 to 2^125), softmax denominators (1 to 32), roots.  tests/test_quotient_gpu.py goes through every x.
 __device__ __forceinline__ float recip(float x) {
     const float r = __builtin_amdgcn_rcpf(x);
     return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
 }
-// 1 / sqrt(x) as a correctly rounded square root and a correctly rounded reciprocal of it (the square root
-// from the hardware's reciprocal root and one residual: exact for 2^-67 <= x < 2^53, checked likewise).
+// 1 / sqrt(x) as a correctly rounded square root and a correctly rounded reciprocal of it, the square root
+// from the hardware's reciprocal root and one residual: for 2^-102 <= x < 2^128 (checked likewise), and 0 for an infinite
+// x, the variance of a row whose squares overflow.  Below 2^-102 (an epsilon of 0, or nearly) the residual loses bits
+// and the last one of the result may differ; 0 and subnormal x give NaN.
 __device__ __forceinline__ float recip_sqrt(float x) {
     const float y = __builtin_amdgcn_rsqf(x);
     const float s0 = x * y;
-    return recip(__builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0));
+    const float r = recip(__builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0));
+    return x == __builtin_inff() ? 0.0f : r;
 }
 
 // The reciprocal of an activation scale in two floats, hi = fl(1 / sa) and lo the rest of it, so that
@@ -188,7 +191,8 @@ __device__ __forceinline__ float recip_sqrt(float x) {
 // rounded quotient, ties included.  The product's own error is 2^-48 of the quotient, so only pairs
 // whose quotient lies that close to the edge of a tie's rounding interval could differ; there are
 // 7564 such pairs of significands within sixteen times that distance, and all agree
-// (tests/test_quotient.py enumerates them; the last term of lo is what two of them need).
+// (tests/test_quotient.py enumerates them; the last term of lo is what two of them need).  For scales above
+// 2^102 lo loses bits to the subnormal range, and a quotient within 2^-20 of a tie may go either way.
 struct Quot { float hi, lo; };
 __device__ __forceinline__ Quot quot_by(float sa) {
     const float hi = recip(sa);

@@ -194,6 +194,28 @@ __global__ void quant_probe(const float* x, float scale, long n4, unsigned* out)
 
 }  // namespace
 
+// recip() and recip_sqrt() on a caller's values
+template <bool ROOT>
+__global__ void recip_probe(const float* x, long n, float* out) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = ROOT ? bf::recip_sqrt(x[i]) : bf::recip(x[i]);
+}
+
+extern "C" int bf_recip_probe(int mode, const float* x, int64_t n, float* out, void* stream) {
+    if (!x || !out || n < 1 || n > (1ll << 30) || ((uintptr_t)x & 3) || ((uintptr_t)out & 3) || (mode != BF_PROBE_RECIP && mode != BF_PROBE_RECIP_SQRT)) {
+        bf::set_error("bf_recip_probe: x and out (4-byte aligned) must not be NULL, n in [1, 2^30], mode BF_PROBE_RECIP or BF_PROBE_RECIP_SQRT");
+        return BF_ERR_ARGUMENT;
+    }
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    if (mode == BF_PROBE_RECIP_SQRT) hipLaunchKernelGGL(recip_probe<true>, grid, block, 0, (hipStream_t)stream, x, (long)n, out);
+    else hipLaunchKernelGGL(recip_probe<false>, grid, block, 0, (hipStream_t)stream, x, (long)n, out);
+    if (hipGetLastError() != hipSuccess) {
+        bf::set_error("bf_recip_probe: launch failed");
+        return BF_ERR_LAUNCH;
+    }
+    return BF_OK;
+}
+
 extern "C" int bf_quant_probe(int mode, const float* x, float scale, int64_t n, uint8_t* out, void* stream) {
     if (!x || !out || n < 4 || (n & 3) || ((uintptr_t)x & 15) || ((uintptr_t)out & 3) || !(scale > 0.0f)) {
         bf::set_error("bf_quant_probe: x (16-byte aligned) and out (4-byte aligned) must not be NULL, n a positive multiple of 4, scale > 0");

@@ -139,6 +139,8 @@ def load_library():
         L.bf_stream_rate.argtypes = [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
         L.bf_quant_probe.restype = C.c_int
         L.bf_quant_probe.argtypes = [C.c_int, C.c_void_p, C.c_float, C.c_int64, C.c_void_p, C.c_void_p]
+        L.bf_recip_probe.restype = C.c_int
+        L.bf_recip_probe.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p]
         L.bf_abi_tag.restype = C.c_uint64
         # the ctypes mirror of bf_eval_args must be the struct the library was compiled with: a
         # shorter one would make the library read pointers from beyond it
@@ -292,6 +294,20 @@ def quant_probe(x, scale: float, mode: str = "s8"):
                                 C.c_void_p(torch.cuda.current_stream(x.device).cuda_stream))
     if rc:
         raise RuntimeError(f"bf_quant_probe failed ({rc}): {lib.bf_last_error().decode()}")
+    return out
+
+
+def recip_probe(x, root: bool = False):
+    """The kernels' ``1 / x``, or with ``root`` their ``1 / sqrt(x)`` (``bf_recip_probe``): ``x`` float32 on the GPU."""
+    if x.dtype is not torch.float32 or not x.is_cuda or x.numel() < 1:
+        raise ValueError("x must be float32 on the GPU")
+    x = x.contiguous()
+    out = torch.empty_like(x)
+    lib = load_library()
+    with torch.cuda.device(x.device):
+        rc = lib.bf_recip_probe(int(root), x.data_ptr(), x.numel(), out.data_ptr(), C.c_void_p(torch.cuda.current_stream(x.device).cuda_stream))
+    if rc:
+        raise RuntimeError(f"bf_recip_probe failed ({rc}): {lib.bf_last_error().decode()}")
     return out
 
 

@@ -87,7 +87,11 @@ enum bf_value_mode {
 
 /* Network shape.  Supported: d_model 256, n_heads 8, d_ff 1024 (all kernels, int8 and e4m3)
  * and d_model 512, n_heads 16, d_ff 2048 (BOARD kernel, int8); head width 32, any
- * n_layers >= 1, n_value 1 (tanh scalar) or 3 (loss/draw/win classes). */
+ * n_layers >= 1, n_value 1 (tanh scalar) or 3 (loss/draw/win classes).
+ * Range of the arithmetic: rows are quantised exactly as stated up to magnitudes of 2^108 (beyond, a value that
+ * lies on a tie may go either way); LayerNorm's
+ * variance + eps is exact from 2^-102 on (eps = 0 is accepted, a constant row then gives NaN), and a row whose
+ * squares overflow normalises to beta. */
 typedef struct {
     int32_t d_model, n_layers, n_heads, d_ff, n_value;
     float eps;
@@ -345,6 +349,10 @@ double bf_stream_rate(const void* buf, size_t bytes, int workgroups, int reps, i
  * :190-227).  Asynchronous on `stream`. */
 enum bf_probe_mode { BF_PROBE_S8 = 0, BF_PROBE_U8_RELU = 1, BF_PROBE_E4M3 = 2 };
 int bf_quant_probe(int mode, const float* x, float scale, int64_t n, uint8_t* out, void* stream);
+/* The kernels' reciprocal and reciprocal square root on their own, for tests: out[i] of x[i] (DEVICE memory).
+ * Asynchronous on `stream`. */
+enum bf_recip_mode { BF_PROBE_RECIP = 0, BF_PROBE_RECIP_SQRT = 1 };
+int bf_recip_probe(int mode, const float* x, int64_t n, float* out, void* stream);
 
 /* In-kernel phase accounting, the counterpart of the reference's profile hooks
  * (reference csrc/encoder.cu:1083-1177 and :1886-1903: set_profile / read_profile /

@@ -30,7 +30,8 @@ def _round32(x: F) -> F:
 
 
 def _quot(v: F, sa: F) -> F:
-    """quot(v, quot_by(sa)) as the device computes it; the reciprocal is correctly rounded (recip)."""
+    """quot(v, quot_by(sa)) as the device computes it; the reciprocal is correctly rounded (recip, which
+    tests/test_quotient_gpu.py holds to that on the device)."""
     hi = _round32(1 / sa)
     rem = _round32(1 - sa * hi)
     lo = _round32(rem * hi + _round32(_round32(rem * hi) * (rem / 2)))
