@@ -167,6 +167,15 @@ __device__ __forceinline__ float div255(float m) {
     return __builtin_fmaf(__builtin_fmaf(-q, 255.0f, m), c, q);
 }
 
+// The activation scale of a row whose largest magnitude is m, and of a row of the hidden layer (unsigned in int8).
+// A row below 2^-118 counts as zero: its scale would be subnormal, which the reciprocal does not take, and what it
+// adds to an output is below 2^-100 of a weight.
+constexpr float LEAST_ROW = 0x1p-118f;
+template <bool FP8>
+__device__ __forceinline__ float row_scale(float m) { return m >= LEAST_ROW ? (FP8 ? m * 0.125f : div127(m)) : 1.0f; }
+template <bool FP8>
+__device__ __forceinline__ float hidden_scale(float m) { return m >= LEAST_ROW ? (FP8 ? m * 0.125f : div255(m)) : 1.0f; }
+
 // 1 / x, correctly rounded for 2^-126 <= |x| <= 2^126: the hardware's reciprocal and one Newton step (the compiler's
 // division takes 11 instructions, four times as many).  Beyond: NaN for 0, subnormal and infinite x, 0 for others.
 // Callers: scales (2^-126 to 2^125), softmax denominators (1 to 32), roots.  tests/test_quotient_gpu.py goes through every x.
@@ -250,7 +259,7 @@ __device__ __forceinline__ void quant_s8(const float (&y)[NTILES][16], int g, v4
 #pragma unroll
         for (int r = 0; r < 16; r++) am = __builtin_fmaxf(am, __builtin_fabsf(y[n][r]));
     am = __builtin_fmaxf(am, partner(am, g));
-    sa = am > 0.0f ? (FP8 ? am * 0.125f : div127(am)) : 1.0f;
+    sa = row_scale<FP8>(am);
     const Quot by = quot_by(sa);
 #pragma unroll
     for (int n = 0; n < NTILES; n++)

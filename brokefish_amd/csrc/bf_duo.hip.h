@@ -317,7 +317,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
             for (int w = 0; w < C::NW; w++) m = __builtin_fmaxf(m, xch[2 * XS + p * PS + w * 64 + lane]);
             m = __builtin_fmaxf(m, partner(m, g));
-            sa[p] = m > 0.0f ? (FP8 ? m * 0.125f : div127(m)) : 1.0f;
+            sa[p] = row_scale<FP8>(m);
             if (publish_scales && wave == 0 && g == 0) tok[p * 32 + t] = sa[p];
             const Quot by = quot_by(sa[p]);
             v4i w;
@@ -720,7 +720,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                         m = __builtin_fmaxf(m, __builtin_fmaxf(xch[xs + p * PS + (2 * c + 4 * u) * 64 + lane],
                                                                xch[xs + p * PS + (2 * c + 1 + 4 * u) * 64 + lane]));
                     m = __builtin_fmaxf(m, partner(m, g));
-                    sh[p][2 * st + c] = m > 0.0f ? (FP8 ? m * 0.125f : div255(m)) : 1.0f;
+                    sh[p][2 * st + c] = hidden_scale<FP8>(m);
                 }
                 const float s8 = q < 2 ? sh[p][2 * st] : sh[p][2 * st + 1];
                 const Quot by = quot_by(s8);

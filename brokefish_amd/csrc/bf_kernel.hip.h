@@ -453,7 +453,7 @@ __global__ __launch_bounds__(THREADS, 1) void eval_kernel(const KArgs a) {
                     // for the signed MFMA, the offset is added back through wsum.
                     // e4m3: the ordinary signed quantiser (the values are non-negative).
                     am = __builtin_fmaxf(am, partner(am, g));
-                    const float s8 = am > 0.0f ? am / (FP8 ? 8.0f : 255.0f) : 1.0f;
+                    const float s8 = hidden_scale<FP8>(am);
                     const Quot by = quot_by(s8);
                     sh[c] = s8;
 #pragma unroll

@@ -305,7 +305,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; r++) am = __builtin_fmaxf(am, __builtin_fabsf(y[p][r]));
         am = chunkmax(am);
-        const float sa = am > 0.0f ? (FP8 ? am * 0.125f : div127(am)) : 1.0f;
+        const float sa = row_scale<FP8>(am);
         if (rg == 0 && rk % (8 / KC) == 0) tok[rk / (8 / KC) * 32 + row] = sa;
         const Quot by = quot_by(sa);
 #pragma unroll
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
             for (int w = 0; w < 8; w++) mx = __builtin_fmaxf(mx, xch[w * 64 + lane]);
             mx = __builtin_fmaxf(mx, partner(mx, g));
-            sh = mx > 0.0f ? (FP8 ? mx * 0.125f : div255(mx)) : 1.0f;
+            sh = hidden_scale<FP8>(mx);
             const Quot by = quot_by(sh);
             v4i w;
 #pragma unroll

@@ -88,8 +88,8 @@ enum bf_value_mode {
 /* Network shape.  Supported: d_model 256, n_heads 8, d_ff 1024 (all kernels, int8 and e4m3)
  * and d_model 512, n_heads 16, d_ff 2048 (BOARD kernel, int8); head width 32, any
  * n_layers >= 1, n_value 1 (tanh scalar) or 3 (loss/draw/win classes).
- * Range of the arithmetic: rows are quantised exactly as stated up to magnitudes of 2^108 (beyond, a value that
- * lies on a tie may go either way); LayerNorm's
+ * Range of the arithmetic: a row to be quantised whose largest magnitude is below 2^-118 counts as zero, up to
+ * 2^108 rows are quantised exactly as stated (beyond, a value that lies on a tie may go either way); LayerNorm's
  * variance + eps is exact from 2^-102 on (eps = 0 is accepted, a constant row then gives NaN), and a row whose
  * squares overflow normalises to beta. */
 typedef struct {

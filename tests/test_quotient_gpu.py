@@ -1,5 +1,5 @@
-"""The kernels' reciprocal and reciprocal square root on the device, every float of their range, and rows at the
-end of the range, whose squares overflow."""
+"""The kernels' reciprocal and reciprocal square root on the device, every float of their range, and rows at the ends of
+the range: squares that overflow, magnitudes too small for a scale."""
 import numpy as np
 import pytest
 import torch
@@ -52,3 +52,20 @@ def test_rows_whose_squares_overflow_normalise_as_in_the_checker(kernel):
     if kernel == "auto":     # and the form that spreads a position over several compute units, through the encoder alone
         octo = encoder_impl("hip")(net, int8=True, kernel="octo")
         assert torch.equal(model.forward(x.cuda()).nan_to_num(7.0), octo.forward(x.cuda()).nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("quant,kernel", [("int8", k) for k in ("auto", "octo", "duo", "twin", "board", "quad")] + [("fp8", k) for k in ("auto", "octo", "duo", "twin", "board", "quad")])
+@pytest.mark.parametrize("tiny", [1e-37, 1e-39, 1e-42])
+def test_rows_too_small_for_a_scale_count_as_zero(quant, kernel, tiny):
+    b, c, r, _ = (t.cuda() for t in positions.random_positions(5, plies=60, seed=4))
+    outs = []
+    for gamma in (tiny, 0.0):
+        torch.manual_seed(0)
+        net = BrokefishNet(n_layers=2).eval().randomise_layers_(seed=4)
+        with torch.no_grad():
+            for layer in net.encoder.layers:
+                layer.norm1.weight.fill_(gamma), layer.norm1.bias.zero_()
+        model = encoder_impl("hip")(net, kernel=kernel, out_dtype=torch.float32, **{quant: True})
+        outs.append([t.clone() for t in model.forward_full(b, c, r)])
+    for got, want in zip(*outs):
+        assert bool(got.isfinite().all()) and torch.equal(got, want)
