@@ -344,7 +344,7 @@ double bf_stream_rate(const void* buf, size_t bytes, int workgroups, int reps, i
  *                     (the row scale keeps |x / scale| <= 127; nothing clamps here)
  *   BF_PROBE_U8_RELU  the unsigned quantiser of the feed-forward hidden row with the ReLU folded
  *                     in: rint(max(x, 0) / scale) saturated to [0, 255]
- *   BF_PROBE_E4M3     OCP e4m3 code of x / scale clamped to +-448
+ *   BF_PROBE_E4M3     OCP e4m3 code of x / scale clamped to +-448 (by the probe: the kernels' quotients end at 8)
  * The device twin of the reference's quantiser unit tests (reference csrc/tests/tint8.cu:39-61,
  * :190-227).  Asynchronous on `stream`. */
 enum bf_probe_mode { BF_PROBE_S8 = 0, BF_PROBE_U8_RELU = 1, BF_PROBE_E4M3 = 2 };

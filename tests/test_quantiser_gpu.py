@@ -1,10 +1,13 @@
 """The kernels' row quantisers on their own (C-ABI ``bf_quant_probe``), against the reference's
 quantiser arithmetic on the host: ``q = clamp(round_half_even(x / s))`` with ``x / s`` a true fp32
 division (reference brokefish/nn/quant.py:246-260; device unit tests csrc/tests/tint8.cu:39-61 for
-the ties and saturation, :190-227 for formula inputs).  The kernels build the quotient from a
-reciprocal and two fused corrections, round by adding 1.5 * 2^23 with a byte-select add (signed) or
-with v_cvt_pk_u8_f32 (unsigned, the ReLU being its saturation at 0), and convert to e4m3 with the
-hardware's OCP conversion: each must give the byte the plain formula gives, ties included.
+the ties and saturation, :190-227 for formula inputs).  The kernels build the quotient from the scale's
+reciprocal in two floats (one multiplication and one fused multiply-add an element; it is the division's
+quotient wherever a rounding decision depends on it, tests/test_quotient.py), round by adding 1.5 * 2^23 with
+a byte-select add (signed) or with v_cvt_pk_u8_f32 (unsigned, the ReLU being its saturation at 0), and
+convert to e4m3 with the hardware's OCP conversion: each must give the byte the plain formula gives, ties
+included.  No kernel meets a quotient beyond what its row's largest magnitude maps to (127, 255, 8), and none
+clamps above it; the e4m3 probe does, before it calls the kernels' code, so that any value may be asked for.
 """
 import numpy as np
 import pytest
@@ -67,7 +70,7 @@ def test_e4m3_quantiser_equals_the_torch_cast(scale):
     s = np.float32(scale)
     g = np.random.default_rng(3)
     x = np.concatenate([(g.uniform(-9, 9, 1_000_000) * np.float64(s)).astype(np.float32),
-                        (g.uniform(-500, 500, 100_000) * np.float64(s)).astype(np.float32),       # beyond the format's range: clamped
+                        (g.uniform(-500, 500, 100_000) * np.float64(s)).astype(np.float32),       # beyond the format's range the probe clamps
                         (g.uniform(-0.02, 0.02, 100_000) * np.float64(s)).astype(np.float32)])    # subnormal codes
     q = torch.from_numpy(x) / torch.tensor(s)
     want = q.clamp(-448.0, 448.0).to(torch.float8_e4m3fn).view(torch.uint8).numpy()
@@ -75,6 +78,17 @@ def test_e4m3_quantiser_equals_the_torch_cast(scale):
     # -0 and +0 are the same number; everything else must be the same code
     same = (got == want) | (((got & 0x7F) == 0) & ((want & 0x7F) == 0))
     assert same.all(), (x[~same][:5], got[~same][:5], want[~same][:5])
+
+
+@pytest.mark.parametrize("mode,top,code", [("s8", 127.0, {127, 129}), ("u8_relu", 255.0, {255, 0}), ("e4m3", 8.0, {0x50, 0xd0})])
+def test_the_largest_magnitude_of_a_row_maps_to_the_top_of_the_range(mode, top, code):
+    # under its own row's scale, with nothing clamped above: a quotient that came out larger would wrap or overflow
+    g = np.random.default_rng(5)
+    for amax in np.concatenate([np.exp2(g.uniform(-110, 90, 150)), np.exp2(g.integers(-110, 90, 20)), 1 + g.uniform(0, 1, 80)]).astype(np.float32):
+        scale = amax / np.float32(top)
+        below = np.nextafter(amax, np.float32(0))
+        got = _run(np.array([amax, -amax, below, -below], np.float32), float(scale), mode)
+        assert set(got.tolist()) == code and got[0] == got[2] and got[1] == got[3], (amax, got)
 
 
 def test_probe_rejects_bad_arguments():
