@@ -16,8 +16,10 @@
 
 #include <algorithm>
 #include <array>
+#include <optional>
 #include <string>
 #include <string_view>
+#include <utility>
 #include <vector>
 
 #include "brokefish_hip.h"
@@ -499,16 +501,37 @@ public:
     static const at::Tensor& tensor(const Param& p) { return THPVariable_Unpack(p.object); }
 };
 
-// A fingerprint under way on a stream: its value is written to pinned host memory
-struct Fingerprint {
+// A fingerprint under way on a stream: a kernel writes its value to pinned host memory.  The host allocator knows nothing
+// of that kernel and hands the memory out again as soon as the tensor is gone, so whoever drops a fingerprint that
+// nobody has read waits for the stream first.
+class Fingerprint {
     torch::Tensor host;
     c10::hip::HIPStreamMasqueradingAsCUDA stream;
+    bool pending = true;
+
+public:
+    explicit Fingerprint(c10::hip::HIPStreamMasqueradingAsCUDA s)
+        : host(at::empty({1}, at::TensorOptions().dtype(torch::kDouble).pinned_memory(true))), stream(s) {}
+    Fingerprint(Fingerprint&& o) noexcept : host(std::move(o.host)), stream(o.stream), pending(std::exchange(o.pending, false)) {}
+    Fingerprint(const Fingerprint&) = delete;
+    Fingerprint& operator=(const Fingerprint&) = delete;
+    ~Fingerprint() {
+        if (!pending) return;
+        try {
+            py::gil_scoped_release no_gil;
+            stream.synchronize();
+        } catch (...) {   // the stream is in error: the memory is not given back
+            new torch::Tensor(std::move(host));
+        }
+    }
+    double* out() { return static_cast<double*>(host.data_ptr()); }
     double value() {
         {
             py::gil_scoped_release no_gil;
             stream.synchronize();
         }
-        return *static_cast<const double*>(host.data_ptr());
+        pending = false;
+        return *out();
     }
 };
 
@@ -532,8 +555,9 @@ c10::optional<Fingerprint> fingerprint(const py::object& net) {
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
     const int n = (int)ptrs.size();
     const torch::Tensor partials = fresh({bf_fingerprint_partials(numel.data(), n)}, torch::kDouble, dev);
-    Fingerprint f{at::empty({1}, at::TensorOptions().dtype(torch::kDouble).pinned_memory(true)), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index())};
-    const int rc = bf_fingerprint(ptrs.data(), numel.data(), n, static_cast<double*>(partials.data_ptr()), static_cast<double*>(f.host.data_ptr()), f.stream.stream());
+    const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
+    c10::optional<Fingerprint> f(std::in_place, stream);
+    const int rc = bf_fingerprint(ptrs.data(), numel.data(), n, static_cast<double*>(partials.data_ptr()), f->out(), stream.stream());
     TORCH_CHECK(rc == BF_OK, "bf_fingerprint failed (", rc, "): ", bf_last_error());
     return f;
 }

@@ -49,3 +49,22 @@ def test_parameters_that_are_unaligned_or_of_another_type_are_taken_as_fp32():
     assert np.array_equal(got_ws.cpu().numpy(), ws) and np.array_equal(got_fp.cpu().numpy().view(np.uint32), fp.view(np.uint32))
     with pytest.raises(ValueError, match="wants"):
         hip_impl.pack_board_on_device(net, net.encoder, hip_impl._Shape(256, 1, 8, 1024, 3, 1e-5), False, torch.device("cuda", 0))
+
+
+def test_a_fingerprint_that_nobody_reads_keeps_its_host_memory_until_it_is_written(monkeypatch):
+    # the value is written to pinned memory by a kernel; here the stream is busy with something else when the
+    # fingerprint is dropped, as it is where packing the same network raises
+    net = BrokefishNet(n_layers=1).eval().randomise_layers_(seed=2).cuda()
+    want = sync.weight_fingerprint(net)
+    monkeypatch.setattr(sync, "encoder_impl", lambda impl: (_ for _ in ()).throw(RuntimeError("no evaluator today")))
+    for how in ("dropped", "raised"):
+        torch.cuda._sleep(100_000_000)
+        if how == "dropped":
+            hip_impl.fingerprint_on_device(net)
+        else:
+            with pytest.raises(RuntimeError, match="no evaluator today"):
+                sync.PackedWeights.pack(net, 1, int8=True)
+        held = [torch.full((1,), 1.0, dtype=torch.float64).pin_memory() for _ in range(64)]
+        torch.cuda.synchronize()
+        assert all(t.item() == 1.0 for t in held), how
+    assert sync.weight_fingerprint(net) == want
