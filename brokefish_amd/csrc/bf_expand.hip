@@ -594,6 +594,50 @@ extern "C" int bf_compact_leaves(const uint8_t* flags, int64_t n, int32_t* leaf_
     return BF_OK;
 }
 
+constexpr int CLEAR_MOST = 8, CLEAR_LANES = 256, CLEAR_PIECES = 4;   // sixteen bytes a piece
+struct KClear {
+    uint8_t* at[CLEAR_MOST];
+    size_t bytes[CLEAR_MOST];
+};
+__global__ __launch_bounds__(CLEAR_LANES) void clear_kernel(const KClear k) {
+    uint8_t* const to = k.at[blockIdx.y];
+    const size_t bytes = k.bytes[blockIdx.y], whole = bytes / 16;
+#pragma unroll
+    for (int i = 0; i < CLEAR_PIECES; i++) {
+        const size_t piece = ((size_t)blockIdx.x * CLEAR_PIECES + i) * CLEAR_LANES + threadIdx.x;
+        if (piece < whole) reinterpret_cast<uint4*>(to)[piece] = uint4{0, 0, 0, 0};
+        else if (piece == whole)
+            for (size_t b = 16 * whole; b < bytes; b++) to[b] = 0;
+    }
+}
+
+extern "C" int bf_clear(void* const* buffers, const size_t* bytes, int n, void* stream) {
+    auto fail = [](int code, const char* msg) {
+        bf::set_error(msg);
+        return code;
+    };
+    if (!buffers || !bytes || n < 1 || n > CLEAR_MOST) return fail(BF_ERR_ARGUMENT, "buffers/bytes must not be NULL, n in [1, 8]");
+    KClear k = {};
+    size_t most = 0;
+    for (int i = 0; i < n; i++) {
+        if ((!buffers[i] && bytes[i]) || ((uintptr_t)buffers[i] & 15)) return fail(BF_ERR_ARGUMENT, "a buffer must be 16-byte aligned and not NULL");
+        k.at[i] = static_cast<uint8_t*>(buffers[i]);
+        k.bytes[i] = bytes[i];
+        most = bytes[i] > most ? bytes[i] : most;
+    }
+    constexpr size_t per = 16 * CLEAR_LANES * CLEAR_PIECES;
+    if (most >= (per << 31)) return fail(BF_ERR_ARGUMENT, "a buffer is too large");
+    if (!most) return BF_OK;
+    hipLaunchKernelGGL(clear_kernel, dim3((unsigned)(most / per + 1), n), dim3(CLEAR_LANES), 0, (hipStream_t)stream, k);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        char msg[256];
+        snprintf(msg, sizeof(msg), "kernel launch failed: %s", hipGetErrorString(e));
+        return fail(BF_ERR_LAUNCH, msg);
+    }
+    return BF_OK;
+}
+
 extern "C" int bf_expand(const bf_expand_args* a, void* stream) {
     auto fail = [](int code, const char* msg) {
         bf::set_error(msg);

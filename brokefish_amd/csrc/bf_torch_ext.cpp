@@ -8,7 +8,7 @@
 
 // PyTorch on ROCm presents its devices under the type name "cuda": these are the guard and stream
 // classes of that arrangement
-#include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
@@ -203,30 +203,34 @@ bool shape_is(const torch::Tensor& t, std::initializer_list<int64_t> want) { ret
 
 void* stream_of(const c10::Device& dev) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream(); }
 
-// a new tensor straight from the caching allocator (at::empty takes the dispatcher's way there)
-torch::Tensor fresh(at::IntArrayRef size, at::ScalarType type, const c10::Device& dev) {
-    return at::detail::empty_cuda(size, type, dev, c10::nullopt);
+// a new tensor straight from the caching allocator, on the current device (at::empty takes the dispatcher's way there)
+torch::Tensor fresh(at::IntArrayRef size, at::ScalarType type) {
+    static c10::Allocator* const allocator = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
+    const size_t bytes = c10::multiply_integers(size) * c10::elementSize(type);
+    torch::Tensor t = at::detail::make_tensor<c10::TensorImpl>(
+        c10::Storage(c10::make_intrusive<c10::StorageImpl>(c10::StorageImpl::use_byte_size_t(), bytes, allocator->allocate(bytes), allocator, true)),
+        c10::DispatchKeySet(c10::DispatchKey::CUDA), c10::scalarTypeToTypeMeta(type));
+    t.unsafeGetTensorImpl()->set_sizes_contiguous(size);
+    return t;
 }
 
-// New tensors that a call returns together, in one allocation (each at a multiple of 512 bytes, as the allocator places
-// them): six allocations of their own were 3 of an expansion call's 7 us.
+// New tensors that a call returns together, each in memory of its own: a caller may keep, save, resize or share one
+// of them and let the others go.  (Views of one allocation are 1 us cheaper for the six of an expansion, of a
+// call's 6; but then keeping the edge counts keeps a hundred times their size.)  Zeroed ones are cleared by one launch.
 struct Want { at::DimVector size; at::ScalarType type; };
 template <size_t N>
 std::array<torch::Tensor, N> fresh_together(const std::array<Want, N>& want, bool zeroed, const c10::Device& dev) {
-    std::array<int64_t, N> at;
-    int64_t bytes = 0;
-    for (size_t i = 0; i < N; i++) {
-        at[i] = bytes;
-        bytes += (c10::multiply_integers(want[i].size) * (int64_t)c10::elementSize(want[i].type) + 511) / 512 * 512;
-    }
-    torch::Tensor all = fresh({bytes}, torch::kByte, dev);
-    if (zeroed) all.zero_();
     std::array<torch::Tensor, N> t;
-    for (size_t i = 0; i < N; i++) {
-        t[i] = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(all.storage()), all.key_set(), c10::scalarTypeToTypeMeta(want[i].type));
-        c10::TensorImpl* const impl = t[i].unsafeGetTensorImpl();
-        impl->set_storage_offset(at[i] / (int64_t)c10::elementSize(want[i].type));
-        impl->set_sizes_contiguous(want[i].size);
+    for (size_t i = 0; i < N; i++) t[i] = fresh(want[i].size, want[i].type);
+    if (zeroed) {
+        void* at[N];
+        size_t bytes[N];
+        for (size_t i = 0; i < N; i++) {
+            at[i] = t[i].data_ptr();
+            bytes[i] = t[i].nbytes();
+        }
+        const int rc = bf_clear(at, bytes, N, stream_of(dev));
+        TORCH_CHECK(rc == BF_OK, "bf_clear failed (", rc, "): ", bf_last_error());
     }
     return t;
 }
@@ -554,7 +558,7 @@ c10::optional<Fingerprint> fingerprint(const py::object& net) {
     }
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
     const int n = (int)ptrs.size();
-    const torch::Tensor partials = fresh({bf_fingerprint_partials(numel.data(), n)}, torch::kDouble, dev);
+    const torch::Tensor partials = fresh({bf_fingerprint_partials(numel.data(), n)}, torch::kDouble);
     const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
     c10::optional<Fingerprint> f(std::in_place, stream);
     const int rc = bf_fingerprint(ptrs.data(), numel.data(), n, static_cast<double*>(partials.data_ptr()), f->out(), stream.stream());

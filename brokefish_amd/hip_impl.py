@@ -126,6 +126,8 @@ def load_library():
         L.bf_fingerprint.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]
         L.bf_expand.restype = C.c_int
         L.bf_expand.argtypes = [C.POINTER(_ExpandArgs), C.c_void_p]
+        L.bf_clear.restype = C.c_int
+        L.bf_clear.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
         L.bf_movegen.restype = C.c_int
         L.bf_movegen.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
         L.bf_compact_leaves.restype = C.c_int

@@ -423,6 +423,11 @@ int bf_expand(const bf_expand_args* args, void* stream);
  * flat staging (brokefish/search/cuda_impl.py:137-145: leaf_flags).  One workgroup; asynchronous. */
 int bf_compact_leaves(const uint8_t* flags, int64_t n, int32_t* leaf_index, int32_t* leaf_count, void* stream);
 
+/* Zero in up to 8 buffers with one launch: buffers and bytes are host arrays of n entries, the buffers 16-byte
+ * aligned DEVICE memory (an entry of 0 bytes may be NULL).  For the outputs of calls that leave rows as they were
+ * (`active`, leaf lists); a kernel and no memset node where it is captured.  Asynchronous on `stream`. */
+int bf_clear(void* const* buffers, const size_t* bytes, int n, void* stream);
+
 /* Legal-move words on the device.  Replaces env.movegen of the reference (reference
  * docs/reference/spec.md:152-172; brokefish/env/torch_impl.py:251-289): for each of n positions
  * (boards [n,32] uint16, control [n] int16) writes mask [n,32] uint64 -- bit s of word p set iff

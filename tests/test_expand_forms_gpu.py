@@ -1,10 +1,12 @@
 """Edge rows in their different forms (whole 16-byte pieces, odd lengths, longer than the LDS row) and the
 leaf compaction at the edges of its workgroups."""
+import ctypes as C
+
 import pytest
 import torch
 
 from brokefish_amd import positions
-from brokefish_amd.hip_impl import compact_leaves, expand_edges
+from brokefish_amd.hip_impl import compact_leaves, expand_edges, load_library, movegen
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +90,32 @@ def test_compaction_at_the_edges_of_its_workgroups(n, shift):
         index, count = compact_leaves(flags)
         want = flags.nonzero().flatten().int()
         assert int(count) == want.numel() and torch.equal(index[:want.numel()], want) and not index[want.numel():].any()
+
+
+@pytest.mark.parametrize("n", [1, 7, 1000])
+def test_outputs_of_a_call_have_memory_of_their_own(n):
+    b, c, _, m = (t.cuda() for t in positions.random_positions(n, plies=60, seed=1))
+    logits = [torch.randn(n, 32, k, device="cuda").half() for k in (64, 4)]
+    on = (torch.arange(n, device="cuda") % 2 == 0)
+    outs = [dict(zip("mk", movegen(b, c)))]
+    outs += [expand_edges(*logits, torch.rand(n, device="cuda"), m, b, c, 96, **kw) for kw in ({}, {"active": on}, {"leaves": compact_leaves(on)})]
+    for out in outs:
+        stores = [t.untyped_storage() for t in out.values()]
+        assert len({s.data_ptr() for s in stores}) == len(stores)
+        assert all(s.nbytes() == t.numel() * t.element_size() and t.storage_offset() == 0 for s, t in zip(stores, out.values()))
+        if len(out) > 2 and out is not outs[1]:      # rows of skipped positions start at zero, the others' are the call's
+            for name, t in out.items():
+                assert not t[~on].any()
+                if name != "node_value":             # (each call had values of its own)
+                    assert torch.equal(t[on], outs[1][name][on])
+
+
+@pytest.mark.parametrize("sizes", [(0, 1, 15, 16, 17), (16383, 16384, 16385), (4096 * 16 + 5, 3, 1 << 22)])
+def test_clear_writes_its_buffers_and_no_more(sizes):
+    room = [torch.full((s + 64,), 7, dtype=torch.uint8, device="cuda") for s in sizes]
+    lib = load_library()
+    at = (C.c_void_p * len(sizes))(*[t.data_ptr() for t in room])
+    assert lib.bf_clear(at, (C.c_size_t * len(sizes))(*sizes), len(sizes), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    for t, s in zip(room, sizes):
+        assert not t[:s].any() and bool((t[s:] == 7).all())
+    assert lib.bf_clear(at, (C.c_size_t * 9)(), 9, None) != 0
