@@ -515,9 +515,11 @@ __global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand
 // load; where they go in the list is the number of live flags in front of them, which every workgroup
 // counts for itself (16 flags per lane and load again: 64 KiB in a microsecond or two), so no workgroup
 // waits for another and nothing is kept between launches.  One workgroup going through all flags, a byte
-// per lane and two barriers per 1024, took 41 us for 65536 flags, this 4.4 us (4096 flags: 10 us
-// before, 3.3).
-constexpr int COMPACT_LANES = 1024, COMPACT_FLAGS = 16;
+// per lane and two barriers per 1024, took 41 us for 65536 flags, this 4.2 us (4096 flags: 10 us
+// before, 3.2).  The counting grows with the square of the workgroups, so there are at most 256 of them, one per
+// compute unit, which beyond 4 M flags take several runs of 16384 each: 2^24 flags take 0.16 ms, 2^28
+// 3 ms (with a workgroup for every 16384: 0.77 and 251; one workgroup: 12 and 237).
+constexpr int COMPACT_LANES = 1024, COMPACT_FLAGS = 16, COMPACT_GROUPS = 256;
 constexpr int COMPACT_CHUNK = COMPACT_LANES * COMPACT_FLAGS;
 
 // the high bit of every non-zero byte
@@ -541,38 +543,54 @@ __device__ __forceinline__ unsigned flag_bits(const uint8_t* flags, long long at
     return bits;
 }
 
-__global__ __launch_bounds__(COMPACT_LANES) void compact_kernel(const uint8_t* flags, int n, int* leaf_index, int* leaf_count) {
-    __shared__ int total[2][COMPACT_LANES / 64];
+template <bool ONE_RUN>   // (the loop costs a launch of few flags 0.4 us)
+__global__ __launch_bounds__(COMPACT_LANES) void compact_kernel(const uint8_t* flags, int n, int chunks_, int* leaf_index, int* leaf_count) {
+    const int chunks = ONE_RUN ? 1 : chunks_;
+    __shared__ int total[2][COMPACT_LANES / 64], ahead[COMPACT_LANES / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const bool aligned = ((uintptr_t)flags & 15) == 0;
-    const long long first = (long long)blockIdx.x * COMPACT_CHUNK;
+    const long long first = (long long)blockIdx.x * chunks * COMPACT_CHUNK;   // this workgroup's flags: `chunks` runs of 16384
     int front = 0;
-    for (long long at = (long long)threadIdx.x * COMPACT_FLAGS; at < first; at += COMPACT_CHUNK)
-        front += __popc(flag_bits(flags, at, n, aligned));
-    const int mine = (int)first + (int)threadIdx.x * COMPACT_FLAGS;
-    unsigned bits = flag_bits(flags, mine, n, aligned);
-    const int cnt = __popc(bits);
-    int inc = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(inc, d);
-        if (lane >= d) inc += o;
+    if (aligned) {
+#pragma unroll 4
+        for (long long at = (long long)threadIdx.x * COMPACT_FLAGS; at < first; at += COMPACT_CHUNK) {
+            const uint4 v = *reinterpret_cast<const uint4*>(flags + at);
+            front += __popc(nonzero_bytes(v.x)) + __popc(nonzero_bytes(v.y)) + __popc(nonzero_bytes(v.z)) + __popc(nonzero_bytes(v.w));
+        }
+    } else {
+#pragma unroll 1
+        for (long long at = (long long)threadIdx.x * COMPACT_FLAGS; at < first; at += COMPACT_CHUNK) front += __popc(flag_bits(flags, at, n, false));
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) front += __shfl_xor(front, d);
-    if (lane == 63) {
-        total[0][wave] = inc;
-        total[1][wave] = front;
-    }
-    __syncthreads();
-    int at = inc - cnt, all = 0;
+    if (lane == 63) ahead[wave] = front;
+    int base = 0;
+    for (int c = 0; c < chunks; c++) {
+        const long long run = first + (long long)c * COMPACT_CHUNK;
+        if (!ONE_RUN && run >= n) break;
+        const int mine = (int)run + (int)threadIdx.x * COMPACT_FLAGS;
+        unsigned bits = flag_bits(flags, mine, n, aligned);
+        const int cnt = __popc(bits);
+        int inc = cnt;
 #pragma unroll
-    for (int w = 0; w < COMPACT_LANES / 64; w++) {
-        at += (w < wave ? total[0][w] : 0) + total[1][w];
-        all += total[0][w] + total[1][w];
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d);
+            if (lane >= d) inc += o;
+        }
+        if (lane == 63) total[c & 1][wave] = inc;
+        __syncthreads();   // one a run: the totals of the run after the next are written behind the next one's
+        int at = inc - cnt, all = 0;
+#pragma unroll
+        for (int w = 0; w < COMPACT_LANES / 64; w++) {
+            base += c == 0 ? ahead[w] : 0;
+            at += w < wave ? total[c & 1][w] : 0;
+            all += total[c & 1][w];
+        }
+        at += base;
+        for (; bits; bits &= bits - 1) leaf_index[at++] = mine + __builtin_ctz(bits);
+        base += all;
     }
-    for (; bits; bits &= bits - 1) leaf_index[at++] = mine + __builtin_ctz(bits);
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *leaf_count = all;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *leaf_count = base;
 }
 
 extern "C" int bf_compact_leaves(const uint8_t* flags, int64_t n, int32_t* leaf_index, int32_t* leaf_count, void* stream) {
@@ -583,8 +601,9 @@ extern "C" int bf_compact_leaves(const uint8_t* flags, int64_t n, int32_t* leaf_
     if (!flags || !leaf_index || !leaf_count) return fail(BF_ERR_ARGUMENT, "flags/leaf_index/leaf_count must not be NULL");
     if (n < 1 || n > (1ll << 28)) return fail(BF_ERR_ARGUMENT, "n must be in [1, 2^28]");
     if (((uintptr_t)leaf_index & 3) || ((uintptr_t)leaf_count & 3)) return fail(BF_ERR_ARGUMENT, "leaf_index / leaf_count must be 4-byte aligned");
-    hipLaunchKernelGGL(compact_kernel, dim3((unsigned)((n + COMPACT_CHUNK - 1) / COMPACT_CHUNK)), dim3(COMPACT_LANES), 0, (hipStream_t)stream,
-                       flags, (int)n, leaf_index, leaf_count);
+    const int runs = (int)((n + COMPACT_CHUNK - 1) / COMPACT_CHUNK), chunks = (runs + COMPACT_GROUPS - 1) / COMPACT_GROUPS;
+    hipLaunchKernelGGL(chunks == 1 ? compact_kernel<true> : compact_kernel<false>, dim3((unsigned)((runs + chunks - 1) / chunks)), dim3(COMPACT_LANES), 0, (hipStream_t)stream,
+                       flags, (int)n, chunks, leaf_index, leaf_count);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         char msg[256];

@@ -420,7 +420,7 @@ int bf_expand(const bf_expand_args* args, void* stream);
  * and the count to leaf_count[0] (both DEVICE memory; leaf_index holds n entries, entries past the
  * count are left as they were).  The "compacted list plus a count" of the reference's design
  * retrospective (reference docs/journal/2026-08-09-kernel-design-retrospective.md:140-154) over its
- * flat staging (brokefish/search/cuda_impl.py:137-145: leaf_flags).  One workgroup; asynchronous. */
+ * flat staging (brokefish/search/cuda_impl.py:137-145: leaf_flags).  One launch; asynchronous on `stream`. */
 int bf_compact_leaves(const uint8_t* flags, int64_t n, int32_t* leaf_index, int32_t* leaf_count, void* stream);
 
 /* Zero in up to 8 buffers with one launch: buffers and bytes are host arrays of n entries, the buffers 16-byte

@@ -119,3 +119,12 @@ def test_clear_writes_its_buffers_and_no_more(sizes):
     for t, s in zip(room, sizes):
         assert not t[:s].any() and bool((t[s:] == 7).all())
     assert lib.bf_clear(at, (C.c_size_t * 9)(), 9, None) != 0
+
+
+@pytest.mark.parametrize("n", [256 * 16384, 256 * 16384 + 1, 257 * 16384 - 5, 512 * 16384 + 40000])
+def test_compaction_of_more_flags_than_its_workgroups_take_in_one_run(n):
+    flags = (torch.rand(n, generator=torch.Generator(device="cuda").manual_seed(n), device="cuda") < 0.3).to(torch.uint8)
+    flags[n // 3:n // 2] = 0                                     # workgroups without a live flag
+    index, count = compact_leaves(flags)
+    want = flags.nonzero().flatten().int()
+    assert int(count) == want.numel() and torch.equal(index[:want.numel()], want) and not index[want.numel():].any()
