@@ -75,20 +75,15 @@ __device__ __forceinline__ u64 antidiagonal(int sq) {   // a8-h1 direction
 
 // What a square decides: its lines (the square itself excluded), the knight's and the king's steps from it.
 struct Square { u64 diag, anti, knight, king, rank, file, s; };
-// Large launches look the first four up: a table of 2 KiB in LDS that the workgroup fills at its start, a field by
+// The first four are looked up: a table of 2 KiB in LDS that the workgroup fills at its start, a field by
 // each of its four wavefronts (a field is 10 to 25 instructions, and a lane asks for three squares).
-template <bool TABLE>
 __device__ __forceinline__ Square square(int sq, const ulonglong2 (*table)[2]) {
     Square q;
     q.s = bit(sq);
     q.rank = (0xFFull << (sq & 56)) ^ q.s;
     q.file = (FILE_A << (sq & 7)) ^ q.s;
-    if constexpr (TABLE) {
-        const ulonglong2 a = table[sq][0], b = table[sq][1];
-        q.diag = a.x; q.anti = a.y; q.knight = b.x; q.king = b.y;
-    } else {
-        q.diag = diagonal(sq); q.anti = antidiagonal(sq); q.knight = knight_pattern(q.s); q.king = king_pattern(q.s);
-    }
+    const ulonglong2 a = table[sq][0], b = table[sq][1];
+    q.diag = a.x; q.anti = a.y; q.knight = b.x; q.king = b.y;
     return q;
 }
 __device__ __forceinline__ u64 rook_attacks(u64 occ, const Square& q) { return line_attacks(occ, q.rank, q.s) | line_attacks(occ, q.file, q.s); }
@@ -124,11 +119,10 @@ __device__ __forceinline__ u64 row_or(u64 v) {
     return ((u64)hi << 32) | lo;
 }
 
-template <bool TABLE>
 __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, const int16_t* control, int n,
                                                       u64* mask, uint8_t* in_check) {
-    __shared__ ulonglong2 table[TABLE ? 64 : 1][2];
-    if constexpr (TABLE) {   // 256 lanes: a wavefront a field
+    __shared__ ulonglong2 table[64][2];
+    {   // 256 lanes: a wavefront a field
         const int sq = threadIdx.x & 63, field = threadIdx.x >> 6;
         reinterpret_cast<u64*>(table[sq])[field] = field == 0 ? diagonal(sq) : field == 1 ? antidiagonal(sq) : field == 2 ? knight_pattern(bit(sq)) : king_pattern(bit(sq));
         __syncthreads();
@@ -166,7 +160,7 @@ __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, co
     const bool rook_long = (__ballot(w == (rookw | home)) >> rowbits) & 0xffff;
 
     // ---- what attacks the king once this lane's piece has left its square (the king's own lane: the check) ----
-    const Square king = square<TABLE>(ksq, table);
+    const Square king = square(ksq, table);
     const u64 att = attackers(e, occ & ~fb, king);
     u64 allowed = ~0ull;
     if (att) allowed = (att & (att - 1)) ? 0 : att | between(king, att);
@@ -193,13 +187,13 @@ __global__ __launch_bounds__(256) void movegen_kernel(const uint16_t* boards, co
         if (!step) occ2 = (occ2 & ~bit(home + (kingside ? 7 : 0))) | bit(home + (kingside ? 5 : 3));
         Enemy e2 = e;
         e2.pawns &= ~tb; e2.knights &= ~tb; e2.diag &= ~tb; e2.orth &= ~tb;
-        const bool ok = may && attackers(e2, occ2, square<TABLE>(at, table)) == 0;
+        const bool ok = may && attackers(e2, occ2, square(at, table)) == 0;
         safe = (unsigned)(__ballot(ok) >> rowbits) & 0xffffu;
     }
 
     // ---- the squares this lane's piece reaches ----
     u64 legal = 0, ep = 0;
-    const Square from = square<TABLE>(sq, table);
+    const Square from = square(sq, table);
     if (mine) {
         if (t == PAWN) {
             const int r = sq >> 3;
@@ -255,11 +249,11 @@ extern "C" int bf_movegen(const uint16_t* boards, const int16_t* control, int64_
     if (!boards || !control || !mask) return fail(BF_ERR_ARGUMENT, "boards/control/mask must not be NULL");
     if (((uintptr_t)boards & 1) || ((uintptr_t)control & 1) || ((uintptr_t)mask & 7))
         return fail(BF_ERR_ARGUMENT, "boards and control must be 2-byte and mask 8-byte aligned");
-    // four positions per wavefront: workgroups of one wavefront while that spreads a small launch over more
-    // compute units (256 of them hold 1024 positions), of four beyond
-    const int waves = n <= 4096 ? 1 : 4;
-    hipLaunchKernelGGL(waves == 1 ? movegen_kernel<false> : movegen_kernel<true>, dim3((unsigned)((n + 4 * waves - 1) / (4 * waves))), dim3(64 * waves), 0,
-                       (hipStream_t)stream, boards, control, (int)n, reinterpret_cast<u64*>(mask), in_check);
+    // Sixteen positions per workgroup, whatever the launch.  Workgroups of one wavefront, which spread a small one over more
+    // compute units and compute the table's fields, are no faster anywhere (64 positions 4.5 us alone against 3.9, 250
+    // 4.6 / 4.3, 1024 4.5 / 4.4, 4096 4.7 / 4.6, 8192 5.8 / 5.5).
+    hipLaunchKernelGGL(movegen_kernel, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, (hipStream_t)stream, boards, control, (int)n, reinterpret_cast<u64*>(mask),
+                       in_check);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         char msg[256];

@@ -67,6 +67,12 @@ def test_every_position_near_the_perft_suite(idx):
     assert want_c.sum() > 0 or idx == 0
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 15, 16, 17, 63, 65, 4095, 4097])
+def test_launches_at_the_edges_of_a_workgroup(n):
+    b, c, _, _ = positions.random_positions_np(n, plies=120, seed=n)
+    _compare(b, c)
+
+
 def test_twenty_thousand_random_playouts():
     b, c, r, m = positions.random_positions_np(20000, plies=200, seed=77, stamp_queen=True)
     want_m, want_c = _compare(b, c)
