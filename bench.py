@@ -46,7 +46,7 @@ def cpu_baseline(net, batch: int, threads: int, budget_s: float = 20.0, mode: st
     from brokefish_amd import positions
     from oracle import emulated
     sd = {k: v.detach() for k, v in net.state_dict().items()}
-    b, c, r, m = positions.random_positions(batch, plies=plies, seed=0)   # configs[0]: playouts of 0-80 plies
+    b, c, r, m = positions.random_positions(batch, plies=plies, seed=0)
     torch.set_num_threads(threads)
     with torch.no_grad():
         t0 = time.perf_counter()
@@ -176,8 +176,8 @@ def main() -> int:
         "value": evals, "unit": "evals/s", "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": ms_step, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "fp8" if fp8 else "int8", "data": "synthetic",
-        "config": {"workload": (f"configs[4]: 16-layer d512 16-head FFN2048 int8 evaluator, batch {a.batch}, " if stress else
-                                f"configs[{3 if fp8 else 1}]: 8-layer d256 8-head FFN1024 {a.quant} evaluator, batch {a.batch}, ")
+        "config": {"workload": (f"16-layer d512 16-head FFN2048 int8 evaluator, batch {a.batch}, " if stress else
+                                f"8-layer d256 8-head FFN1024 {a.quant} evaluator, batch {a.batch}, ")
                                + f"kernel {kname}, binding {model.binding}, "
                                "seeded random playouts 0-120 plies, legal-move mask ANDed in-kernel, "
                                "fp16 logits out, seed-0 random-init weights"},
@@ -213,7 +213,7 @@ def main() -> int:
                           "share_of_total": {k: round(v / ph["total"], 4) for k, v in ph.items() if k != "total"}}
     del model, bd, cd, rd, md
     if headline and not a.no_extras:
-        # configurations 3, 4 and 5 timed in interleaved rounds (every point once per round, median over the
+        # the other configurations timed in interleaved rounds (every point once per round, median over the
         # rounds), as the reference's bench does for its variants (bench/bench_model.py:167-193): the batch
         # sweep (small-batch latency regime; same net, same generator), e4m3 at batch 4096 (products on the
         # fp16 matrix instruction: quoted against both peaks), the 16-layer 512-wide network at batch 16384
@@ -231,7 +231,7 @@ def main() -> int:
                 times[(name, nb)].append(mdl.time_kernel_ms(*inputs[nb], warmup=2, iters=iters))
         med = {k: sorted(v)[len(v) // 2] for k, v in times.items()}
         line["sweep"] = [{"batch": nb, "ms_per_launch": med[("sweep", nb)], "evals_per_s": nb / med[("sweep", nb)] * 1e3,
-                          "kernel": mdl8.kernel_choice(nb), "frac_int8_peak": OPS_PER_EVAL * nb / (med[("sweep", nb)] * 1e-3) / PEAK_INT8_OPS,
+                          "kernel": mdl8.kernel_choice(nb), "form": mdl8.launch_form(nb), "frac_int8_peak": OPS_PER_EVAL * nb / (med[("sweep", nb)] * 1e-3) / PEAK_INT8_OPS,
                           "ms_min_max": [min(times[("sweep", nb)]), max(times[("sweep", nb)])]}
                          for nb in (64, 256, 1024, 4096, 16384, 65536)]
         line["timing_protocol"] = f"{rounds} interleaved rounds over the sweep, e4m3 and stress points, median; HIP events on the launch stream"
@@ -252,7 +252,7 @@ def main() -> int:
         threads = max(1, min(cores, int(os.environ.get("OMP_NUM_THREADS", "16"))))
         line["cpu_baseline"] = cpu_baseline(net, a.cpu_batch, threads, mode=a.quant, budget_s=12.0)
         line["cpu_baseline"]["physical_cores"] = cores
-        if headline and not a.no_extras:      # configuration 1 names fp32 and the int8 simulation
+        if headline and not a.no_extras:      # the CPU forward is quoted in fp32 and in the int8 simulation
             f32 = cpu_baseline(net, a.cpu_batch, threads, mode="fp32", budget_s=4.0)
             line["cpu_baseline"]["fp32"] = {"value": f32["value"], "unit": "evals/s", "sample": f32["sample"]}
     print(json.dumps(line))

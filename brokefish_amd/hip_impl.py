@@ -934,7 +934,8 @@ class FusedEncoder:
         return ws
 
     def kernel_choice(self, n: int) -> str:
-        """Which kernel a call with ``n`` positions runs ("quad", "board", "twin", "octo" or "duo")."""
+        """Which kernel a call with ``n`` positions runs ("quad", "board", "twin", "octo" or "duo").  "octo" counts the
+        form that spreads a position over several compute units too; :meth:`launch_form` tells them apart."""
         a = _Args()
         a.n, a.shape, a.quant, a.kernel = n, self._shape, (1 if self.fp8 else 0), self.KERNELS[self.kernel]
         a.wstream = a.fparams = 16 if self.wstream is not None else None        # only tested for NULL
@@ -943,6 +944,15 @@ class FusedEncoder:
         if rc < 0:
             raise RuntimeError(f"bf_kernel_choice failed ({rc}): {self._lib.bf_last_error().decode()}")
         return {1: "quad", 2: "board", 3: "twin", 4: "octo", 5: "duo"}[rc]
+
+    def launch_form(self, n: int) -> str:
+        """:meth:`kernel_choice`, with "team" for launches that go to the form that spreads a position over several
+        compute units (the smallest ones, without taps and profile)."""
+        kind = self.kernel_choice(n)
+        if kind != "octo" or not self._team_bytes:
+            return kind
+        most = self._team_bytes // int(self._lib.bf_team_position_bytes(C.byref(self._shape)))
+        return "team" if n <= most * (2 if self.d_model != self.D else 1) else kind
 
     def forward_expand(self, boards, control, rep, mask=None, max_edges: int = 96, active=None, out=None, leaves=None):
         """``forward_full`` followed on the same stream by the search's expand step

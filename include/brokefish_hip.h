@@ -275,7 +275,8 @@ uint64_t bf_abi_tag(void);
 
 /* Largest n for which AUTO prefers OCTO over DUO / TWIN on the 256-wide network. */
 int64_t bf_board_max_n(void);
-/* The kernel AUTO would run for these arguments (enum bf_kernel), or a negative bf_status. */
+/* The kernel AUTO would run for these arguments (enum bf_kernel), or a negative bf_status.  The form that spreads a
+ * position over several compute units (team_workspace) counts as OCTO, whose launches it takes. */
 int bf_kernel_choice(const bf_eval_args* args);
 
 /* The evaluator.  Replaces model_forward of the reference extension

@@ -149,3 +149,11 @@ def test_the_count_of_layers_wraps(shape, start):
             assert_same(team.forward_full(*x[:3]), single.forward_full(*x[:3]))
         else:
             assert_same(team.forward_masked(*x), want)
+
+
+def test_launch_form_names_the_form_that_runs():
+    team, single = pair()
+    assert [team.launch_form(n) for n in (1, 64, 65, 256, 257)] == ["team", "team", "octo", "octo", "duo"]
+    assert single.launch_form(1) == "octo" and [team.kernel_choice(n) for n in (1, 65)] == ["octo", "octo"]
+    wide, _ = pair("wide")
+    assert [wide.launch_form(n) for n in (1, 32, 64, 65)] == ["team", "team", "team", "octo"]
