@@ -454,7 +454,7 @@ __global__ __launch_bounds__(THREADS, 1) void eval_kernel(const KArgs a) {
                     // e4m3: the ordinary signed quantiser (the values are non-negative).
                     am = __builtin_fmaxf(am, partner(am, g));
                     const float s8 = hidden_scale<FP8>(am);
-                    const Quot by = quot_by(s8);
+                    const auto by = quad_quotient<FP8>(s8);
                     sh[c] = s8;
 #pragma unroll
                     for (int s2 = 0; s2 < 8; s2++)
