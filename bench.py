@@ -27,14 +27,13 @@ OPS_PER_EVAL_STRESS = 3_221_225_472   # 2 * 32 tokens * 16 layers * 12 * 512^2 (
 PEAK_INT8_OPS = 5.0e15                # MI355X dense int8 MFMA, ops/s
 PEAK_FP16_OPS = 2.5e15                # dense fp16 MFMA: the e4m3 format's products run on the fp16 instruction
 # HBM bytes per launch from the FETCH_SIZE / WRITE_SIZE counter runs summarised under profiles/
-# (calibrated on a 1 GiB copy), by (network shape, kernel, batch).
-MEASURED_TRAFFIC_BYTES = {("base", "duo", 4096): 0.445e9, ("base", "twin", 4096): 0.78e9, ("base", "quad", 4096): 3.07e9,
-                          ("base", "board", 256): 5.5e7, ("base", "octo", 256): 5.5e7, ("stress", "board", 16384): 2.66e10,
-                          ("stress", "octo", 16384): 2.95e10}
+# (calibrated on a copy of known size), by (network shape, kernel, batch).
+MEASURED_TRAFFIC_BYTES = {("base", "duo", 4096): 0.445e9, ("base", "twin", 4096): 0.77e9, ("base", "quad", 4096): 3.08e9,
+                          ("base", "octo", 256): 5.5e7, ("stress", "octo", 16384): 2.87e10}
 MEASURED_TRAFFIC_BYTES_E4M3 = {("base", "twin", 4096): 0.97e9}
 # vector-ALU instructions per launch (SQ_INSTS_VALU of the same counter runs), by (network shape, kernel, batch):
 # with the matrix products hidden, the launch cannot be shorter than these instructions' issue time
-MEASURED_VALU_INSTS = {("base", "duo", 4096): 5.938e8, ("base", "twin", 4096): 5.513e8}
+MEASURED_VALU_INSTS = {("base", "duo", 4096): 5.486e8, ("base", "twin", 4096): 5.131e8}
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 PEAK_HBM_BPS = 8.0e12                 # MI355X HBM3E, bytes/s
 

@@ -20,7 +20,7 @@
 // En passant, where two pieces leave the board's lines at once, is replayed (a loop that hardly ever
 // runs).  Integer work, bound by the vector ALU: one wavefront per position (its boards built on the
 // scalar unit, each of some 31 moves replayed) took 119 us for 65536 positions, this 24 us, and with the squares'
-// diagonals, knight's and king's steps looked up (839 instead of 1016 vector instructions a wavefront) 19 us (1.1 TB/s
+// diagonals, knight's and king's steps looked up (651 vector instructions a wavefront, by counter) 19 us (1.1 TB/s
 // of its bytes).
 #include <hip/hip_runtime.h>
 
