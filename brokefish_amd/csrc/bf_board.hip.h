@@ -41,7 +41,8 @@
 #include "bf_device.hip.h"
 
 // TWIN form: workgroups per compute unit, and register sets of the weight prefetch (one set =
-// half a block; SETS - 1 half-blocks are in flight).  Measured on MI355X at batch 4096: three
+// half a block; SETS - 1 half-blocks are in flight).  Measured on MI355X at batch 4096 (with the division's
+// quotients, which took 4 % more): three
 // workgroups per unit spill too much (81-103 registers); three sets run without a spill
 // (1.717 ms), four spill 8 registers (1.741 ms), six 61 (2.10 ms).
 #ifndef BF_TWIN_SETS

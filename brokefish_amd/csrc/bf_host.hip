@@ -309,8 +309,8 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
                                  "are NaN (see team_workspace of bf_eval_args); nothing was launched now");
     const bool enc = !k.profile && enc_build(a, kind);
     // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
-    // position 124 -> 84 us, e4m3 155 -> 96; 512 wide 750 -> 275 us), and so does what is left of the 512-wide
-    // network's rounds of 256 positions (727 us each) where two team launches (328 us each) hold it.
+    // position 120 -> 82 us, e4m3 155 -> 96; 512 wide 738 -> 272 us), and so does what is left of the 512-wide
+    // network's rounds of 256 positions (738 us each) where two team launches (328 us each) hold it.
     const int team = team_limit(a, k, enc);
     if (kind == BF_KERNEL_OCTO && team > 0) {
         const int left = k.n <= team ? k.n : a->shape.d_model == 512 && !k.leaf_index ? k.n % (int)kBoardMaxN : 0;   // a list's length is on the device

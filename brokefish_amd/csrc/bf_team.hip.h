@@ -15,8 +15,8 @@
 // So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
 // tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
 // except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
-// 124 -> 82 us, e4m3 155 -> 96, width 512 with 16 layers 750 -> 271; 64 positions 120 -> 87, e4m3 155 -> 99; 32 of the
-// wide network 727 -> 321.  The arithmetic is that of the other kernels, operation for operation: the results are
+// 120 -> 82 us, e4m3 155 -> 96, width 512 with 16 layers 738 -> 272; 64 positions 120 -> 87, e4m3 155 -> 99; 32 of the
+// wide network 738 -> 328.  The arithmetic is that of the other kernels, operation for operation: the results are
 // bit-identical to theirs.
 //
 // Rows and tiles.  For everything per row (LayerNorm, quantisers, residual sums) a wavefront owns the rows of four
