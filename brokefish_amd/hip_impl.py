@@ -681,7 +681,12 @@ def fingerprint_on_device(net):
 # --------------------------------------------------------------------------- #
 
 class FusedEncoder:
-    """Boards to logits in one launch (see the module docstring)."""
+    """Boards to logits in one launch (see the module docstring).
+
+    With ``kernel="auto"`` the smallest launches spread a position over several compute units, whose workgroups
+    wait for one another.  A device holds ten such launches at a time, four of the 512-wide network: one process
+    stays below that by itself, more processes on one GPU than that should construct with ``kernel="octo"``.  A
+    launch that could not finish leaves NaN, and the next call raises ``RuntimeError`` (``BF_ERR_TEAM``)."""
 
     D, DFF, T, H = 256, 1024, 32, 8
     SHAPES = ((256, 1024, 8), (512, 2048, 16))     # (d_model, d_ff, heads) the library carries
