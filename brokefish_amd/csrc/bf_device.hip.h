@@ -30,6 +30,43 @@ __device__ __forceinline__ float partner(float v, int g) {
     return __int_as_float(g ? r[0] : r[1]);
 }
 
+// The lower and the upper halves of a and b side by side: lo = [a's lower half | b's lower half], hi = [a's upper | b's
+// upper].  One instruction, and every use of it below is symmetric in the halves, so no lane has to choose (partner()
+// costs two moves and a select beside it).
+struct Halves { float lo, hi; };
+__device__ __forceinline__ Halves halves_of(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false);
+    return {__int_as_float(r[0]), __int_as_float(r[1])};
+}
+// max without the quieting of its operands that fmaxf costs (an instruction for every value that comes from memory): for
+// values the kernel computed itself.  A NaN loses against a number, as in fmaxf.
+__device__ __forceinline__ float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// A row statistic (one value per token) of one or two positions.  A token's two lanes (t, t + 32) hold partial results of
+// every position; `row` combines them, and with two positions leaves position 0's rows in the lower lanes and position 1's
+// in the upper ones, so that what is computed from them (a root, a scale, its reciprocal) is computed once for both;
+// `each` hands them out again, to both lanes of the token.
+template <int NP> struct Rows;
+template <> struct Rows<1> {
+    static __device__ __forceinline__ float sum(const float (&v)[1]) { const Halves h = halves_of(v[0], v[0]); return h.lo + h.hi; }
+    static __device__ __forceinline__ float max(const float (&v)[1]) { const Halves h = halves_of(v[0], v[0]); return vmax(h.lo, h.hi); }
+    static __device__ __forceinline__ void each(float row, float (&v)[1]) { v[0] = row; }
+};
+template <> struct Rows<2> {
+    static __device__ __forceinline__ float sum(const float (&v)[2]) { const Halves h = halves_of(v[0], v[1]); return h.lo + h.hi; }
+    static __device__ __forceinline__ float max(const float (&v)[2]) { const Halves h = halves_of(v[0], v[1]); return vmax(h.lo, h.hi); }
+    static __device__ __forceinline__ void each(float row, float (&v)[2]) { const Halves h = halves_of(row, row); v[0] = h.lo; v[1] = h.hi; }
+};
+
 // exp(x) for x <= 0; same operation sequence as the CPU checker's bfo_exp_neg
 __device__ __forceinline__ float exp_neg(float x) {
     const float t = x * 1.44269504088896341f;

@@ -12,24 +12,38 @@
 // workgroup barrier.  The arithmetic is that of the other kernels operation for operation, so
 // the results are bit-identical to theirs.
 //
+// What bounds it (4096 positions, 8 layers, clocks of a SIMD per layer of some 54,000): the vector ALU's issue port, which
+// retires additions, products and fused ones every 2.4 clocks from two wavefronts, everything else every 4.4, fp32 matrix
+// steps (64 clocks, nothing beside them) and, of every int8 matrix step, 24 of its 33 clocks: together 45,000.  The rest
+// are the thirteen exchanges of a layer, whose latencies both wavefronts of a SIMD wait out at the same time, and weights
+// coming out of L2 in bursts.  So an exchange asks for everything at once, a row's statistics are computed once for both
+// positions (Rows), and addresses are made without vector instructions: 1573 us -> 1500.
+//
 // NPOS = 1 is the same kernel with one position per workgroup: the latency form for launches of
 // at most one workgroup per compute unit (each wavefront one tile of the width, every product
 // issued under the previous product's epilogue, and the workgroups of an XCD warming the L2
 // with the next layer's weights one layer ahead).
 //
-// LDS map (bytes): [xch: 3 slots x 2 positions x 8 waves x 64 floats] [hid: the quantised hidden
-// row, 32 KiB per position] [act: the quantised row of the width, 8 KiB per position] [par: one
+// LDS map (bytes): [xch: 3 slots x 2 positions x 8 waves x 64 floats] [act: the quantised row of the
+// width, 8 KiB per position] [hid: the quantised hidden row, 32 KiB per position] [par: one
 // copy of each quarter's side parameters, shared by its two wavefronts and both positions]
-// [tok: the activation scale of every token of the row that feeds QKV, per position].
+// [tok: the activation scale of every token of the row that feeds QKV, per position]
+// [key: what masks every token's scores as a key, per position].
 // During the heads the normalised stream of a position (32 KiB, fp32) overlays its hidden row.
 #pragma once
 
 #include "bf_board.hip.h"
 
-// register sets of the weight prefetch (one set = half a block; a set is refilled the moment its
-// half-block has been consumed, so all of them are in flight or full between products)
-#ifndef BF_DUO_SETS
-#define BF_DUO_SETS 3
+// Weight fragments (four registers each) a wave has in flight or in use.  What the loads cost is their rate out of L2 and
+// not their latency (a build without them runs 8 % shorter, one whose loads all hit L1 as well): at 4096 positions 8
+// places run 1507 us, 12 run 1498; 16 spill.
+#ifndef BF_DUO_RING
+#define BF_DUO_RING 12
+#endif
+// Steps between the LDS fetch of an operand fragment and its use.  4096 positions: 1496 us with one, 1498 with three (a
+// SIMD's other wavefront covers the latency); the one-position form at 100 positions: 118.3 and 116.7.
+#ifndef BF_DUO_AHEAD
+#define BF_DUO_AHEAD 3
 #endif
 
 namespace bf {
@@ -37,7 +51,6 @@ namespace duo {
 
 using board::block_at;
 using board::BlockAt;
-using board::dma;
 using board::frag_mma;
 using board::lds;
 using board::lds_barrier;
@@ -49,17 +62,18 @@ struct Cfg : Layout<256> {
     static constexpr int NP = NP_, NW = 8;   // positions per workgroup (2; 1: the latency form), wavefronts
     static constexpr int XS = NP * NW * 64;               // floats of one exchange slot
     static constexpr int XCH_OFF = 0;
-    static constexpr int HID_OFF = XCH_OFF + 3 * XS * 4;
-    static constexpr int HID_P = (F / 32) * FRAG;         // a position's hidden row
-    static constexpr int ACT_OFF = HID_OFF + NP * HID_P;
+    static constexpr int ACT_OFF = XCH_OFF + 3 * XS * 4;
     // a position's quantised row of the width: operand bytes; in the e4m3 format widened to fp16 on
     // the way in (every e4m3 value is an fp16 value), so that the products read ready-made operands
     static constexpr int ACT_FRAG = FP8 ? 2 * FRAG : FRAG;
     static constexpr int ACT_P = NT * ACT_FRAG;
-    static constexpr int PAR_OFF = ACT_OFF + NP * ACT_P;
+    static constexpr int HID_OFF = ACT_OFF + NP * ACT_P;
+    static constexpr int HID_P = (F / 32) * FRAG;         // a position's hidden row
+    static constexpr int PAR_OFF = HID_OFF + NP * HID_P;
     static constexpr int PWL_FLOATS = A_FLOATS + B_FLOATS;
     static constexpr int TOK_OFF = PAR_OFF + 4 * PWL_FLOATS * 4;   // activation scale of every token, per position
-    static constexpr int USED_BYTES = TOK_OFF + NP * 32 * 4;
+    static constexpr int KEY_OFF = TOK_OFF + NP * 32 * 4;          // what is added to the scores of every key: 0, or -inf for a dead token
+    static constexpr int USED_BYTES = KEY_OFF + NP * 32 * 4;
     // The one-position form serves launches of at most one workgroup per compute unit: asking for
     // more than half of a unit's LDS keeps the dispatcher from placing two of them on one unit
     // while another unit stays empty.
@@ -87,12 +101,12 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     constexpr int STEPS = C::STEPS, BPW = C::BPW, HB = C::HB;
     constexpr int NB = BPW / 2;      // weight blocks a wave consumes per layer
     constexpr int HT = 2;            // hidden tiles a wave computes per feed-forward step
-    constexpr int NSETS = BF_DUO_SETS;
+    constexpr int RING = BF_DUO_RING, AHEAD = BF_DUO_AHEAD;
     constexpr int XS = C::XS, PS = C::NW * 64;   // floats of an exchange slot; of one position's part of it
-    constexpr int HALF = BLOCK / 2;
     static_assert(C::KC == 1 && STEPS == TW && KCF == 2 * STEPS, "the 256-wide network");
-    static_assert((2 * NB) % NSETS == 0, "register set of a half-block must not depend on the layer");
-    static_assert(NSETS - 1 <= 2 * HB + 2, "the first prefetches of the heads stay inside the head blocks");
+    static_assert(8 % (AHEAD + 1) == 0, "an operand's place must not depend on the product");
+    static_assert((8 * NB) % RING == 0, "a fragment's place in the ring must not depend on the layer");
+    static_assert(RING <= 8 * HB + 8, "the first prefetches of the heads stay inside the head blocks");
     static_assert(board::block_at_covers_layer<1, TW, 2, BPW, true>(), "block_at must enumerate a layer's blocks exactly once");
 
     const int lane = threadIdx.x & 63;
@@ -172,41 +186,69 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         }
     };
 
+    // the lane's offsets, as opaque values: known bits would let the compiler make a base register out of every sum
+    // of them with a constant instead of using the instructions' own offsets
+    int lane16 = lane * 16, lane4 = lane * 4;
+    asm volatile("" : "+v"(lane16));
+    asm volatile("" : "+v"(lane4));
     float* const xch = reinterpret_cast<float*>(lds + C::XCH_OFF);
+    const float* const xlane = reinterpret_cast<const float*>(lds + C::XCH_OFF + lane4);
     uint8_t* const hid = lds + C::HID_OFF;
     uint8_t* const act = lds + C::ACT_OFF;
     float* const tok = reinterpret_cast<float*>(lds + C::TOK_OFF);
+    float* const key = reinterpret_cast<float*>(lds + C::KEY_OFF);
     const bool par_owner = sub == 0;
     float* const pA = reinterpret_cast<float*>(lds + C::PAR_OFF) + q * C::PWL_FLOATS;
     float* const pB = pA + C::A_FLOATS;
+    // LDS addresses that a layer uses once or twice are made where they are used (one vector addition): the empty asm
+    // keeps the compiler from hoisting them all out of the layer loop, where two dozen of them hold a register each
+    // that the operand and weight rings need.
+    auto here = [&](const void* at) -> uint8_t* {
+        int off = (int)(static_cast<const uint8_t*>(at) - lds);
+        asm volatile("" : "+s"(off));
+        return lds + off;
+    };
+    auto here_f = [&](const float* at) -> float* { return reinterpret_cast<float*>(here(at)); };
     const uint8_t* const wsrc =
-        a.wstream + ((size_t)q * ((size_t)a.n_layers * BPW + HB + 1) + (size_t)a.l0 * BPW) * BLOCK + lane * 16;
-    const float* const wpar = a.fparams + (size_t)q * a.n_layers * C::PW_FLOATS;
+        a.wstream + ((size_t)q * ((size_t)a.n_layers * BPW + HB + 1) + (size_t)a.l0 * BPW) * BLOCK;   // uniform
+    // the quarter's stream as a buffer: a load's address is a uniform offset and the lane's own, with no vector
+    // arithmetic and no address registers
+    const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wsrc), 0, ((a.n_layers - a.l0) * BPW + HB + 1) * BLOCK, 0x00027000);
+    const __amdgpu_buffer_rsrc_t pbuf = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a.fparams + (size_t)q * a.n_layers * C::PW_FLOATS), 0, a.n_layers * C::PW_FLOATS * 4, 0x00027000);
+    // `nfloats` of the quarter's side parameters, from float `at` on, straight into LDS
+    auto fetch_par = [&](int at, float* dst, int nfloats) {
+        uint8_t* const d = reinterpret_cast<uint8_t*>(dst);
+        const int bytes = nfloats * 4, full = bytes / FRAG, rem = (bytes % FRAG) / 16;
+#pragma unroll
+        for (int i = 0; i <= full; i++)
+            if (i < full || lane < rem)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(pbuf, (__attribute__((address_space(3))) void*)(d + i * FRAG), 16, lane16, at * 4 + i * FRAG, 0, 0);
+    };
     const float* const gp = a.fparams + (size_t)4 * a.n_layers * C::PW_FLOATS;
 
-    // half-block `hseq` of the quarter's stream into register set `set`
-    v4i frt[NSETS][4];
-    auto load_half = [&](int hseq, int set) {
+    // The weight fragments in flight: a ring of RING registers-of-four, refilled one by one.  Fragment `fseq` of the
+    // quarter's stream into place `at`.
+    v4i frt[RING];
+    auto load_frag = [&](int fseq, int at) {
 #ifdef BF_EXP_SAMEBLOCK   // timing experiment: every load reads the wave's first half-block (an L1 hit)
-        const uint8_t* src = wsrc + (size_t)(hseq & 0) * HALF;
+        const int src = (fseq & 3) * FRAG;
 #else
-        const uint8_t* src = wsrc + (size_t)hseq * HALF;
+        const int src = fseq * FRAG;
 #endif
 #ifdef BF_EXP_NOLOAD   // timing experiment: no weight traffic
         (void)src;
-#pragma unroll
-        for (int s = 0; s < 4; s++) asm volatile("" : "=v"(frt[set][s]));
+        asm volatile("" : "=v"(frt[at]));
 #else
-#pragma unroll
-        for (int s = 0; s < 4; s++) frt[set][s] = *reinterpret_cast<const v4i*>(src + s * FRAG);
+        frt[at] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane16, src, 0));
 #endif
     };
-    // the wave's hh-th half-block of the layer whose stream starts at block `base` (hh may run into
-    // the following layer, whose stream starts at block `next`)
-    auto fetch_half = [&](int hh, int base, int next) {
-        const int n = hh / 2;
+    // the wave's ff-th fragment of the layer whose stream starts at block `base` (ff may run into the following layer,
+    // whose stream starts at block `next`)
+    auto fetch_frag = [&](int ff, int base, int next) {
+        const int n = ff / 8;
         const BlockAt at = block_at<1, TW, 2, true>(n % NB);
-        load_half(2 * ((n < NB ? base : next) + at.a + sub * at.b) + hh % 2, hh % NSETS);
+        load_frag(8 * ((n < NB ? base : next) + at.a + sub * at.b) + ff % 8, ff % RING);
     };
 
     // L2 warm-up for launches of one wave of workgroups (NP == 1): such a launch moves through the
@@ -250,18 +292,32 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     // two tile sums of a quarter are added, then the four quarter sums in order.  One exchange slot
     // per call site, so that a fast wave's next partial cannot overwrite what a slow wave still
     // reads: between two uses of a slot lies at least one other workgroup barrier.
-    auto xsum2 = [&](const float (&part)[NP], int slot, float (&out)[NP]) {
+    // An exchange is a chain of latencies that both wavefronts of a SIMD wait out together, so everything a
+    // wave reads behind the barrier is asked for at once, before the first value is used.
+    auto xsum2 = [&](const float (&part)[NP], int slot) -> float {
 #pragma unroll
-        for (int p = 0; p < NP; p++) xch[slot * XS + p * PS + wave * 64 + lane] = part[p];
+        for (int p = 0; p < NP; p++) here_f(xch + slot * XS + p * PS + wave * 64)[lane] = part[p];
         barrier();
+        float s[NP][8], out[NP];
 #pragma unroll
-        for (int p = 0; p < NP; p++) {
-            const float* s = xch + slot * XS + p * PS + lane;
-            out[p] = (((s[0] + s[256]) + (s[64] + s[320])) + (s[128] + s[384])) + (s[192] + s[448]);
-        }
+        for (int p = 0; p < NP; p++)
+#pragma unroll
+            for (int w = 0; w < C::NW; w++) s[p][w] = xlane[slot * XS + p * PS + w * 64];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = 0; p < NP; p++) out[p] = (((s[p][0] + s[p][4]) + (s[p][1] + s[p][5])) + (s[p][2] + s[p][6])) + (s[p][3] + s[p][7]);
+        return Rows<NP>::sum(out);
+    };
+    // Largest value of the rows over waves [W0, W0 + 1, ...]: a wave publishes, for two positions, one value a row
+    // (Rows<2>::max, half the traffic of the lanes' own), for one position its lanes' own.
+    auto xmax_put = [&](const float (&am)[NP], int at) { here_f(xch + at + wave * 64)[lane] = NP == 2 ? Rows<NP>::max(am) : am[0]; };
+    auto xmax_row = [&](float m) -> float {
+        if constexpr (NP == 2) return m;
+        const float v[1] = {m};
+        return Rows<1>::max(v);
     };
     auto layernorm2 = [&](const float (&x)[NP][16], const float* gamma, const float* beta, float (&y)[NP][16]) {
-        float part[NP], s[NP], mean[NP], v[NP], rstd[NP];
+        float part[NP], mean[NP], rstd[NP];
 #pragma unroll
         for (int p = 0; p < NP; p++) {
             float acc = 0.0f;
@@ -269,10 +325,9 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             for (int r = 0; r < 16; r++) acc = acc + x[p][r];
             part[p] = acc;
         }
-        xsum2(part, 0, s);
+        Rows<NP>::each(xsum2(part, 0) * (1.0f / D), mean);
 #pragma unroll
         for (int p = 0; p < NP; p++) {
-            mean[p] = (s[p] + partner(s[p], g)) * (1.0f / D);
             float acc = 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -281,12 +336,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             }
             part[p] = acc;
         }
-        xsum2(part, 1, v);
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-            const float var = (v[p] + partner(v[p], g)) * (1.0f / D);
-            rstd[p] = recip_sqrt(var + a.eps);
-        }
+        Rows<NP>::each(recip_sqrt(xsum2(part, 1) * (1.0f / D) + a.eps), rstd);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const v4f ga = ldg4(gamma + 8 * j + 4 * g);
@@ -303,23 +353,28 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     // signed quantiser of both positions' rows: one scale per row; this wave's bytes go to the
     // position's activation buffer, from which every wave reads its B operands
     auto quant_exchange2 = [&](const float (&y)[NP][16], float (&sa)[NP], int8_t* tap, const size_t (&tap_row)[NP], bool publish_scales) {
+        float am[NP];
 #pragma unroll
         for (int p = 0; p < NP; p++) {
-            float am = 0.0f;
+            am[p] = 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; r++) am = __builtin_fmaxf(am, __builtin_fabsf(y[p][r]));
-            xch[2 * XS + p * PS + wave * 64 + lane] = am;
+            for (int r = 0; r < 16; r++) am[p] = __builtin_fmaxf(am[p], __builtin_fabsf(y[p][r]));
         }
+        xmax_put(am, 2 * XS);
         barrier();
+        float mw[8];
+#pragma unroll
+        for (int w = 0; w < C::NW; w++) mw[w] = xlane[2 * XS + w * 64];
+        const float sr = row_scale<FP8>(xmax_row(vmax3(vmax3(mw[0], mw[1], mw[2]), vmax3(mw[3], mw[4], mw[5]), vmax(mw[6], mw[7]))));
+        Rows<NP>::each(sr, sa);
+        if (publish_scales && wave == 0 && lane < 32 * NP) here_f(tok)[lane] = sr;
+        const Quot br = quot_by(sr);
+        float hi[NP], lo[NP];
+        Rows<NP>::each(br.hi, hi);
+        Rows<NP>::each(br.lo, lo);
 #pragma unroll
         for (int p = 0; p < NP; p++) {
-            float m = 0.0f;
-#pragma unroll
-            for (int w = 0; w < C::NW; w++) m = __builtin_fmaxf(m, xch[2 * XS + p * PS + w * 64 + lane]);
-            m = __builtin_fmaxf(m, partner(m, g));
-            sa[p] = row_scale<FP8>(m);
-            if (publish_scales && wave == 0 && g == 0) tok[p * 32 + t] = sa[p];
-            const Quot by = quot_by(sa[p]);
+            const Quot by = {hi[p], lo[p]};
             v4i w;
 #pragma unroll
             for (int j = 0; j < 4; j++)
@@ -328,9 +383,9 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                 const v2l wl = __builtin_bit_cast(v2l, w);
 #pragma unroll
                 for (int h = 0; h < 2; h++)
-                    *reinterpret_cast<v8h*>(act + p * C::ACT_P + (2 * tile + h) * FRAG + lane * 16) = e4m3x8_as_f16(wl[h]);
+                    *reinterpret_cast<v8h*>(here(act + p * C::ACT_P + (2 * tile + h) * FRAG) + lane16) = e4m3x8_as_f16(wl[h]);
             } else {
-                *reinterpret_cast<v4i*>(act + p * C::ACT_P + tile * FRAG + lane * 16) = w;
+                *reinterpret_cast<v4i*>(here(act + p * C::ACT_P + tile * FRAG) + lane16) = w;
             }
             if (TAPS && tap && live[p])
 #pragma unroll
@@ -339,18 +394,18 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         }
         barrier();
     };
-    const uint8_t* const act0 = act + lane * 16;
-    const uint8_t* const hid0 = hid + lane * 16;
+    const uint8_t* const act0 = act + lane16;
+    const uint8_t* const hid0 = hid + lane16;
     auto ldsfrag = [&](const uint8_t* p) -> v4i { return *reinterpret_cast<const v4i*>(p); };
 
     // ---- start the weight stream and the first layer's parameters --------------------------------
     if (nl_run > 0) {
 #pragma unroll
-        for (int j = 0; j < NSETS; j++) fetch_half(j, 0, BPW);
+        for (int j = 0; j < RING; j++) fetch_frag(j, 0, BPW);
         warm_l2(a.l0 * BPW);
         if (par_owner) {
-            dma(wpar + (size_t)a.l0 * C::PW_FLOATS, pA, C::A_FLOATS, lane);
-            dma(wpar + (size_t)a.l0 * C::PW_FLOATS + C::A_FLOATS, pB, C::B_FLOATS, lane);
+            fetch_par(a.l0 * C::PW_FLOATS, pA, C::A_FLOATS);
+            fetch_par(a.l0 * C::PW_FLOATS + C::A_FLOATS, pB, C::B_FLOATS);
         }
     }
 
@@ -368,6 +423,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         const unsigned word = enc_only ? (a.taps.alive[(size_t)b * T + t] ? 0u : 0x800u) : a.boards[(size_t)b * T + t];
         ctrl[p] = enc_only ? 1 : a.control[b];
         alive[p] = (unsigned)__ballot(((word >> 11) & 1) == 0 && g == 0);
+        if (wave == 0 && g == 0) key[p * 32 + t] = ((word >> 11) & 1) == 0 ? 0.0f : -__builtin_inff();
         if (ENC || (TAPS && a.taps.x_in)) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -426,31 +482,30 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #endif
         // One position's product with the wave's k-th block of this layer: eight 32-deep steps against
         // the operand row whose fragment 0 is at BSRC (lane offset included), each fragment fetched
-        // from LDS one step ahead.  The block's two halves sit in register sets 2k % NSETS and
-        // (2k + 1) % NSETS; the last position refills each of them as soon as it has consumed it (with
-        // the half-blocks NSETS on), so every set is in flight or full across the phases between
-        // products (attention, the LayerNorms).
+        // from LDS one step ahead.  The last position refills a fragment's place in the ring as soon as it has
+        // consumed it, with the fragment RING further on, so every place is in flight or full across the phases
+        // between products (attention, the LayerNorms).
         // BETWEEN(s) runs after step s has been issued: an eighth of the previous product's epilogue,
         // which the vector ALU works through while the matrix pipe runs; nothing is scheduled across
         // the end of a step.
-#ifndef BF_DUO_AHEAD
-#define BF_DUO_AHEAD 1   // steps between the LDS fetch of an operand fragment and its use
-#endif
-#define BF_DUO_CHAIN(SWAP, k, p, BSRC, INIT, R, BETWEEN)                                             \
+        // The operand fragments come from LDS AHEAD steps early, also across the products of a phase: in its last
+        // steps a product fetches the first operands of the next one (at NEXT, if there is one whose operands are
+        // written already: MORE).  BF_DUO_OPERANDS opens a phase with the first product's.
+#define BF_DUO_OPERANDS(BSRC)                                                                        \
+    v4i ops_[AHEAD + 1];                                                                             \
+    _Pragma("unroll") for (int u_ = 0; u_ < AHEAD; u_++) ops_[u_] = ldsfrag((BSRC) + u_ * FRAG)
+#define BF_DUO_CHAIN(SWAP, k, p, BSRC, MORE, NEXT, INIT, R, BETWEEN)                                 \
     do {                                                                                             \
-        constexpr int A_ = BF_DUO_AHEAD;                                                             \
-        const uint8_t* const b_ = (BSRC);                                                            \
-        v4i ring_[A_ + 1];                                                                           \
-        _Pragma("unroll") for (int u_ = 0; u_ < A_; u_++) ring_[u_] = ldsfrag(b_ + u_ * FRAG);       \
+        const uint8_t *const b_ = (BSRC), *const n_ = (NEXT);                                        \
         (R) = (INIT);                                                                                \
         _Pragma("unroll") for (int s_ = 0; s_ < 8; s_++) {                                           \
-            if (s_ + A_ < 8) ring_[(s_ + A_) % (A_ + 1)] = ldsfrag(b_ + (s_ + A_) * FRAG);           \
-            (R) = frag_mma<SWAP>(frt[(2 * (k) + s_ / 4) % NSETS][s_ % 4], ring_[s_ % (A_ + 1)], (R)); \
+            if (s_ + AHEAD < 8) ops_[(s_ + AHEAD) % (AHEAD + 1)] = ldsfrag(b_ + (s_ + AHEAD) * FRAG); \
+            else if (MORE) ops_[(s_ + AHEAD) % (AHEAD + 1)] = ldsfrag(n_ + (s_ + AHEAD - 8) * FRAG);   \
+            (R) = frag_mma<SWAP>(frt[(8 * (k) + s_) % RING], ops_[s_ % (AHEAD + 1)], (R));           \
             BETWEEN(s_);                                                                             \
             __builtin_amdgcn_sched_barrier(0);                                                       \
-            if ((p) == NP - 1 && s_ == 3) fetch_half(2 * (k) + NSETS, lbase, lfollow);               \
+            if ((p) == NP - 1) fetch_frag(8 * (k) + s_ + RING, lbase, lfollow);                      \
         }                                                                                            \
-        if ((p) == NP - 1) fetch_half(2 * (k) + NSETS + 1, lbase, lfollow);                          \
     } while (0)
         // e4m3: both positions' products with the wave's k-th block, step by step.  A weight fragment is
         // widened to fp16 once and multiplied with both positions' operands; these come from LDS
@@ -470,7 +525,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             _Pragma("unroll") for (int p_ = 0; p_ < 2; p_++)                                         \
                 _Pragma("unroll") for (int h_ = 0; h_ < ((A16) ? 2 : 1); h_++)                       \
                     nxt_[p_][h_] = s_ + 1 < 8 ? ldsfrag(bp_[p_] + ((A16) ? 2 * (s_ + 1) + h_ : s_ + 1) * FRAG) : cur_[p_][h_]; \
-            const v2l wl_ = __builtin_bit_cast(v2l, frt[(2 * (k) + s_ / 4) % NSETS][s_ % 4]);        \
+            const v2l wl_ = __builtin_bit_cast(v2l, frt[(8 * (k) + s_) % RING]);                      \
             _Pragma("unroll") for (int h_ = 0; h_ < 2; h_++) {                                       \
                 const v8h wh_ = e4m3x8_as_f16(wl_[h_]);                                              \
                 _Pragma("unroll") for (int p_ = 0; p_ < 2; p_++) {                                   \
@@ -483,9 +538,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             __builtin_amdgcn_sched_barrier(0);                                                       \
             _Pragma("unroll") for (int p_ = 0; p_ < 2; p_++)                                         \
                 _Pragma("unroll") for (int h_ = 0; h_ < ((A16) ? 2 : 1); h_++) cur_[p_][h_] = nxt_[p_][h_]; \
-            if (s_ == 3) fetch_half(2 * (k) + NSETS, lbase, lfollow);                                \
+            fetch_frag(8 * (k) + s_ + RING, lbase, lfollow);                                         \
         }                                                                                            \
-        fetch_half(2 * (k) + NSETS + 1, lbase, lfollow);                                             \
     } while (0)
         const acc_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         auto none = [&](int) {};
@@ -495,13 +549,13 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         float sa[NP];
         {
             float y[NP][16];
-            layernorm2(x, pA + C::A_LN1G + 32 * sub, pA + C::A_LN1B + 32 * sub, y);
+            layernorm2(x, here_f(pA + C::A_LN1G + 32 * sub), here_f(pA + C::A_LN1B + 32 * sub), y);
             quant_exchange2(y, sa, TAPS ? a.taps.qa_qkv : nullptr, bl, true);
         }
         // the quarter's feed-forward parameters of this layer (the first layer's came with the start)
         if (par_owner && li > 0) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            dma(wpar + (size_t)l * C::PW_FLOATS + C::A_FLOATS, pB, C::B_FLOATS, lane);
+            fetch_par(l * C::PW_FLOATS + C::A_FLOATS, pB, C::B_FLOATS);
         }
         BF_PHASE(PH_LN1);
 
@@ -509,8 +563,9 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         float o[NP][16];
         {
             float qf[NP][16], kf[NP][16], vf[NP][16];
-            const float swq = pA[C::A_SW + sub], swk = pA[C::A_SW + TW + sub], swv = pA[C::A_SW + 2 * TW + sub];
-            const float bv = pA[C::A_BV + 32 * sub + t];
+            const float* const sw3 = here_f(pA + C::A_SW + sub);
+            const float swq = sw3[0], swk = sw3[TW], swv = sw3[2 * TW];
+            const float bv = here_f(pA + C::A_BV + 32 * sub)[t];
             acc_t acc[2];   // product n of a sequence uses accumulator n & 1; the previous one's epilogue runs under it
             v4f bq[4], bk[4], stok[NP][4];
             // the epilogues, two accumulator registers at a time (slice s of eight)
@@ -544,70 +599,81 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                 else if (tq == 1) epi_k(p, s, ai);
                 else epi_v(p, s, ai);
             };
-            load_tile16(pA + C::A_BQ + 32 * sub, g, bq);
+            load_tile16(here_f(pA + C::A_BQ + 32 * sub), g, bq);
             if constexpr (FP8) {
                 // e4m3: a block's two products share the widening of its weight fragments, the
                 // epilogues of both positions follow
                 BF_DUO_PAIR_F8(false, 0, true, act0, act1, acc);
 #pragma unroll
                 for (int s = 0; s < 8; s++) { epi_q(0, s, 0); epi_q(1, s, 1); }
-                load_tile16(pA + C::A_BK + 32 * sub, g, bk);
+                load_tile16(here_f(pA + C::A_BK + 32 * sub), g, bk);
                 BF_DUO_PAIR_F8(false, 1, true, act0, act1, acc);
 #pragma unroll
                 for (int s = 0; s < 8; s++) { epi_k(0, s, 0); epi_k(1, s, 1); }
-                load_tile16(tok, g, stok[0]);
-                load_tile16(tok + 32, g, stok[1]);
+                load_tile16(here_f(tok), g, stok[0]);
+                load_tile16(here_f(tok + 32), g, stok[1]);
                 BF_DUO_PAIR_F8(true, 2, true, act0, act1, acc);
 #pragma unroll
                 for (int s = 0; s < 8; s++) { epi_v(0, s, 0); epi_v(1, s, 1); }
             } else {
                 // Q, K, V blocks in turn, each for every position: 3 NP products
+                BF_DUO_OPERANDS(act0);
 #pragma unroll
                 for (int n = 0; n < 3 * NP; n++) {
                     const int tq = n / NP, p = n % NP;
-                    if (n == NP) load_tile16(pA + C::A_BK + 32 * sub, g, bk);
-                    if (tq == 2) load_tile16(tok + 32 * p, g, stok[p]);
+                    if (n == NP) load_tile16(here_f(pA + C::A_BK + 32 * sub), g, bk);
+                    if (tq == 2) load_tile16(here_f(tok + 32 * p), g, stok[p]);
                     auto between = [&](int s) {
                         if (n > 0) epi_qkv((n - 1) / NP, (n - 1) % NP, s, (n - 1) & 1);
                     };
-                    if (tq == 2) BF_DUO_CHAIN(true, 2, p, act0 + p * C::ACT_P, zero, acc[n & 1], between);
-                    else BF_DUO_CHAIN(false, tq, p, act0 + p * C::ACT_P, zero, acc[n & 1], between);
+                    const uint8_t* const next = act0 + (n + 1) % NP * C::ACT_P;
+                    if (tq == 2) BF_DUO_CHAIN(true, 2, p, act0 + p * C::ACT_P, n + 1 < 3 * NP, next, zero, acc[n & 1], between);
+                    else BF_DUO_CHAIN(false, tq, p, act0 + p * C::ACT_P, n + 1 < 3 * NP, next, zero, acc[n & 1], between);
                 }
 #pragma unroll
                 for (int s = 0; s < 8; s++) epi_v(NP - 1, s, (3 * NP - 1) & 1);
             }
             BF_PHASE(PH_QKV);
             if (l + 1 < a.l1) warm_l2((l + 1) * BPW);   // the sets are full and the next weight wait is an attention away
+            v16f sc[NP];   // scores, transposed: lane = query token, register r = key ch(r, g)
+            auto scores = [&](int p) {
+                sc[p] = v16f{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-            for (int p = 0; p < NP; p++) {
-                // scores, transposed: lane = query token, register r = key ch(r, g)
-                v16f sc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-                for (int r = 0; r < 16; r++) sc = BF_F32MMA(kf[p][r], qf[p][r], sc);
-                float pr[16];
+                for (int r = 0; r < 16; r++) sc[p] = BF_F32MMA(kf[p][r], qf[p][r], sc[p]);
+            };
+            float pr[NP][16], rl[NP];
+            auto softmax = [&](int p) {
                 float mx = -__builtin_inff();
+                v4f kb[4];
+                load_tile16(here_f(key + 32 * p), g, kb);
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    float s = sc[r] * 0.17677669529663687f;
-                    s = ((alive[p] >> ch(r, g)) & 1u) ? s : -__builtin_inff();
-                    pr[r] = s;
-                    mx = __builtin_fmaxf(mx, s);
+                    // scaled and masked in one operation: adding 0 changes nothing, a dead key's -inf (or what an infinite
+                    // score makes of it, NaN) loses in the maximum and has probability 0
+                    pr[p][r] = __builtin_fmaf(sc[p][r], 0.17677669529663687f, kb[r / 4][r % 4]);
+                    mx = __builtin_fmaxf(mx, pr[p][r]);
                 }
-                mx = __builtin_fmaxf(mx, partner(mx, g));
+                const float mx1[1] = {mx};
+                mx = Rows<1>::max(mx1);
                 float lsum = 0.0f;
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    pr[r] = exp_neg(pr[r] - mx);
-                    lsum = lsum + pr[r];
+                    pr[p][r] = exp_neg(pr[p][r] - mx);
+                    lsum = lsum + pr[p][r];
                 }
-                const float rl = recip(lsum + partner(lsum, g));
+                const float ls1[1] = {lsum};
+                rl[p] = recip(Rows<1>::sum(ls1));
+            };
+            auto weigh = [&](int p) {
                 v16f oa = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-                for (int r = 0; r < 16; r++) oa = BF_F32MMA(vf[p][r], pr[r] * rl, oa);
+                for (int r = 0; r < 16; r++) oa = BF_F32MMA(vf[p][r], pr[p][r] * rl[p], oa);
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[p][r] = oa[r];
                 pin16(o[p]);
-            }
+            };
+#pragma unroll
+            for (int p = 0; p < NP; p++) { scores(p); softmax(p); weigh(p); }
             BF_PHASE(PH_ATTN);
         }
 
@@ -617,8 +683,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             quant_exchange2(o, so, TAPS ? a.taps.qa_out : nullptr, bl, false);
             acc_t acc[2];
             v4f bo[4];
-            load_tile16(pA + C::A_BOUT + 32 * sub, g, bo);
-            const float sw = pA[C::A_SW + 3 * TW + sub];
+            load_tile16(here_f(pA + C::A_BOUT + 32 * sub), g, bo);
+            const float sw = *here_f(pA + C::A_SW + 3 * TW + sub);
             auto epi_o = [&](int p, int s, int ai) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
@@ -632,12 +698,13 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
                 for (int s = 0; s < 8; s++) epi_o(0, s, 0);
             } else {
+                BF_DUO_OPERANDS(act0);
 #pragma unroll
                 for (int p = 0; p < NP; p++) {
                     auto between = [&](int s) {
                         if (p > 0) epi_o(p - 1, s, (p - 1) & 1);
                     };
-                    BF_DUO_CHAIN(false, 3, p, act0 + p * C::ACT_P, zero, acc[p & 1], between);
+                    BF_DUO_CHAIN(false, 3, p, act0 + p * C::ACT_P, p + 1 < NP, act0 + C::ACT_P, zero, acc[p & 1], between);
                 }
             }
 #pragma unroll
@@ -648,13 +715,13 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         // ---- feed-forward ---------------------------------------------------------------------------------
         {
             float y[NP][16];
-            layernorm2(x, pB + C::B_LN2G + 32 * sub, pB + C::B_LN2B + 32 * sub, y);
+            layernorm2(x, here_f(pB + C::B_LN2G + 32 * sub), here_f(pB + C::B_LN2B + 32 * sub), y);
             quant_exchange2(y, sa, TAPS ? a.taps.qa_ff1 : nullptr, bl, false);
         }
         // the attention-phase parameters are dead for both waves of the quarter: fetch the next layer's
         if (par_owner) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            dma(wpar + (size_t)lnext * C::PW_FLOATS, pA, C::A_FLOATS, lane);
+            fetch_par(lnext * C::PW_FLOATS, pA, C::A_FLOATS);
         }
         BF_PHASE(PH_LN2);
         // First matmul, step by step: each step's two 256-wide chunks are quantised as soon as the step
@@ -663,6 +730,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         float sh[NP][KCF];
 #pragma unroll
         for (int st = 0; st < STEPS; st++) {
+            BF_DUO_OPERANDS(act0);
             float hf[NP][HT][16];
             float am[NP];
 #pragma unroll
@@ -685,8 +753,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             };
 #pragma unroll
             for (int i = 0; i < HT; i++) {
-                load_tile16(pB + C::B_BFF1 + 128 * st + 32 * (HT * sub + i), g, b1[i]);
-                sw1[i] = pB[C::B_SW + 4 * st + HT * sub + i];
+                load_tile16(here_f(pB + C::B_BFF1 + 128 * st + 32 * (HT * sub + i)), g, b1[i]);
+                sw1[i] = *here_f(pB + C::B_SW + 4 * st + HT * sub + i);
                 if constexpr (FP8) {
                     BF_DUO_PAIR_F8(false, 4 + HT * st + i, true, act0, act1, acc);
 #pragma unroll
@@ -698,7 +766,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                         auto between = [&](int s) {
                             if (n > 0) epi_f((n - 1) / NP, (n - 1) % NP, s, (n - 1) & 1);
                         };
-                        BF_DUO_CHAIN(false, 4 + HT * st + i, p, act0 + p * C::ACT_P, zero, acc[n & 1], between);
+                        BF_DUO_CHAIN(false, 4 + HT * st + i, p, act0 + p * C::ACT_P, n + 1 < NP * HT, act0 + (p + 1) % NP * C::ACT_P, zero, acc[n & 1],
+                                     between);
                     }
                 }
             }
@@ -707,23 +776,28 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                 for (int s = 0; s < 8; s++) epi_f(HT - 1, NP - 1, s, (NP * HT - 1) & 1);
             // the maxima of consecutive steps go through different exchange slots
             const int xs = (st & 1) ? 0 : 2 * XS;
-#pragma unroll
-            for (int p = 0; p < NP; p++) xch[xs + p * PS + wave * 64 + lane] = am[p];
+            xmax_put(am, xs);
             barrier();
+            float hi[NP], lo[NP];
+            {
+                float mw[8], sc[2];
+#pragma unroll
+                for (int w = 0; w < C::NW; w++) mw[w] = xlane[xs + w * 64];
+#pragma unroll
+                for (int c = 0; c < 2; c++) {   // chunk c: quarters 2c and 2c + 1 (hidden values are >= 0)
+                    float each[NP];
+                    sc[c] = hidden_scale<FP8>(xmax_row(vmax(vmax3(mw[2 * c], mw[2 * c + 1], mw[2 * c + 4]), mw[2 * c + 5])));
+                    Rows<NP>::each(sc[c], each);
+#pragma unroll
+                    for (int p = 0; p < NP; p++) sh[p][2 * st + c] = each[p];
+                }
+                const Quot br = quot_by(q < 2 ? sc[0] : sc[1]);
+                Rows<NP>::each(br.hi, hi);
+                Rows<NP>::each(br.lo, lo);
+            }
 #pragma unroll
             for (int p = 0; p < NP; p++) {
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    float m = 0.0f;   // hidden values are >= 0
-#pragma unroll
-                    for (int u = 0; u < 2; u++)
-                        m = __builtin_fmaxf(m, __builtin_fmaxf(xch[xs + p * PS + (2 * c + 4 * u) * 64 + lane],
-                                                               xch[xs + p * PS + (2 * c + 1 + 4 * u) * 64 + lane]));
-                    m = __builtin_fmaxf(m, partner(m, g));
-                    sh[p][2 * st + c] = hidden_scale<FP8>(m);
-                }
-                const float s8 = q < 2 ? sh[p][2 * st] : sh[p][2 * st + 1];
-                const Quot by = quot_by(s8);
+                const Quot by = {hi[p], lo[p]};
 #pragma unroll
                 for (int i = 0; i < HT; i++) {
                     v4i w;
@@ -736,7 +810,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                             *reinterpret_cast<unsigned*>(a.taps.qa_ff2 + (bl[p] * T + t) * F + 512 * st + 128 * q + 32 * (HT * sub + i) + 8 * j + 4 * g) = u;
                         w[j] = (int)(FP8 ? u : (u ^ 0x80808080u));
                     }
-                    *reinterpret_cast<v4i*>(hid + p * C::HID_P + (16 * st + 4 * q + HT * sub + i) * FRAG + lane * 16) = w;
+                    *reinterpret_cast<v4i*>(here(hid + p * C::HID_P + (16 * st + 4 * q + HT * sub + i) * FRAG) + lane16) = w;
                 }
             }
         }
@@ -750,10 +824,11 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             float o32[NP][16];
             acc_t acc[2];
             acc_t init = zero;
+            BF_DUO_OPERANDS(hid0);
             float sw2[KCF];   // e4m3: one weight scale per k-chunk
             if constexpr (FP8)
 #pragma unroll
-                for (int cc = 0; cc < KCF; cc++) sw2[cc] = pB[C::B_SW + 16 + sub * KCF + cc];
+                for (int cc = 0; cc < KCF; cc++) sw2[cc] = here_f(pB + C::B_SW + 16 + sub * KCF)[cc];
             auto epi_2 = [&](int cc, int p, int s, int ai) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
@@ -778,10 +853,10 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                 } else {
 #pragma unroll
                     for (int p = 0; p < NP; p++) {
-                        const int n = NP * cc + p;
+                        const int n = NP * cc + p, cn = (n + 1) / NP, pn = (n + 1) % NP;
                         if (p == 0) {
                             v4i w0[4];
-                            load_tile16i(pB + C::B_WSUM + cc * CW + 32 * sub, g, w0);
+                            load_tile16i(here_f(pB + C::B_WSUM + cc * CW + 32 * sub), g, w0);
 #pragma unroll
                             for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -790,7 +865,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                         auto between = [&](int s) {
                             if (n > 0) epi_2((n - 1) / NP, (n - 1) % NP, s, (n - 1) & 1);
                         };
-                        BF_DUO_CHAIN(false, 4 + HT * STEPS + cc, p, hid0 + p * C::HID_P + 8 * cc * FRAG, init, acc[n & 1], between);
+                        BF_DUO_CHAIN(false, 4 + HT * STEPS + cc, p, hid0 + p * C::HID_P + 8 * cc * FRAG,
+                                     cn < KCF, hid0 + pn * C::HID_P + 8 * cn * FRAG, init, acc[n & 1], between);
                     }
                 }
             }
@@ -798,8 +874,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
                 for (int s = 0; s < 8; s++) epi_2(KCF - 1, NP - 1, s, (NP * KCF - 1) & 1);
             v4f b2[4];
-            load_tile16(pB + C::B_BFF2 + 32 * sub, g, b2);
-            const float sw = pB[C::B_SW + 16 + sub];
+            load_tile16(here_f(pB + C::B_BFF2 + 32 * sub), g, b2);
+            const float sw = *here_f(pB + C::B_SW + 16 + sub);
 #pragma unroll
             for (int p = 0; p < NP; p++) {
 #pragma unroll
@@ -816,6 +892,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         }
         BF_PHASE(PH_FF2);
         warm_done();
+#undef BF_DUO_OPERANDS
 #undef BF_DUO_CHAIN
 #undef BF_DUO_PAIR_F8
         if (TAPS && a.taps.resid)
@@ -848,10 +925,10 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     // ---- final norm and heads --------------------------------------------------------------------------
     // The weight stream is restarted at the head blocks (after the last layer the prefetch ran on
     // into a layer that is not used).
-    const int hseq0 = (a.n_layers - a.l0) * BPW;
+    const int hblk0 = (a.n_layers - a.l0) * BPW;
     wait_vm<0>();   // also: no parameter copy is still landing
 #pragma unroll
-    for (int j = 0; j < NSETS - 1; j++) load_half(2 * hseq0 + j, j);
+    for (int j = 0; j < RING; j++) load_frag(8 * hblk0 + j, j);
     float hn[NP][16];
     layernorm2(x, gp + C::G_NFG + 32 * tile, gp + C::G_NFB + 32 * tile, hn);
     // publish as B-operand fragments (n, j): lane holds the four floats of register quad j
@@ -880,16 +957,12 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     v16f head = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (q < 3 && heads_here) {
 #pragma unroll
-        for (int hi = 0; hi < 2 * HB; hi++) {
-            // the stream is padded by one block: two half-blocks past the last head block exist
-            if (hi + NSETS - 1 < 2 * HB + 2) load_half(2 * hseq0 + hi + NSETS - 1, (hi + NSETS - 1) % NSETS);
+        for (int f = 0; f < 8 * HB; f++) {
+            const v4f w = __builtin_bit_cast(v4f, frt[f % RING]);
+            const v4f hv = *reinterpret_cast<const v4f*>(hnb + (f * 64 + lane) * 4);
 #pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const v4f w = __builtin_bit_cast(v4f, frt[hi % NSETS][s]);
-                const v4f hv = *reinterpret_cast<const v4f*>(hnb + ((hi * 4 + s) * 64 + lane) * 4);
-#pragma unroll
-                for (int k = 0; k < 4; k++) head = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k], hv[k], head, 0, 0, 0);
-            }
+            for (int k = 0; k < 4; k++) head = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k], hv[k], head, 0, 0, 0);
+            if (f + RING < 8 * HB) load_frag(8 * hblk0 + f + RING, f % RING);
         }
     }
     BF_PHASE(PH_HEADS);
@@ -1012,7 +1085,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             // its blocks are read straight from the stream, in the same order as above
             v16f hd = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
             for (int f = 0; f < 8 * HB; f++) {
-                const v4f w = *reinterpret_cast<const v4f*>(wsrc + (size_t)hseq0 * BLOCK + (size_t)f * FRAG);
+                const v4f w = *reinterpret_cast<const v4f*>(wsrc + (size_t)hblk0 * BLOCK + (size_t)f * FRAG + lane16);
                 const v4f hvv = *reinterpret_cast<const v4f*>(hnb + (f * 64 + lane) * 4);
 #pragma unroll
                 for (int k = 0; k < 4; k++) hd = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k], hvv[k], hd, 0, 0, 0);
