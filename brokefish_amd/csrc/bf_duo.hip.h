@@ -599,6 +599,10 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                 else if (tq == 1) epi_k(p, s, ai);
                 else epi_v(p, s, ai);
             };
+            // A SIMD favours its older wavefront, which then waits at the next exchange for a partner that has the SIMD to
+            // itself: the younger one goes first here, the older one in the attention behind (4096 positions -1.3 to
+            // -2.9 %, e4m3 -1.8 %; first in the attention too: +5 to +10 %; in other phases: nothing)
+            if (sub) __builtin_amdgcn_s_setprio(2);
             load_tile16(here_f(pA + C::A_BQ + 32 * sub), g, bq);
             if constexpr (FP8) {
                 // e4m3: a block's two products share the widening of its weight fragments, the
@@ -633,6 +637,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
                 for (int s = 0; s < 8; s++) epi_v(NP - 1, s, (3 * NP - 1) & 1);
             }
+            __builtin_amdgcn_s_setprio(0);
             BF_PHASE(PH_QKV);
             if (l + 1 < a.l1) warm_l2((l + 1) * BPW);   // the sets are full and the next weight wait is an attention away
             v16f sc[NP];   // scores, transposed: lane = query token, register r = key ch(r, g)
