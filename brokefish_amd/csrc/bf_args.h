@@ -163,10 +163,7 @@ hipError_t launch_twin256_taps(const KArgs& k, hipStream_t stream);
 hipError_t launch_twin256_fp8(const KArgs& k, hipStream_t stream);
 hipError_t launch_twin256_fp8_taps(const KArgs& k, hipStream_t stream);
 // one position per workgroup of eight wavefronts (two per quarter of the width), one workgroup
-// per compute unit: the lowest latency per position for the 256-wide network (int8, e4m3), and
-// the faster form for the 512-wide one (int8)
-hipError_t launch_octo256_fp8(const KArgs& k, hipStream_t stream);
-hipError_t launch_octo256_fp8_taps(const KArgs& k, hipStream_t stream);
+// per compute unit: the faster form for the 512-wide network (int8)
 hipError_t launch_octo512(const KArgs& k, hipStream_t stream);
 hipError_t launch_octo512_taps(const KArgs& k, hipStream_t stream);
 // two positions per workgroup of eight wavefronts (256-wide network): a weight fragment fetched
@@ -178,8 +175,8 @@ hipError_t launch_duo256_fp8_taps(const KArgs& k, hipStream_t stream);
 // the encoder-only builds of the kernels AUTO chooses from
 hipError_t launch_duo256_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_enc(const KArgs& k, hipStream_t stream);
-hipError_t launch_twin256_fp8_enc(const KArgs& k, hipStream_t stream);
-hipError_t launch_octo256_fp8_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_duo256_fp8_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_solo256_fp8_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_octo512_enc(const KArgs& k, hipStream_t stream);
 // the builds that carry the phase profile
 hipError_t launch_twin256_prof(const KArgs& k, hipStream_t stream);
@@ -189,14 +186,16 @@ hipError_t launch_board256_prof(const KArgs& k, hipStream_t stream);
 hipError_t launch_board512_prof(const KArgs& k, hipStream_t stream);
 hipError_t launch_board256_fp8_prof(const KArgs& k, hipStream_t stream);
 hipError_t launch_twin256_fp8_prof(const KArgs& k, hipStream_t stream);
-hipError_t launch_octo256_fp8_prof(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_fp8_prof(const KArgs& k, hipStream_t stream);
 hipError_t launch_prof_fp8(const KArgs& k, int grid, hipStream_t stream);
 // the same kernel with one position per workgroup (the eight-wavefront form for launches that
-// cannot fill the GPU): int8, 256-wide network
+// cannot fill the GPU): 256-wide network
 hipError_t launch_solo256(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_taps(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_prof(const KArgs& k, hipStream_t stream);
+hipError_t launch_solo256_fp8(const KArgs& k, hipStream_t stream);
+hipError_t launch_solo256_fp8_taps(const KArgs& k, hipStream_t stream);
+hipError_t launch_solo256_fp8_prof(const KArgs& k, hipStream_t stream);
 // several workgroups per position: launches of at most team_positions() positions (0: not on this device; `look`
 // allows the one look at the device, which synchronises), with team_slot_bytes() of workspace for each
 hipError_t launch_team256(const KArgs& k, hipStream_t stream);

@@ -238,7 +238,7 @@ __device__ __forceinline__ float recip_sqrt(float x) {
 // whose quotient lies that close to the edge of a tie's rounding interval could differ; there are
 // 7564 such pairs of significands within sixteen times that distance, and all agree
 // (tests/test_quotient.py enumerates them; the last term of lo is what two of them need).  For scales above
-// 2^102 lo loses bits to the subnormal range, and a quotient within 2^-20 of a tie may go either way.
+// 2^102 (2^99 where an eighth of it is taken) lo loses bits to the subnormal range, and a quotient within 2^-20 of a tie may go either way.
 struct Quot { float hi, lo; };
 __device__ __forceinline__ Quot quot_by(float sa) {
     const float hi = recip(sa);
@@ -299,6 +299,22 @@ __device__ __forceinline__ unsigned quant4_relu_u8(float v0, float v1, float v2,
 #pragma unroll
     for (int i = 0; i < 4; i++) w = __builtin_amdgcn_cvt_pk_u8_f32(quot(v[i], by), i, w);
     return w;
+}
+
+// The e4m3 quantiser of the hidden row with the ReLU folded in: the quotients are taken at an eighth, where the range [0, 8]
+// is what the multiplication's own clamp saturates to, and the conversion scales them back.  (A power of two either way;
+// the clamp takes the place of a maximum for every element.)
+__device__ __forceinline__ unsigned quant4_relu_e4m3(float v0, float v1, float v2, float v3, const Quot& by) {
+    const Quot e = {by.hi * 0.125f, by.lo * 0.125f};
+    const float v[4] = {v0, v1, v2, v3};
+    float q[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[i] = __builtin_amdgcn_fmed3f(quot(v[i], e), 0.0f, 1.0f);
+    typedef short v2s __attribute__((ext_vector_type(2)));
+    v2s w = {0, 0};
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(w, q[0], q[1], 0.125f, false);
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(w, q[2], q[3], 0.125f, true);
+    return __builtin_bit_cast(unsigned, w);
 }
 
 // signed quantiser (int8: amax -> 127, e4m3: amax -> 8) of one token row spread over two

@@ -30,6 +30,12 @@
 // [tok: the activation scale of every token of the row that feeds QKV, per position]
 // [key: what masks every token's scores as a key, per position].
 // During the heads the normalised stream of a position (32 KiB, fp32) overlays its hidden row.
+//
+// The e4m3 format widens each weight fragment to fp16 once for every position of the workgroup and keeps the row of the
+// width widened in LDS; epilogues run under the next block's products here too (two pairs of accumulators, for which
+// the weight ring gives up four places): 2143 us (TWIN) -> 1956.  The same vector ALU bounds it: a layer's 4,600 vector
+// instructions per wavefront and 384 + 64 matrix steps are some 57,000 of 68,000 clocks.  Tried: chunks of the hidden row kept
+// widened in LDS (-0.4 %: LDS then delivers as much as it can), two blocks side by side against each operand (-0.3 %).
 #pragma once
 
 #include "bf_board.hip.h"
@@ -95,13 +101,13 @@ template <int MODE, bool FP8, bool PROF = false, int NPOS = 2>
 __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     constexpr bool TAPS = MODE == MODE_TAPS, ENC = MODE == MODE_ENC;
     typedef Cfg<FP8, NPOS> C;
-    static_assert(NPOS == 2 || (NPOS == 1 && !FP8), "one position per workgroup: the int8 format");
+    static_assert(NPOS == 1 || NPOS == 2, "positions per workgroup");
     typedef typename Acc<FP8>::type acc_t;
     constexpr int NP = C::NP, D = C::D, F = C::F, NT = C::NT, TW = C::TW, CW = C::CW, KCF = C::KCF;
     constexpr int STEPS = C::STEPS, BPW = C::BPW, HB = C::HB;
     constexpr int NB = BPW / 2;      // weight blocks a wave consumes per layer
     constexpr int HT = 2;            // hidden tiles a wave computes per feed-forward step
-    constexpr int RING = BF_DUO_RING, AHEAD = BF_DUO_AHEAD;
+    constexpr int RING = FP8 && NP == 2 ? 8 : BF_DUO_RING, AHEAD = BF_DUO_AHEAD;
     constexpr int XS = C::XS, PS = C::NW * 64;   // floats of an exchange slot; of one position's part of it
     static_assert(C::KC == 1 && STEPS == TW && KCF == 2 * STEPS, "the 256-wide network");
     static_assert(8 % (AHEAD + 1) == 0, "an operand's place must not depend on the product");
@@ -507,43 +513,43 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             if ((p) == NP - 1) fetch_frag(8 * (k) + s_ + RING, lbase, lfollow);                      \
         }                                                                                            \
     } while (0)
-        // e4m3: both positions' products with the wave's k-th block, step by step.  A weight fragment is
-        // widened to fp16 once and multiplied with both positions' operands; these come from LDS
-        // already widened (A16: the row of the width) or as bytes (the hidden row).  Each accumulator
-        // sees its sixteen 16-deep steps in order, as in the other kernels.
-#define BF_DUO_PAIR_F8(SWAP, k, A16, B0, B1, R)                                                      \
+        // e4m3: the positions' products with the wave's k-th block, step by step.  A weight fragment is widened to
+        // fp16 once and multiplied with every position's operands; these come from LDS already widened
+        // (A16: the row of the width) or as bytes (the hidden row), position p's STRIDE bytes on.  Each accumulator
+        // sees its sixteen 16-deep steps in order, as in the other kernels.  BETWEEN(s): an eighth of the
+        // previous product's epilogues, as above.
+#define BF_DUO_PRODUCT_F8(SWAP, k, A16, B, STRIDE, R, BETWEEN)                                       \
     do {                                                                                             \
-        const uint8_t* const bp_[2] = {(B0), (B1)};                                                  \
-        (R)[0] = zero;                                                                               \
-        (R)[1] = zero;                                                                               \
-        /* the operands of a step are fetched from LDS one step ahead: [position][half] */           \
-        v4i cur_[2][2], nxt_[2][2];                                                                  \
-        _Pragma("unroll") for (int p_ = 0; p_ < 2; p_++)                                             \
-            _Pragma("unroll") for (int h_ = 0; h_ < ((A16) ? 2 : 1); h_++)                           \
-                cur_[p_][h_] = ldsfrag(bp_[p_] + ((A16) ? h_ : 0) * FRAG);                           \
+        const uint8_t* const b_ = (B);                                                               \
+        constexpr int PER_ = (A16) ? 2 : 1;   /* operand fragments of a step */                      \
+        v4i cur_[NP], nxt_[NP];                                                                      \
+        _Pragma("unroll") for (int p_ = 0; p_ < NP; p_++) {                                          \
+            (R)[p_] = zero;                                                                          \
+            cur_[p_] = ldsfrag(b_ + p_ * (STRIDE));                                                  \
+        }                                                                                            \
         _Pragma("unroll") for (int s_ = 0; s_ < 8; s_++) {                                           \
-            _Pragma("unroll") for (int p_ = 0; p_ < 2; p_++)                                         \
-                _Pragma("unroll") for (int h_ = 0; h_ < ((A16) ? 2 : 1); h_++)                       \
-                    nxt_[p_][h_] = s_ + 1 < 8 ? ldsfrag(bp_[p_] + ((A16) ? 2 * (s_ + 1) + h_ : s_ + 1) * FRAG) : cur_[p_][h_]; \
             const v2l wl_ = __builtin_bit_cast(v2l, frt[(8 * (k) + s_) % RING]);                      \
             _Pragma("unroll") for (int h_ = 0; h_ < 2; h_++) {                                       \
+                const bool new_ = h_ == 1 || (A16);                                                  \
+                const int u_ = PER_ * s_ + (h_ + 1) * PER_ / 2;   /* the fragment after this one */  \
+                if (new_ && u_ < 8 * PER_)                                                           \
+                    _Pragma("unroll") for (int p_ = 0; p_ < NP; p_++) nxt_[p_] = ldsfrag(b_ + p_ * (STRIDE) + u_ * FRAG); \
                 const v8h wh_ = e4m3x8_as_f16(wl_[h_]);                                              \
-                _Pragma("unroll") for (int p_ = 0; p_ < 2; p_++) {                                   \
+                _Pragma("unroll") for (int p_ = 0; p_ < NP; p_++) {                                  \
                     v8h ah_;                                                                         \
-                    if (A16) ah_ = __builtin_bit_cast(v8h, cur_[p_][h_]);                            \
-                    else ah_ = e4m3x8_as_f16(__builtin_bit_cast(v2l, cur_[p_][0])[h_]);              \
+                    if (A16) ah_ = __builtin_bit_cast(v8h, cur_[p_]);                                \
+                    else ah_ = e4m3x8_as_f16(__builtin_bit_cast(v2l, cur_[p_])[h_]);                 \
                     (R)[p_] = f16_step<SWAP>(wh_, ah_, (R)[p_]);                                     \
+                    if (new_) cur_[p_] = nxt_[p_];                                                   \
                 }                                                                                    \
             }                                                                                        \
+            BETWEEN(s_);                                                                             \
             __builtin_amdgcn_sched_barrier(0);                                                       \
-            _Pragma("unroll") for (int p_ = 0; p_ < 2; p_++)                                         \
-                _Pragma("unroll") for (int h_ = 0; h_ < ((A16) ? 2 : 1); h_++) cur_[p_][h_] = nxt_[p_][h_]; \
             fetch_frag(8 * (k) + s_ + RING, lbase, lfollow);                                         \
         }                                                                                            \
     } while (0)
         const acc_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         auto none = [&](int) {};
-        const uint8_t* const act1 = act0 + C::ACT_P;
 
         // ---- LayerNorm 1, quantise, exchange -----------------------------------------------------------
         float sa[NP];
@@ -569,35 +575,35 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             acc_t acc[2];   // product n of a sequence uses accumulator n & 1; the previous one's epilogue runs under it
             v4f bq[4], bk[4], stok[NP][4];
             // the epilogues, two accumulator registers at a time (slice s of eight)
-            auto epi_q = [&](int p, int s, int ai) {
+            auto epi_q = [&](int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    qf[p][e] = accf(acc[ai], e) * sa[p] * swq + bq[e / 4][e % 4];
+                    qf[p][e] = accf(ac, e) * sa[p] * swq + bq[e / 4][e % 4];
                     if (TAPS && a.taps.acc_qkv && live[p])
-                        a.taps.acc_qkv[(bl[p] * T + t) * 3 * D + 32 * tile + ch(e, g)] = tapbits<false>(acc[ai], e);
+                        a.taps.acc_qkv[(bl[p] * T + t) * 3 * D + 32 * tile + ch(e, g)] = tapbits<false>(ac, e);
                 }
             };
-            auto epi_k = [&](int p, int s, int ai) {
+            auto epi_k = [&](int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    kf[p][e] = accf(acc[ai], e) * sa[p] * swk + bk[e / 4][e % 4];
+                    kf[p][e] = accf(ac, e) * sa[p] * swk + bk[e / 4][e % 4];
                     if (TAPS && a.taps.acc_qkv && live[p])
-                        a.taps.acc_qkv[(bl[p] * T + t) * 3 * D + D + 32 * tile + ch(e, g)] = tapbits<false>(acc[ai], e);
+                        a.taps.acc_qkv[(bl[p] * T + t) * 3 * D + D + 32 * tile + ch(e, g)] = tapbits<false>(ac, e);
                 }
             };
             // V tile: rows are tokens, so the activation scale is that of token ch(e, g)
-            auto epi_v = [&](int p, int s, int ai) {
+            auto epi_v = [&](int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    vf[p][e] = accf(acc[ai], e) * stok[p][e / 4][e % 4] * swv + bv;
+                    vf[p][e] = accf(ac, e) * stok[p][e / 4][e % 4] * swv + bv;
                     if (TAPS && a.taps.acc_qkv && live[p])
-                        a.taps.acc_qkv[(bl[p] * T + ch(e, g)) * 3 * D + 2 * D + 32 * tile + t] = tapbits<false>(acc[ai], e);
+                        a.taps.acc_qkv[(bl[p] * T + ch(e, g)) * 3 * D + 2 * D + 32 * tile + t] = tapbits<false>(ac, e);
                 }
             };
-            auto epi_qkv = [&](int tq, int p, int s, int ai) {
-                if (tq == 0) epi_q(p, s, ai);
-                else if (tq == 1) epi_k(p, s, ai);
-                else epi_v(p, s, ai);
+            auto epi_qkv = [&](int tq, int p, int s, const acc_t& ac) {
+                if (tq == 0) epi_q(p, s, ac);
+                else if (tq == 1) epi_k(p, s, ac);
+                else epi_v(p, s, ac);
             };
             // A SIMD favours its older wavefront, which then waits at the next exchange for a partner that has the SIMD to
             // itself: the younger one goes first here, the older one in the attention behind (4096 positions -1.3 to
@@ -605,20 +611,27 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             if (sub) __builtin_amdgcn_s_setprio(2);
             load_tile16(here_f(pA + C::A_BQ + 32 * sub), g, bq);
             if constexpr (FP8) {
-                // e4m3: a block's two products share the widening of its weight fragments, the
-                // epilogues of both positions follow
-                BF_DUO_PAIR_F8(false, 0, true, act0, act1, acc);
-#pragma unroll
-                for (int s = 0; s < 8; s++) { epi_q(0, s, 0); epi_q(1, s, 1); }
+                // e4m3: a block's two products share the widening of its weight fragments; the epilogues of both
+                // positions run under the next block's
+                acc_t pair[2][NP];
+                BF_DUO_PRODUCT_F8(false, 0, true, act0, C::ACT_P, pair[0], none);
                 load_tile16(here_f(pA + C::A_BK + 32 * sub), g, bk);
-                BF_DUO_PAIR_F8(false, 1, true, act0, act1, acc);
+                auto with_q = [&](int s) {
 #pragma unroll
-                for (int s = 0; s < 8; s++) { epi_k(0, s, 0); epi_k(1, s, 1); }
-                load_tile16(here_f(tok), g, stok[0]);
-                load_tile16(here_f(tok + 32), g, stok[1]);
-                BF_DUO_PAIR_F8(true, 2, true, act0, act1, acc);
+                    for (int p = 0; p < NP; p++) epi_q(p, s, pair[0][p]);
+                };
+                BF_DUO_PRODUCT_F8(false, 1, true, act0, C::ACT_P, pair[1], with_q);
 #pragma unroll
-                for (int s = 0; s < 8; s++) { epi_v(0, s, 0); epi_v(1, s, 1); }
+                for (int p = 0; p < NP; p++) load_tile16(here_f(tok + 32 * p), g, stok[p]);
+                auto with_k = [&](int s) {
+#pragma unroll
+                    for (int p = 0; p < NP; p++) epi_k(p, s, pair[1][p]);
+                };
+                BF_DUO_PRODUCT_F8(true, 2, true, act0, C::ACT_P, pair[0], with_k);
+#pragma unroll
+                for (int s = 0; s < 8; s++)
+#pragma unroll
+                    for (int p = 0; p < NP; p++) epi_v(p, s, pair[0][p]);
             } else {
                 // Q, K, V blocks in turn, each for every position: 3 NP products
                 BF_DUO_OPERANDS(act0);
@@ -628,14 +641,14 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                     if (n == NP) load_tile16(here_f(pA + C::A_BK + 32 * sub), g, bk);
                     if (tq == 2) load_tile16(here_f(tok + 32 * p), g, stok[p]);
                     auto between = [&](int s) {
-                        if (n > 0) epi_qkv((n - 1) / NP, (n - 1) % NP, s, (n - 1) & 1);
+                        if (n > 0) epi_qkv((n - 1) / NP, (n - 1) % NP, s, acc[(n - 1) & 1]);
                     };
                     const uint8_t* const next = act0 + (n + 1) % NP * C::ACT_P;
                     if (tq == 2) BF_DUO_CHAIN(true, 2, p, act0 + p * C::ACT_P, n + 1 < 3 * NP, next, zero, acc[n & 1], between);
                     else BF_DUO_CHAIN(false, tq, p, act0 + p * C::ACT_P, n + 1 < 3 * NP, next, zero, acc[n & 1], between);
                 }
 #pragma unroll
-                for (int s = 0; s < 8; s++) epi_v(NP - 1, s, (3 * NP - 1) & 1);
+                for (int s = 0; s < 8; s++) epi_v(NP - 1, s, acc[(3 * NP - 1) & 1]);
             }
             __builtin_amdgcn_s_setprio(0);
             BF_PHASE(PH_QKV);
@@ -690,30 +703,31 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             v4f bo[4];
             load_tile16(here_f(pA + C::A_BOUT + 32 * sub), g, bo);
             const float sw = *here_f(pA + C::A_SW + 3 * TW + sub);
-            auto epi_o = [&](int p, int s, int ai) {
+            auto epi_o = [&](int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    x[p][e] = x[p][e] + (accf(acc[ai], e) * so[p] * sw + bo[e / 4][e % 4]);
+                    x[p][e] = x[p][e] + (accf(ac, e) * so[p] * sw + bo[e / 4][e % 4]);
                     if (TAPS && a.taps.acc_out && live[p])
-                        a.taps.acc_out[(bl[p] * T + t) * D + 32 * tile + ch(e, g)] = tapbits<false>(acc[ai], e);
+                        a.taps.acc_out[(bl[p] * T + t) * D + 32 * tile + ch(e, g)] = tapbits<false>(ac, e);
                 }
             };
             if constexpr (FP8) {
-                BF_DUO_PAIR_F8(false, 3, true, act0, act1, acc);
+                BF_DUO_PRODUCT_F8(false, 3, true, act0, C::ACT_P, acc, none);
+                if (NP > 1)
 #pragma unroll
-                for (int s = 0; s < 8; s++) epi_o(0, s, 0);
+                    for (int s = 0; s < 8; s++) epi_o(0, s, acc[0]);
             } else {
                 BF_DUO_OPERANDS(act0);
 #pragma unroll
                 for (int p = 0; p < NP; p++) {
                     auto between = [&](int s) {
-                        if (p > 0) epi_o(p - 1, s, (p - 1) & 1);
+                        if (p > 0) epi_o(p - 1, s, acc[(p - 1) & 1]);
                     };
                     BF_DUO_CHAIN(false, 3, p, act0 + p * C::ACT_P, p + 1 < NP, act0 + C::ACT_P, zero, acc[p & 1], between);
                 }
             }
 #pragma unroll
-            for (int s = 0; s < 8; s++) epi_o(NP - 1, s, (NP - 1) & 1);
+            for (int s = 0; s < 8; s++) epi_o(NP - 1, s, acc[(NP - 1) & 1]);
         }
         BF_PHASE(PH_OUT);
 
@@ -740,20 +754,19 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             float am[NP];
 #pragma unroll
             for (int p = 0; p < NP; p++) am[p] = 0.0f;
-            acc_t acc[2];
+            acc_t acc[2], pair[2][NP];   // e4m3: a block's products at a time
             v4f b1[HT][4];
             float sw1[HT];
-            auto epi_f = [&](int i, int p, int s, int ai) {
+            auto epi_f = [&](int i, int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    // int8: the ReLU is the saturation of the unsigned quantiser below, and the
-                    // running maximum starts at 0, so negative values need no clamp here
-                    float v = accf(acc[ai], e) * sa[p] * sw1[i] + b1[i][e / 4][e % 4];
-                    if constexpr (FP8) v = __builtin_fmaxf(v, 0.0f);
+                    // the ReLU is in the hidden quantiser's saturation, and the running maximum starts at 0,
+                    // so negative values need no clamp here
+                    const float v = accf(ac, e) * sa[p] * sw1[i] + b1[i][e / 4][e % 4];
                     hf[p][i][e] = v;
                     am[p] = __builtin_fmaxf(am[p], v);
                     if (TAPS && a.taps.acc_ff1 && live[p])
-                        a.taps.acc_ff1[(bl[p] * T + t) * F + 512 * st + 128 * q + 32 * (HT * sub + i) + ch(e, g)] = tapbits<false>(acc[ai], e);
+                        a.taps.acc_ff1[(bl[p] * T + t) * F + 512 * st + 128 * q + 32 * (HT * sub + i) + ch(e, g)] = tapbits<false>(ac, e);
                 }
             };
 #pragma unroll
@@ -761,24 +774,32 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                 load_tile16(here_f(pB + C::B_BFF1 + 128 * st + 32 * (HT * sub + i)), g, b1[i]);
                 sw1[i] = *here_f(pB + C::B_SW + 4 * st + HT * sub + i);
                 if constexpr (FP8) {
-                    BF_DUO_PAIR_F8(false, 4 + HT * st + i, true, act0, act1, acc);
+                    auto with_f = [&](int s) {
+                        if (i > 0)
 #pragma unroll
-                    for (int s = 0; s < 8; s++) { epi_f(i, 0, s, 0); epi_f(i, 1, s, 1); }
+                            for (int p = 0; p < NP; p++) epi_f(i - 1, p, s, pair[(i - 1) & 1][p]);
+                    };
+                    BF_DUO_PRODUCT_F8(false, 4 + HT * st + i, true, act0, C::ACT_P, pair[i & 1], with_f);
                 } else {
 #pragma unroll
                     for (int p = 0; p < NP; p++) {
                         const int n = NP * i + p;   // product number within the step; the previous one's epilogue runs under it
                         auto between = [&](int s) {
-                            if (n > 0) epi_f((n - 1) / NP, (n - 1) % NP, s, (n - 1) & 1);
+                            if (n > 0) epi_f((n - 1) / NP, (n - 1) % NP, s, acc[(n - 1) & 1]);
                         };
                         BF_DUO_CHAIN(false, 4 + HT * st + i, p, act0 + p * C::ACT_P, n + 1 < NP * HT, act0 + (p + 1) % NP * C::ACT_P, zero, acc[n & 1],
                                      between);
                     }
                 }
             }
-            if constexpr (!FP8)
+            if constexpr (FP8)
 #pragma unroll
-                for (int s = 0; s < 8; s++) epi_f(HT - 1, NP - 1, s, (NP * HT - 1) & 1);
+                for (int s = 0; s < 8; s++)
+#pragma unroll
+                    for (int p = 0; p < NP; p++) epi_f(HT - 1, p, s, pair[(HT - 1) & 1][p]);
+            else
+#pragma unroll
+                for (int s = 0; s < 8; s++) epi_f(HT - 1, NP - 1, s, acc[(NP * HT - 1) & 1]);
             // the maxima of consecutive steps go through different exchange slots
             const int xs = (st & 1) ? 0 : 2 * XS;
             xmax_put(am, xs);
@@ -809,7 +830,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         unsigned u;
-                        if constexpr (FP8) u = quant4<true>(hf[p][i][4 * j], hf[p][i][4 * j + 1], hf[p][i][4 * j + 2], hf[p][i][4 * j + 3], by);
+                        if constexpr (FP8) u = quant4_relu_e4m3(hf[p][i][4 * j], hf[p][i][4 * j + 1], hf[p][i][4 * j + 2], hf[p][i][4 * j + 3], by);
                         else u = quant4_relu_u8(hf[p][i][4 * j], hf[p][i][4 * j + 1], hf[p][i][4 * j + 2], hf[p][i][4 * j + 3], by);
                         if (TAPS && a.taps.qa_ff2 && live[p])
                             *reinterpret_cast<unsigned*>(a.taps.qa_ff2 + (bl[p] * T + t) * F + 512 * st + 128 * q + 32 * (HT * sub + i) + 8 * j + 4 * g) = u;
@@ -827,34 +848,37 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         {
             double o64[NP][16];
             float o32[NP][16];
-            acc_t acc[2];
+            acc_t acc[2], pair[2][NP];
             acc_t init = zero;
             BF_DUO_OPERANDS(hid0);
             float sw2[KCF];   // e4m3: one weight scale per k-chunk
             if constexpr (FP8)
 #pragma unroll
                 for (int cc = 0; cc < KCF; cc++) sw2[cc] = here_f(pB + C::B_SW + 16 + sub * KCF)[cc];
-            auto epi_2 = [&](int cc, int p, int s, int ai) {
+            auto epi_2 = [&](int cc, int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
                     if constexpr (FP8) {
-                        const float part = (accf(acc[ai], e) * sh[p][cc]) * sw2[cc];
+                        const float part = (accf(ac, e) * sh[p][cc]) * sw2[cc];
                         o32[p][e] = cc == 0 ? part : o32[p][e] + part;
                     } else {
                         const double sc = (double)sh[p][cc];
-                        const int full = accbits(acc[ai], e);
+                        const int full = accbits(ac, e);
                         o64[p][e] = cc == 0 ? (double)full * sc : __builtin_fma((double)full, sc, o64[p][e]);
                     }
                     if (TAPS && a.taps.acc_ff2 && live[p])
-                        a.taps.acc_ff2[((bl[p] * KCF + cc) * T + t) * D + 32 * tile + ch(e, g)] = accbits(acc[ai], e);
+                        a.taps.acc_ff2[((bl[p] * KCF + cc) * T + t) * D + 32 * tile + ch(e, g)] = accbits(ac, e);
                 }
             };
 #pragma unroll
             for (int cc = 0; cc < KCF; cc++) {
                 if constexpr (FP8) {
-                    BF_DUO_PAIR_F8(false, 4 + HT * STEPS + cc, false, hid0 + 8 * cc * FRAG, hid0 + C::HID_P + 8 * cc * FRAG, acc);
+                    auto with_2 = [&](int s) {
+                        if (cc > 0)
 #pragma unroll
-                    for (int s = 0; s < 8; s++) { epi_2(cc, 0, s, 0); epi_2(cc, 1, s, 1); }
+                            for (int p = 0; p < NP; p++) epi_2(cc - 1, p, s, pair[(cc - 1) & 1][p]);
+                    };
+                    BF_DUO_PRODUCT_F8(false, 4 + HT * STEPS + cc, false, hid0 + 8 * cc * FRAG, C::HID_P, pair[cc & 1], with_2);
                 } else {
 #pragma unroll
                     for (int p = 0; p < NP; p++) {
@@ -868,16 +892,21 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                                 for (int k = 0; k < 4; k++) init[4 * j + k] = w0[j][k];
                         }
                         auto between = [&](int s) {
-                            if (n > 0) epi_2((n - 1) / NP, (n - 1) % NP, s, (n - 1) & 1);
+                            if (n > 0) epi_2((n - 1) / NP, (n - 1) % NP, s, acc[(n - 1) & 1]);
                         };
                         BF_DUO_CHAIN(false, 4 + HT * STEPS + cc, p, hid0 + p * C::HID_P + 8 * cc * FRAG,
                                      cn < KCF, hid0 + pn * C::HID_P + 8 * cn * FRAG, init, acc[n & 1], between);
                     }
                 }
             }
-            if constexpr (!FP8)
+            if constexpr (FP8)
 #pragma unroll
-                for (int s = 0; s < 8; s++) epi_2(KCF - 1, NP - 1, s, (NP * KCF - 1) & 1);
+                for (int s = 0; s < 8; s++)
+#pragma unroll
+                    for (int p = 0; p < NP; p++) epi_2(KCF - 1, p, s, pair[(KCF - 1) & 1][p]);
+            else
+#pragma unroll
+                for (int s = 0; s < 8; s++) epi_2(KCF - 1, NP - 1, s, acc[(NP * KCF - 1) & 1]);
             v4f b2[4];
             load_tile16(here_f(pB + C::B_BFF2 + 32 * sub), g, b2);
             const float sw = *here_f(pB + C::B_SW + 16 + sub);
@@ -899,7 +928,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         warm_done();
 #undef BF_DUO_OPERANDS
 #undef BF_DUO_CHAIN
-#undef BF_DUO_PAIR_F8
+#undef BF_DUO_PRODUCT_F8
         if (TAPS && a.taps.resid)
 #pragma unroll
             for (int p = 0; p < NP; p++)

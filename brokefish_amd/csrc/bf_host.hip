@@ -139,9 +139,9 @@ static int choose_kernel(const bf_eval_args* a) {
             return fail(BF_ERR_UNSUPPORTED, "the two-positions-per-workgroup kernel needs the 256-wide network and board_wstream/board_fparams");
         return BF_KERNEL_DUO;
     case BF_KERNEL_AUTO:
-        // above one position per compute unit: two positions per workgroup for int8 (2-4 % faster
-        // than TWIN from 512 positions up and half its L2 traffic), TWIN for e4m3 (whose operand
-        // conversions leave the two-position form short of registers)
+        // above one position per compute unit: two positions per workgroup (int8: 5 to 8 % faster than TWIN from 512
+        // positions up and half its L2 traffic).  For e4m3 the answer is still TWIN, what AUTO ran before the two-position
+        // kernel overtook it; check_args() gives those launches to DUO (same bits; 4096 positions 2142 -> 1985 us).
         if (octo_can) return (twin_can && a->n > kBoardMaxN) ? (a->quant == BF_QUANT_INT8 ? BF_KERNEL_DUO : BF_KERNEL_TWIN) : BF_KERNEL_OCTO;
         if (quad_can) return BF_KERNEL_QUAD;
         return fail(BF_ERR_ARGUMENT, shape512(&a->shape)
@@ -162,12 +162,14 @@ static bool enc_build(const bf_eval_args* a, int kind) {
         t->acc_ff2 || t->resid || t->normed)
         return false;
     if (a->shape.d_model == 512) return kind == BF_KERNEL_OCTO;
-    return a->quant == BF_QUANT_INT8 ? kind == BF_KERNEL_OCTO || kind == BF_KERNEL_DUO : kind == BF_KERNEL_OCTO || kind == BF_KERNEL_TWIN;
+    // TWIN in e4m3: the two-position build serves it (same bits)
+    return kind == BF_KERNEL_OCTO || kind == BF_KERNEL_DUO || (kind == BF_KERNEL_TWIN && a->quant == BF_QUANT_E4M3);
 }
 
 static int check_args(const bf_eval_args* a, bf::KArgs* k, int* kind) {
     *kind = choose_kernel(a);
     if (*kind < 0) return *kind;
+    if (a->kernel == BF_KERNEL_AUTO && *kind == BF_KERNEL_TWIN) *kind = BF_KERNEL_DUO;
     const bool board = *kind == BF_KERNEL_BOARD || *kind == BF_KERNEL_TWIN || *kind == BF_KERNEL_OCTO || *kind == BF_KERNEL_DUO;
     if (a->n < 1 || a->n > (1ll << 28)) return fail(BF_ERR_ARGUMENT, "n must be in [1, 2^28]");
     // encoder-only launch: residual stream in and out through the tap table, no board words, no heads
@@ -327,11 +329,12 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
         }
     }
     // When the library chose the two-position kernel itself, a last round of at most 256 positions goes to the
-    // one-position form in a second launch on the same stream (640 positions: 0.33 ms instead of 0.39).  With
+    // one-position form in a second launch on the same stream (640 positions: 0.33 ms instead of 0.39, e4m3 0.39 instead of
+    // 0.48).  With
     // a leaf list the count is on the device: both forms are launched and each takes its share of the list
     // (a launch that finds nothing to do costs 3 us; 200 live leaves of 1000 take a third less).  Not
     // with other taps or the profile.
-    if (kind == BF_KERNEL_DUO && a->kernel == BF_KERNEL_AUTO && a->quant == BF_QUANT_INT8 && (!a->taps || enc) && !k.profile) {
+    if (kind == BF_KERNEL_DUO && a->kernel == BF_KERNEL_AUTO && (!a->taps || enc) && !k.profile) {
         const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n);
         if (rest) {
             bf::KArgs front = k, back = k;
@@ -342,9 +345,11 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
                 front = slice(k, bf::D, 0, k.n - rest);
                 back = slice(k, bf::D, k.n - rest, rest);
             }
-            e = (enc ? bf::launch_duo256_enc : bf::launch_duo256)(front, stream);
+            const bool f8 = a->quant == BF_QUANT_E4M3;
+            e = (f8 ? (enc ? bf::launch_duo256_fp8_enc : bf::launch_duo256_fp8) : enc ? bf::launch_duo256_enc : bf::launch_duo256)(front, stream);
             if (e == hipSuccess)
-                e = !k.leaf_index && rest <= team ? launch_team(a, back, enc, stream) : (enc ? bf::launch_solo256_enc : bf::launch_solo256)(back, stream);
+                e = !k.leaf_index && rest <= team ? launch_team(a, back, enc, stream)
+                    : (f8 ? (enc ? bf::launch_solo256_fp8_enc : bf::launch_solo256_fp8) : enc ? bf::launch_solo256_enc : bf::launch_solo256)(back, stream);
             if (e != hipSuccess) {
                 snprintf(g_err, sizeof(g_err), "kernel launch failed: %s", hipGetErrorString(e));
                 return BF_ERR_LAUNCH;
@@ -354,20 +359,20 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
     }
     if (enc) {
         if (a->shape.d_model == 512) e = bf::launch_octo512_enc(k, stream);
-        else if (a->quant == BF_QUANT_E4M3) e = (kind == BF_KERNEL_OCTO ? bf::launch_octo256_fp8_enc : bf::launch_twin256_fp8_enc)(k, stream);
+        else if (a->quant == BF_QUANT_E4M3) e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_fp8_enc : bf::launch_duo256_fp8_enc)(k, stream);
         else e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_enc : bf::launch_duo256_enc)(k, stream);
     } else if (kind == BF_KERNEL_OCTO) {
-        // eight wavefronts per position: the 512-wide network and the e4m3 format on the board kernel's
-        // eight-wavefront form; the 256-wide int8 network on the two-position kernel's one-position
-        // form, which issues each product under the previous one's epilogue
+        // eight wavefronts per position: the 512-wide network on the board kernel's eight-wavefront form; the
+        // 256-wide one on the two-position kernel's one-position form, which issues each product under the
+        // previous one's epilogue
         if (k.profile && a->shape.d_model == 512)
             e = bf::launch_octo512_prof(k, stream);
         else if (a->shape.d_model == 512)
             e = a->taps ? bf::launch_octo512_taps(k, stream) : bf::launch_octo512(k, stream);
         else if (a->quant == BF_QUANT_E4M3)
-            e = k.profile ? bf::launch_octo256_fp8_prof(k, stream)
-              : a->taps   ? bf::launch_octo256_fp8_taps(k, stream)
-                          : bf::launch_octo256_fp8(k, stream);
+            e = k.profile ? bf::launch_solo256_fp8_prof(k, stream)
+              : a->taps   ? bf::launch_solo256_fp8_taps(k, stream)
+                          : bf::launch_solo256_fp8(k, stream);
         else if (k.profile)
             e = bf::launch_solo256_prof(k, stream);
         else

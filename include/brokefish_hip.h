@@ -48,19 +48,19 @@ enum bf_quant {
  *          per compute unit: low latency per position (launches that cannot fill the GPU);
  *          both network widths.
  *   TWIN   the BOARD decomposition shaped so that two workgroups share a compute unit (each SIMD
- *          holds two wavefronts that cover each other's waits): the highest throughput
- *          (256-wide network).
+ *          holds two wavefronts that cover each other's waits; 256-wide network).
  *   OCTO   eight wavefronts per position, one workgroup per compute unit: the lowest latency per
- *          position for the 256-wide network (int8: the DUO kernel with one position per
- *          workgroup; e4m3: the BOARD decomposition with two wavefronts per quarter of the
- *          width), and the faster kernel for the 512-wide one (BOARD decomposition likewise).
+ *          position for the 256-wide network (the DUO kernel with one position per workgroup), and
+ *          the faster kernel for the 512-wide one (the BOARD decomposition with two wavefronts per
+ *          quarter of the width).
  *   DUO    two positions per workgroup of eight wavefronts (the OCTO decomposition, every
  *          wavefront doing its share for both positions), so that a weight fragment fetched from
  *          L2 serves two positions (256-wide network, int8 and e4m3).
  * BOARD, TWIN, OCTO and DUO read the same blobs (board_wstream / board_fparams).  The 256-wide network
  * runs in int8 and e4m3 on all four; the 512-wide network in int8 on OCTO and BOARD.  Kernels that
  * carry a network and a format return bit-identical results for it, so AUTO may pick by batch
- * size: OCTO up to 256 positions, above that DUO (int8) or TWIN (e4m3).  DUO runs in rounds of 512
+ * size: OCTO up to 256 positions, above that DUO (for e4m3 bf_kernel_choice still answers TWIN, which
+ * DUO has overtaken there).  DUO runs in rounds of 512
  * positions; when AUTO has chosen it and the last round would hold at most 256 positions, those
  * are given to the one-position form in a second launch on the same stream (bf_kernel_choice
  * still answers DUO). */
@@ -229,7 +229,7 @@ typedef struct {
     const uint8_t* active;
     int32_t kernel;         /* enum bf_kernel; AUTO with the board blobs: OCTO for
                              * n <= bf_board_max_n() and for the 512-wide network, above that
-                             * DUO (int8) or TWIN (e4m3); without the board blobs QUAD */
+                             * DUO; without the board blobs QUAD */
     /* which tokens the value rows read (reference brokefish/nn/model.py:551-617): the king of the
      * side to move (BF_VALUE_KING, the default), the mean of the final-normed live tokens
      * (BF_VALUE_POOLED), or the final norm of the mean of the live tokens' residual stream
@@ -276,7 +276,8 @@ uint64_t bf_abi_tag(void);
 /* Largest n for which AUTO prefers OCTO over DUO / TWIN on the 256-wide network. */
 int64_t bf_board_max_n(void);
 /* The kernel AUTO would run for these arguments (enum bf_kernel), or a negative bf_status.  The form that spreads a
- * position over several compute units (team_workspace) counts as OCTO, whose launches it takes. */
+ * position over several compute units (team_workspace) counts as OCTO, whose launches it takes; DUO's e4m3 launches
+ * count as TWIN, whose they were. */
 int bf_kernel_choice(const bf_eval_args* args);
 
 /* The evaluator.  Replaces model_forward of the reference extension
