@@ -167,8 +167,8 @@ def main() -> int:
     traffic = (MEASURED_TRAFFIC_BYTES_E4M3 if fp8 else MEASURED_TRAFFIC_BYTES).get((a.shape, kname, a.batch))
     # each workgroup streams its own copy of the weights from L2
     # (four positions share one copy in the quad kernel, two in the duo kernel)
-    weight_bytes = (6_389_760 * ((a.batch + 3) // 4) if kname == "quad" else 6_455_296 * ((a.batch + 1) // 2) if kname == "duo"
-                    else (50_626_560 if stress else 6_455_296) * a.batch)
+    weight_bytes = (6_389_760 * ((a.batch + 3) // 4) if kname == "quad"
+                    else (50_626_560 if stress else 6_455_296) * ((a.batch + 1) // 2 if kname == "duo" else a.batch))
     line = {
         "metric": (f"network evals/sec at batch {a.batch} int8, 16-layer width-512 stress shape, on 1 MI355X" if stress
                    else f"network evals/sec at batch 4096 {'fp8 e4m3' if fp8 else 'int8'} on 1 MI355X"),

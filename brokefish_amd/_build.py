@@ -26,6 +26,7 @@ TORCH_EXT = os.path.join(HERE, "_bf_torch.so")
 HIP_SOURCES = ["bf_variant_prod_fp8.hip", "bf_variant_taps_fp8.hip", "bf_variant_prof_fp8.hip",
                "bf_variant_prod.hip", "bf_variant_taps.hip", "bf_variant_prof.hip",
                "bf_variant_board512.hip", "bf_variant_board512_taps.hip", "bf_variant_board512_prof.hip",
+               "bf_variant_wide512.hip", "bf_variant_wide512_enc.hip", "bf_variant_wide512_prof.hip",
                "bf_host.hip", "bf_expand.hip", "bf_movegen.hip", "bf_probe.hip", "bf_pack.hip",
                "bf_variant_board256.hip", "bf_variant_board256_taps.hip", "bf_variant_board256_prof.hip",
                "bf_variant_twin256.hip", "bf_variant_twin256_taps.hip", "bf_variant_twin256_prof.hip",

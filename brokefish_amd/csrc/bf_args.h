@@ -172,6 +172,10 @@ hipError_t launch_duo256(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_taps(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_fp8(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_fp8_taps(const KArgs& k, hipStream_t stream);
+// the same for the 512-wide network
+hipError_t launch_wide512(const KArgs& k, hipStream_t stream);
+hipError_t launch_wide512_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_wide512_prof(const KArgs& k, hipStream_t stream);
 // the encoder-only builds of the kernels AUTO chooses from
 hipError_t launch_duo256_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_enc(const KArgs& k, hipStream_t stream);

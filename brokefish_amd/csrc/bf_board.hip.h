@@ -281,7 +281,9 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
     // before any barrier
     int b = blockIdx.x;
     if (a.leaf_index) {
-        if (b >= *a.leaf_count) return;
+        const int cnt = *a.leaf_count < a.n ? *a.leaf_count : a.n;   // the list has n entries whatever the count says
+        if (OCTO && a.list_split) b += cnt - round_rest(cnt);
+        if (b >= cnt) return;
         b = __builtin_amdgcn_readfirstlane(a.leaf_index[b]);
         if ((unsigned)b >= (unsigned)a.n) return;   // not a position of this launch
     }
@@ -1360,7 +1362,7 @@ hipError_t launch_board(const KArgs& k, hipStream_t stream) {
         if (e != hipSuccess) return e;
         lds_set.fetch_or(bit, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((board_kernel<DM, MODE, TWIN, FP8, OCTO, PROF>), dim3(k.n), dim3(OCTO ? 2 * THREADS : THREADS), lds_bytes, stream, k);
+    hipLaunchKernelGGL((board_kernel<DM, MODE, TWIN, FP8, OCTO, PROF>), dim3(k.grid ? k.grid : k.n), dim3(OCTO ? 2 * THREADS : THREADS), lds_bytes, stream, k);
     return hipGetLastError();
 }
 

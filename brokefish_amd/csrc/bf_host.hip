@@ -311,63 +311,55 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
                                  "are NaN (see team_workspace of bf_eval_args); nothing was launched now");
     const bool enc = !k.profile && enc_build(a, kind);
     // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
-    // position 120 -> 82 us, e4m3 155 -> 96; 512 wide 738 -> 272 us), and so does what is left of the 512-wide
-    // network's rounds of 256 positions (738 us each) where two team launches (328 us each) hold it.
+    // position 120 -> 82 us, e4m3 155 -> 96; 512 wide 738 -> 272 us), and 512 wide so does one that two team launches hold
+    // (328 us each; the one-position form takes 738 for up to 256).
+    const bool wide = a->shape.d_model == 512;
     const int team = team_limit(a, k, enc);
-    if (kind == BF_KERNEL_OCTO && team > 0) {
-        const int left = k.n <= team ? k.n : a->shape.d_model == 512 && !k.leaf_index ? k.n % (int)kBoardMaxN : 0;   // a list's length is on the device
-        if (left && left <= (a->shape.d_model == 512 ? 2 : 1) * team) {
-            e = hipSuccess;
-            if (left < k.n) e = (enc ? bf::launch_octo512_enc : bf::launch_octo512)(slice(k, a->shape.d_model, 0, k.n - left), stream);
-            for (int at = k.n - left; at < k.n && e == hipSuccess; at += team)
-                e = launch_team(a, left <= team && left == k.n ? k : slice(k, a->shape.d_model, at, k.n - at < team ? k.n - at : team), enc, stream);
-            if (e != hipSuccess) {
-                snprintf(g_err, sizeof(g_err), "kernel launch failed: %s", hipGetErrorString(e));
-                return BF_ERR_LAUNCH;
-            }
-            return BF_OK;
-        }
-    }
-    // When the library chose the two-position kernel itself, a last round of at most 256 positions goes to the
-    // one-position form in a second launch on the same stream (640 positions: 0.33 ms instead of 0.39, e4m3 0.39 instead of
-    // 0.48).  With
-    // a leaf list the count is on the device: both forms are launched and each takes its share of the list
-    // (a launch that finds nothing to do costs 3 us; 200 live leaves of 1000 take a third less).  Not
-    // with other taps or the profile.
-    if (kind == BF_KERNEL_DUO && a->kernel == BF_KERNEL_AUTO && (!a->taps || enc) && !k.profile) {
+    auto launch_teams = [&](const bf::KArgs& s) {
+        hipError_t r = hipSuccess;
+        for (int at = 0; at < s.n && r == hipSuccess; at += team)
+            r = launch_team(a, s.n <= team ? s : slice(s, a->shape.d_model, at, s.n - at < team ? s.n - at : team), enc, stream);
+        return r;
+    };
+    const auto by_teams = [&](const bf::KArgs& s) { return team > 0 && !(s.leaf_index && s.n > team) && s.n <= (wide ? 2 : 1) * team; };
+    const bool by_rounds = a->kernel == BF_KERNEL_AUTO && (!a->taps || enc) && !k.profile && k.n > (int)kBoardMaxN && (wide || kind == BF_KERNEL_DUO);
+    if (kind == BF_KERNEL_OCTO && !by_rounds && by_teams(k)) {
+        e = launch_teams(k);
+    } else if (by_rounds) {
+        // Two positions per workgroup, in rounds of 512 positions that cost the same full or not: a last round of at most 256
+        // goes to the one-position form in a second launch on the same stream (640 positions: 0.33 ms instead of 0.39, e4m3
+        // 0.39 instead of 0.48).  With a leaf list the count is on the device: both forms are launched and each
+        // takes its share of the list (a launch that finds nothing to do costs 3 us; 200 live leaves of 1000 take a third
+        // less).  Not with other taps or the profile.
         const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n);
-        if (rest) {
-            bf::KArgs front = k, back = k;
-            if (k.leaf_index) {
-                front.list_split = back.list_split = 1;
-                back.grid = rest;
-            } else {
-                front = slice(k, bf::D, 0, k.n - rest);
-                back = slice(k, bf::D, k.n - rest, rest);
-            }
-            const bool f8 = a->quant == BF_QUANT_E4M3;
-            e = (f8 ? (enc ? bf::launch_duo256_fp8_enc : bf::launch_duo256_fp8) : enc ? bf::launch_duo256_enc : bf::launch_duo256)(front, stream);
-            if (e == hipSuccess)
-                e = !k.leaf_index && rest <= team ? launch_team(a, back, enc, stream)
-                    : (f8 ? (enc ? bf::launch_solo256_fp8_enc : bf::launch_solo256_fp8) : enc ? bf::launch_solo256_enc : bf::launch_solo256)(back, stream);
-            if (e != hipSuccess) {
-                snprintf(g_err, sizeof(g_err), "kernel launch failed: %s", hipGetErrorString(e));
-                return BF_ERR_LAUNCH;
-            }
-            return BF_OK;
+        bf::KArgs front = k, back = k;
+        if (k.leaf_index) {
+            front.list_split = back.list_split = 1;
+            back.grid = rest;
+        } else if (rest) {
+            front = slice(k, a->shape.d_model, 0, k.n - rest);
+            back = slice(k, a->shape.d_model, k.n - rest, rest);
         }
-    }
-    if (enc) {
-        if (a->shape.d_model == 512) e = bf::launch_octo512_enc(k, stream);
+        const bool f8 = a->quant == BF_QUANT_E4M3;
+        e = (wide ? (enc ? bf::launch_wide512_enc : bf::launch_wide512)
+             : f8 ? (enc ? bf::launch_duo256_fp8_enc : bf::launch_duo256_fp8)
+                  : (enc ? bf::launch_duo256_enc : bf::launch_duo256))(front, stream);
+        if (rest && e == hipSuccess)
+            e = !k.leaf_index && by_teams(back) ? launch_teams(back)
+                : (wide ? (enc ? bf::launch_octo512_enc : bf::launch_octo512)
+                   : f8 ? (enc ? bf::launch_solo256_fp8_enc : bf::launch_solo256_fp8)
+                        : (enc ? bf::launch_solo256_enc : bf::launch_solo256))(back, stream);
+    } else if (enc) {
+        if (wide) e = bf::launch_octo512_enc(k, stream);
         else if (a->quant == BF_QUANT_E4M3) e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_fp8_enc : bf::launch_duo256_fp8_enc)(k, stream);
         else e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_enc : bf::launch_duo256_enc)(k, stream);
     } else if (kind == BF_KERNEL_OCTO) {
         // eight wavefronts per position: the 512-wide network on the board kernel's eight-wavefront form; the
         // 256-wide one on the two-position kernel's one-position form, which issues each product under the
         // previous one's epilogue
-        if (k.profile && a->shape.d_model == 512)
-            e = bf::launch_octo512_prof(k, stream);
-        else if (a->shape.d_model == 512)
+        if (k.profile && wide)
+            e = (a->kernel == BF_KERNEL_AUTO && k.n > (int)kBoardMaxN ? bf::launch_wide512_prof : bf::launch_octo512_prof)(k, stream);
+        else if (wide)
             e = a->taps ? bf::launch_octo512_taps(k, stream) : bf::launch_octo512(k, stream);
         else if (a->quant == BF_QUANT_E4M3)
             e = k.profile ? bf::launch_solo256_fp8_prof(k, stream)

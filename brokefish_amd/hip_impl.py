@@ -810,8 +810,8 @@ class FusedEncoder:
             self.board_wstream, self.board_fparams = pack_board_on_device(net, net.encoder if net is not None else source,
                                                                           self._shape, self.fp8, self.device)
         self._buffered_full = 0
-        # launches of more positions than this run the two-position kernel (kernel="auto", 256 wide)
-        self._pair_above = int(self._lib.bf_board_max_n()) if kernel == "auto" and not wide else 1 << 62
+        # launches of more positions than this run the two-position kernel (kernel="auto")
+        self._pair_above = int(self._lib.bf_board_max_n()) if kernel == "auto" else 1 << 62
         # exchange memory of the form that spreads a position over several compute units: one per stream,
         # as launches on different streams may overlap
         with torch.cuda.device(self.device):
@@ -940,8 +940,8 @@ class FusedEncoder:
 
     def kernel_choice(self, n: int) -> str:
         """Which kernel a call with ``n`` positions runs ("quad", "board", "twin", "octo" or "duo").  "octo" counts the
-        form that spreads a position over several compute units too, "twin" in e4m3 the two-position kernel that has
-        taken over its launches; :meth:`launch_form` tells them apart."""
+        form that spreads a position over several compute units too, and "octo" of the 512-wide network and "twin" in e4m3
+        the two-position kernels that have taken over their larger launches; :meth:`launch_form` tells them apart."""
         a = _Args()
         a.n, a.shape, a.quant, a.kernel = n, self._shape, (1 if self.fp8 else 0), self.KERNELS[self.kernel]
         a.wstream = a.fparams = 16 if self.wstream is not None else None        # only tested for NULL
@@ -953,10 +953,11 @@ class FusedEncoder:
 
     def launch_form(self, n: int) -> str:
         """:meth:`kernel_choice`, with "team" for launches that go to the form that spreads a position over several
-        compute units (the smallest ones, without taps and profile) and "duo" where kernel="auto" answers "twin"."""
-        kind = self.kernel_choice(n)
-        if self.kernel == "auto" and kind == "twin":
+        compute units (the smallest ones, without taps and profile) and "duo" for those with two positions per
+        workgroup (of kernel="auto", all of more than 256 positions)."""
+        if n > self._pair_above:
             return "duo"
+        kind = self.kernel_choice(n)
         if kind != "octo" or not self._team_bytes:
             return kind
         most = self._team_bytes // int(self._lib.bf_team_position_bytes(C.byref(self._shape)))
@@ -1153,9 +1154,7 @@ class FusedEncoder:
 
     def _launch_waves(self, n: int) -> int:
         """Wavefronts in a launch of ``n`` positions of the kernel such a call runs."""
-        kind = self.kernel_choice(n)
-        if self.kernel == "auto" and kind == "twin":
-            kind = "duo"
+        kind = "duo" if n > self._pair_above else self.kernel_choice(n)
         return {"board": 4 * n, "twin": 4 * n, "octo": 8 * n, "duo": 8 * ((n + 1) // 2), "quad": 4 * ((n + 3) // 4)}[kind]
 
     def profile_phase_names(self):

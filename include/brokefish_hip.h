@@ -59,11 +59,11 @@ enum bf_quant {
  * BOARD, TWIN, OCTO and DUO read the same blobs (board_wstream / board_fparams).  The 256-wide network
  * runs in int8 and e4m3 on all four; the 512-wide network in int8 on OCTO and BOARD.  Kernels that
  * carry a network and a format return bit-identical results for it, so AUTO may pick by batch
- * size: OCTO up to 256 positions, above that DUO (for e4m3 bf_kernel_choice still answers TWIN, which
- * DUO has overtaken there).  DUO runs in rounds of 512
- * positions; when AUTO has chosen it and the last round would hold at most 256 positions, those
- * are given to the one-position form in a second launch on the same stream (bf_kernel_choice
- * still answers DUO). */
+ * size: OCTO up to 256 positions, above that two positions per workgroup: DUO, and a form of its own for the
+ * 512-wide network (bf_kernel_choice still answers TWIN for e4m3 and OCTO for that network, whose
+ * launches these were).  They run in rounds of 512 positions; when AUTO has chosen them and the last round
+ * would hold at most 256 positions, those are given to the one-position form in a second launch on the
+ * same stream. */
 enum bf_kernel {
     BF_KERNEL_AUTO = 0,
     BF_KERNEL_QUAD = 1,
@@ -228,8 +228,8 @@ typedef struct {
      * QUAD: the wavefront runs on, storing nothing) */
     const uint8_t* active;
     int32_t kernel;         /* enum bf_kernel; AUTO with the board blobs: OCTO for
-                             * n <= bf_board_max_n() and for the 512-wide network, above that
-                             * DUO; without the board blobs QUAD */
+                             * n <= bf_board_max_n(), above that two positions per workgroup
+                             * (DUO); without the board blobs QUAD */
     /* which tokens the value rows read (reference brokefish/nn/model.py:551-617): the king of the
      * side to move (BF_VALUE_KING, the default), the mean of the final-normed live tokens
      * (BF_VALUE_POOLED), or the final norm of the mean of the live tokens' residual stream
@@ -273,11 +273,11 @@ typedef struct {
 #define BF_ABI_TAG (((uint64_t)BF_ABI_VERSION << 32) | (uint64_t)sizeof(bf_eval_args))
 uint64_t bf_abi_tag(void);
 
-/* Largest n for which AUTO prefers OCTO over DUO / TWIN on the 256-wide network. */
+/* Largest n for which AUTO gives a workgroup one position. */
 int64_t bf_board_max_n(void);
 /* The kernel AUTO would run for these arguments (enum bf_kernel), or a negative bf_status.  The form that spreads a
  * position over several compute units (team_workspace) counts as OCTO, whose launches it takes; DUO's e4m3 launches
- * count as TWIN, whose they were. */
+ * count as TWIN, those of the 512-wide network with two positions per workgroup as OCTO, whose they were. */
 int bf_kernel_choice(const bf_eval_args* args);
 
 /* The evaluator.  Replaces model_forward of the reference extension
