@@ -15,8 +15,8 @@
 // So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
 // tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
 // except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
-// 120 -> 82 us, e4m3 155 -> 96, width 512 with 16 layers 738 -> 272; 64 positions 120 -> 87, e4m3 155 -> 99; 32 of the
-// wide network 738 -> 328.  The arithmetic is that of the other kernels, operation for operation: the results are
+// 120 -> 76 us, e4m3 155 -> 92, width 512 with 16 layers 738 -> 266; 64 positions 120 -> 81, e4m3 155 -> 95; 32 of the
+// wide network 738 -> 321.  The arithmetic is that of the other kernels, operation for operation: the results are
 // bit-identical to theirs.
 //
 // Rows and tiles.  For everything per row (LayerNorm, quantisers, residual sums) a wavefront owns the rows of four
@@ -27,8 +27,15 @@
 // the L2, where pieces are laid out so that four tokens, 64 bytes, stay together on either side.
 //
 // What bounds it now: a layer is some 20 k clocks at width 256, of which the waits for other members are 1.5 k; the unit's
-// path to the L2 moves 400 KB in it (6.3 k clocks, most of it under something else), two LayerNorms, three
-// quantisers and the epilogues are some 7 k of vector work, attention 2.8 k.
+// path to the L2 moves 370 KB in it (5.8 k clocks, most of it under something else), two LayerNorms, three
+// quantisers and the epilogues are some 7 k of vector work, attention 2.8 k.  Outside the layers: 8.7 k to the first one (two
+// loads that depend on each other, then the first weights), 8.3 k of final norm and head chain, 3.3 k for the best move.
+// The path takes a 16-byte load of 64 lanes in 16 clocks and a wavefront stops at the load that finds it busy, so where the
+// loads stand matters as much as how many they are (one position, 82.3 us before):
+//   - a layer's parameters, asked for right before the Q, K, V products, made those wait for them (all loads return in order);
+//     the four wavefronts without attention ask for the next layer's in that time: 81.5, width 512 273 -> 265;
+//   - weights between the vector instructions of the LayerNorms and the softmax instead of all at once: 78.7;
+//   - a member's own piece of exchange B through LDS (96 KB instead of 128), each copy of the sum in the order of the loads: 76.4.
 //
 // An exchange: a wavefront stores its piece, waits until the L2 has it (vmcnt), and stores a flag; the wavefronts that
 // need the piece poll the flags past their L1 (sc1) and then load the piece past it (polling tags inside the data
@@ -178,15 +185,21 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     const float* const gp = a.fparams + (size_t)4 * a.n_layers * C::PW_FLOATS;
     const int fq = 2 * (m & 1) + (wave >> 2), fh = wave & 3, fst = m >> 1;   // hidden tile 8 m + wave: its quarter, number there, step
     auto par = [&](int l, int quarter) { return reinterpret_cast<const float*>(lds + C::PAR_OFF + (l & 1) * C::PAR_BYTES) + quarter * C::P_FLOATS; };
-    auto fetch_par = [&](int l) {   // a quarter's part A by its first wave, the rest by its second
-        const float* src = a.fparams + ((size_t)q * a.n_layers + l) * C::PW_FLOATS;
-        float* dst = const_cast<float*>(par(l, q));
-        if (wave & 1) {
-            src += C::A_FLOATS;
-            dma(src, dst + C::P_B, C::B_LDS_FLOATS, lane);
-            dma(src + C::B_WSUM + m * CW, dst + C::P_WSUM, CW, lane);
-            dma(src + C::B_BFF1 + 128 * fst, dst + C::P_BFF1, 128, lane);
-        } else dma(src, dst, C::A_FLOATS, lane);
+    auto fetch_par = [&](int l, int quarter, bool first, bool rest) {   // of a quarter: part A, and what follows it
+        const float* const src = a.fparams + ((size_t)quarter * a.n_layers + l) * C::PW_FLOATS;
+        float* const dst = const_cast<float*>(par(l, quarter));
+        if (first) dma(src, dst, C::A_FLOATS, lane);
+        if (rest) {
+            dma(src + C::A_FLOATS, dst + C::P_B, C::B_LDS_FLOATS, lane);
+            dma(src + C::A_FLOATS + C::B_WSUM + m * CW, dst + C::P_WSUM, CW, lane);
+            dma(src + C::A_FLOATS + C::B_BFF1 + 128 * fst, dst + C::P_BFF1, 128, lane);
+        }
+    };
+    float* const fin = const_cast<float*>(par(a.l1, 0));   // the final norm's, after the last layer: [gamma][beta]
+    static_assert(2 * D <= 4 * C::P_FLOATS, "they fit a copy");
+    auto fetch_final = [&]() {
+        dma(gp + C::G_NFG, fin, D, lane);
+        dma(gp + C::G_NFB, fin + D, D, lane);
     };
     // block `idx` of layer l in a quarter's stream.  Buffer loads with the block's place in a scalar register: one
     // vector register of addresses for all of them (the stream is far below 4 GiB).
@@ -198,14 +211,24 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
 #pragma unroll
         for (int s = 0; s < 8; s++) w[s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane16 + s % 4 * FRAG, at + s / 4 * 4 * FRAG, 0));
     };
-    // Two register sets of KC blocks: SA serves QKV, (width 512) the second tile of the output projection, and
-    // the second feed-forward matmul; SB the output projection and the first.  A set is filled as soon as it is
-    // free, a LayerNorm, an attention or an exchange ahead of its use.
-    v4i SA[KC][8], SB[KC][8];
+    // Register sets of KC blocks.  Width 512, two: SA serves QKV, the second tile of the output projection, and the second
+    // feed-forward matmul; SB the output projection and the first.  A set is filled as soon as it is free, a LayerNorm, an
+    // attention or an exchange ahead of its use.  Width 256, three: SA QKV and the second feed-forward matmul, SB the output
+    // projection, SC the first feed-forward matmul.  Each is filled where the wavefront has vector work to put between the loads
+    // (spaced() below): SA and SB in LayerNorm 1, SC in the softmax, SA again in LayerNorm 2 -- or has nothing to do: SC by the
+    // four that have no attention.  Filled at once, as soon as free: one position 82.3 us instead of 78.7.
+    v4i SA[KC][8], SB[KC][8], SC[TWW == 1 ? KC : 1][8];
+    auto& SF = [&]() -> auto& { if constexpr (TWW == 1) return SC; else return SB; }();
     const int hh = wave & 1, tq = wave >> 1;        // QKV: waves 0..5 take tile tq (Q, K, V) of head hh
+    // the stream as waves 6 and 7 see it in fetch_qkv: empty, their loads move nothing (a branch around them could not be scheduled into)
+    const __amdgpu_buffer_rsrc_t wq = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.wstream), 0, tq < 3 ? 4 * stride_q * BLOCK : 0, 0x00020000);
     const int head = 2 * m + hh, hq = head / TW, hi = head % TW;
     auto fetch_qkv = [&](int l) {
-        if (tq < 3) {
+        if constexpr (TWW == 1) {
+            const int at = tq < 3 ? (hq * stride_q + l * BPW + 3 * hi + tq) * BLOCK : 0, hop = tq < 3 ? 4 * FRAG : 0;
+#pragma unroll
+            for (int s = 0; s < 8; s++) SA[0][s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wq, lane16 + s % 4 * FRAG, at + s / 4 * hop, 0));
+        } else if (tq < 3) {
 #pragma unroll
             for (int c = 0; c < KC; c++) load_block(SA[c], hq, l, 3 * KC * hi + tq * KC + c);
         } else {   // nothing: the set's old contents end here, or they would stay in registers up to this point
@@ -221,13 +244,22 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     };
     auto fetch_ff1 = [&](int l) {
 #pragma unroll
-        for (int c = 0; c < KC; c++) load_block(SB[c], fq, l, BASE + fst * SSTR + KC * fh + c);
+        for (int c = 0; c < KC; c++) load_block(SF[c], fq, l, BASE + fst * SSTR + KC * fh + c);
     };
     auto fetch_ff2 = [&](int l) {
 #pragma unroll
         for (int i = 0; i < TWW; i++) load_block(SA[i], q, l, BASE + fst * SSTR + 4 * KC + (m & 1) * TW + iq0 + i);
     };
     static_assert(TWW <= KC, "the second feed-forward matmul's blocks fit the set");
+    // `count` loads one at a time among the vector instructions of the code around (to the next barrier), `every` of those apart: the
+    // unit takes a load in 16 clocks, so a set's eight at once, by all wavefronts, stop the wavefronts for a thousand.
+    auto spaced = [&](auto every, auto count) {
+#pragma unroll
+        for (int i = 0; i < decltype(count)::value; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x002, decltype(every)::value, 0);   // vector instructions
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                        // a load
+        }
+    };
     auto product = [&](auto swap, const v4i (&w)[8], const uint8_t* from, acc_t acc) -> acc_t {
 #pragma unroll
         for (int s = 0; s < 8; s++) acc = frag_mma<decltype(swap)::value>(w[s], *reinterpret_cast<const v4i*>(from + s * FRAG + lane * 16), acc);
@@ -246,7 +278,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         const v2u r = rows_of(v);
         const float lo = __int_as_float(r[0]), hi = __int_as_float(r[1]);
         float s = ((lo + dpp<SHL + 8>(lo)) + hi) + dpp<SHL + 8>(hi);
-        s = s + partner(s, rg);
+        s = Rows<1>::sum({s});
         int u = __float_as_int(s);
         u = __builtin_amdgcn_update_dpp(u, u, SHR + 4, 0xf, 0x2, false);
         u = __builtin_amdgcn_update_dpp(u, u, SHR + 8, 0xf, 0xc, false);
@@ -254,12 +286,12 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     };
     // largest value of a row's 256-wide chunk
     auto chunkmax = [&](float v) -> float {
-        v = __builtin_fmaxf(v, dpp<ROR + 4>(v));
-        v = __builtin_fmaxf(v, dpp<ROR + 8>(v));
-        v = __builtin_fmaxf(v, partner(v, rg));
+        v = vmax(v, dpp<ROR + 4>(v));
+        v = vmax(v, dpp<ROR + 8>(v));
+        v = Rows<1>::max({v});
         if constexpr (KC == 1) {
             const v2u r = rows_of(v);
-            v = __builtin_fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
+            v = vmax(__int_as_float(r[0]), __int_as_float(r[1]));
         }
         return v;
     };
@@ -350,7 +382,8 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     auto tile_at = [&](int tile) { return tile % NP * FRAG + tile / NP * 64; };
 
     // ---- start: parameters of the first layer; its weights follow the embedding's loads, which return in order ----
-    if (a.l1 > a.l0) fetch_par(a.l0);
+    if (a.l1 > a.l0) fetch_par(a.l0, q, !(wave & 1), wave & 1);
+    else if (!ENC && wave == 4) fetch_final();
 
     // ---- embedding, or the caller's stream -------------------------------------------------------------
     float x[NP][16];
@@ -401,10 +434,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     }
 #pragma unroll
     for (int p = 0; p < NP; p++) pin16(x[p]);   // has arrived, and with it the parameters, which were asked for before
-    if (a.l1 > a.l0) {
-        fetch_qkv(a.l0);
-        if constexpr (TWW == 1) fetch_out(SB, a.l0, 0);
-    }
+    if constexpr (TWW > 1) if (a.l1 > a.l0) fetch_qkv(a.l0);
     lds_barrier();
 
     for (int l = a.l0; l < a.l1; l++) {
@@ -416,11 +446,16 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         // ---- LayerNorm 1, quantise ---------------------------------------------------------------------
         {
             float y[NP][16];
+            if constexpr (TWW == 1) {
+                fetch_qkv(l);
+                fetch_out(SB, l, 0);
+            }
             layernorm(x, pr + C::A_LN1G, pr + C::A_LN1B, y);
+            if constexpr (TWW == 1) spaced(std::integral_constant<int, 5>(), std::integral_constant<int, 16>());
+            __builtin_amdgcn_sched_barrier(0);
             quantise(y);
         }
         lds_barrier();
-        if (lnext != l) fetch_par(lnext);   // the other copy's last reads lie before the barriers above
 
         __builtin_amdgcn_sched_barrier(0);
         // ---- Q, K, V tiles of this member's heads ------------------------------------------------------
@@ -460,8 +495,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 for (int iq = 0; iq < 2; iq++)
                     *reinterpret_cast<v4f*>(to + ((g * 2 + odd) * 2 + iq) * 128) = v4f{v[8 * iq + odd], v[8 * iq + 2 + odd], v[8 * iq + 4 + odd], v[8 * iq + 6 + odd]};
         }
-        if constexpr (TWW == 1) fetch_ff2(l);
-        else {
+        if constexpr (TWW > 1) {
             fetch_out(SB, l, 0);
             fetch_out(SA, l, 1);
         }
@@ -491,6 +525,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             for (int i = 0; i < 8; i++)
 #pragma unroll
                 for (int u = 0; u < 2; u++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[u][i], qv[i], sc[u], 0, 0, 0);
+            if constexpr (TWW == 1) fetch_ff1(l);
             float p[8];
             float mx = -__builtin_inff();
 #pragma unroll
@@ -498,11 +533,11 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 float s = sc[i / 4][i % 4] * 0.17677669529663687f;
                 s = ((alive >> ch(2 * i + (G >> 1), G & 1)) & 1u) ? s : -__builtin_inff();
                 p[i] = s;
-                mx = __builtin_fmaxf(mx, s);
+                mx = vmax(mx, s);
             }
-            mx = __builtin_fmaxf(mx, partner(mx, g));
+            mx = Rows<1>::max({mx});
             const v2u mr = rows_of(mx);
-            mx = __builtin_fmaxf(__int_as_float(mr[0]), __int_as_float(mr[1]));
+            mx = vmax(__int_as_float(mr[0]), __int_as_float(mr[1]));
             // a lane half's chain runs over r = 0 .. 15: even r in lane rows 0 and 1, odd r in rows 2 and 3
             float lsum = 0.0f;
 #pragma unroll
@@ -515,6 +550,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             }
             const v2u lr = rows_of(lsum);
             const float rl = recip(__int_as_float(lr[0]) + __int_as_float(lr[1]));
+            if constexpr (TWW == 1) spaced(std::integral_constant<int, 14>(), std::integral_constant<int, 8>());
             float vv[2][8];
 #pragma unroll
             for (int u = 0; u < 2; u++) operand(2, 16 * u + c16, vv[u]);
@@ -532,6 +568,12 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, oa[u]), wsr,
                                                        piece_at(c16, G & 1) + (G >> 1) * C::ROWS_Q, C::WS_A + 4 * qb * C::ROWS_W + 2 * u * C::ROWS_Q + tile_at(tile), 0);
             raise_flag(C::FLAG_A + qb * NT + tile, tag);
+        }
+        if (wave >= 4) {
+            // the other copy's last reads lie before the barriers above
+            if (lnext != l) fetch_par(lnext, wave & 3, true, true);
+            else if (!ENC && wave == 4) fetch_final();
+            if constexpr (TWW == 1) fetch_ff1(l);
         }
 
         // ---- exchange A, output projection + residual --------------------------------------------------
@@ -555,7 +597,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 acc_t acc[KC];
 #pragma unroll
                 for (int c = 0; c < KC; c++) acc[c] = product(std::false_type(), i == 0 ? SB[c] : SA[c], act + 8 * c * FRAG, zero);
-                if (i == 0) fetch_ff1(l);
+                if (TWW > 1 && i == 0) fetch_ff1(l);
                 v4f bo[4];
                 load_tile16(pq + C::A_BOUT + 32 * (iq0 + i), g, bo);
                 const float sw = pq[C::A_SW + 3 * TW + iq0 + i];
@@ -582,7 +624,10 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         // ---- LayerNorm 2, quantise, this member's chunk of the hidden row ---------------------------------
         {
             float y[NP][16];
+            if constexpr (TWW == 1) fetch_ff2(l);
             layernorm(x, pr + C::P_B + C::B_LN2G, pr + C::P_B + C::B_LN2B, y);
+            if constexpr (TWW == 1) spaced(std::integral_constant<int, 10>(), std::integral_constant<int, 8>());
+            __builtin_amdgcn_sched_barrier(0);
             quantise(y);
         }
         lds_barrier();
@@ -595,7 +640,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             float sa[KC];
             scales(sa);
 #pragma unroll
-            for (int c = 0; c < KC; c++) acc[c] = product(std::false_type(), SB[c], act + 8 * c * FRAG, zero);
+            for (int c = 0; c < KC; c++) acc[c] = product(std::false_type(), SF[c], act + 8 * c * FRAG, zero);
             v4f b1[4];
             load_tile16(pF + C::P_BFF1 + 32 * fh, g, b1);
             const float sw1 = pF[C::P_B + C::B_SW + 4 * fst + fh];
@@ -613,7 +658,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             float mx = 0.0f;
 #pragma unroll
             for (int w = 0; w < 8; w++) mx = __builtin_fmaxf(mx, xch[w * 64 + lane]);
-            mx = __builtin_fmaxf(mx, partner(mx, g));
+            mx = Rows<1>::max({mx});
             sh = hidden_scale<FP8>(mx);
             const Quot by = quot_by(sh);
             v4i w;
@@ -646,7 +691,12 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                     if constexpr (C::TWO_STEPS) __builtin_amdgcn_raw_buffer_store_b128(v, wsr, lane16, C::piece_b(m, tile, j), 0);
                     else __builtin_amdgcn_raw_buffer_store_b128(v, wsr, piece_at(t, g), C::WS_B + m * C::ROWS + j * C::ROWS_Q + tile_at(tile), 0);
                 }
+                if constexpr (!C::TWO_STEPS)   // this member's own piece: through LDS
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        *reinterpret_cast<v4i*>(ex + wave * C::EX_TILE + j * FRAG + lane16) = v4i{accbits(acc, 4 * j), accbits(acc, 4 * j + 1), accbits(acc, 4 * j + 2), accbits(acc, 4 * j + 3)};
             }
+            if constexpr (!C::TWO_STEPS) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the flag stands for it, too
             if (wave == 0 && g == 0) __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(sh), wsr, t * 4, C::scales_b(m), 0);
             raise_flag(C::flag_b(m, wave), tag);
             wait_flags(C::awaited_b(m, lane), C::FLAGS_B, tag, reached);
@@ -687,44 +737,50 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                 float shc[NWG];
 #pragma unroll
                 for (int c = 0; c < NWG; c++) shc[c] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(wsr, row * 4, C::scales_b(c), SC1));
-                v4i piece[NWG][4];
+                // the others' pieces in order, and this member's own
+                v4i piece[NWG - 1][4], own[4];
 #pragma unroll
-                for (int c = 0; c < NWG; c++)
+                for (int j = 0; j < 4; j++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++) piece[c][j] = take(C::WS_B + c * C::ROWS, 0, j);
-                double o64[16];
-                float o32[16];
+                    for (int c = 0; c < NWG - 1; c++) piece[c][j] = take(C::WS_B + (c + (c >= m)) * C::ROWS, 0, j);
 #pragma unroll
-                for (int c = 0; c < NWG; c++) {
-                    if constexpr (FP8) {
-                        const float sw2 = prB[C::B_SW + 16 + ri * KCF + c];
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const float part = (__int_as_float(piece[c][r / 4][r % 4]) * shc[c]) * sw2;
-                            o32[r] = c == 0 ? part : o32[r] + part;
-                        }
-                    } else {
-                        const double sc = (double)shc[c];
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const double full = (double)piece[c][r / 4][r % 4];
-                            o64[r] = c == 0 ? full * sc : __builtin_fma(full, sc, o64[r]);
-                        }
-                    }
-                }
+                for (int j = 0; j < 4; j++) own[j] = *reinterpret_cast<const v4i*>(ex + rk * C::EX_TILE + j * FRAG + (rg * 32 + row) * 16);
                 const float sw = prB[C::B_SW + 16 + ri];
+                auto sum_as = [&](auto member) {   // the sum runs over the members in order: one copy of it per place of the own piece
+                    constexpr int M = decltype(member)::value;
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const v4f b2 = ldg4(pr + C::P_B + C::B_BFF2 + 8 * j);
+                    for (int j = 0; j < 4; j++) {
+                        if constexpr (!FP8)   // its work stays in this copy, in the order of the loads (e4m3 is the faster without: 91.7 us against 92.9)
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const int r = 4 * j + k;
-                        float upd;
-                        if constexpr (FP8) upd = o32[r] + b2[k];
-                        else upd = (float)o64[r] * sw + b2[k];
-                        x[0][r] = x[0][r] + upd;
+                            for (int c = 0; c < NWG - 1; c++) asm volatile("" : "+v"(piece[c][j]));
+                        const v4f b2 = ldg4(pr + C::P_B + C::B_BFF2 + 8 * j);
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            double o64 = 0.0;
+                            float upd = 0.0f;
+#pragma unroll
+                            for (int c = 0; c < NWG; c++) {
+                                const int v = c == M ? own[j][k] : piece[c - (c > M)][j][k];
+                                if constexpr (FP8) {
+                                    const float part = (__int_as_float(v) * shc[c]) * prB[C::B_SW + 16 + ri * KCF + c];
+                                    upd = c == 0 ? part : upd + part;
+                                } else {
+                                    const double full = (double)v, sc = (double)shc[c];
+                                    o64 = c == 0 ? full * sc : __builtin_fma(full, sc, o64);
+                                }
+                            }
+                            if constexpr (FP8) upd = upd + b2[k];
+                            else upd = (float)o64 * sw + b2[k];
+                            x[0][4 * j + k] = x[0][4 * j + k] + upd;
+                        }
                     }
-                }
+                    asm volatile("; %0" ::"n"(M));   // differs from copy to copy, or the compiler makes one of them and selects its operands, behind the last load
+                };
+                static_assert(C::TWO_STEPS || NWG == 4, "a copy per member");
+                if (m == 0) sum_as(std::integral_constant<int, 0>());
+                else if (m == 1) sum_as(std::integral_constant<int, 1>());
+                else if (m == 2) sum_as(std::integral_constant<int, 2>());
+                else sum_as(std::integral_constant<int, 3>());
             }
 #pragma unroll
             for (int p = 0; p < NP; p++) {
@@ -733,8 +789,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                     for (int r = 0; r < 16; r++) x[p][r] = __builtin_nanf("");
                 pin16(x[p]);
             }
-            fetch_qkv(lnext);
-            if constexpr (TWW == 1) fetch_out(SB, lnext, 0);
+            if constexpr (TWW > 1) fetch_qkv(lnext);
         }
     }
     if (wave == 0 && lane == 0) flags[m] = tag0 + (a.l1 - a.l0);
@@ -769,8 +824,8 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     const int ht = job >> 2, rh = job < 8 ? (job >> 1) & 1 : 0, th = job & 1;   // job < 10: rows 16 rh .. of head tile ht, tokens 16 th ..
     if (job < 10) load_head(ht, rh, 0);
     float hn[NP][16];
-    const float* const gn = gp + 32 * NP * rk + 4 * rg;
-    layernorm(x, gn + C::G_NFG, gn + C::G_NFB, hn);
+    const float* const gn = fin + 32 * NP * rk + 4 * rg;
+    layernorm(x, gn, gn + D, hn);
     // as operand fragments (tile, quad)
     float* const hnb = reinterpret_cast<float*>(ex);
     auto publish = [&](const float (&v)[NP][16]) {
@@ -919,7 +974,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                     const v4f s = *reinterpret_cast<const v4f*>(ex + (NP * rk + p) * C::EX_TILE + j * FRAG + (rg * 32 + row) * 16);
                     v[p][4 * j] = s[0]; v[p][4 * j + 2] = s[1]; v[p][4 * j + 1] = s[2]; v[p][4 * j + 3] = s[3];
                 }
-            layernorm(v, gn + C::G_NFG, gn + C::G_NFB, hv);
+            layernorm(v, gn, gn + D, hv);
             lds_barrier();
             publish(hv);
             lds_barrier();
