@@ -925,7 +925,7 @@ class FusedEncoder:
         if not self._team_bytes:
             return None
         wide = self.d_model != self.D
-        left = n % 256 if wide else n if self.fp8 else n % 512
+        left = n % 256 if wide else n % 512
         if not 0 < left <= 64:
             return None
         if torch.cuda.is_current_stream_capturing():
