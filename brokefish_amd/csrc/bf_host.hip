@@ -311,8 +311,8 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
                                  "are NaN (see team_workspace of bf_eval_args); nothing was launched now");
     const bool enc = !k.profile && enc_build(a, kind);
     // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
-    // position 120 -> 82 us, e4m3 155 -> 96; 512 wide 738 -> 272 us), and 512 wide so does one that two team launches hold
-    // (328 us each; the one-position form takes 738 for up to 256).
+    // position 120 -> 76 us, e4m3 155 -> 92; 512 wide 738 -> 265 us), and 512 wide so does one that two team launches hold
+    // (320 us each; the one-position form takes 738 for up to 256).
     const bool wide = a->shape.d_model == 512;
     const int team = team_limit(a, k, enc);
     auto launch_teams = [&](const bf::KArgs& s) {

@@ -15,8 +15,8 @@
 // So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
 // tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
 // except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
-// 120 -> 76 us, e4m3 155 -> 92, width 512 with 16 layers 738 -> 266; 64 positions 120 -> 81, e4m3 155 -> 95; 32 of the
-// wide network 738 -> 321.  The arithmetic is that of the other kernels, operation for operation: the results are
+// 120 -> 76 us, e4m3 155 -> 92, width 512 with 16 layers 738 -> 265; 64 positions 120 -> 81, e4m3 155 -> 95; 32 of the
+// wide network 738 -> 320.  The arithmetic is that of the other kernels, operation for operation: the results are
 // bit-identical to theirs.
 //
 // Rows and tiles.  For everything per row (LayerNorm, quantisers, residual sums) a wavefront owns the rows of four
@@ -212,8 +212,9 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         for (int s = 0; s < 8; s++) w[s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane16 + s % 4 * FRAG, at + s / 4 * 4 * FRAG, 0));
     };
     // Register sets of KC blocks.  Width 512, two: SA serves QKV, the second tile of the output projection, and the second
-    // feed-forward matmul; SB the output projection and the first.  A set is filled as soon as it is free, a LayerNorm, an
-    // attention or an exchange ahead of its use.  Width 256, three: SA QKV and the second feed-forward matmul, SB the output
+    // feed-forward matmul; SB the output projection and the first.  A set is filled as soon as it is free, an attention or an
+    // exchange ahead of its use; SA for QKV between the vector instructions of LayerNorm 1 (spaced() below; 32 positions 322.6 ->
+    // 319.5 us).  Width 256, three: SA QKV and the second feed-forward matmul, SB the output
     // projection, SC the first feed-forward matmul.  Each is filled where the wavefront has vector work to put between the loads
     // (spaced() below): SA and SB in LayerNorm 1, SC in the softmax, SA again in LayerNorm 2 -- or has nothing to do: SC by the
     // four that have no attention.  Filled at once, as soon as free: one position 82.3 us instead of 78.7.
@@ -224,19 +225,9 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     const __amdgpu_buffer_rsrc_t wq = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.wstream), 0, tq < 3 ? 4 * stride_q * BLOCK : 0, 0x00020000);
     const int head = 2 * m + hh, hq = head / TW, hi = head % TW;
     auto fetch_qkv = [&](int l) {
-        if constexpr (TWW == 1) {
-            const int at = tq < 3 ? (hq * stride_q + l * BPW + 3 * hi + tq) * BLOCK : 0, hop = tq < 3 ? 4 * FRAG : 0;
+        const int at = tq < 3 ? (hq * stride_q + l * BPW + 3 * KC * hi + tq * KC) * BLOCK : 0, hop = tq < 3 ? 4 * FRAG : 0;
 #pragma unroll
-            for (int s = 0; s < 8; s++) SA[0][s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wq, lane16 + s % 4 * FRAG, at + s / 4 * hop, 0));
-        } else if (tq < 3) {
-#pragma unroll
-            for (int c = 0; c < KC; c++) load_block(SA[c], hq, l, 3 * KC * hi + tq * KC + c);
-        } else {   // nothing: the set's old contents end here, or they would stay in registers up to this point
-#pragma unroll
-            for (int c = 0; c < KC; c++)
-#pragma unroll
-                for (int s = 0; s < 8; s++) asm volatile("" : "=v"(SA[c][s]));
-        }
+        for (int s = 0; s < 8 * KC; s++) SA[s / 8][s % 8] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wq, lane16 + s % 4 * FRAG, at + s / 4 * hop, 0));
     };
     auto fetch_out = [&](v4i (&w)[KC][8], int l, int i) {
 #pragma unroll
@@ -434,7 +425,6 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     }
 #pragma unroll
     for (int p = 0; p < NP; p++) pin16(x[p]);   // has arrived, and with it the parameters, which were asked for before
-    if constexpr (TWW > 1) if (a.l1 > a.l0) fetch_qkv(a.l0);
     lds_barrier();
 
     for (int l = a.l0; l < a.l1; l++) {
@@ -446,12 +436,10 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
         // ---- LayerNorm 1, quantise ---------------------------------------------------------------------
         {
             float y[NP][16];
-            if constexpr (TWW == 1) {
-                fetch_qkv(l);
-                fetch_out(SB, l, 0);
-            }
+            fetch_qkv(l);
+            if constexpr (TWW == 1) fetch_out(SB, l, 0);
             layernorm(x, pr + C::A_LN1G, pr + C::A_LN1B, y);
-            if constexpr (TWW == 1) spaced(std::integral_constant<int, 5>(), std::integral_constant<int, 16>());
+            spaced(std::integral_constant<int, TWW == 1 ? 5 : 12>(), std::integral_constant<int, 16>());
             __builtin_amdgcn_sched_barrier(0);
             quantise(y);
         }
@@ -789,7 +777,6 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
                     for (int r = 0; r < 16; r++) x[p][r] = __builtin_nanf("");
                 pin16(x[p]);
             }
-            if constexpr (TWW > 1) fetch_qkv(lnext);
         }
     }
     if (wave == 0 && lane == 0) flags[m] = tag0 + (a.l1 - a.l0);
