@@ -20,13 +20,12 @@
 //                 waits (LDS round trips, barriers, MFMA results) are covered by the other's
 //                 work.  Weight fragments go from L2 straight to registers (half a block = four
 //                 fragments at a time, prefetched through a rotation of register sets).
-//                 Highest throughput.
 //   OCTO          (with TWIN's register weight path) eight wavefronts per position, one workgroup
 //                 per compute unit: a quarter belongs to two wavefronts, `sub` = 0 and 1, each
 //                 owning half of the quarter's tiles in every matmul and reading its blocks out
-//                 of the quarter's stream where they lie (block_at).  A quarter's LayerNorm chain
-//                 is started by its first wavefront and continued by its second.  Lowest latency
-//                 per position (launches of up to one position per compute unit).
+//                 of the quarter's stream where they lie (block_at).  The 512-wide network's launches of up
+//                 to one position per compute unit, and larger ones where it is asked for by name; the 256-wide
+//                 network's eight-wavefront form is the one-position form of bf_duo.hip.h.
 //
 // LDS map (bytes): [ring: 4 waves x SLOTS x 8 KiB, absent in the TWIN form] [xch: 3 slots of
 // 64 floats per wave] [hid: the whole quantised hidden row (32 KiB at width 256, 64 KiB at width
@@ -51,9 +50,6 @@
 #ifndef BF_TWIN_OCC
 #define BF_TWIN_OCC 2
 #endif
-// Eight-wavefront form: register sets of its weight prefetch.  Measured: 256-wide network, 64
-// positions: 0.136 ms with four sets, 0.137 with three, 0.138 with six; 512-wide network, 4096
-// positions: 12.5 ms with four, 12.8 with three, 16.0 with six (68 spilled registers).
 #ifndef BF_TWIN_AHEAD_FFN
 #define BF_TWIN_AHEAD_FFN 1
 #endif
@@ -62,9 +58,6 @@
 #endif
 #ifndef BF_FORCE_ACTL
 #define BF_FORCE_ACTL 0
-#endif
-#ifndef BF_OCTO_SETS
-#define BF_OCTO_SETS 4
 #endif
 
 // Timing experiments (BF_EXP_*): compile-time switches that replace a part of a kernel by a
@@ -96,7 +89,7 @@ struct Cfg : Layout<DM> {
     // the quantised hidden row of the feed-forward block: the whole row (F / 32 tiles) where it fits
     // -- the 256-wide network (32 KiB), and the 512-wide one (64 KiB) with eight wavefronts, no
     // weight ring and one parameter copy per quarter; otherwise one step of 512 channels (16 tiles)
-    static constexpr bool FULLHID = DM == 256 || (OCTO && DM == 512);
+    static constexpr bool FULLHID = DM == 256 || OCTO;
     static constexpr int HID_FRAGS = FULLHID ? L::F / 32 : 16;
     static constexpr int ACT_OFF = HID_OFF + HID_FRAGS * FRAG;
     static constexpr int PAR_OFF = ACT_OFF + L::NT * FRAG;
@@ -242,9 +235,9 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
     constexpr int HT = 4 / SUB;               // hidden tiles a wave computes per feed-forward step
     constexpr int NB = BPW / SUB;             // weight blocks a wave consumes per layer
     // register sets of the prefetch: NSETS - 1 half-blocks in flight
-    // (the 512-wide network's eight-wave form: three sets measure the same as four and spill
-    // 15 registers instead of 26)
-    constexpr int NSETS = OCTO ? (DM == 512 ? 3 : BF_OCTO_SETS) : BF_TWIN_SETS;
+    // (the eight-wave form: three sets measure the same as four and spill 15 registers instead of 26)
+    constexpr int NSETS = OCTO ? 3 : BF_TWIN_SETS;
+    static_assert(!OCTO || DM == 512, "eight wavefronts: the 512-wide network");
     static_assert(TW % SUB == 0 && (2 * NB) % NSETS == 0, "tiles and register sets must split evenly");
     constexpr bool FULLHID = C::FULLHID;      // the whole quantised hidden row stays in LDS
     static_assert(block_at_covers_layer<KC, TW, SUB, BPW, FULLHID>(), "block_at must enumerate a layer's blocks exactly once");
@@ -253,7 +246,7 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
     constexpr int XS = NW * 64;               // floats of one exchange slot
     // Eight wavefronts on the 512-wide network: a wave has 256 registers and the quantised row alone
     // would take 64 of them, so the activation fragments are read from LDS at each MFMA instead.
-    constexpr bool ACTL = (OCTO && DM == 512) || BF_FORCE_ACTL;
+    constexpr bool ACTL = OCTO || BF_FORCE_ACTL;
     // One wave per SIMD (!TWIN, 512 registers): a tile's product is issued before the previous
     // tile's epilogue, and Q, K and V together, so the matrix pipe works under the vector work of
     // the same wave.  Two waves per SIMD (256 registers each): one product at a time, issued after
