@@ -17,7 +17,7 @@
 // steps (64 clocks, nothing beside them) and, of every int8 matrix step, 24 of its 33 clocks: together 45,000.  The rest
 // are the thirteen exchanges of a layer, whose latencies both wavefronts of a SIMD wait out at the same time, and weights
 // coming out of L2 in bursts.  So an exchange asks for everything at once, a row's statistics are computed once for both
-// positions (Rows), and addresses are made without vector instructions: 1573 us -> 1500.
+// positions (Rows), addresses are made without vector instructions, and an accumulator is descaled without being converted: 1573 us -> 1463.
 //
 // NPOS = 1 is the same kernel with one position per workgroup: the latency form for launches of
 // at most one workgroup per compute unit (each wavefront one tile of the width, every product
@@ -39,18 +39,6 @@
 #pragma once
 
 #include "bf_board.hip.h"
-
-// Weight fragments (four registers each) a wave has in flight or in use.  What the loads cost is their rate out of L2 and
-// not their latency (a build without them runs 8 % shorter, one whose loads all hit L1 as well): at 4096 positions 8
-// places run 1507 us, 12 run 1498; 16 spill.
-#ifndef BF_DUO_RING
-#define BF_DUO_RING 12
-#endif
-// Steps between the LDS fetch of an operand fragment and its use.  4096 positions: 1496 us with one, 1498 with three (a
-// SIMD's other wavefront covers the latency); the one-position form at 100 positions: 118.3 and 116.7.
-#ifndef BF_DUO_AHEAD
-#define BF_DUO_AHEAD 3
-#endif
 
 namespace bf {
 namespace duo {
@@ -107,7 +95,11 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     constexpr int STEPS = C::STEPS, BPW = C::BPW, HB = C::HB;
     constexpr int NB = BPW / 2;      // weight blocks a wave consumes per layer
     constexpr int HT = 2;            // hidden tiles a wave computes per feed-forward step
-    constexpr int RING = FP8 && NP == 2 ? 8 : BF_DUO_RING, AHEAD = BF_DUO_AHEAD;
+    // Weight fragments (four registers each) in flight or in use, and steps between the LDS fetch of an operand fragment and its use
+    // (4096 positions: 1496 us with one, 1498 with three, as a SIMD's other wavefront covers the latency; the one-position form at 100
+    // positions: 118.3 and 116.7; encoder-only, two positions, 512 of them: 179.0, and 179.8 with a register spilled)
+    constexpr int RING = NP == 2 ? 8 : 12, AHEAD = NP == 2 && ENC ? 1 : 3;
+    constexpr bool SUBN = !FP8 && !TAPS;   // how accumulators are descaled, see descale() (tapped accumulators are stored as they are)
     constexpr int XS = C::XS, PS = C::NW * 64;   // floats of an exchange slot; of one position's part of it
     static_assert(C::KC == 1 && STEPS == TW && KCF == 2 * STEPS, "the 256-wide network");
     static_assert(8 % (AHEAD + 1) == 0, "an operand's place must not depend on the product");
@@ -233,7 +225,19 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     };
     const float* const gp = a.fparams + (size_t)4 * a.n_layers * C::PW_FLOATS;
 
-    // The weight fragments in flight: a ring of RING registers-of-four, refilled one by one.  Fragment `fseq` of the
+    // What descaled accumulators start from: the integer whose bits are the smallest normal float (see descale())
+    acc_t start = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if constexpr (SUBN)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            int v = 0x00800000;
+            asm volatile("" : "+v"(v));   // kept, not made anew for every product
+            start[i] = v;
+        }
+    // The weight fragments in flight: a ring of RING registers-of-four, refilled one by one.  What the loads cost is their rate
+    // out of L2 and not their latency (a build without them runs 8 % shorter, one whose loads all hit L1 as well): two
+    // positions, 4096 of them: 8 places 1463 us, 12 with the sixteen registers of `start` beside them 1489 (14 spilled), without
+    // 1481.  One position: 12 places 120.3 us, 16 120.7, 24 128.6 (spilled).  Fragment `fseq` of the
     // quarter's stream into place `at`.
     v4i frt[RING];
     auto load_frag = [&](int fseq, int at) {
@@ -358,7 +362,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     };
     // signed quantiser of both positions' rows: one scale per row; this wave's bytes go to the
     // position's activation buffer, from which every wave reads its B operands
-    auto quant_exchange2 = [&](const float (&y)[NP][16], float (&sa)[NP], int8_t* tap, const size_t (&tap_row)[NP], bool publish_scales) {
+    auto quant_exchange2 = [&](const float (&y)[NP][16], float (&sa)[NP], float (&ex)[NP], int8_t* tap, const size_t (&tap_row)[NP], bool publish_scales) {
         float am[NP];
 #pragma unroll
         for (int p = 0; p < NP; p++) {
@@ -372,7 +376,11 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
         for (int w = 0; w < C::NW; w++) mw[w] = xlane[2 * XS + w * 64];
         const float sr = row_scale<FP8>(xmax_row(vmax3(vmax3(mw[0], mw[1], mw[2]), vmax3(mw[3], mw[4], mw[5]), vmax(mw[6], mw[7]))));
-        Rows<NP>::each(sr, sa);
+        if constexpr (SUBN) {   // the scale in two parts: its significand times 2^126 (NaN: NaN), its exponent and 23
+            const int bits = __float_as_int(sr);
+            Rows<NP>::each(__builtin_fmaf(sr, 0.0f, __int_as_float((bits & 0x007fffff) | 0x7e800000)), sa);
+            Rows<NP>::each(__int_as_float((bits >> 23) - 127 + 23), ex);
+        } else Rows<NP>::each(sr, sa);
         if (publish_scales && wave == 0 && lane < 32 * NP) here_f(tok)[lane] = sr;
         const Quot br = quot_by(sr);
         float hi[NP], lo[NP];
@@ -549,14 +557,33 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         }                                                                                            \
     } while (0)
         const acc_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        // An accumulator a times its row's scale s and its channel's w: fl(fl(a s) w).  int8: the sum of a matmul of the width is
+        // below 2^22, and the products start at 2^23, so that what comes out, 2^23 + a, is the bit pattern of the float
+        // (2^23 + a) 2^-149: up to 2^24 the bits of subnormal and smallest normal floats count linearly.  One fused operation takes
+        // the offset off and multiplies: with s = m 2^e, fma(x, m 2^126, -m) = fl(a m) 2^-23, exactly rounded as fl(a s) is, and
+        // 2^(e + 23) goes into w (ldexp, once a tile).  That takes the place of a conversion, 4.4 clocks, and a product: 4096
+        // positions 1481 -> 1463 us, 200 positions 115.2 -> 113.6, same bits (for s w below 2^104, where such a matmul's
+        // results reach a float's range; rows without a largest value, NaN, stay NaN).
+        auto descale = [&](const acc_t& ac, int e, float s, float off, float w) -> float {
+            if constexpr (SUBN) return __builtin_fmaf(__int_as_float(accbits(ac, e)), s, off) * w;
+            else return accf(ac, e) * s * w;
+        };
+        auto offsets = [&](const float (&sa)[NP], float (&off)[NP]) {
+#pragma unroll
+            for (int p = 0; p < NP; p++) off[p] = SUBN ? sa[p] * -0x1p-126f : 0.0f;
+        };
+        auto scaled = [&](float w, const float (&ex)[NP], float (&to)[NP]) {
+#pragma unroll
+            for (int p = 0; p < NP; p++) to[p] = SUBN ? __builtin_ldexpf(w, __float_as_int(ex[p])) : w;
+        };
         auto none = [&](int) {};
 
         // ---- LayerNorm 1, quantise, exchange -----------------------------------------------------------
-        float sa[NP];
+        float sa[NP], ex[NP];
         {
             float y[NP][16];
             layernorm2(x, here_f(pA + C::A_LN1G + 32 * sub), here_f(pA + C::A_LN1B + 32 * sub), y);
-            quant_exchange2(y, sa, TAPS ? a.taps.qa_qkv : nullptr, bl, true);
+            quant_exchange2(y, sa, ex, TAPS ? a.taps.qa_qkv : nullptr, bl, true);
         }
         // the quarter's feed-forward parameters of this layer (the first layer's came with the start)
         if (par_owner && li > 0) {
@@ -572,13 +599,17 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             const float* const sw3 = here_f(pA + C::A_SW + sub);
             const float swq = sw3[0], swk = sw3[TW], swv = sw3[2 * TW];
             const float bv = here_f(pA + C::A_BV + 32 * sub)[t];
+            float off[NP], wq[NP], wk[NP];
+            offsets(sa, off);
+            scaled(swq, ex, wq);
+            scaled(swk, ex, wk);
             acc_t acc[2];   // product n of a sequence uses accumulator n & 1; the previous one's epilogue runs under it
             v4f bq[4], bk[4], stok[NP][4];
             // the epilogues, two accumulator registers at a time (slice s of eight)
             auto epi_q = [&](int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    qf[p][e] = accf(ac, e) * sa[p] * swq + bq[e / 4][e % 4];
+                    qf[p][e] = descale(ac, e, sa[p], off[p], wq[p]) + bq[e / 4][e % 4];
                     if (TAPS && a.taps.acc_qkv && live[p])
                         a.taps.acc_qkv[(bl[p] * T + t) * 3 * D + 32 * tile + ch(e, g)] = tapbits<false>(ac, e);
                 }
@@ -586,7 +617,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             auto epi_k = [&](int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    kf[p][e] = accf(ac, e) * sa[p] * swk + bk[e / 4][e % 4];
+                    kf[p][e] = descale(ac, e, sa[p], off[p], wk[p]) + bk[e / 4][e % 4];
                     if (TAPS && a.taps.acc_qkv && live[p])
                         a.taps.acc_qkv[(bl[p] * T + t) * 3 * D + D + 32 * tile + ch(e, g)] = tapbits<false>(ac, e);
                 }
@@ -645,7 +676,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                     };
                     const uint8_t* const next = act0 + (n + 1) % NP * C::ACT_P;
                     if (tq == 2) BF_DUO_CHAIN(true, 2, p, act0 + p * C::ACT_P, n + 1 < 3 * NP, next, zero, acc[n & 1], between);
-                    else BF_DUO_CHAIN(false, tq, p, act0 + p * C::ACT_P, n + 1 < 3 * NP, next, zero, acc[n & 1], between);
+                    else BF_DUO_CHAIN(false, tq, p, act0 + p * C::ACT_P, n + 1 < 3 * NP, next, start, acc[n & 1], between);
                 }
 #pragma unroll
                 for (int s = 0; s < 8; s++) epi_v(NP - 1, s, acc[(3 * NP - 1) & 1]);
@@ -697,16 +728,18 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 
         // ---- output projection + residual (this wave's tile) --------------------------------------------
         {
-            float so[NP];
-            quant_exchange2(o, so, TAPS ? a.taps.qa_out : nullptr, bl, false);
+            float so[NP], eo[NP], off[NP], wo[NP];
+            quant_exchange2(o, so, eo, TAPS ? a.taps.qa_out : nullptr, bl, false);
             acc_t acc[2];
             v4f bo[4];
             load_tile16(here_f(pA + C::A_BOUT + 32 * sub), g, bo);
             const float sw = *here_f(pA + C::A_SW + 3 * TW + sub);
+            offsets(so, off);
+            scaled(sw, eo, wo);
             auto epi_o = [&](int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
-                    x[p][e] = x[p][e] + (accf(ac, e) * so[p] * sw + bo[e / 4][e % 4]);
+                    x[p][e] = x[p][e] + (descale(ac, e, so[p], off[p], wo[p]) + bo[e / 4][e % 4]);
                     if (TAPS && a.taps.acc_out && live[p])
                         a.taps.acc_out[(bl[p] * T + t) * D + 32 * tile + ch(e, g)] = tapbits<false>(ac, e);
                 }
@@ -723,7 +756,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                     auto between = [&](int s) {
                         if (p > 0) epi_o(p - 1, s, acc[(p - 1) & 1]);
                     };
-                    BF_DUO_CHAIN(false, 3, p, act0 + p * C::ACT_P, p + 1 < NP, act0 + C::ACT_P, zero, acc[p & 1], between);
+                    BF_DUO_CHAIN(false, 3, p, act0 + p * C::ACT_P, p + 1 < NP, act0 + C::ACT_P, start, acc[p & 1], between);
                 }
             }
 #pragma unroll
@@ -735,7 +768,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         {
             float y[NP][16];
             layernorm2(x, here_f(pB + C::B_LN2G + 32 * sub), here_f(pB + C::B_LN2B + 32 * sub), y);
-            quant_exchange2(y, sa, TAPS ? a.taps.qa_ff1 : nullptr, bl, false);
+            quant_exchange2(y, sa, ex, TAPS ? a.taps.qa_ff1 : nullptr, bl, false);
         }
         // the attention-phase parameters are dead for both waves of the quarter: fetch the next layer's
         if (par_owner) {
@@ -756,13 +789,14 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             for (int p = 0; p < NP; p++) am[p] = 0.0f;
             acc_t acc[2], pair[2][NP];   // e4m3: a block's products at a time
             v4f b1[HT][4];
-            float sw1[HT];
+            float off[NP], sw1[HT][NP];
+            offsets(sa, off);
             auto epi_f = [&](int i, int p, int s, const acc_t& ac) {
 #pragma unroll
                 for (int e = 2 * s; e < 2 * s + 2; e++) {
                     // the ReLU is in the hidden quantiser's saturation, and the running maximum starts at 0,
                     // so negative values need no clamp here
-                    const float v = accf(ac, e) * sa[p] * sw1[i] + b1[i][e / 4][e % 4];
+                    const float v = descale(ac, e, sa[p], off[p], sw1[i][p]) + b1[i][e / 4][e % 4];
                     hf[p][i][e] = v;
                     am[p] = __builtin_fmaxf(am[p], v);
                     if (TAPS && a.taps.acc_ff1 && live[p])
@@ -772,7 +806,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
             for (int i = 0; i < HT; i++) {
                 load_tile16(here_f(pB + C::B_BFF1 + 128 * st + 32 * (HT * sub + i)), g, b1[i]);
-                sw1[i] = *here_f(pB + C::B_SW + 4 * st + HT * sub + i);
+                scaled(*here_f(pB + C::B_SW + 4 * st + HT * sub + i), ex, sw1[i]);
                 if constexpr (FP8) {
                     auto with_f = [&](int s) {
                         if (i > 0)
@@ -787,7 +821,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                         auto between = [&](int s) {
                             if (n > 0) epi_f((n - 1) / NP, (n - 1) % NP, s, acc[(n - 1) & 1]);
                         };
-                        BF_DUO_CHAIN(false, 4 + HT * st + i, p, act0 + p * C::ACT_P, n + 1 < NP * HT, act0 + (p + 1) % NP * C::ACT_P, zero, acc[n & 1],
+                        BF_DUO_CHAIN(false, 4 + HT * st + i, p, act0 + p * C::ACT_P, n + 1 < NP * HT, act0 + (p + 1) % NP * C::ACT_P, start, acc[n & 1],
                                      between);
                     }
                 }
