@@ -33,7 +33,7 @@ MEASURED_TRAFFIC_BYTES = {("base", "duo", 4096): 0.445e9, ("base", "twin", 4096)
 MEASURED_TRAFFIC_BYTES_E4M3 = {("base", "twin", 4096): 0.97e9}
 # vector-ALU instructions per launch (SQ_INSTS_VALU of the same counter runs), by (network shape, kernel, batch):
 # with the matrix products hidden, the launch cannot be shorter than these instructions' issue time
-MEASURED_VALU_INSTS = {("base", "duo", 4096): 5.139e8, ("base", "twin", 4096): 5.131e8}
+MEASURED_VALU_INSTS = {("base", "duo", 4096): 4.897e8, ("base", "twin", 4096): 5.131e8}
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 PEAK_HBM_BPS = 8.0e12                 # MI355X HBM3E, bytes/s
 
