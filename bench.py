@@ -31,6 +31,8 @@ PEAK_FP16_OPS = 2.5e15                # dense fp16 MFMA: the e4m3 format's produ
 MEASURED_TRAFFIC_BYTES = {("base", "duo", 4096): 0.445e9, ("base", "twin", 4096): 0.77e9, ("base", "quad", 4096): 3.08e9,
                           ("base", "octo", 256): 5.5e7, ("stress", "octo", 16384): 2.87e10}
 MEASURED_TRAFFIC_BYTES_E4M3 = {("base", "twin", 4096): 0.97e9}
+# ... and of the forms with two positions per workgroup that AUTO runs above 256 positions, by format too
+MEASURED_TRAFFIC_BYTES_PAIRS = {("base", "duo", 4096, "e4m3"): 0.445e9, ("stress", "wide", 16384, "int8"): 1.33e10}
 # vector-ALU instructions per launch (SQ_INSTS_VALU of the same counter runs), by (network shape, kernel, batch):
 # with the matrix products hidden, the launch cannot be shorter than these instructions' issue time
 MEASURED_VALU_INSTS = {("base", "duo", 4096): 4.897e8, ("base", "twin", 4096): 5.131e8}
@@ -144,7 +146,7 @@ def main() -> int:
     # a running search or serving loop sees it.  Short launches are timed over enough repetitions
     # for the clocks to settle.
     from brokefish_amd.hip_impl import mfma_rate, stream_rate
-    kname = {"team": "octo"}.get(model.launch_form(a.batch), model.launch_form(a.batch))
+    kname = model.launch_form(a.batch)      # what runs: a kernel's name, "team" or "wide"
     kern_ms = model.time_kernel_ms(bd, cd, rd, md, warmup=10 if a.batch <= 1024 else 3 if stress else 40,
                                    iters=max(a.steps, 200 if a.batch <= 1024 else 10))
     stream_ceiling = stream_rate(6_389_760 if kname == "quad" else 50_626_560 if stress else 6_455_296, workgroups=min(a.batch, 4096),
@@ -164,11 +166,12 @@ def main() -> int:
     evals = a.batch * a.steps / dt
     achieved = ops_per_eval * a.batch / (kern_ms * 1e-3) / 1e12
     peak = PEAK_FP16_OPS if fp8 else PEAK_INT8_OPS
-    traffic = (MEASURED_TRAFFIC_BYTES_E4M3 if fp8 else MEASURED_TRAFFIC_BYTES).get((a.shape, kname, a.batch))
+    traffic = MEASURED_TRAFFIC_BYTES_PAIRS.get((a.shape, kname, a.batch, a.quant)) or \
+        (MEASURED_TRAFFIC_BYTES_E4M3 if fp8 else MEASURED_TRAFFIC_BYTES).get((a.shape, kname, a.batch))
     # each workgroup streams its own copy of the weights from L2
-    # (four positions share one copy in the quad kernel, two in the duo kernel)
+    # (four positions share one copy in the quad kernel, two in the duo kernel and the wide form)
     weight_bytes = (6_389_760 * ((a.batch + 3) // 4) if kname == "quad"
-                    else (50_626_560 if stress else 6_455_296) * ((a.batch + 1) // 2 if kname == "duo" else a.batch))
+                    else (50_626_560 if stress else 6_455_296) * ((a.batch + 1) // 2 if kname in ("duo", "wide") else a.batch))
     line = {
         "metric": (f"network evals/sec at batch {a.batch} int8, 16-layer width-512 stress shape, on 1 MI355X" if stress
                    else f"network evals/sec at batch 4096 {'fp8 e4m3' if fp8 else 'int8'} on 1 MI355X"),
@@ -208,7 +211,8 @@ def main() -> int:
                              "the kernel timing and the ceiling probes ran before them (device at its steady clocks)")
     if a.phases:
         ph = model.profile_phases(bd, cd, rd, md)
-        line["phases"] = {"kernel": kname, "ticks_per_wavefront": {k: round(v, 1) for k, v in ph.items()},
+        line["phases"] = {"kernel": "octo" if kname == "team" else kname,     # the team form has no profile build
+                           "ticks_per_wavefront": {k: round(v, 1) for k, v in ph.items()},
                           "share_of_total": {k: round(v / ph["total"], 4) for k, v in ph.items() if k != "total"}}
     del model, bd, cd, rd, md
     if headline and not a.no_extras:
@@ -240,7 +244,7 @@ def main() -> int:
                         "frac_fp16_peak_2.5PF": tops / PEAK_FP16_OPS, "frac_fp8_peak_5.0PF": tops / 5.0e15,
                         "measured_mfma_rate": mfma_rate("e4m3")}
         ms = med[("stress", 16384)]
-        line["stress"] = {"batch": 16384, "kernel": mdlw.kernel_choice(16384), "kernel_ms": ms, "evals_per_s": 16384 / ms * 1e3,
+        line["stress"] = {"batch": 16384, "kernel": mdlw.kernel_choice(16384), "form": mdlw.launch_form(16384), "kernel_ms": ms, "evals_per_s": 16384 / ms * 1e3,
                           "achieved_TOPs": OPS_PER_EVAL_STRESS * 16384 / (ms * 1e-3) / 1e12,
                           "frac_int8_peak": OPS_PER_EVAL_STRESS * 16384 / (ms * 1e-3) / PEAK_INT8_OPS}
         line["neighbours"] = neighbours(mdl8, inputs)

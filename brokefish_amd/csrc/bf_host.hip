@@ -33,8 +33,7 @@ static bool board_shape_ok(const bf_shape* s) { return shape_ok(s) || shape512(s
 
 // AUTO runs one workgroup of eight wavefronts per compute unit (lowest latency per position) up
 // to this many positions, which is one per compute unit of an MI355X; above it, the forms built
-// for throughput (256-wide network): two positions per workgroup (int8) or two workgroups of
-// four wavefronts per compute unit (e4m3).
+// for throughput, with two positions per workgroup.
 static const int64_t kBoardMaxN = 256;
 
 template <int DM>
@@ -103,7 +102,7 @@ extern "C" double bf_fp8_q_max(void) { return 8.0; }
 
 extern "C" const char* bf_last_error(void) { return g_err; }
 
-// Which kernel runs for these arguments (enum bf_kernel), or a negative status.
+// The kernel these arguments ask for, or whose launches they are (enum bf_kernel), or a negative status.
 static int choose_kernel(const bf_eval_args* a) {
     if (!a) return fail(BF_ERR_ARGUMENT, "args is NULL");
     if (!board_shape_ok(&a->shape))
@@ -141,7 +140,7 @@ static int choose_kernel(const bf_eval_args* a) {
     case BF_KERNEL_AUTO:
         // above one position per compute unit: two positions per workgroup (int8: 5 to 8 % faster than TWIN from 512
         // positions up and half its L2 traffic).  For e4m3 the answer is still TWIN, what AUTO ran before the two-position
-        // kernel overtook it; check_args() gives those launches to DUO (same bits; 4096 positions 2142 -> 1985 us).
+        // kernel overtook it; run_kernel() gives those launches to DUO.
         if (octo_can) return (twin_can && a->n > kBoardMaxN) ? (a->quant == BF_QUANT_INT8 ? BF_KERNEL_DUO : BF_KERNEL_TWIN) : BF_KERNEL_OCTO;
         if (quad_can) return BF_KERNEL_QUAD;
         return fail(BF_ERR_ARGUMENT, shape512(&a->shape)
@@ -166,10 +165,16 @@ static bool enc_build(const bf_eval_args* a, int kind) {
     return kind == BF_KERNEL_OCTO || kind == BF_KERNEL_DUO || (kind == BF_KERNEL_TWIN && a->quant == BF_QUANT_E4M3);
 }
 
+// What AUTO makes of choose_kernel()'s answer: TWIN's launches are the two-position kernel's (same bits; e4m3, 4096
+// positions: 2142 -> 1962 us).
+static int run_kernel(const bf_eval_args* a) {
+    const int kind = choose_kernel(a);
+    return a && a->kernel == BF_KERNEL_AUTO && kind == BF_KERNEL_TWIN ? BF_KERNEL_DUO : kind;
+}
+
 static int check_args(const bf_eval_args* a, bf::KArgs* k, int* kind) {
-    *kind = choose_kernel(a);
+    *kind = run_kernel(a);
     if (*kind < 0) return *kind;
-    if (a->kernel == BF_KERNEL_AUTO && *kind == BF_KERNEL_TWIN) *kind = BF_KERNEL_DUO;
     const bool board = *kind == BF_KERNEL_BOARD || *kind == BF_KERNEL_TWIN || *kind == BF_KERNEL_OCTO || *kind == BF_KERNEL_DUO;
     if (a->n < 1 || a->n > (1ll << 28)) return fail(BF_ERR_ARGUMENT, "n must be in [1, 2^28]");
     // encoder-only launch: residual stream in and out through the tap table, no board words, no heads
@@ -288,11 +293,33 @@ static bf::KArgs slice(const bf::KArgs& k, int d_model, int first, int count) {
 
 // Positions a team launch of this call may hold: 0 unless AUTO chose, a workspace came along and nothing but the
 // stream is tapped.
-static int team_limit(const bf_eval_args* a, const bf::KArgs& k, bool enc) {
-    if (a->kernel != BF_KERNEL_AUTO || !k.team_ws || k.profile || (a->taps && !enc)) return 0;
+static int team_limit(const bf_eval_args* a, bool profile, bool enc) {
+    if (a->kernel != BF_KERNEL_AUTO || !a->team_workspace || profile || (a->taps && !enc)) return 0;
     const size_t fits = a->team_workspace_bytes / bf::team_slot_bytes(a->shape.d_model);
     const int most = bf::team_positions(a->shape.d_model, false);
     return fits < (size_t)most ? (int)fits : most;
+}
+
+// How a launch of kernel `kind` is carried out: launch() follows it and bf_launch_form() tells it.
+struct Route {
+    int form;       // enum bf_form
+    bool enc;       // the encoder-only build
+    bool rounds;    // whole rounds of two positions per workgroup (form), the rest in a launch of its own
+    int team;       // positions a team launch may hold, 0: none
+    bool by_teams(const bf_eval_args* a, int64_t n) const {   // whether n of the launch's positions go to teams
+        return team > 0 && !(a->leaf_index && n > team) && n <= (a->shape.d_model == 512 ? 2 : 1) * team;
+    }
+};
+static Route route(const bf_eval_args* a, int kind, bool profile) {
+    const bool wide = a->shape.d_model == 512, pairs = a->kernel == BF_KERNEL_AUTO && a->n > kBoardMaxN && (wide || kind == BF_KERNEL_DUO);
+    Route r;
+    r.enc = !profile && enc_build(a, kind);
+    r.team = team_limit(a, profile, r.enc);
+    r.rounds = pairs && (!a->taps || r.enc) && !profile;
+    r.form = kind;   // the forms named after a kernel have its number
+    if (wide && (r.rounds || (pairs && profile))) r.form = BF_FORM_WIDE;
+    else if (kind == BF_KERNEL_OCTO && !r.rounds && r.by_teams(a, a->n)) r.form = BF_FORM_TEAM;
+    return r;
 }
 
 static hipError_t launch_team(const bf_eval_args* a, bf::KArgs k, bool enc, hipStream_t stream) {
@@ -309,23 +336,21 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
     if (bf::team_gave_up())
         return fail(BF_ERR_TEAM, "an earlier launch on this device gave up waiting for compute units held by other launches and its outputs "
                                  "are NaN (see team_workspace of bf_eval_args); nothing was launched now");
-    const bool enc = !k.profile && enc_build(a, kind);
+    const bool wide = a->shape.d_model == 512;
+    const Route to = route(a, kind, k.profile != nullptr);
+    const bool enc = to.enc;
     // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
     // position 120 -> 76 us, e4m3 155 -> 92; 512 wide 738 -> 265 us), and 512 wide so does one that two team launches hold
     // (320 us each; the one-position form takes 738 for up to 256).
-    const bool wide = a->shape.d_model == 512;
-    const int team = team_limit(a, k, enc);
     auto launch_teams = [&](const bf::KArgs& s) {
         hipError_t r = hipSuccess;
-        for (int at = 0; at < s.n && r == hipSuccess; at += team)
-            r = launch_team(a, s.n <= team ? s : slice(s, a->shape.d_model, at, s.n - at < team ? s.n - at : team), enc, stream);
+        for (int at = 0; at < s.n && r == hipSuccess; at += to.team)
+            r = launch_team(a, s.n <= to.team ? s : slice(s, a->shape.d_model, at, s.n - at < to.team ? s.n - at : to.team), enc, stream);
         return r;
     };
-    const auto by_teams = [&](const bf::KArgs& s) { return team > 0 && !(s.leaf_index && s.n > team) && s.n <= (wide ? 2 : 1) * team; };
-    const bool by_rounds = a->kernel == BF_KERNEL_AUTO && (!a->taps || enc) && !k.profile && k.n > (int)kBoardMaxN && (wide || kind == BF_KERNEL_DUO);
-    if (kind == BF_KERNEL_OCTO && !by_rounds && by_teams(k)) {
+    if (to.form == BF_FORM_TEAM) {
         e = launch_teams(k);
-    } else if (by_rounds) {
+    } else if (to.rounds) {
         // Two positions per workgroup, in rounds of 512 positions that cost the same full or not: a last round of at most 256
         // goes to the one-position form in a second launch on the same stream (640 positions: 0.33 ms instead of 0.39, e4m3
         // 0.39 instead of 0.48).  With a leaf list the count is on the device: both forms are launched and each
@@ -345,7 +370,7 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
              : f8 ? (enc ? bf::launch_duo256_fp8_enc : bf::launch_duo256_fp8)
                   : (enc ? bf::launch_duo256_enc : bf::launch_duo256))(front, stream);
         if (rest && e == hipSuccess)
-            e = !k.leaf_index && by_teams(back) ? launch_teams(back)
+            e = !k.leaf_index && to.by_teams(a, back.n) ? launch_teams(back)
                 : (wide ? (enc ? bf::launch_octo512_enc : bf::launch_octo512)
                    : f8 ? (enc ? bf::launch_solo256_fp8_enc : bf::launch_solo256_fp8)
                         : (enc ? bf::launch_solo256_enc : bf::launch_solo256))(back, stream);
@@ -358,7 +383,7 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
         // 256-wide one on the two-position kernel's one-position form, which issues each product under the
         // previous one's epilogue
         if (k.profile && wide)
-            e = (a->kernel == BF_KERNEL_AUTO && k.n > (int)kBoardMaxN ? bf::launch_wide512_prof : bf::launch_octo512_prof)(k, stream);
+            e = (to.form == BF_FORM_WIDE ? bf::launch_wide512_prof : bf::launch_octo512_prof)(k, stream);
         else if (wide)
             e = a->taps ? bf::launch_octo512_taps(k, stream) : bf::launch_octo512(k, stream);
         else if (a->quant == BF_QUANT_E4M3)
@@ -407,6 +432,11 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
         return BF_ERR_LAUNCH;
     }
     return BF_OK;
+}
+
+extern "C" int bf_launch_form(const bf_eval_args* args) {
+    const int kind = run_kernel(args);
+    return kind < 0 ? kind : route(args, kind, false).form;
 }
 
 extern "C" int bf_model_forward(const bf_eval_args* args, void* stream) {

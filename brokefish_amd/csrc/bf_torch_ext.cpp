@@ -727,5 +727,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         const int rc = bf_kernel_choice(&a);
         TORCH_CHECK(rc >= 0, "bf_kernel_choice failed (", rc, "): ", bf_last_error());
         return rc;
-    }, "which kernel (enum bf_kernel) a call with these arguments runs");
+    }, "the kernel (enum bf_kernel) these arguments name or, for AUTO, whose launches they are");
 }

@@ -135,6 +135,8 @@ def load_library():
         L.bf_board_max_n.restype = C.c_int64
         L.bf_kernel_choice.restype = C.c_int
         L.bf_kernel_choice.argtypes = [C.POINTER(_Args)]
+        L.bf_launch_form.restype = C.c_int
+        L.bf_launch_form.argtypes = [C.POINTER(_Args)]
         L.bf_mfma_rate.restype = C.c_double
         L.bf_mfma_rate.argtypes = [C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_void_p]
         L.bf_stream_rate.restype = C.c_double
@@ -831,10 +833,8 @@ class FusedEncoder:
             per = names[self.kernel]
         elif self.board_wstream is None:
             per = names["quad"]
-        elif self.d_model != self.D:
-            per = names["octo"]
         else:
-            per = "1 board/workgroup, 1 or 2 workgroups/CU by batch size"
+            per = "1 or 2 boards/workgroup of 8 wavefronts by batch size"
         return f"{fmt} FFN+QKV+out_proj, {per} (gfx950)"
 
     # -- buffers and checks ---------------------------------------------------
@@ -938,30 +938,36 @@ class FusedEncoder:
             ws = self._team.setdefault(key, torch.zeros(self._team_bytes, dtype=torch.uint8, device=self.device))
         return ws
 
-    def kernel_choice(self, n: int) -> str:
-        """Which kernel a call with ``n`` positions runs ("quad", "board", "twin", "octo" or "duo").  "octo" counts the
-        form that spreads a position over several compute units too, and "octo" of the 512-wide network and "twin" in e4m3
-        the two-position kernels that have taken over their larger launches; :meth:`launch_form` tells them apart."""
+    def _choice_args(self, n: int) -> _Args:
         a = _Args()
         a.n, a.shape, a.quant, a.kernel = n, self._shape, (1 if self.fp8 else 0), self.KERNELS[self.kernel]
         a.wstream = a.fparams = 16 if self.wstream is not None else None        # only tested for NULL
         a.board_wstream = a.board_fparams = 16 if self.board_wstream is not None else None
+        return a
+
+    def kernel_choice(self, n: int) -> str:
+        """The kernel a call with ``n`` positions names or, with kernel="auto", the one whose launches those are ("quad",
+        "board", "twin", "octo" or "duo").  kernel="auto" hands some of them on to forms that return the same bits
+        faster: :meth:`launch_form` says what runs."""
+        a = self._choice_args(n)
         rc = self._lib.bf_kernel_choice(C.byref(a))
         if rc < 0:
             raise RuntimeError(f"bf_kernel_choice failed ({rc}): {self._lib.bf_last_error().decode()}")
         return {1: "quad", 2: "board", 3: "twin", 4: "octo", 5: "duo"}[rc]
 
     def launch_form(self, n: int) -> str:
-        """:meth:`kernel_choice`, with "team" for launches that go to the form that spreads a position over several
-        compute units (the smallest ones, without taps and profile) and "duo" for those with two positions per
-        workgroup (of kernel="auto", all of more than 256 positions)."""
-        if n > self._pair_above:
-            return "duo"
-        kind = self.kernel_choice(n)
-        if kind != "octo" or not self._team_bytes:
-            return kind
-        most = self._team_bytes // int(self._lib.bf_team_position_bytes(C.byref(self._shape)))
-        return "team" if n <= most * (2 if self.d_model != self.D else 1) else kind
+        """What runs in a ``forward_full`` of ``n`` positions (``bf_launch_form``): one of the kernels' names; of
+        kernel="auto" also "team", the form that spreads a position over several compute units (the smallest launches, without
+        taps and profile), and "wide", the 512-wide network's with two positions per workgroup (above 256).  A last round
+        that goes to another form does not count."""
+        a = self._choice_args(n)
+        if self._team_bytes:
+            a.team_workspace, a.team_workspace_bytes = 256, self._team_bytes    # tested for NULL and size
+        with torch.cuda.device(self.device):     # what may be a team depends on the device
+            rc = self._lib.bf_launch_form(C.byref(a))
+        if rc < 0:
+            raise RuntimeError(f"bf_launch_form failed ({rc}): {self._lib.bf_last_error().decode()}")
+        return {1: "quad", 2: "board", 3: "twin", 4: "octo", 5: "duo", 6: "team", 7: "wide"}[rc]
 
     def forward_expand(self, boards, control, rep, mask=None, max_edges: int = 96, active=None, out=None, leaves=None):
         """``forward_full`` followed on the same stream by the search's expand step
@@ -1154,8 +1160,9 @@ class FusedEncoder:
 
     def _launch_waves(self, n: int) -> int:
         """Wavefronts in a launch of ``n`` positions of the kernel such a call runs."""
-        kind = "duo" if n > self._pair_above else self.kernel_choice(n)
-        return {"board": 4 * n, "twin": 4 * n, "octo": 8 * n, "duo": 8 * ((n + 1) // 2), "quad": 4 * ((n + 3) // 4)}[kind]
+        pairs = 8 * ((n + 1) // 2)
+        return {"board": 4 * n, "twin": 4 * n, "octo": 8 * n, "team": 8 * n, "duo": pairs, "wide": pairs,
+                "quad": 4 * ((n + 3) // 4)}[self.launch_form(n)]     # the profile of a "team" launch is the "octo" kernel's
 
     def profile_phase_names(self):
         """Names of the counters of :meth:`read_profile`, in order (reference csrc/encoder.cu:1910)."""

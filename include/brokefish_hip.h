@@ -60,8 +60,7 @@ enum bf_quant {
  * runs in int8 and e4m3 on all four; the 512-wide network in int8 on OCTO and BOARD.  Kernels that
  * carry a network and a format return bit-identical results for it, so AUTO may pick by batch
  * size: OCTO up to 256 positions, above that two positions per workgroup: DUO, and a form of its own for the
- * 512-wide network (bf_kernel_choice still answers TWIN for e4m3 and OCTO for that network, whose
- * launches these were).  They run in rounds of 512 positions; when AUTO has chosen them and the last round
+ * 512-wide network (bf_launch_form tells).  They run in rounds of 512 positions; when AUTO has chosen them and the last round
  * would hold at most 256 positions, those are given to the one-position form in a second launch on the
  * same stream. */
 enum bf_kernel {
@@ -275,10 +274,24 @@ uint64_t bf_abi_tag(void);
 
 /* Largest n for which AUTO gives a workgroup one position. */
 int64_t bf_board_max_n(void);
-/* The kernel AUTO would run for these arguments (enum bf_kernel), or a negative bf_status.  The form that spreads a
- * position over several compute units (team_workspace) counts as OCTO, whose launches it takes; DUO's e4m3 launches
- * count as TWIN, those of the 512-wide network with two positions per workgroup as OCTO, whose they were. */
+/* The kernel these arguments name or, for AUTO, the one whose launches they are (enum bf_kernel), or a negative bf_status.
+ * AUTO has handed some of those launches on to forms that return the same bits faster, and the answer does not tell:
+ * bf_launch_form does. */
 int bf_kernel_choice(const bf_eval_args* args);
+/* What runs for these arguments: the kernels by their enum bf_kernel numbers and, of AUTO only, the form that spreads a position
+ * over several compute units (needs team_workspace) and the 512-wide network's with two positions per workgroup.  A launch whose
+ * last round is given to another form counts as that of its whole rounds; bf_profile_phases never runs TEAM, but OCTO
+ * in its place.  Or a negative bf_status. */
+enum bf_form {
+    BF_FORM_QUAD = BF_KERNEL_QUAD,
+    BF_FORM_BOARD = BF_KERNEL_BOARD,
+    BF_FORM_TWIN = BF_KERNEL_TWIN,
+    BF_FORM_OCTO = BF_KERNEL_OCTO,
+    BF_FORM_DUO = BF_KERNEL_DUO,
+    BF_FORM_TEAM = 6,
+    BF_FORM_WIDE = 7
+};
+int bf_launch_form(const bf_eval_args* args);
 
 /* The evaluator.  Replaces model_forward of the reference extension
  * (reference csrc/encoder.cu:1770-1876, bound at :1918-1925; called from

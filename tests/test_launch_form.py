@@ -1,0 +1,67 @@
+"""bf_launch_form: what runs for given arguments, where the answer of bf_kernel_choice names the kernel whose launches those
+are.  The library answers without a device; the forms' outputs are held against one another in the GPU tests."""
+import ctypes
+import importlib.util
+import os
+import re
+
+import pytest
+
+from brokefish_amd import hip_impl
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+QUAD, BOARD, TWIN, OCTO, DUO, TEAM, WIDE = range(1, 8)
+BASE, BIG = (256, 8, 8, 1024), (512, 16, 16, 2048)
+
+
+def args(shape, n, quant=0, kernel=0):
+    a = hip_impl._Args()
+    d, layers, heads, f = shape
+    a.shape = hip_impl._Shape(d, layers, heads, f, 1, 1e-5)
+    a.board_wstream = a.board_fparams = 16                     # only tested for NULL
+    a.n, a.quant, a.kernel = n, quant, kernel
+    return a
+
+
+def form(a):
+    return hip_impl.load_library().bf_launch_form(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("shape,quant,small,large", [(BASE, 0, OCTO, DUO), (BASE, 1, OCTO, DUO), (BIG, 0, OCTO, WIDE)])
+def test_auto_by_size(shape, quant, small, large):
+    for n, want in ((1, small), (256, small), (257, large), (512, large), (513, large), (16384, large)):
+        assert form(args(shape, n, quant)) == want
+
+
+@pytest.mark.parametrize("shape,quant,kernels", [(BASE, 0, (BOARD, TWIN, OCTO, DUO)), (BASE, 1, (BOARD, TWIN, OCTO, DUO)), (BIG, 0, (BOARD, OCTO))])
+def test_a_kernel_asked_for_by_name_runs(shape, quant, kernels):
+    for kernel in kernels:
+        for n in (1, 300, 4096):
+            assert form(args(shape, n, quant, kernel)) == kernel
+
+
+def test_the_taps_of_the_wide_network_are_the_one_position_forms():
+    a = args(BIG, 4096)
+    taps = hip_impl._Taps()
+    taps.resid = 16
+    a.taps = ctypes.pointer(taps)
+    assert form(a) == OCTO
+    taps.resid, taps.alive = None, 16                          # the stack alone: a build of every form AUTO takes
+    assert form(a) == WIDE
+
+
+def test_refused_arguments():
+    assert form(args((384, 8, 12, 1536), 4)) == -2
+    assert form(args(BIG, 4, quant=1)) < 0 and form(args(BASE, 4, kernel=7)) == -1
+    assert hip_impl.load_library().bf_launch_form(None) == -1
+
+
+def test_the_traffic_of_the_two_position_forms_is_quoted_from_their_profiles():
+    spec = importlib.util.spec_from_file_location("bench_module", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    where = {("base", "duo", 4096, "e4m3"): "duo_kernel_e4m3_batch4096.md", ("stress", "wide", 16384, "int8"): "wide_kernel_512_int8_batch16384.md"}
+    assert set(where) == set(bench.MEASURED_TRAFFIC_BYTES_PAIRS)
+    for key, name in where.items():
+        text = open(os.path.join(ROOT, "profiles", name)).read()
+        assert bench.MEASURED_TRAFFIC_BYTES_PAIRS[key] in {float(x) for x in re.findall(r"\d+(?:\.\d+)?e\d+", text)}, key
