@@ -176,11 +176,12 @@ hipError_t launch_duo256_fp8_taps(const KArgs& k, hipStream_t stream);
 hipError_t launch_wide512(const KArgs& k, hipStream_t stream);
 hipError_t launch_wide512_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_wide512_prof(const KArgs& k, hipStream_t stream);
-// the encoder-only builds of the kernels AUTO chooses from
+// the encoder-only builds
 hipError_t launch_duo256_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_fp8_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_fp8_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_twin256_fp8_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_octo512_enc(const KArgs& k, hipStream_t stream);
 // the builds that carry the phase profile
 hipError_t launch_twin256_prof(const KArgs& k, hipStream_t stream);

@@ -154,14 +154,14 @@ static int choose_kernel(const bf_eval_args* a) {
 extern "C" int bf_kernel_choice(const bf_eval_args* args) { return choose_kernel(args); }
 
 // Whether the encoder-only build of kernel `kind` serves this launch: nothing but the stream is tapped, and the
-// kernel is one of those AUTO chooses from (the others run their taps build, whose every phase tests for taps).
+// kernel is one that AUTO chooses from, or TWIN in e4m3, which AUTO chose before DUO carried that format (the others run
+// their taps build, whose every phase tests for taps).
 static bool enc_build(const bf_eval_args* a, int kind) {
     const bf_taps* t = a->taps;
     if (!t || !t->alive || t->embed || t->qa_qkv || t->acc_qkv || t->qa_out || t->acc_out || t->qa_ff1 || t->acc_ff1 || t->qa_ff2 ||
         t->acc_ff2 || t->resid || t->normed)
         return false;
     if (a->shape.d_model == 512) return kind == BF_KERNEL_OCTO;
-    // TWIN in e4m3: the two-position build serves it (same bits)
     return kind == BF_KERNEL_OCTO || kind == BF_KERNEL_DUO || (kind == BF_KERNEL_TWIN && a->quant == BF_QUANT_E4M3);
 }
 
@@ -376,7 +376,8 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
                         : (enc ? bf::launch_solo256_enc : bf::launch_solo256))(back, stream);
     } else if (enc) {
         if (wide) e = bf::launch_octo512_enc(k, stream);
-        else if (a->quant == BF_QUANT_E4M3) e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_fp8_enc : bf::launch_duo256_fp8_enc)(k, stream);
+        else if (a->quant == BF_QUANT_E4M3)
+            e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_fp8_enc : kind == BF_KERNEL_TWIN ? bf::launch_twin256_fp8_enc : bf::launch_duo256_fp8_enc)(k, stream);
         else e = (kind == BF_KERNEL_OCTO ? bf::launch_solo256_enc : bf::launch_duo256_enc)(k, stream);
     } else if (kind == BF_KERNEL_OCTO) {
         // eight wavefronts per position: the 512-wide network on the board kernel's eight-wavefront form; the

@@ -1,9 +1,11 @@
 """The encoder-only builds (half-precision stream in and out, split last round) against the taps builds of the
 other kernels, bit for bit."""
+import ctypes
+
 import pytest
 import torch
 
-from brokefish_amd import encoder_impl
+from brokefish_amd import encoder_impl, hip_impl
 from brokefish_amd.net import BrokefishNet
 
 pytestmark = pytest.mark.gpu
@@ -32,3 +34,20 @@ def test_encoder_only_builds_return_the_bits_of_the_taps_builds(wide, fmt, other
         assert model.forward(xh, alive, out=xh) is xh and torch.equal(xh, want.half()), n     # in place
     xb = (0.2 * torch.randn(5, 32, d, device="cuda")).bfloat16()
     assert torch.equal(model.forward(xb), ref.forward(xb.float()).bfloat16())                 # a type with passes of its own
+
+
+@pytest.mark.parametrize("kernel", ["twin", "octo", "duo"])
+def test_a_kernel_asked_for_by_name_takes_a_half_precision_stream_in_e4m3(kernel):
+    torch.manual_seed(0)
+    net = BrokefishNet(n_layers=3).eval().randomise_layers_(seed=4)
+    model, ref = encoder_impl("hip")(net, fp8=True, kernel=kernel), encoder_impl("hip")(net, fp8=True, kernel="board")
+    assert hasattr(model._lib, f"_ZN2bf{len('launch_twin256_fp8_enc')}launch_twin256_fp8_encERKNS_5KArgsEP12ihipStream_t")
+    for n in (1, 2, 300, 513):
+        x = 0.2 * torch.randn(n, 32, 256, device="cuda").half()
+        alive = (torch.rand(n, 32, device="cuda") < 0.8).to(torch.int8)
+        want = ref.forward(x.float(), alive).half()
+        taps, a, got = hip_impl._Taps(), model._choice_args(n), torch.empty_like(x)
+        taps.alive, taps.x_in_h, taps.resid_last_h = alive.data_ptr(), x.data_ptr(), got.data_ptr()
+        a.board_wstream, a.board_fparams, a.taps = model.board_wstream.data_ptr(), model.board_fparams.data_ptr(), ctypes.pointer(taps)
+        model._call(a)
+        assert torch.equal(got, want), n
