@@ -165,11 +165,21 @@ static bool enc_build(const bf_eval_args* a, int kind) {
     return kind == BF_KERNEL_OCTO || kind == BF_KERNEL_DUO || (kind == BF_KERNEL_TWIN && a->quant == BF_QUANT_E4M3);
 }
 
+// Whether AUTO keeps this launch on one position per workgroup (e4m3: TWIN; 512 wide: OCTO) where it would pair them: flags
+// without a list.  A workgroup of one position leaves when its flag is 0; a pair of neighbours runs when either is live.
+// 4000 flags, scattered, of which 5 % / a third / two thirds / all are set: e4m3 281 / 986 / 1693 / 2174 us against 476 /
+// 1616 / 1891 / 1959 of pairs, 512 wide 1.45 / 5.67 / 9.99 / 12.1 ms against 2.04 / 7.54 / 9.14 / 9.50: flags are there for
+// the launches of which most is not live.  int8 of the 256-wide network: 356 / 1227 / 1503 / 1481 us in pairs, which
+// AUTO has given it since it has had them; as a list 129 / 561 / 1098 / 1537.
+static bool unpaired(const bf_eval_args* a) {
+    return a->active && (a->quant == BF_QUANT_E4M3 || a->shape.d_model == 512);
+}
+
 // What AUTO makes of choose_kernel()'s answer: TWIN's launches are the two-position kernel's (same bits; e4m3, 4096
 // positions: 2142 -> 1962 us).
 static int run_kernel(const bf_eval_args* a) {
     const int kind = choose_kernel(a);
-    return a && a->kernel == BF_KERNEL_AUTO && kind == BF_KERNEL_TWIN ? BF_KERNEL_DUO : kind;
+    return a && a->kernel == BF_KERNEL_AUTO && kind == BF_KERNEL_TWIN && !unpaired(a) ? BF_KERNEL_DUO : kind;
 }
 
 static int check_args(const bf_eval_args* a, bf::KArgs* k, int* kind) {
@@ -311,7 +321,7 @@ struct Route {
     }
 };
 static Route route(const bf_eval_args* a, int kind, bool profile) {
-    const bool wide = a->shape.d_model == 512, pairs = a->kernel == BF_KERNEL_AUTO && a->n > kBoardMaxN && (wide || kind == BF_KERNEL_DUO);
+    const bool wide = a->shape.d_model == 512, pairs = a->kernel == BF_KERNEL_AUTO && a->n > kBoardMaxN && (wide ? !unpaired(a) : kind == BF_KERNEL_DUO);
     Route r;
     r.enc = !profile && enc_build(a, kind);
     r.team = team_limit(a, profile, r.enc);

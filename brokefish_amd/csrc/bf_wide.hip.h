@@ -104,9 +104,9 @@ __global__ __launch_bounds__(512, 1) void wide_kernel(const KArgs a) {
     const int tile0 = TW * q + TWW * sub, t0 = TWW * sub;   // first tile of the width; within the quarter
     const int t = lane & 31, g = lane >> 5;
 
-    // the positions of this workgroup: its two slots of the launch, or those entries of the compacted leaf list.  A slot
-    // without a position computes its neighbour's again and stores nothing; a workgroup without any leaves before the
-    // first barrier.
+    // the positions of this workgroup: its two slots of the launch, or those entries of the compacted leaf list (flags
+    // without a list go to the one-position form).  A slot without a position computes its neighbour's again and stores
+    // nothing; a workgroup without any leaves before the first barrier.
     int bp[NP];
     bool live[NP];
     {
@@ -126,7 +126,6 @@ __global__ __launch_bounds__(512, 1) void wide_kernel(const KArgs a) {
                 b = ok ? __builtin_amdgcn_readfirstlane(a.leaf_index[j]) : 0;
                 ok = ok && (unsigned)b < (unsigned)a.n;
             }
-            if (ok && a.active) ok = a.active[b] != 0;
             bp[p] = ok ? b : 0;
             live[p] = ok;
             if (ok) { any = true; some = b; }

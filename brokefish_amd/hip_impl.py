@@ -955,12 +955,14 @@ class FusedEncoder:
             raise RuntimeError(f"bf_kernel_choice failed ({rc}): {self._lib.bf_last_error().decode()}")
         return {1: "quad", 2: "board", 3: "twin", 4: "octo", 5: "duo"}[rc]
 
-    def launch_form(self, n: int) -> str:
-        """What runs in a ``forward_full`` of ``n`` positions (``bf_launch_form``): one of the kernels' names; of
+    def launch_form(self, n: int, flags: bool = False) -> str:
+        """What runs in a launch of ``n`` positions (``bf_launch_form``): one of the kernels' names; of
         kernel="auto" also "team", the form that spreads a position over several compute units (the smallest launches, without
         taps and profile), and "wide", the 512-wide network's with two positions per workgroup (above 256).  A last round
-        that goes to another form does not count."""
+        that goes to another form does not count.  ``flags``: with ``active`` flags that are passed on to the library as they
+        are (:meth:`forward_full` compacts them above 256 positions)."""
         a = self._choice_args(n)
+        a.active = 256 if flags else None                                       # only tested for NULL
         if self._team_bytes:
             a.team_workspace, a.team_workspace_bytes = 256, self._team_bytes    # tested for NULL and size
         with torch.cuda.device(self.device):     # what may be a team depends on the device
@@ -1113,7 +1115,7 @@ class FusedEncoder:
                                                  C.c_void_p(self._profile.data_ptr()))
             if rc:
                 raise RuntimeError(f"bf_profile_phases failed ({rc}): {self._lib.bf_last_error().decode()}")
-            self._profile_waves += self._launch_waves(n)
+            self._profile_waves += self._launch_waves(n, active is not None)
         elif self.binding == "torch":
             for name, t in (("boards", boards), ("control", control), ("rep", rep), ("mask", mask), ("active", active)):
                 if t is not None and t.device != self.device:
@@ -1158,11 +1160,11 @@ class FusedEncoder:
             raise RuntimeError(f"bf_time_kernel_ms failed ({ms}): {self._lib.bf_last_error().decode()}")
         return ms
 
-    def _launch_waves(self, n: int) -> int:
+    def _launch_waves(self, n: int, flags: bool = False) -> int:
         """Wavefronts in a launch of ``n`` positions of the kernel such a call runs."""
         pairs = 8 * ((n + 1) // 2)
         return {"board": 4 * n, "twin": 4 * n, "octo": 8 * n, "team": 8 * n, "duo": pairs, "wide": pairs,
-                "quad": 4 * ((n + 3) // 4)}[self.launch_form(n)]     # the profile of a "team" launch is the "octo" kernel's
+                "quad": 4 * ((n + 3) // 4)}[self.launch_form(n, flags)]     # the profile of a "team" launch is the "octo" kernel's
 
     def profile_phase_names(self):
         """Names of the counters of :meth:`read_profile`, in order (reference csrc/encoder.cu:1910)."""

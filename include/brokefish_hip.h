@@ -222,9 +222,12 @@ typedef struct {
     const float* board_fparams;
     /* optional [n] uint8: positions with 0 are skipped and their outputs left untouched -- the
      * flat leaf staging of the reference's search (brokefish/search/cuda_impl.py:137-145:
-     * leaf_board / leaf_control / leaf_rep / leaf_flags) evaluated without compaction and without
-     * paying for the leaves that need no evaluation (BOARD / TWIN: the workgroup exits at once;
-     * QUAD: the wavefront runs on, storing nothing) */
+     * leaf_board / leaf_control / leaf_rep / leaf_flags) evaluated without compaction.  Forms with one position
+     * per workgroup do not pay for the leaves that need no evaluation (their workgroups exit at once); DUO pays for
+     * one whose neighbour (2 i, 2 i + 1) is live, QUAD for one in a workgroup with a live one.  AUTO gives launches
+     * with flags to one position per workgroup in e4m3 (above 256 positions: TWIN) and for the 512-wide network
+     * (OCTO), int8 of the 256-wide one above 256 positions to DUO.  A list (below) costs less than flags wherever a
+     * good part of the leaves is not live. */
     const uint8_t* active;
     int32_t kernel;         /* enum bf_kernel; AUTO with the board blobs: OCTO for
                              * n <= bf_board_max_n(), above that two positions per workgroup

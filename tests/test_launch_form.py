@@ -50,6 +50,16 @@ def test_the_taps_of_the_wide_network_are_the_one_position_forms():
     assert form(a) == WIDE
 
 
+@pytest.mark.parametrize("shape,quant,want", [(BASE, 0, DUO), (BASE, 1, TWIN), (BIG, 0, OCTO)])
+def test_flags_without_a_list_are_not_paired_where_a_pair_costs_more(shape, quant, want):
+    for n in (257, 512, 4096):
+        a = args(shape, n, quant)
+        a.active = 16
+        assert form(a) == want
+        a.active, a.leaf_index, a.leaf_count = None, 16, 16        # a list: pairs of live ones
+        assert form(a) in (DUO, WIDE)
+
+
 def test_refused_arguments():
     assert form(args((384, 8, 12, 1536), 4)) == -2
     assert form(args(BIG, 4, quant=1)) < 0 and form(args(BASE, 4, kernel=7)) == -1

@@ -49,6 +49,34 @@ def test_live_counts_at_the_edges_of_a_round(made, live):
             assert torch.equal(g[on], w[on]) and bool((g[~on] == 7.0).all()), how
 
 
+@pytest.mark.parametrize("profile", [False, True])
+@pytest.mark.parametrize("n,live", [(600, 0), (600, 1), (600, 200), (N, 430), (N, N)])
+def test_flags_passed_to_the_library_as_they_are(made, n, live, profile):
+    # FusedEncoder compacts flags above 256 positions; a C caller need not, and the profile does not
+    auto, batch, want = made
+    b, c, r, m = [t[:n] for t in batch]
+    flags = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    flags[torch.randperm(n, generator=torch.Generator().manual_seed(live))[:live].cuda()] = 3
+    on = flags != 0
+    auto.forward_masked(b, c, r, m)                            # the buffers exist
+    outs = (auto.policy_out, auto.promo_out, auto.value_out, auto.best_out)
+    for t in outs:
+        t.fill_(7)
+    if profile:
+        auto.set_profile(True)
+        try:
+            auto.forward_full(b, c, r, m, active=flags)
+        finally:
+            cycles, waves = auto.read_profile()
+            auto.set_profile(False)
+            auto.reset_profile()
+        assert waves == (4 if auto.fp8 else 8) * n and (int(cycles[-1]) > 0) == (live > 0)
+    else:
+        auto._call(auto._args(b, c, r, m, *outs, active=flags))
+    for g, w in zip(outs, want):
+        assert torch.equal(g[on], w[:n][on]) and bool((g[~on] == 7).all())
+
+
 @pytest.mark.parametrize("head,n_value", [("pooled", 1), ("prenorm", 1), ("pooled", 3), ("king", 3)])
 def test_value_heads_of_the_wide_network(head, n_value):
     auto, board = _models(WIDE, "int8", value_head=head, n_value=n_value)
