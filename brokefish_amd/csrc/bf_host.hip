@@ -47,6 +47,13 @@ static size_t board_fparams_floats(int n_layers) {
     return (size_t)4 * n_layers * L::PW_FLOATS + L::GLOBAL_FLOATS;
 }
 
+// Whether the kernels that reach their weights by 32-bit offsets carry a network of this depth: DUO, its one-position form and
+// the 512-wide one with two positions, from the start of a quarter's stream (10,922 layers; 512 wide 2,730); the team form
+// from the start of all four (2,730; 682).  Deeper networks stay on BOARD, TWIN and, 512 wide, OCTO.
+static bool offsets_reach(const bf_shape* s, int quarters) {
+    return bf_board_wstream_bytes(s) / 4 * quarters <= 0x7fffffff;
+}
+
 extern "C" size_t bf_board_wstream_bytes(const bf_shape* s) {
     if (shape_ok(s)) return board_wstream_bytes<256>(s->n_layers);
     if (shape512(s)) return board_wstream_bytes<512>(s->n_layers);
@@ -116,8 +123,9 @@ static int choose_kernel(const bf_eval_args* a) {
     // the board blobs are packed for one format; the 512-wide network runs int8 only
     const bool board_can = have_board && (a->quant == BF_QUANT_INT8 || shape_ok(&a->shape));
     const bool twin_can = have_board && shape_ok(&a->shape);
-    const bool octo_can = board_can;   // the same networks and formats as BOARD
-    const bool duo_can = twin_can;     // the 256-wide network, both formats
+    const bool reach = offsets_reach(&a->shape, 1);
+    const bool octo_can = board_can && (reach || shape512(&a->shape));   // the same networks and formats as BOARD
+    const bool duo_can = twin_can && reach;                              // the 256-wide network, both formats
     switch (a->kernel) {
     case BF_KERNEL_QUAD:
         if (!quad_can) return fail(BF_ERR_UNSUPPORTED, "the four-positions-per-workgroup kernel needs the 256-wide network and wstream/fparams");
@@ -131,17 +139,18 @@ static int choose_kernel(const bf_eval_args* a) {
         return BF_KERNEL_TWIN;
     case BF_KERNEL_OCTO:
         if (!octo_can)
-            return fail(BF_ERR_UNSUPPORTED, "the eight-wavefronts-per-position kernel needs board_wstream/board_fparams (512-wide network: the int8 format)");
+            return fail(BF_ERR_UNSUPPORTED, "the eight-wavefronts-per-position kernel needs board_wstream/board_fparams (512-wide network: the int8 format; 256-wide: at most 10922 layers)");
         return BF_KERNEL_OCTO;
     case BF_KERNEL_DUO:
         if (!duo_can)
-            return fail(BF_ERR_UNSUPPORTED, "the two-positions-per-workgroup kernel needs the 256-wide network and board_wstream/board_fparams");
+            return fail(BF_ERR_UNSUPPORTED, "the two-positions-per-workgroup kernel needs the 256-wide network, of at most 10922 layers, and board_wstream/board_fparams");
         return BF_KERNEL_DUO;
     case BF_KERNEL_AUTO:
         // above one position per compute unit: two positions per workgroup (int8: 5 to 8 % faster than TWIN from 512
         // positions up and half its L2 traffic).  For e4m3 the answer is still TWIN, what AUTO ran before the two-position
         // kernel overtook it; run_kernel() gives those launches to DUO.
         if (octo_can) return (twin_can && a->n > kBoardMaxN) ? (a->quant == BF_QUANT_INT8 ? BF_KERNEL_DUO : BF_KERNEL_TWIN) : BF_KERNEL_OCTO;
+        if (board_can) return a->n > kBoardMaxN ? BF_KERNEL_TWIN : BF_KERNEL_BOARD;   // too deep for those
         if (quad_can) return BF_KERNEL_QUAD;
         return fail(BF_ERR_ARGUMENT, shape512(&a->shape)
                         ? "the 512-wide network runs on the one-position-per-workgroup kernel: int8, board_wstream/board_fparams required"
@@ -165,14 +174,14 @@ static bool enc_build(const bf_eval_args* a, int kind) {
     return kind == BF_KERNEL_OCTO || kind == BF_KERNEL_DUO || (kind == BF_KERNEL_TWIN && a->quant == BF_QUANT_E4M3);
 }
 
-// Whether AUTO keeps this launch on one position per workgroup (e4m3: TWIN; 512 wide: OCTO) where it would pair them: flags
-// without a list.  A workgroup of one position leaves when its flag is 0; a pair of neighbours runs when either is live.
+// Whether AUTO keeps this launch on one position per workgroup (256 wide: TWIN; 512 wide: OCTO) where it would pair them: too
+// many layers for the kernels that do, or (e4m3 and 512 wide) flags without a list.  A workgroup of one position leaves when its flag is 0; a pair of neighbours runs when either is live.
 // 4000 flags, scattered, of which 5 % / a third / two thirds / all are set: e4m3 281 / 986 / 1693 / 2174 us against 476 /
 // 1616 / 1891 / 1959 of pairs, 512 wide 1.45 / 5.67 / 9.99 / 12.1 ms against 2.04 / 7.54 / 9.14 / 9.50: flags are there for
 // the launches of which most is not live.  int8 of the 256-wide network: 356 / 1227 / 1503 / 1481 us in pairs, which
 // AUTO has given it since it has had them; as a list 129 / 561 / 1098 / 1537.
 static bool unpaired(const bf_eval_args* a) {
-    return a->active && (a->quant == BF_QUANT_E4M3 || a->shape.d_model == 512);
+    return !offsets_reach(&a->shape, 1) || (a->active && (a->quant == BF_QUANT_E4M3 || a->shape.d_model == 512));
 }
 
 // What AUTO makes of choose_kernel()'s answer: TWIN's launches are the two-position kernel's (same bits; e4m3, 4096
@@ -304,7 +313,7 @@ static bf::KArgs slice(const bf::KArgs& k, int d_model, int first, int count) {
 // Positions a team launch of this call may hold: 0 unless AUTO chose, a workspace came along and nothing but the
 // stream is tapped.
 static int team_limit(const bf_eval_args* a, bool profile, bool enc) {
-    if (a->kernel != BF_KERNEL_AUTO || !a->team_workspace || profile || (a->taps && !enc)) return 0;
+    if (a->kernel != BF_KERNEL_AUTO || !a->team_workspace || profile || (a->taps && !enc) || !offsets_reach(&a->shape, 4)) return 0;
     const size_t fits = a->team_workspace_bytes / bf::team_slot_bytes(a->shape.d_model);
     const int most = bf::team_positions(a->shape.d_model, false);
     return fits < (size_t)most ? (int)fits : most;

@@ -180,7 +180,8 @@ typedef struct {
                          * heads run -- boards, control, rep, mask, policy, promo and value of
                          * bf_eval_args are ignored and may be NULL */
     const void* x_in_h;  /* encoder-only launches of AUTO, with no other tap: the stream in fp16 instead of */
-    void* resid_last_h;  /* x_in, and the result in fp16 instead of resid_last (8-byte aligned)             */
+    void* resid_last_h;  /* x_in, and the result in fp16 instead of resid_last (8-byte aligned; where AUTO   */
+                         /* runs BOARD or int8 TWIN, above 10,922 layers, BF_ERR_UNSUPPORTED)              */
 } bf_taps;
 
 typedef struct {

@@ -60,6 +60,38 @@ def test_flags_without_a_list_are_not_paired_where_a_pair_costs_more(shape, quan
         assert form(a) in (DUO, WIDE)
 
 
+def deep(shape, layers):
+    return shape[:1] + (layers,) + shape[2:]
+
+
+@pytest.mark.parametrize("shape,quant,most,small,large,deep_small,deep_large", [
+    (BASE, 0, 10922, OCTO, DUO, BOARD, TWIN), (BASE, 1, 10922, OCTO, DUO, BOARD, TWIN), (BIG, 0, 2730, OCTO, WIDE, OCTO, OCTO)])
+def test_networks_too_deep_for_32_bit_offsets(shape, quant, most, small, large, deep_small, deep_large):
+    lib = hip_impl.load_library()
+    for layers in (most, most + 1, 2 ** 28, 2 ** 31 - 1):
+        fits = layers == most
+        s = args(deep(shape, layers), 1).shape
+        assert (lib.bf_board_wstream_bytes(ctypes.byref(s)) // 4 < 2 ** 31) == fits      # a quarter's stream
+        for n in (1, 256, 257, 4096):
+            want = (small if n <= 256 else large) if fits else (deep_small if n <= 256 else deep_large)
+            assert form(args(deep(shape, layers), n, quant)) == want
+        if shape is BASE:
+            for kernel in (OCTO, DUO):
+                assert form(args(deep(shape, layers), 300, quant, kernel)) == (kernel if fits else -2)
+            for kernel in (BOARD, TWIN):
+                assert form(args(deep(shape, layers), 300, quant, kernel)) == kernel
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,most,other", [(BASE, 2730, OCTO), (BIG, 682, OCTO)])
+def test_teams_reach_all_four_quarters_by_32_bit_offsets(shape, most, other):
+    lib = hip_impl.load_library()
+    for layers, want in ((most, TEAM), (most + 1, other)):
+        a = args(deep(shape, layers), 8)
+        a.team_workspace, a.team_workspace_bytes = 256, lib.bf_team_workspace_bytes(ctypes.byref(a.shape))
+        assert a.team_workspace_bytes and form(a) == want
+
+
 def test_refused_arguments():
     assert form(args((384, 8, 12, 1536), 4)) == -2
     assert form(args(BIG, 4, quant=1)) < 0 and form(args(BASE, 4, kernel=7)) == -1
