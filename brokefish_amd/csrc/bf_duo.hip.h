@@ -562,8 +562,9 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         // (2^23 + a) 2^-149: up to 2^24 the bits of subnormal and smallest normal floats count linearly.  One fused operation takes
         // the offset off and multiplies: with s = m 2^e, fma(x, m 2^126, -m) = fl(a m) 2^-23, exactly rounded as fl(a s) is, and
         // 2^(e + 23) goes into w (ldexp, once a tile).  That takes the place of a conversion, 4.4 clocks, and a product: 4096
-        // positions 1481 -> 1463 us, 200 positions 115.2 -> 113.6, same bits (for s w below 2^104, where such a matmul's
-        // results reach a float's range; rows without a largest value, NaN, stay NaN).
+        // positions 1481 -> 1463 us, 200 positions 115.2 -> 113.6, same bits for 2^-149 <= s w < 2^104:
+        // above, w 2^(e + 23) overflows (infinite results, and NaN for a = 0) though fl(fl(a s) w) may be finite yet; below, it
+        // loses bits to the subnormal range.  Rows without a largest value, NaN, stay NaN.
         auto descale = [&](const acc_t& ac, int e, float s, float off, float w) -> float {
             if constexpr (SUBN) return __builtin_fmaf(__int_as_float(accbits(ac, e)), s, off) * w;
             else return accf(ac, e) * s * w;

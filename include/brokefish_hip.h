@@ -58,7 +58,7 @@ enum bf_quant {
  *          L2 serves two positions (256-wide network, int8 and e4m3).
  * BOARD, TWIN, OCTO and DUO read the same blobs (board_wstream / board_fparams).  The 256-wide network
  * runs in int8 and e4m3 on all four; the 512-wide network in int8 on OCTO and BOARD.  Kernels that
- * carry a network and a format return bit-identical results for it, so AUTO may pick by batch
+ * carry a network and a format return bit-identical results for it (in the range given at bf_shape), so AUTO may pick by batch
  * size: OCTO up to 256 positions, above that two positions per workgroup: DUO, and a form of its own for the
  * 512-wide network (bf_launch_form tells).  They run in rounds of 512 positions; when AUTO has chosen them and the last round
  * would hold at most 256 positions, those are given to the one-position form in a second launch on the
@@ -85,11 +85,15 @@ enum bf_value_mode {
 #define BF_PROMO 4
 
 /* Network shape.  Supported: d_model 256, n_heads 8, d_ff 1024 (all kernels, int8 and e4m3)
- * and d_model 512, n_heads 16, d_ff 2048 (BOARD kernel, int8); head width 32, any
- * n_layers >= 1, n_value 1 (tanh scalar) or 3 (loss/draw/win classes).
+ * and d_model 512, n_heads 16, d_ff 2048 (BOARD and OCTO kernels, int8); head width 32, any
+ * n_layers >= 1, n_value 1 (tanh scalar) or 3 (loss/draw/win classes).  DUO and, of the 256-wide network, OCTO carry up to
+ * 10,922 layers; AUTO gives deeper networks (512 wide: above 2,730) to BOARD, TWIN and OCTO at any size.
  * Range of the arithmetic: a row to be quantised whose largest magnitude is below 2^-118 counts as zero, up to
- * 2^108 rows are quantised exactly as stated (beyond, a value that lies on a tie may go either way); LayerNorm's
- * variance + eps is exact from 2^-102 on (eps = 0 is accepted, a constant row then gives NaN), and a row whose
+ * 2^108 (e4m3 2^105, its hidden rows 2^102) rows are quantised exactly as stated (beyond, a value that lies on a tie may go
+ * either way).  int8 of the 256-wide network on DUO and OCTO: a row's scale times a weight block's lies between 2^-149 and 2^104
+ * (largest magnitude / 127 each); above, results of these two become infinite or NaN that other kernels still return finite,
+ * below, they differ in their subnormal bits.  LayerNorm's variance + eps is exact from 2^-102 on (eps = 0 is accepted, a
+ * constant row then gives NaN), and a row whose
  * squares overflow normalises to beta. */
 typedef struct {
     int32_t d_model, n_layers, n_heads, d_ff, n_value;
