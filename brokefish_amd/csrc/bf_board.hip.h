@@ -60,19 +60,13 @@
 #define BF_FORCE_ACTL 0
 #endif
 
-// Timing experiments (BF_EXP_*): compile-time switches that replace a part of a kernel by a
-// cheaper stand-in to measure what that part costs.  Their results are wrong by construction, so
-// they compile only together with BF_TIMING_BUILD, which the library's own build never defines
-// (brokefish_amd/_build.py refuses both).
+// What a part of a kernel costs is measured on copies of these sources, in which a cheaper stand-in takes its place.  The switches
+// that such copies have had are refused by name: no build of the library can ask for one and go on without it.
 #if (defined(BF_EXP_NOF32) || defined(BF_EXP_NOMFMA) || defined(BF_EXP_SAMEBLOCK) || defined(BF_EXP_NOLOAD) || \
-     defined(BF_EXP_HALFLOAD) || defined(BF_EXP_NOBARRIER) || defined(BF_EXP_SAMELAYER) || defined(BF_EXP_NOWARM)) && !defined(BF_TIMING_BUILD)
-#error "BF_EXP_* switches give wrong results: they need BF_TIMING_BUILD and never go into the library"
+     defined(BF_EXP_HALFLOAD) || defined(BF_EXP_NOBARRIER) || defined(BF_EXP_SAMELAYER) || defined(BF_EXP_NOWARM))
+#error "BF_EXP_* switches give wrong results: they are no part of these sources"
 #endif
-#ifdef BF_EXP_NOF32   // timing experiment: one vector instruction in place of an fp32 matrix step
-#define BF_F32MMA(a_, b_, c_) ([&]() { v16f r_ = (c_); r_[0] = __builtin_fmaf((a_), (b_), r_[0]); return r_; }())
-#else
 #define BF_F32MMA(a_, b_, c_) __builtin_amdgcn_mfma_f32_32x32x2f32((a_), (b_), (c_), 0, 0, 0)
-#endif
 
 namespace bf {
 namespace board {
@@ -137,11 +131,6 @@ __device__ __forceinline__ void dma(const float* src, float* dst, int nfloats, i
 // one 16-byte fragment step of a block product: a 32-deep int8 MFMA, or two 16-deep e4m3 steps
 template <bool SWAP>
 __device__ __forceinline__ v16i frag_mma(const v4i& w, const v4i& act, const v16i& acc) {
-#ifdef BF_EXP_NOMFMA   // timing experiment: one vector instruction in place of the product
-    v16i r = acc;
-    r[0] += w[0] ^ act[0];
-    return r;
-#endif
     return SWAP ? __builtin_amdgcn_mfma_i32_32x32x32_i8(act, w, acc, 0, 0, 0)
                 : __builtin_amdgcn_mfma_i32_32x32x32_i8(w, act, acc, 0, 0, 0);
 }
@@ -333,25 +322,9 @@ __global__ __launch_bounds__(OCTO ? 2 * THREADS : THREADS, TWIN && !OCTO ? BF_TW
     // TWIN: half-block `hseq` of this wave's stream (consumption order) into register set `set`
     v4i frt[NSETS][4];
     auto load_half = [&](int hseq, int set) {
-#ifdef BF_EXP_SAMEBLOCK   // timing experiment: every weight load hits the same 4 KiB (L1 hits)
-        const uint8_t* src = wsrc + (size_t)(hseq & 1) * HALF;
-#else
         const uint8_t* src = wsrc + (size_t)hseq * HALF;
-#endif
-#ifdef BF_EXP_NOLOAD   // timing experiment: no weight traffic
-        (void)src;
-#pragma unroll
-        for (int s = 0; s < 4; s++) asm volatile("" : "=v"(frt[set][s]));
-#elif defined(BF_EXP_HALFLOAD)   // timing experiment: half of the weight traffic
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            if (s & 1) asm volatile("" : "=v"(frt[set][s]));
-            else frt[set][s] = *reinterpret_cast<const v4i*>(src + s * FRAG);
-        }
-#else
 #pragma unroll
         for (int s = 0; s < 4; s++) frt[set][s] = *reinterpret_cast<const v4i*>(src + s * FRAG);
-#endif
     };
     // the wave's hh-th half-block of the layer whose stream starts at block `base` (hh may run into
     // the following layer, whose stream starts at block `next`) into its register set

@@ -176,11 +176,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             lds_barrier();
             t_sync += __builtin_readcyclecounter() - t0_;
         } else {
-#ifdef BF_EXP_NOBARRIER   // timing experiment: no workgroup barriers (results are wrong)
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#else
             lds_barrier();
-#endif
         }
     };
 
@@ -241,17 +237,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     // quarter's stream into place `at`.
     v4i frt[RING];
     auto load_frag = [&](int fseq, int at) {
-#ifdef BF_EXP_SAMEBLOCK   // timing experiment: every load reads the wave's first half-block (an L1 hit)
-        const int src = (fseq & 3) * FRAG;
-#else
         const int src = fseq * FRAG;
-#endif
-#ifdef BF_EXP_NOLOAD   // timing experiment: no weight traffic
-        (void)src;
-        asm volatile("" : "=v"(frt[at]));
-#else
         frt[at] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane16, src, 0));
-#endif
     };
     // the wave's ff-th fragment of the layer whose stream starts at block `base` (ff may run into the following layer,
     // whose stream starts at block `next`)
@@ -269,11 +256,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     // touches (workgroups that left early, another dispatch order) costs time, not correctness.
     // Below four workgroups per XCD the touches cover too little to pay for the loads they delay
     // (loads return in order), above one workgroup per compute unit the launch is not in step.
-#ifdef BF_EXP_NOWARM   // timing experiment: no warm-up touches (results stay right)
-    constexpr int WARM = 0;
-#else
     constexpr int WARM = NP == 1 ? 2 : 0;
-#endif
     constexpr int LAYER_LINES = BPW * BLOCK / 128;   // per quarter
     int warm[WARM > 0 ? WARM : 1] = {};
     auto warm_l2 = [&](int blk0) {
@@ -489,11 +472,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #pragma unroll
         for (int p = 0; p < NP; p++) bl[p] = (size_t)bp[p] * nl_run + li;
         const int lnext = l + 1 < a.l1 ? l + 1 : l;   // after the last layer the same layer is fetched again (and never used)
-#ifdef BF_EXP_SAMELAYER   // timing experiment: every layer streams the first layer's blocks (they stay in L2)
-        const int lbase = 0 * li, lfollow = 0 * lnext;
-#else
         const int lbase = li * BPW, lfollow = (lnext - a.l0) * BPW;
-#endif
         // One position's product with the wave's k-th block of this layer: eight 32-deep steps against
         // the operand row whose fragment 0 is at BSRC (lane offset included), each fragment fetched
         // from LDS one step ahead.  The last position refills a fragment's place in the ring as soon as it has

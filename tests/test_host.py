@@ -138,8 +138,8 @@ def test_kernel_choice_follows_shape_blobs_and_batch_size():
 
 
 def test_timing_experiments_cannot_reach_the_library():
-    """The kernels' BF_EXP_* switches give wrong results by construction: the build refuses them,
-    and the sources refuse to compile them without BF_TIMING_BUILD."""
+    """The BF_EXP_* switches of timing copies give wrong results by construction: the build refuses them,
+    and the sources, which hold none any more, refuse to compile under their names."""
     from brokefish_amd import _build
     assert not any("BF_EXP" in f or "BF_TIMING" in f for f in _build.HIPCC_FLAGS)
     for extra in (["-DBF_EXP_NOLOAD"], ["-DBF_TIMING_BUILD"]):
