@@ -21,7 +21,7 @@
 // runs).  Integer work, bound by the vector ALU: one wavefront per position (its boards built on the
 // scalar unit, each of some 31 moves replayed) took 119 us for 65536 positions, this 24 us, with the squares'
 // diagonals, knight's and king's steps looked up (651 vector instructions a wavefront, by counter) 19 us, and with
-// three-operand logic, sums for differences and pawns' squares from the king's steps (634) 17 us (1.25 TB/s of its
+// three-operand logic, sums for differences and pawns' squares from the king's steps (547) 17 us (1.25 TB/s of its
 // bytes).
 #include <hip/hip_runtime.h>
 

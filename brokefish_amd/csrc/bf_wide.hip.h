@@ -19,8 +19,8 @@
 //
 // What bounds it: a layer is 144,000 clocks of a SIMD, of which its two wavefronts' vector work is some 75,000 (the float64
 // sums of two chunks alone 27,000: six instructions an element), fp32 matrix steps 16,500, int8 ones 50,000 less what runs
-// under them, and fifteen exchanges some 15,000.  1500 positions: 4346 us with one position per workgroup, 3287.  The 50 KB
-// loop body matters: with every loop of a layer unrolled (95 KB, against 64 KiB of instruction cache for two compute
+// under them, and fifteen exchanges some 15,000.  A call of 1500 positions: 4.38 ms with one position per workgroup, 3.40.  The 50 KB
+// loop body matters (kernel alone, 3287 us): with every loop of a layer unrolled (95 KB, against 64 KiB of instruction cache for two compute
 // units) and 50 registers spilled for it, 3776.  The weights' first touches are misses in every layer; sharing them out a
 // phase ahead changed nothing (3327 against 3325).
 //

@@ -41,7 +41,7 @@ enum bf_quant {
     BF_QUANT_E4M3 = 1
 };
 
-/* Five kernels compute the same function.
+/* Five kernels that can be asked for by name, and two forms that only AUTO runs (enum bf_form), compute the same function.
  *   QUAD   four positions per workgroup, one wavefront each, weights shared through LDS
  *          (256-wide network, int8 and e4m3).
  *   BOARD  one position per workgroup, the four wavefronts split the model width; one workgroup
