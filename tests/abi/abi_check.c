@@ -11,6 +11,7 @@ int main(void) {
     bf_eval_args args;
     bf_expand_args ex;
     double s8 = 0.0, u8 = 0.0;
+    int64_t numel[2];
 
     memset(&shape, 0, sizeof shape);
     shape.d_model = 256; shape.n_layers = 8; shape.n_heads = 8; shape.d_ff = 1024; shape.n_value = 1; shape.eps = 1e-5f;
@@ -45,6 +46,13 @@ int main(void) {
     if (bf_stream_rate(NULL, 32768, 4, 1, NULL, NULL) >= 0.0) return 18;
     if (bf_abi_tag() != BF_ABI_TAG || (bf_abi_tag() >> 32) != BF_ABI_VERSION) return 19;    /* this client and the library agree */
     if (bf_quant_probe(BF_PROBE_S8, NULL, 1.0f, 4, NULL, NULL) != BF_ERR_ARGUMENT) return 20;
+    if (bf_recip_probe(BF_PROBE_RECIP, NULL, 4, NULL, NULL) != BF_ERR_ARGUMENT) return 21;
+    if (bf_launch_form(&args) != BF_ERR_UNSUPPORTED || bf_launch_form(NULL) != BF_ERR_ARGUMENT) return 22;
+    if (bf_team_workspace_bytes(&shape) != 0 || bf_team_position_bytes(&shape) != 0 || bf_team_gave_up() != 0) return 23;   /* 384 wide */
+    if (bf_pack_scratch_floats(&shape) != 0 || bf_pack_board(&shape, BF_QUANT_INT8, NULL, NULL, NULL, NULL, NULL, NULL) != BF_ERR_UNSUPPORTED) return 24;
+    numel[0] = 8192; numel[1] = 8193;
+    if (bf_fingerprint_partials(numel, 2) != 3 || bf_fingerprint(NULL, numel, 2, NULL, NULL, NULL) != BF_ERR_ARGUMENT) return 25;
+    if (bf_clear(NULL, NULL, 1, NULL) != BF_ERR_ARGUMENT) return 26;
     printf("abi ok: %s\n", bf_last_error());
     return 0;
 }
