@@ -40,6 +40,8 @@
 
 #include "bf_board.hip.h"
 
+typedef float v2f __attribute__((ext_vector_type(2)));
+
 namespace bf {
 namespace duo {
 
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     static_assert(C::KC == 1 && STEPS == TW && KCF == 2 * STEPS, "the 256-wide network");
     static_assert(8 % (AHEAD + 1) == 0, "an operand's place must not depend on the product");
     static_assert((8 * NB) % RING == 0, "a fragment's place in the ring must not depend on the layer");
-    static_assert(RING <= 8 * HB + 8, "the first prefetches of the heads stay inside the head blocks");
+    static_assert(RING <= 8 * HB, "the first prefetches of the heads stay inside the head blocks");
     static_assert(board::block_at_covers_layer<1, TW, 2, BPW, true>(), "block_at must enumerate a layer's blocks exactly once");
 
     const int lane = threadIdx.x & 63;
@@ -309,7 +311,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         const float v[1] = {m};
         return Rows<1>::max(v);
     };
-    auto layernorm2 = [&](const float (&x)[NP][16], const float* gamma, const float* beta, float (&y)[NP][16]) {
+    auto layernorm2_by = [&](const float (&x)[NP][16], auto gamma, auto beta, float (&y)[NP][16]) {   // gamma(j), beta(j): of register quad j
         float part[NP], mean[NP], rstd[NP];
 #pragma unroll
         for (int p = 0; p < NP; p++) {
@@ -332,8 +334,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         Rows<NP>::each(recip_sqrt(xsum2(part, 1) * (1.0f / D) + a.eps), rstd);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const v4f ga = ldg4(gamma + 8 * j + 4 * g);
-            const v4f be = ldg4(beta + 8 * j + 4 * g);
+            const v4f ga = gamma(j), be = beta(j);
 #pragma unroll
             for (int p = 0; p < NP; p++)
 #pragma unroll
@@ -342,6 +343,9 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
                     y[p][4 * j + k] = __builtin_fmaf(d * rstd[p], ga[k], be[k]);
                 }
         }
+    };
+    auto layernorm2 = [&](const float (&x)[NP][16], const float* gamma, const float* beta, float (&y)[NP][16]) {
+        layernorm2_by(x, [&](int j) { return ldg4(gamma + 8 * j + 4 * g); }, [&](int j) { return ldg4(beta + 8 * j + 4 * g); }, y);
     };
     // signed quantiser of both positions' rows: one scale per row; this wave's bytes go to the
     // position's activation buffer, from which every wave reads its B operands
@@ -971,123 +975,193 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     if (enc_only) return;   // the same for every wave of the launch
 
     // ---- final norm and heads --------------------------------------------------------------------------
-    // The weight stream is restarted at the head blocks (after the last layer the prefetch ran on
-    // into a layer that is not used).
-    const int hblk0 = (a.n_layers - a.l0) * BPW;
-    wait_vm<0>();   // also: no parameter copy is still landing
+    // The products of the heads come in pieces of 16 rows of a head tile and 16 tokens (v_mfma_f32_16x16x4f32: the
+    // fused-multiply-add chain of the 32x32x2 form, four links a step).  A wave takes 16 rows of a policy tile for both
+    // halves of its position's tokens (one position: for one half), and one wave of each SIMD (one position: of two) a half of a
+    // position's tokens with the first rows of tile 2, where promotion and value lie.  For two positions that is 10.2 k clocks of every
+    // SIMD; as 32x32 products of whole tiles (tile 2's 25 rows of zeros among them) it was 16.4 k of three SIMDs, and the fourth idled.
+    // With the final norm's parameters and the legal moves asked for ahead and the best move found without LDS permutations: phases
+    // heads + stores 29.9 k -> 24.7 k ticks of 483 k; 300 positions 171.6 -> 169.6 us, 100 115.4 -> 114.4, 4096 1434 -> 1425, e4m3 1911 -> 1904.
+    constexpr int HALVES = NP;                       // token halves of a policy wave
+    const int ht = q & 1, rh = q >> 1;               // its rows: 16 rh .. of head tile ht
+    const int mine = NP == 2 ? sub : 0;              // its position
+    const bool extra = sub == 1 && (NP == 2 || q < 2);
+    const int xmine = NP == 2 ? q & 1 : 0, xth = NP == 2 ? q >> 1 : q;   // tile 2: position, token half
+    const int G = lane >> 4, c16 = lane & 15;
+    const int b = mine ? bp[NP - 1] : bp[0], xb = xmine ? bp[NP - 1] : bp[0];
+    const bool store = mine ? live[NP - 1] : live[0], xstore = xmine ? live[NP - 1] : live[0];
+    const int xctrl = xmine ? ctrl[NP - 1] : ctrl[0];
+    // Lane (row, k) reads, of fragment f, the lane of its row and of half k % 2, from element k / 2 on: what it multiplies lies in places 0
+    // and 2 then.  (The last lanes' reads end four bytes behind the fragment, in the next one or the block of padding.)
+    const size_t qstride = (size_t)a.n_layers * BPW + HB + 1;
+    auto head_tile = [&](int n) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.wstream + (n * qstride + (size_t)a.n_layers * BPW) * BLOCK), 0, HB * BLOCK + 16, 0x00027000);
+    };
+    const __amdgpu_buffer_rsrc_t policy_tile = head_tile(ht), tile2 = head_tile(2);
+    const int from0 = (c16 + 32 * (G & 1)) * 16 + 4 * (G >> 1), from = from0 + 256 * rh;
+    auto load_head = [&](const __amdgpu_buffer_rsrc_t& buf, int lane_at, int f, int at) {
+        frt[at] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(buf, lane_at, f * FRAG, 0));
+    };
+    // the final norm's parameters, a quarter's worth of exchanges ahead of their use
+    v4f nfg[4], nfb[4];
+    load_tile16(gp + C::G_NFG + 32 * tile, g, nfg);
+    load_tile16(gp + C::G_NFB + 32 * tile, g, nfb);
 #pragma unroll
-    for (int j = 0; j < RING; j++) load_frag(8 * hblk0 + j, j);
+    for (int j = 0; j < RING; j++) load_head(policy_tile, from, j, j);
+    unsigned long long legal[HALVES];
+    const bool masked = a.mask != nullptr;
+#pragma unroll
+    for (int i = 0; i < HALVES; i++) legal[i] = masked ? a.mask[(size_t)b * T + 16 * (NP == 2 ? i : sub) + c16] : ~0ull;
+    __builtin_amdgcn_sched_barrier(0);
+    auto final_norm = [&](const float (&of)[NP][16], float (&y)[NP][16]) {
+        layernorm2_by(of, [&](int j) { return nfg[j]; }, [&](int j) { return nfb[j]; }, y);
+    };
     float hn[NP][16];
-    layernorm2(x, gp + C::G_NFG + 32 * tile, gp + C::G_NFB + 32 * tile, hn);
-    // publish as B-operand fragments (n, j): lane holds the four floats of register quad j
+    final_norm(x, hn);
+    // A position's row as operand fragments (n, j): lane (t, g) holds the four floats of register quad j, elements 0 and 2 together
+    auto publish = [&](int p, const float (&v)[16]) {
+        float* const to = reinterpret_cast<float*>(hid + p * C::HID_P);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            *reinterpret_cast<v4f*>(to + ((tile * 4 + j) * 64 + lane) * 4) = v4f{v[4 * j], v[4 * j + 2], v[4 * j + 1], v[4 * j + 3]};
+    };
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-        float* const hnb = reinterpret_cast<float*>(hid + p * C::HID_P);
         if (TAPS && a.taps.normed && live[p])
 #pragma unroll
             for (int r = 0; r < 16; r++)
                 a.taps.normed[((size_t)bp[p] * T + t) * D + 32 * tile + ch(r, g)] = hn[p][r];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const v4f v = {hn[p][4 * j], hn[p][4 * j + 1], hn[p][4 * j + 2], hn[p][4 * j + 3]};
-            *reinterpret_cast<v4f*>(hnb + ((tile * 4 + j) * 64 + lane) * 4) = v;
-        }
+        publish(p, hn[p]);
     }
     barrier();
-    // Wave (m, p) multiplies head tile m (rows 32m..32m+31 of [policy; promo; value; 0]) with the
-    // normalised stream of position p over the whole width, one fused-multiply-add chain in (tile,
-    // quad, element) order; quarter 3's tile is zero and stores nothing, so it is not computed.
-    // With one position per workgroup the second wave of a quarter has nothing to do here but
-    // meet the barriers.
-    const int mine = NP == 2 ? sub : 0;   // the position whose heads this wave computes
-    const bool heads_here = NP == 2 || sub == 0;
-    const float* const hnb = reinterpret_cast<const float*>(hid + mine * C::HID_P);
-    v16f head = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (q < 3 && heads_here) {
+    // lane (token, k) of a step: element k / 2 (and 2 + k / 2 in the next step) of the fragment lane of half k % 2
+    auto operands_of = [&](int pos) {
+        int at = C::HID_OFF + pos * C::HID_P + (32 * (G & 1) + c16) * 16 + 8 * (G >> 1);
+        asm volatile("" : "+v"(at));   // one address register; the rest are the instructions' own offsets
+        return lds + at;
+    };
+    auto operand = [&](const uint8_t* of, int th, int f) { return *reinterpret_cast<const v2f*>(of + f * FRAG + th * 256); };
+    auto steps = [&](const v4i& w, const v2f& h, v4f& acc) {
+        const v4f wf = __builtin_bit_cast(v4f, w);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[0], h[0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[2], h[1], acc, 0, 0, 0);
+    };
+    constexpr int EARLY = 4;   // operands come from LDS this many fragments early
+    constexpr int RING_POOL = 8;   // fragments of a set in the pooled heads
+    static_assert(RING_POOL <= RING && (8 * HB) % RING_POOL == 0, "whole sets");
+    v4f head[HALVES];
+#pragma unroll
+    for (int i = 0; i < HALVES; i++) head[i] = v4f{0, 0, 0, 0};
+    {
+        const uint8_t* const of = operands_of(mine) + (NP == 2 ? 0 : 256 * sub);
+        v2f h[EARLY][HALVES];
+#pragma unroll
+        for (int f = 0; f < EARLY; f++)
+#pragma unroll
+            for (int i = 0; i < HALVES; i++) h[f][i] = operand(of, i, f);
 #pragma unroll
         for (int f = 0; f < 8 * HB; f++) {
-            const v4f w = __builtin_bit_cast(v4f, frt[f % RING]);
-            const v4f hv = *reinterpret_cast<const v4f*>(hnb + (f * 64 + lane) * 4);
 #pragma unroll
-            for (int k = 0; k < 4; k++) head = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k], hv[k], head, 0, 0, 0);
-            if (f + RING < 8 * HB) load_frag(8 * hblk0 + f + RING, f % RING);
+            for (int i = 0; i < HALVES; i++) {
+                steps(frt[f % RING], h[f % EARLY][i], head[i]);
+                if (f + EARLY < 8 * HB) h[f % EARLY][i] = operand(of, i, f + EARLY);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (f + RING < 8 * HB) load_head(policy_tile, from, f + RING, f % RING);
+            else if (extra) load_head(tile2, from0, f + RING - 8 * HB, (f + RING) % RING);
+        }
+    }
+    v4f rest = {0, 0, 0, 0};
+    if (extra) {
+        const uint8_t* const of = operands_of(xmine) + 256 * xth;
+        v2f h[EARLY];
+#pragma unroll
+        for (int f = 0; f < EARLY; f++) h[f] = operand(of, 0, f);
+#pragma unroll
+        for (int f = 0; f < 8 * HB; f++) {
+            steps(frt[(8 * HB + f) % RING], h[f % EARLY], rest);
+            if (f + EARLY < 8 * HB) h[f % EARLY] = operand(of, 0, f + EARLY);
+            __builtin_amdgcn_sched_barrier(0);
+            if (f + RING < 8 * HB) load_head(tile2, from0, f + RING, (8 * HB + f) % RING);
         }
     }
     BF_PHASE(PH_HEADS);
-    const int b = mine ? bp[NP - 1] : bp[0];
-    const bool store = heads_here && (mine ? live[NP - 1] : live[0]);
-    const int ctrl_m = mine ? ctrl[NP - 1] : ctrl[0];
-    auto value_of = [&](const v16f& hd) -> float {
+    auto value_of = [&](const v4f& hd) -> float {
         if (a.n_value == 1) return tanh_dev(hd[0]);
         const float r0 = hd[0], r1 = hd[1], r2 = hd[2];   // classes loss, draw, win
         const float mx = __builtin_fmaxf(__builtin_fmaxf(r0, r1), r2);
         const float e0 = exp_neg(r0 - mx), e1 = exp_neg(r1 - mx), e2 = exp_neg(r2 - mx);
         return (e2 - e0) / ((e0 + e1) + e2);
     };
-    // value (king head): king token of the side to move, lane half 1 of head tile 2 holds rows 68..70
-    if (q == 2 && store) {
-        const int king = ctrl_m < 0 ? 31 : 15;
-        if (a.vmode == 0 && lane == 32 + king) a.value[b] = value_of(head);
-        if (g == 0) {   // promo: rows 64..67 are registers 0..3 of lane half 0
-            if (a.out_fp32) {
-                const v4f v = {head[0], head[1], head[2], head[3]};
-                *reinterpret_cast<v4f*>((float*)a.promo + ((size_t)b * T + t) * 4) = v;
-            } else {
-                const v4h v = {(_Float16)head[0], (_Float16)head[1], (_Float16)head[2], (_Float16)head[3]};
-                *reinterpret_cast<v4h*>((_Float16*)a.promo + ((size_t)b * T + t) * 4) = v;
-            }
+    // tile 2: rows 64 .. 67 (lanes G = 0) are the promotions, rows 68 .. 70 (G = 1) the value, whose token is the mover's king
+    if (extra && xstore) {
+        const int tk = 16 * xth + c16;
+        if (a.vmode == 0 && G == 1 && tk == (xctrl < 0 ? 31 : 15)) a.value[xb] = value_of(rest);
+        if (G == 0) {
+            if (a.out_fp32) *reinterpret_cast<v4f*>((float*)a.promo + ((size_t)xb * T + tk) * 4) = rest;
+            else *reinterpret_cast<v4h*>((_Float16*)a.promo + ((size_t)xb * T + tk) * 4) = v4h{(_Float16)rest[0], (_Float16)rest[1], (_Float16)rest[2], (_Float16)rest[3]};
         }
     }
-    // policy (quarters 0 and 1: squares 0..31 and 32..63), optional legal-move AND and argmax
+    // policy: squares 32 ht + 16 rh + 4 G .. of the wave's tokens, optional legal-move AND and argmax
+    constexpr int NONE = 0x7fffffff;
     float bv = -__builtin_inff();
-    int bi = 0x7fffffff;
-    if (q < 2 && heads_here) {
-        unsigned long long mw = ~0ull;
-        if (a.mask) mw = a.mask[(size_t)b * T + t];
+    int bi = NONE;
+    const int sq0 = 32 * ht + 16 * rh + 4 * G;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float v[4];
+    for (int i = 0; i < HALVES; i++) {
+        const int tk = 16 * (NP == 2 ? i : sub) + c16;
+        const unsigned here_legal = (unsigned)(legal[i] >> sq0);
+        float v[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int sq = 32 * q + 8 * j + 4 * g + k;
-                const bool legal = (mw >> sq) & 1ull;
-                v[k] = legal ? head[4 * j + k] : -__builtin_inff();
-                // squares are visited in increasing order within a lane, so '>' keeps the lowest
-                if (legal && (bi == 0x7fffffff || v[k] > bv)) { bv = v[k]; bi = t * 64 + sq; }
-            }
-            const size_t at = ((size_t)b * T + t) * 64 + 32 * q + 8 * j + 4 * g;
-            if (store) {
-                if (a.out_fp32) {
-                    const v4f vv = {v[0], v[1], v[2], v[3]};
-                    *reinterpret_cast<v4f*>((float*)a.policy + at) = vv;
-                } else {
-                    const v4h vv = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-                    *reinterpret_cast<v4h*>((_Float16*)a.policy + at) = vv;
-                }
-            }
+        for (int k = 0; k < 4; k++) {
+            const bool ok = (here_legal >> k) & 1u;
+            v[k] = ok ? head[i][k] : -__builtin_inff();
+            // a lane visits its moves in increasing order, so '>' keeps the lowest
+            if (ok && (bi == NONE || v[k] > bv)) { bv = v[k]; bi = tk * 64 + sq0 + k; }
+        }
+        const size_t at = ((size_t)b * T + tk) * 64 + sq0;
+        if (store) {
+            if (a.out_fp32) *reinterpret_cast<v4f*>((float*)a.policy + at) = v4f{v[0], v[1], v[2], v[3]};
+            else *reinterpret_cast<v4h*>((_Float16*)a.policy + at) = v4h{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
         }
     }
-    if (a.mask && a.best) {
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            const float ov = __shfl_xor(bv, d);
-            const int oi = __shfl_xor(bi, d);
-            const bool take = (oi != 0x7fffffff) && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi));
+    if (masked && a.best) {
+        auto merge = [&](float ov, int oi) {
+            const bool take = oi != NONE && (bi == NONE || ov > bv || (ov == bv && oi < bi));
             bv = take ? ov : bv;
             bi = take ? oi : bi;
-        }
-        // the two policy waves' winners of a position meet in the exchange slot no row sum uses
-        if (q < 2 && heads_here && lane == 0) {
-            xch[2 * XS + mine * 4 + q * 2] = bv;
-            xch[2 * XS + mine * 4 + q * 2 + 1] = __int_as_float(bi);
+        };
+        auto over_dpp = [&](auto ctrl_) {   // another lane of the row of 16
+            constexpr int c = decltype(ctrl_)::value;
+            const int ov = __builtin_amdgcn_update_dpp(0, __float_as_int(bv), c, 0xf, 0xf, true), oi = __builtin_amdgcn_update_dpp(0, bi, c, 0xf, 0xf, true);
+            merge(__int_as_float(ov), oi);
+        };
+        auto over_swap = [&](auto swap) {   // both lanes get both values and keep the better one
+            const auto v2 = swap(__float_as_int(bv)), i2 = swap(bi);
+            bv = __int_as_float((int)v2[0]);
+            bi = (int)i2[0];
+            merge(__int_as_float((int)v2[1]), (int)i2[1]);
+        };
+        over_dpp(std::integral_constant<int, 0xb1>());    // xor 1
+        over_dpp(std::integral_constant<int, 0x4e>());    // xor 2
+        over_dpp(std::integral_constant<int, 0x141>());   // the mirrored eight
+        over_dpp(std::integral_constant<int, 0x140>());   // the mirrored sixteen
+        over_swap([](int v) { return __builtin_amdgcn_permlane16_swap(v, v, false, false); });
+        over_swap([](int v) { return __builtin_amdgcn_permlane32_swap(v, v, false, false); });
+        // the winners of a position's waves meet in the exchange slot no row sum uses
+        int* const met = reinterpret_cast<int*>(xch + 2 * XS);
+        if (lane == 0) {
+            met[2 * wave] = __float_as_int(bv);
+            met[2 * wave + 1] = bi;
         }
         barrier();
-        if (q == 0 && lane == 0 && store) {
-            const float ov = xch[2 * XS + mine * 4 + 2];
-            const int oi = __float_as_int(xch[2 * XS + mine * 4 + 3]);
-            const bool take = (oi != 0x7fffffff) && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi));
-            bi = take ? oi : bi;
-            a.best[b] = bi == 0x7fffffff ? -1 : bi;
+        if (q == 0 && (NP == 2 || sub == 0) && store) {
+#pragma unroll
+            for (int w = 1; w < 8 / NP; w++) {
+                const int o = NP == 2 ? 4 * sub + w : w;
+                merge(__int_as_float(met[2 * o]), met[2 * o + 1]);
+            }
+            if (lane == 0) a.best[b] = bi == NONE ? -1 : bi;
         }
     }
     // ---- pooled value heads (reference brokefish/nn/model.py:576-617) --------------------------------
@@ -1110,7 +1184,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
             }
         }
         if (a.vmode == 2) {
-            layernorm2(pv, gp + C::G_NFG + 32 * tile, gp + C::G_NFB + 32 * tile, hv);
+            final_norm(pv, hv);
         } else {
 #pragma unroll
             for (int p = 0; p < NP; p++)
@@ -1119,28 +1193,21 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
         }
         barrier();   // every wave has finished reading the normalised streams
 #pragma unroll
-        for (int p = 0; p < NP; p++) {
-            float* const dst = reinterpret_cast<float*>(hid + p * C::HID_P);
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const v4f v = {hv[p][4 * j], hv[p][4 * j + 1], hv[p][4 * j + 2], hv[p][4 * j + 3]};
-                *reinterpret_cast<v4f*>(dst + ((tile * 4 + j) * 64 + lane) * 4) = v;
-            }
-        }
+        for (int p = 0; p < NP; p++) publish(p, hv[p]);
         barrier();
-        if (q == 2 && heads_here) {
-            // head tile 2 once more, against the pooled row (every token column holds the same row);
-            // its blocks are read straight from the stream, in the same order as above
-            v16f hd = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            for (int f = 0; f < 8 * HB; f++) {
-                const v4f w = *reinterpret_cast<const v4f*>(wsrc + (size_t)hblk0 * BLOCK + (size_t)f * FRAG + lane16);
-                const v4f hvv = *reinterpret_cast<const v4f*>(hnb + (f * 64 + lane) * 4);
+        if (extra && xth == 0) {
+            // tile 2's rows once more, against the pooled row (every token column holds the same row), in the same order as above
+            v4f hd = {0, 0, 0, 0};
+            const uint8_t* const of = operands_of(xmine);
+            for (int f0 = 0; f0 < 8 * HB; f0 += RING_POOL) {
 #pragma unroll
-                for (int k = 0; k < 4; k++) hd = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k], hvv[k], hd, 0, 0, 0);
+                for (int j = 0; j < RING_POOL; j++) load_head(tile2, from0, f0 + j, j);
+#pragma unroll
+                for (int j = 0; j < RING_POOL; j++) steps(frt[j], operand(of, 0, f0 + j), hd);
             }
-            if (lane == 32 && store) {
+            if (lane == 16 && xstore) {
                 const float v = value_of(hd);
-                a.value[b] = ctrl_m > 0 ? v : -v;
+                a.value[xb] = xctrl > 0 ? v : -v;
             }
         }
     }
