@@ -15,8 +15,8 @@
 // So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
 // tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
 // except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
-// 120 -> 76 us, e4m3 155 -> 92, width 512 with 16 layers 738 -> 265; 64 positions 120 -> 81, e4m3 155 -> 95; 32 of the
-// wide network 738 -> 320.  The arithmetic is that of the other kernels, operation for operation: the results are
+// 120 -> 74.5 us, e4m3 155 -> 90, width 512 with 16 layers 738 -> 255; 64 positions 120 -> 80, e4m3 155 -> 94.5; 32 of the
+// wide network 738 -> 314.  The arithmetic is that of the other kernels, operation for operation: the results are
 // bit-identical to theirs.
 //
 // Rows and tiles.  For everything per row (LayerNorm, quantisers, residual sums) a wavefront owns the rows of four
@@ -28,8 +28,11 @@
 //
 // What bounds it now: a layer is some 20 k clocks at width 256, of which the waits for other members are 1.5 k; the unit's
 // path to the L2 moves 370 KB in it (5.8 k clocks, most of it under something else), two LayerNorms, three
-// quantisers and the epilogues are some 7 k of vector work, attention 2.8 k.  Outside the layers: 8.7 k to the first one (two
-// loads that depend on each other, then the first weights), 8.3 k of final norm and head chain, 3.3 k for the best move.
+// quantisers and the epilogues are some 7 k of vector work, attention 2.8 k.  Outside the layers: 7.6 k to the first one (two
+// loads that depend on each other; 8.5 k with every wavefront asking for the rows that all tokens share), 6.9 k of final norm and head
+// chain (8.3 k while the chain waited for its operands out of LDS at every step), 3 k for the best move: together 75.5 -> 74.5 us, 64
+// positions 81.1 -> 79.9, 20 of the wide network 300 -> 291.  (Lines of the first layer's weights and of the head tiles
+// asked for ahead: 75.7.  The output projection's weights moved out of LayerNorm 1, into the QKV phase or the attention: 76.7 to 81.9.)
 // The path takes a 16-byte load of 64 lanes in 16 clocks and a wavefront stops at the load that finds it busy, so where the
 // loads stand matters as much as how many they are (one position, 82.3 us before):
 //   - a layer's parameters, asked for right before the Q, K, V products, made those wait for them (all loads return in order);
@@ -372,53 +375,79 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     auto piece_at = [&](int tk, int half) { return (tk >> 2) * C::ROWS_W + (half * 32 + (tk & 3)) * 16; };
     auto tile_at = [&](int tile) { return tile % NP * FRAG + tile / NP * 64; };
 
-    // ---- start: parameters of the first layer; its weights follow the embedding's loads, which return in order ----
-    if (a.l1 > a.l0) fetch_par(a.l0, q, !(wave & 1), wave & 1);
-    else if (!ENC && wave == 4) fetch_final();
-
-    // ---- embedding, or the caller's stream -------------------------------------------------------------
-    float x[NP][16];
+    // ---- start: the board's words, then the first layer's parameters, which come while the rows that the words name are
+    // asked for; its weights follow (all loads return in order) ----
     const unsigned own_word = ENC ? (a.taps.alive[(size_t)b * T + t] ? 0u : 0x800u) : a.boards[(size_t)b * T + t];
     const unsigned row_word = ENC ? 0u : a.boards[(size_t)b * T + row];
     const int ctrl = ENC ? 1 : a.control[b];
     int rp = ENC ? 0 : a.rep[b];
     rp = rp > 2 ? 2 : rp;
+    __builtin_amdgcn_sched_barrier(0);
+    if (a.l1 > a.l0) fetch_par(a.l0, q, !(wave & 1), wave & 1);
+    else if (!ENC && wave == 4) fetch_final();
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- embedding, or the caller's stream -------------------------------------------------------------
+    // The rows that all tokens share (clock and repetition, added; the two of colour) come once, four bytes a thread, by way of
+    // LDS: a load of sixteen bytes a lane takes the unit's path 16 clocks, and five rows for every token are 20 of them in each wave.
+    float x[NP][16];
     const unsigned alive = (unsigned)__ballot(((own_word >> 11) & 1) == 0 && g == 0);
+    if constexpr (ENC) {
 #pragma unroll
-    for (int p = 0; p < NP; p++) {
-        const size_t at = ((size_t)b * T + row) * D + 32 * (NP * rk + p) + 4 * rg;
-        if constexpr (ENC) {
+        for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const v4f v = stream_in(a.taps, at + 8 * j);
+                const v4f v = stream_in(a.taps, ((size_t)b * T + row) * D + 32 * (NP * rk + p) + 4 * rg + 8 * j);
 #pragma unroll
                 for (int k = 0; k < 4; k++) x[p][4 * j + k] = v[k];
             }
-        } else {
-            const unsigned word = row_word;
-            const int stm = ctrl < 0;
-            int clock = (ctrl < 0 ? -ctrl : ctrl) - 1;
-            clock = clock < 0 ? 0 : (clock > 100 ? 100 : clock);
-            int ts = ((word >> 6) & 7) * 2 + ((word >> 9) & 1);
-            ts = ts > 11 ? 11 : ts;
-            const int ct = ((word >> 10) & 1) * 2 + stm;
+    } else {
+        float* const shared_rows = reinterpret_cast<float*>(ex);   // [clock + repetition][colour, bit 10 clear][set]
+        static_assert(3 * D * 4 <= C::EX_BYTES && (D == 256 || D == 512), "shared rows");
+        const int stm = ctrl < 0;
+        int clock = (ctrl < 0 ? -ctrl : ctrl) - 1;
+        clock = clock < 0 ? 0 : (clock > 100 ? 100 : clock);
+        const int c = (int)threadIdx.x & (D - 1);
+        const bool first = D == 512 || threadIdx.x < D, second = D == 512 || threadIdx.x >= D;   // whose share
+        float once[4] = {};
+        if (first) {
+            once[0] = gp[C::G_CLOCK + clock * D + c];
+            once[1] = gp[C::G_REP + rp * D + c];
+        }
+        if (second) {
+            once[2] = gp[C::G_CT + stm * D + c];
+            once[3] = gp[C::G_CT + (2 + stm) * D + c];
+        }
+        int ts = ((row_word >> 6) & 7) * 2 + ((row_word >> 9) & 1);
+        ts = ts > 11 ? 11 : ts;
+        v4f vs[NP][4], vt[NP][4];
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
             const int own = 32 * (NP * rk + p) + 4 * rg;
-            const float* e_sq = gp + C::G_SQ + (word & 63) * D + own;
-            const float* e_ts = gp + C::G_TS + ts * D + own;
-            const float* e_ct = gp + C::G_CT + ct * D + own;
-            const float* e_ck = gp + C::G_CLOCK + clock * D + own;
-            const float* e_rp = gp + C::G_REP + rp * D + own;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int c = 8 * j;
-                const v4f vs = ldg4(e_sq + c), vt = ldg4(e_ts + c), vc = ldg4(e_ct + c);
-                const v4f vk = ldg4(e_ck + c), vr = ldg4(e_rp + c);
+                vs[p][j] = ldg4(gp + C::G_SQ + (row_word & 63) * D + own + 8 * j);
+                vt[p][j] = ldg4(gp + C::G_TS + ts * D + own + 8 * j);
+            }
+        }
+        if (first) shared_rows[c] = once[0] + once[1];
+        if (second) {
+            shared_rows[D + c] = once[2];
+            shared_rows[2 * D + c] = once[3];
+        }
+        lds_barrier();
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            const float* const of = shared_rows + 32 * (NP * rk + p) + 4 * rg;
+            const float* const colour = of + D + ((row_word >> 10) & 1) * D;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const v4f vb = ldg4(of + 8 * j), vc = ldg4(colour + 8 * j);
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const float per_board = vk[k] + vr[k];
-                    float v = vs[k] + vt[k];
+                    float v = vs[p][j][k] + vt[p][j][k];
                     v = v + vc[k];
-                    x[p][4 * j + k] = v + per_board;
+                    x[p][4 * j + k] = v + vb[k];
                 }
             }
         }
@@ -798,18 +827,22 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     // and value (the first rows of tile 2).
     const int job = wave * NWG + m;
     const int G = lane >> 4, c16 = lane & 15;
-    // the head tile's fragments, HEAD_SET of them; the first ones now
-    constexpr int HEAD_SET = 32;
-    static_assert(8 * HB % HEAD_SET == 0, "whole sets");
-    v4i hw[HEAD_SET];
-    auto load_head = [&](int ht, int rh, int f0) {
-        const int at = (ht * stride_q + a.n_layers * BPW) * BLOCK + f0 * FRAG, lane_at = (16 * rh + c16 + 32 * (G & 1)) * 16;
+    // A head tile's fragments, HR of them in flight; the first ones now.  Lane (row, k) reads the fragment's lane of its row and of half
+    // k % 2, from element k / 2 on, so that what it multiplies lies in places 0 and 2.  (The last lanes' reads end four bytes behind
+    // the fragment, in the next one or the stream's block of padding.)
+    constexpr int HR = 16;
+    static_assert(8 * HB % HR == 0, "whole rounds");
+    v4i hw[HR];
+    auto load_head = [&](int ht, int rh, int f) {
+        const int at = (ht * stride_q + a.n_layers * BPW) * BLOCK, lane_at = (16 * rh + c16 + 32 * (G & 1)) * 16 + 4 * (G >> 1);
+        hw[f % HR] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane_at + f % 4 * FRAG, at + f / 4 * 4 * FRAG, 0));
+    };
+    auto load_first = [&](int ht, int rh) {
 #pragma unroll
-        for (int f = 0; f < HEAD_SET; f++)
-            hw[f] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane_at + f % 4 * FRAG, at + f / 4 * 4 * FRAG, 0));
+        for (int f = 0; f < HR; f++) load_head(ht, rh, f);
     };
     const int ht = job >> 2, rh = job < 8 ? (job >> 1) & 1 : 0, th = job & 1;   // job < 10: rows 16 rh .. of head tile ht, tokens 16 th ..
-    if (job < 10) load_head(ht, rh, 0);
+    if (job < 10) load_first(ht, rh);
     float hn[NP][16];
     const float* const gn = fin + 32 * NP * rk + 4 * rg;
     layernorm(x, gn, gn + D, hn);
@@ -831,19 +864,22 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
     // Rows 16 rh .. of head tile `ht` times tokens 16 th ..: the chain of the 32x32x2 form, two of whose steps (four k) are
     // one step here.  Lane (row or token, k) takes element k / 2 and 2 + k / 2 of the fragment lane of half k % 2.
     auto head_product = [&](int ht, int rh, int th) -> v4f {
-        const float* hp = hnb + (16 * th + c16 + 32 * (G & 1)) * 4 + 2 * (G >> 1);
-        const bool up = G >> 1;
+        int from = C::EX_OFF + (16 * th + c16 + 32 * (G & 1)) * 16 + 8 * (G >> 1);
+        asm volatile("" : "+v"(from));   // one address register; the rest are the instructions' own offsets
+        auto operand = [&](int f) { return *reinterpret_cast<const v2f*>(lds + from + f / 4 * C::EX_TILE + f % 4 * FRAG); };
+        constexpr int EARLY = 8;   // operands come from LDS this many fragments early: the chain waits for its matrix steps only
+        v2f h[EARLY];
+#pragma unroll
+        for (int f = 0; f < EARLY; f++) h[f] = operand(f);
         v4f acc = {0, 0, 0, 0};
 #pragma unroll
-        for (int f0 = 0; f0 < 8 * HB; f0 += HEAD_SET) {
-            if (f0) load_head(ht, rh, f0);
-#pragma unroll
-            for (int f = 0; f < HEAD_SET; f++) {
-                const v4f w = __builtin_bit_cast(v4f, hw[f]);
-                const v2f h = *reinterpret_cast<const v2f*>(hp + (f0 + f) / 4 * (C::EX_TILE / 4) + (f0 + f) % 4 * 256);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(up ? w[1] : w[0], h[0], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(up ? w[3] : w[2], h[1], acc, 0, 0, 0);
-            }
+        for (int f = 0; f < 8 * HB; f++) {
+            const v4f w = __builtin_bit_cast(v4f, hw[f % HR]);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[0], h[f % EARLY][0], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[2], h[f % EARLY][1], acc, 0, 0, 0);
+            if (f + EARLY < 8 * HB) h[f % EARLY] = operand(f + EARLY);
+            __builtin_amdgcn_sched_barrier(0);
+            if (f + HR < 8 * HB) load_head(ht, rh, f + HR);
         }
         return acc;
     };
@@ -886,8 +922,14 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             };
             over_lanes_of_row();
             over_dpp(std::integral_constant<int, 0x140>());
-            merge(__shfl_xor(bv, 16), __shfl_xor(bi, 16));
-            merge(__shfl_xor(bv, 32), __shfl_xor(bi, 32));
+            auto over_swap = [&](auto swap) {   // both lanes get both values and keep the better one
+                const auto v2 = swap(__float_as_int(bv)), i2 = swap(bi);
+                bv = __int_as_float((int)v2[0]);
+                bi = (int)i2[0];
+                merge(__int_as_float((int)v2[1]), (int)i2[1]);
+            };
+            over_swap([](int v) { return __builtin_amdgcn_permlane16_swap(v, v, false, false); });
+            over_swap([](int v) { return __builtin_amdgcn_permlane32_swap(v, v, false, false); });
             // the eight wavefronts' winners meet in member 0
             const unsigned tag = tag0 + (a.l1 - a.l0);
             if (lane == 0) __builtin_amdgcn_raw_buffer_store_b64(v2u{(unsigned)__float_as_int(bv), (unsigned)bi}, wsr, 0, C::WS_H + job * 16, 0);
@@ -967,7 +1009,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             lds_barrier();
         }
         if (job == 8) {
-            if constexpr (8 * HB > HEAD_SET) load_head(2, 0, 0);   // else they are still there
+            load_first(2, 0);
             const v4f hd = head_product(2, 0, 0);
             if (lane == 16) {
                 const float v = value_of(hd);
