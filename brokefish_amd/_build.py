@@ -37,6 +37,7 @@ HIP_SOURCES = ["bf_variant_prod_fp8.hip", "bf_variant_taps_fp8.hip", "bf_variant
                "bf_variant_duo256_fp8.hip", "bf_variant_duo256_fp8_taps.hip", "bf_variant_duo256_fp8_prof.hip",
                "bf_variant_solo256.hip", "bf_variant_solo256_taps.hip", "bf_variant_solo256_prof.hip",
                "bf_variant_solo256_fp8.hip", "bf_variant_solo256_fp8_taps.hip", "bf_variant_solo256_fp8_prof.hip",
+               "bf_variant_ragged256_fp8.hip", "bf_variant_ragged256.hip", "bf_variant_ragged256_fp8_enc.hip", "bf_variant_ragged256_enc.hip",
                "bf_variant_duo256_enc.hip", "bf_variant_solo256_enc.hip", "bf_variant_duo256_fp8_enc.hip",
                "bf_variant_solo256_fp8_enc.hip", "bf_variant_twin256_fp8_enc.hip", "bf_variant_octo512_enc.hip", "bf_variant_team.hip"]
 # -ffp-contract=off: the kernel's fp32 arithmetic is specified operation by operation

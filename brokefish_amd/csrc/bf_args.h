@@ -121,6 +121,7 @@ struct KArgs {
     // the former takes whole rounds, the latter what round_rest() leaves.
     int list_split;
     int grid;                     // workgroups of the one-position form, 0: one per position
+    int pairs, single_from;       // both forms in one launch: workgroups of two positions in front; without a list, the first position behind theirs
     int n;
     const uint8_t* wstream;
     const float* fparams;
@@ -178,6 +179,11 @@ hipError_t launch_wide512_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_wide512_prof(const KArgs& k, hipStream_t stream);
 // the encoder-only builds
 hipError_t launch_duo256_enc(const KArgs& k, hipStream_t stream);
+// both of the above and their last round's in one launch
+hipError_t launch_ragged256(const KArgs& k, hipStream_t stream);
+hipError_t launch_ragged256_enc(const KArgs& k, hipStream_t stream);
+hipError_t launch_ragged256_fp8(const KArgs& k, hipStream_t stream);
+hipError_t launch_ragged256_fp8_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_duo256_fp8_enc(const KArgs& k, hipStream_t stream);
 hipError_t launch_solo256_fp8_enc(const KArgs& k, hipStream_t stream);

@@ -88,7 +88,7 @@ template <bool SWAP>
 __device__ __forceinline__ v16i f16_step(const v8h&, const v8h&, const v16i& acc) { return acc; }
 
 template <int MODE, bool FP8, bool PROF = false, int NPOS = 2>
-__global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
+__device__ __forceinline__ void evaluate(const KArgs& a, const int block, const int blocks) {   // workgroup `block` of `blocks`
     constexpr bool TAPS = MODE == MODE_TAPS, ENC = MODE == MODE_ENC;
     typedef Cfg<FP8, NPOS> C;
     static_assert(NPOS == 1 || NPOS == 2, "positions per workgroup");
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     int bp[NP];
     bool live[NP];
     {
-        int cnt = a.n, first = NP * (int)blockIdx.x;
+        int cnt = a.n, first = (NP == 1 ? a.single_from : 0) + NP * block;
         if (a.leaf_index) {
             cnt = *a.leaf_count < a.n ? *a.leaf_count : a.n;   // the list has n entries whatever the count says
             if (a.list_split) {
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     // L2 warm-up for launches of one wave of workgroups (NP == 1): such a launch moves through the
     // layers in step, so every first touch of a weight line would be an L2 miss that all the
     // workgroups behind that L2 wait for.  The workgroups of an XCD (dispatched round-robin, so
-    // blockIdx / 8 numbers them) each touch a share of the lines of a layer's blocks one layer ahead,
+    // block / 8 numbers them) each touch a share of the lines of a layer's blocks one layer ahead,
     // one dword per 128-byte line; the values are never used.  A hint only: a share that nobody
     // touches (workgroups that left early, another dispatch order) costs time, not correctness.
     // Below four workgroups per XCD the touches cover too little to pay for the loads they delay
@@ -263,11 +263,11 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
     int warm[WARM > 0 ? WARM : 1] = {};
     auto warm_l2 = [&](int blk0) {
         if constexpr (WARM > 0) {
-            const int per = ((int)gridDim.x + 7) >> 3;
+            const int per = (blocks + 7) >> 3;
 #pragma unroll
             for (int j = 0; j < WARM; j++) {
-                const int line = ((j * per + ((int)blockIdx.x >> 3)) * 8 + wave) * 64 + lane;
-                if (line < 4 * LAYER_LINES && gridDim.x > 24 && gridDim.x <= 256) {
+                const int line = ((j * per + (block >> 3)) * 8 + wave) * 64 + lane;
+                if (line < 4 * LAYER_LINES && blocks > 24 && blocks <= 256) {
                     const int qq = line / LAYER_LINES, off = line % LAYER_LINES;
                     warm[j] = *reinterpret_cast<const int*>(
                         a.wstream + ((size_t)qq * ((size_t)a.n_layers * BPW + HB + 1) + (size_t)blk0) * BLOCK + (size_t)off * 128);
@@ -1249,22 +1249,48 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 #undef BF_PHASE
 }
 
-template <int MODE, bool FP8 = false, bool PROF = false, int NPOS = 2>
-hipError_t launch_duo(const KArgs& k, hipStream_t stream) {
-    // more than 64 KiB of dynamic LDS has to be requested once per kernel and device
-    static std::atomic<unsigned long long> lds_set{0};
-    constexpr int lds_bytes = Cfg<FP8, NPOS>::LDS_BYTES;
+template <int MODE, bool FP8, bool PROF = false, int NPOS = 2>
+__global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
+    evaluate<MODE, FP8, PROF, NPOS>(a, (int)blockIdx.x, (int)gridDim.x);
+}
+
+// Both forms in one launch: a.pairs workgroups of two positions, and behind them those of one position that carry the last
+// round.  As a launch of its own the last round waited until every pair was done, and over a leaf list (whose count is on
+// the device, so that either may have nothing to do) it cost a launch: MEASURED.
+template <int MODE, bool FP8>
+__global__ __launch_bounds__(512, 1) void ragged_kernel(const KArgs a) {
+    const int block = (int)blockIdx.x;
+    if (block < a.pairs) evaluate<MODE, FP8, false, 2>(a, block, a.pairs);
+    else evaluate<MODE, FP8, false, 1>(a, block - a.pairs, (int)gridDim.x - a.pairs);
+}
+
+// One launch of `kernel`; `lds_set`: the devices on which its dynamic LDS has been asked for (more than 64 KiB has to be, once
+// per kernel and device)
+inline hipError_t launch_kernel(void (*kernel)(KArgs), std::atomic<unsigned long long>& lds_set, int lds_bytes, int grid, const KArgs& k, hipStream_t stream) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
     const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
     if (!(lds_set.load(std::memory_order_relaxed) & bit)) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_kernel<MODE, FP8, PROF, NPOS>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (e != hipSuccess) return e;
         lds_set.fetch_or(bit, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((duo_kernel<MODE, FP8, PROF, NPOS>), dim3(k.grid ? k.grid : (k.n + NPOS - 1) / NPOS), dim3(512), lds_bytes, stream, k);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds_bytes, stream, k);
     return hipGetLastError();
+}
+
+template <int MODE, bool FP8 = false, bool PROF = false, int NPOS = 2>
+hipError_t launch_duo(const KArgs& k, hipStream_t stream) {
+    static std::atomic<unsigned long long> lds_set{0};
+    return launch_kernel(&duo_kernel<MODE, FP8, PROF, NPOS>, lds_set, Cfg<FP8, NPOS>::LDS_BYTES, k.grid ? k.grid : (k.n + NPOS - 1) / NPOS, k, stream);
+}
+
+// k.pairs workgroups of two positions and k.grid of one
+template <int MODE, bool FP8>
+hipError_t launch_ragged(const KArgs& k, hipStream_t stream) {
+    static std::atomic<unsigned long long> lds_set{0};
+    static_assert(Cfg<FP8, 2>::LDS_BYTES >= Cfg<FP8, 1>::LDS_BYTES, "both forms");
+    return launch_kernel(&ragged_kernel<MODE, FP8>, lds_set, Cfg<FP8, 2>::LDS_BYTES, k.pairs + k.grid, k, stream);
 }
 
 }  // namespace duo

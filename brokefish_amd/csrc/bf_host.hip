@@ -375,7 +375,8 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
         // 0.39 instead of 0.48).  With a leaf list the count is on the device: both forms are launched and each
         // takes its share of the list (a launch that finds nothing to do costs 3 us; 200 live leaves of 1000 take a third
         // less).  Not with other taps or the profile.
-        const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n);
+        const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n), pairs = (k.leaf_index ? k.n + 1 : k.n - rest) / 2;
+        const bool f8 = a->quant == BF_QUANT_E4M3, teams = rest && !k.leaf_index && to.by_teams(a, rest);
         bf::KArgs front = k, back = k;
         if (k.leaf_index) {
             front.list_split = back.list_split = 1;
@@ -384,15 +385,19 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
             front = slice(k, a->shape.d_model, 0, k.n - rest);
             back = slice(k, a->shape.d_model, k.n - rest, rest);
         }
-        const bool f8 = a->quant == BF_QUANT_E4M3;
-        e = (wide ? (enc ? bf::launch_wide512_enc : bf::launch_wide512)
-             : f8 ? (enc ? bf::launch_duo256_fp8_enc : bf::launch_duo256_fp8)
-                  : (enc ? bf::launch_duo256_enc : bf::launch_duo256))(front, stream);
-        if (rest && e == hipSuccess)
-            e = !k.leaf_index && to.by_teams(a, back.n) ? launch_teams(back)
-                : (wide ? (enc ? bf::launch_octo512_enc : bf::launch_octo512)
-                   : f8 ? (enc ? bf::launch_solo256_fp8_enc : bf::launch_solo256_fp8)
-                        : (enc ? bf::launch_solo256_enc : bf::launch_solo256))(back, stream);
+        if (rest && !wide && !teams) {   // the 256-wide network has both forms in one launch
+            bf::KArgs both = k;
+            both.list_split = front.list_split;
+            both.pairs = pairs;
+            both.single_from = k.leaf_index ? 0 : k.n - rest;
+            both.grid = rest;
+            e = (f8 ? (enc ? bf::launch_ragged256_fp8_enc : bf::launch_ragged256_fp8) : (enc ? bf::launch_ragged256_enc : bf::launch_ragged256))(both, stream);
+        } else {
+            e = (wide ? (enc ? bf::launch_wide512_enc : bf::launch_wide512)
+                 : f8 ? (enc ? bf::launch_duo256_fp8_enc : bf::launch_duo256_fp8)
+                      : (enc ? bf::launch_duo256_enc : bf::launch_duo256))(front, stream);
+            if (rest && e == hipSuccess) e = teams ? launch_teams(back) : (enc ? bf::launch_octo512_enc : bf::launch_octo512)(back, stream);
+        }
     } else if (enc) {
         if (wide) e = bf::launch_octo512_enc(k, stream);
         else if (a->quant == BF_QUANT_E4M3)

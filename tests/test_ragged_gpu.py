@@ -1,0 +1,31 @@
+"""Sizes whose last round of 512 positions goes to workgroups of one position, in the same launch as the pairs: outputs and the
+encoder alone against the kernel of one position per workgroup of four wavefronts, bit for bit.  (Leaf lists:
+test_leaf_split_gpu.py, test_rounds_gpu.py.)"""
+import pytest
+import torch
+
+from brokefish_amd import encoder_impl, positions
+from brokefish_amd.net import BrokefishNet
+
+pytestmark = pytest.mark.gpu
+N = 1281
+
+
+@pytest.fixture(scope="module", params=["int8", "fp8"])
+def made(request):
+    torch.manual_seed(0)
+    net = BrokefishNet(n_layers=2).eval().randomise_layers_(seed=9)
+    auto, board = (encoder_impl("hip")(net, out_dtype=torch.float32, kernel=k, **{request.param: True}) for k in ("auto", "board"))
+    batch = [t.cuda() for t in positions.random_positions(N, plies=100, seed=9)]
+    x = torch.randn(N, 32, 256, device="cuda", generator=torch.Generator("cuda").manual_seed(9)) * 0.14
+    alive = ((batch[0].to(torch.int32) >> 11) & 1) == 0
+    return auto, batch, [t.clone() for t in board.forward_masked(*batch)], x, alive, board.forward(x, alive).clone()
+
+
+# the smallest and largest last round that pairs leave (65 to 256), its neighbours on either side, behind one round and two
+@pytest.mark.parametrize("n", [576, 577, 600, 767, 768, 769, 1088, 1089, 1280, N])
+def test_a_last_round_in_the_same_launch(made, n):
+    auto, batch, want, x, alive, stream = made
+    for g, w in zip(auto.forward_masked(*[t[:n] for t in batch]), want):
+        assert torch.equal(g, w[:n])
+    assert torch.equal(auto.forward(x[:n].contiguous(), alive[:n].contiguous()), stream[:n])
