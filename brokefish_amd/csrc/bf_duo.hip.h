@@ -1021,10 +1021,12 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
     // Lane (row, k) reads, of fragment f, the lane of its row and of half k % 2, from element k / 2 on: what it multiplies lies in places 0
     // and 2 then.  (The last lanes' reads end four bytes behind the fragment, in the next one or the block of padding.)
     const size_t qstride = (size_t)a.n_layers * BPW + HB + 1;
-    auto head_tile = [&](int n) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.wstream + (n * qstride + (size_t)a.n_layers * BPW) * BLOCK), 0, HB * BLOCK + 16, 0x00027000);
+    // A wave without a piece of tile 2 sees it empty, and its loads move nothing: with a branch around them the number of loads under way
+    // would not be known, and the chains behind would wait for all of them at every step.
+    auto head_tile = [&](int n, bool used) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.wstream + (n * qstride + (size_t)a.n_layers * BPW) * BLOCK), 0, used ? HB * BLOCK + 16 : 0, 0x00027000);
     };
-    const __amdgpu_buffer_rsrc_t policy_tile = head_tile(ht), tile2 = head_tile(2);
+    const __amdgpu_buffer_rsrc_t policy_tile = head_tile(ht, true), tile2 = head_tile(2, extra);
     const int from0 = (c16 + 32 * (G & 1)) * 16 + 4 * (G >> 1), from = from0 + 256 * rh;
     auto load_head = [&](const __amdgpu_buffer_rsrc_t& buf, int lane_at, int f, int at) {
         frt[at] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(buf, lane_at, f * FRAG, 0));
@@ -1095,7 +1097,7 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
             }
             __builtin_amdgcn_sched_barrier(0);
             if (f + RING < 8 * HB) load_head(policy_tile, from, f + RING, f % RING);
-            else if (extra) load_head(tile2, from0, f + RING - 8 * HB, (f + RING) % RING);
+            else load_head(tile2, from0, f + RING - 8 * HB, (f + RING) % RING);
         }
     }
     v4f rest = {0, 0, 0, 0};
