@@ -38,9 +38,7 @@
 // widened in LDS (-0.4 %: LDS then delivers as much as it can), two blocks side by side against each operand (-0.3 %).
 #pragma once
 
-#include "bf_board.hip.h"
-
-typedef float v2f __attribute__((ext_vector_type(2)));
+#include "bf_heads.hip.h"
 
 namespace bf {
 namespace duo {
@@ -1002,58 +1000,19 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
     if (enc_only) return;   // the same for every wave of the launch
 
     // ---- final norm and heads --------------------------------------------------------------------------
-    // The products of the heads come in pieces of 16 rows of a head tile and 16 tokens (v_mfma_f32_16x16x4f32: the
-    // fused-multiply-add chain of the 32x32x2 form, four links a step).  A wave takes 16 rows of a policy tile for both
-    // halves of its position's tokens (one position: for one half), and one wave of each SIMD (one position: of two) a half of a
-    // position's tokens with the first rows of tile 2, where promotion and value lie.  For two positions that is 10.2 k clocks of every
-    // SIMD; as 32x32 products of whole tiles (tile 2's 25 rows of zeros among them) it was 16.4 k of three SIMDs, and the fourth idled.
-    // With the final norm's parameters and the legal moves asked for ahead and the best move found without LDS permutations: phases
-    // heads + stores 29.9 k -> 24.7 k ticks of 483 k; 300 positions 171.6 -> 169.6 us, 100 115.4 -> 114.4, 4096 1434 -> 1425, e4m3 1911 -> 1904.
-    constexpr int HALVES = NP;                       // token halves of a policy wave
-    const int ht = q & 1, rh = q >> 1;               // its rows: 16 rh .. of head tile ht
-    const int mine = NP == 2 ? sub : 0;              // its position
-    const bool extra = sub == 1 && (NP == 2 || q < 2);
-    const int xmine = NP == 2 ? q & 1 : 0, xth = NP == 2 ? q >> 1 : q;   // tile 2: position, token half
-    const int G = lane >> 4, c16 = lane & 15;
-    const int b = mine ? bp[NP - 1] : bp[0], xb = xmine ? bp[NP - 1] : bp[0];
-    const bool store = mine ? live[NP - 1] : live[0], xstore = xmine ? live[NP - 1] : live[0];
-    const int xctrl = xmine ? ctrl[NP - 1] : ctrl[0];
-    // Lane (row, k) reads, of fragment f, the lane of its row and of half k % 2, from element k / 2 on: what it multiplies lies in places 0
-    // and 2 then.  (The last lanes' reads end four bytes behind the fragment, in the next one or the block of padding.)
-    const size_t qstride = (size_t)a.n_layers * BPW + HB + 1;
-    // A wave without a piece of tile 2 sees it empty, and its loads move nothing: with a branch around them the number of loads under way
-    // would not be known, and the chains behind would wait for all of them at every step.
-    auto head_tile = [&](int n, bool used) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.wstream + (n * qstride + (size_t)a.n_layers * BPW) * BLOCK), 0, used ? HB * BLOCK + 16 : 0, 0x00027000);
-    };
-    const __amdgpu_buffer_rsrc_t policy_tile = head_tile(ht, true), tile2 = head_tile(2, extra);
-    const int from0 = (c16 + 32 * (G & 1)) * 16 + 4 * (G >> 1), from = from0 + 256 * rh;
-    auto load_head = [&](const __amdgpu_buffer_rsrc_t& buf, int lane_at, int f, int at) {
-        frt[at] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(buf, lane_at, f * FRAG, 0));
-    };
+    Heads<NP, HB, RING> heads(a, BPW, lane, wave, bp, live, ctrl, C::HID_OFF, C::HID_P);
     // the final norm's parameters, a quarter's worth of exchanges ahead of their use
     v4f nfg[4], nfb[4];
     load_tile16(gp + C::G_NFG + 32 * tile, g, nfg);
     load_tile16(gp + C::G_NFB + 32 * tile, g, nfb);
-#pragma unroll
-    for (int j = 0; j < RING; j++) load_head(policy_tile, from, j, j);
-    unsigned long long legal[HALVES];
-    const bool masked = a.mask != nullptr;
-#pragma unroll
-    for (int i = 0; i < HALVES; i++) legal[i] = masked ? a.mask[(size_t)b * T + 16 * (NP == 2 ? i : sub) + c16] : ~0ull;
+    heads.ask();
     __builtin_amdgcn_sched_barrier(0);
     auto final_norm = [&](const float (&of)[NP][16], float (&y)[NP][16]) {
         layernorm2_by(of, [&](int j) { return nfg[j]; }, [&](int j) { return nfb[j]; }, y);
     };
     float hn[NP][16];
     final_norm(x, hn);
-    // A position's row as operand fragments (n, j): lane (t, g) holds the four floats of register quad j, elements 0 and 2 together
-    auto publish = [&](int p, const float (&v)[16]) {
-        float* const to = reinterpret_cast<float*>(hid + p * C::HID_P);
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            *reinterpret_cast<v4f*>(to + ((tile * 4 + j) * 64 + lane) * 4) = v4f{v[4 * j], v[4 * j + 2], v[4 * j + 1], v[4 * j + 3]};
-    };
+    auto publish = [&](int p, const float (&v)[16]) { heads.publish(p, tile, v); };
 #pragma unroll
     for (int p = 0; p < NP; p++) {
         if (TAPS && a.taps.normed && live[p])
@@ -1063,136 +1022,9 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
         publish(p, hn[p]);
     }
     barrier();
-    // lane (token, k) of a step: element k / 2 (and 2 + k / 2 in the next step) of the fragment lane of half k % 2
-    auto operands_of = [&](int pos) {
-        int at = C::HID_OFF + pos * C::HID_P + (32 * (G & 1) + c16) * 16 + 8 * (G >> 1);
-        asm volatile("" : "+v"(at));   // one address register; the rest are the instructions' own offsets
-        return lds + at;
-    };
-    auto operand = [&](const uint8_t* of, int th, int f) { return *reinterpret_cast<const v2f*>(of + f * FRAG + th * 256); };
-    auto steps = [&](const v4i& w, const v2f& h, v4f& acc) {
-        const v4f wf = __builtin_bit_cast(v4f, w);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[0], h[0], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[2], h[1], acc, 0, 0, 0);
-    };
-    constexpr int EARLY = 4;   // operands come from LDS this many fragments early
-    constexpr int RING_POOL = 8;   // fragments of a set in the pooled heads
-    static_assert(RING_POOL <= RING && (8 * HB) % RING_POOL == 0, "whole sets");
-    v4f head[HALVES];
-#pragma unroll
-    for (int i = 0; i < HALVES; i++) head[i] = v4f{0, 0, 0, 0};
-    {
-        const uint8_t* const of = operands_of(mine) + (NP == 2 ? 0 : 256 * sub);
-        v2f h[EARLY][HALVES];
-#pragma unroll
-        for (int f = 0; f < EARLY; f++)
-#pragma unroll
-            for (int i = 0; i < HALVES; i++) h[f][i] = operand(of, i, f);
-#pragma unroll
-        for (int f = 0; f < 8 * HB; f++) {
-#pragma unroll
-            for (int i = 0; i < HALVES; i++) {
-                steps(frt[f % RING], h[f % EARLY][i], head[i]);
-                if (f + EARLY < 8 * HB) h[f % EARLY][i] = operand(of, i, f + EARLY);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if (f + RING < 8 * HB) load_head(policy_tile, from, f + RING, f % RING);
-            else load_head(tile2, from0, f + RING - 8 * HB, (f + RING) % RING);
-        }
-    }
-    v4f rest = {0, 0, 0, 0};
-    if (extra) {
-        const uint8_t* const of = operands_of(xmine) + 256 * xth;
-        v2f h[EARLY];
-#pragma unroll
-        for (int f = 0; f < EARLY; f++) h[f] = operand(of, 0, f);
-#pragma unroll
-        for (int f = 0; f < 8 * HB; f++) {
-            steps(frt[(8 * HB + f) % RING], h[f % EARLY], rest);
-            if (f + EARLY < 8 * HB) h[f % EARLY] = operand(of, 0, f + EARLY);
-            __builtin_amdgcn_sched_barrier(0);
-            if (f + RING < 8 * HB) load_head(tile2, from0, f + RING, (8 * HB + f) % RING);
-        }
-    }
+    heads.products();
     BF_PHASE(PH_HEADS);
-    auto value_of = [&](const v4f& hd) -> float {
-        if (a.n_value == 1) return tanh_dev(hd[0]);
-        const float r0 = hd[0], r1 = hd[1], r2 = hd[2];   // classes loss, draw, win
-        const float mx = __builtin_fmaxf(__builtin_fmaxf(r0, r1), r2);
-        const float e0 = exp_neg(r0 - mx), e1 = exp_neg(r1 - mx), e2 = exp_neg(r2 - mx);
-        return (e2 - e0) / ((e0 + e1) + e2);
-    };
-    // tile 2: rows 64 .. 67 (lanes G = 0) are the promotions, rows 68 .. 70 (G = 1) the value, whose token is the mover's king
-    if (extra && xstore) {
-        const int tk = 16 * xth + c16;
-        if (a.vmode == 0 && G == 1 && tk == (xctrl < 0 ? 31 : 15)) a.value[xb] = value_of(rest);
-        if (G == 0) {
-            if (a.out_fp32) *reinterpret_cast<v4f*>((float*)a.promo + ((size_t)xb * T + tk) * 4) = rest;
-            else *reinterpret_cast<v4h*>((_Float16*)a.promo + ((size_t)xb * T + tk) * 4) = v4h{(_Float16)rest[0], (_Float16)rest[1], (_Float16)rest[2], (_Float16)rest[3]};
-        }
-    }
-    // policy: squares 32 ht + 16 rh + 4 G .. of the wave's tokens, optional legal-move AND and argmax
-    constexpr int NONE = 0x7fffffff;
-    float bv = -__builtin_inff();
-    int bi = NONE;
-    const int sq0 = 32 * ht + 16 * rh + 4 * G;
-#pragma unroll
-    for (int i = 0; i < HALVES; i++) {
-        const int tk = 16 * (NP == 2 ? i : sub) + c16;
-        const unsigned here_legal = (unsigned)(legal[i] >> sq0);
-        float v[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const bool ok = (here_legal >> k) & 1u;
-            v[k] = ok ? head[i][k] : -__builtin_inff();
-            // a lane visits its moves in increasing order, so '>' keeps the lowest
-            if (ok && (bi == NONE || v[k] > bv)) { bv = v[k]; bi = tk * 64 + sq0 + k; }
-        }
-        const size_t at = ((size_t)b * T + tk) * 64 + sq0;
-        if (store) {
-            if (a.out_fp32) *reinterpret_cast<v4f*>((float*)a.policy + at) = v4f{v[0], v[1], v[2], v[3]};
-            else *reinterpret_cast<v4h*>((_Float16*)a.policy + at) = v4h{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-        }
-    }
-    if (masked && a.best) {
-        auto merge = [&](float ov, int oi) {
-            const bool take = oi != NONE && (bi == NONE || ov > bv || (ov == bv && oi < bi));
-            bv = take ? ov : bv;
-            bi = take ? oi : bi;
-        };
-        auto over_dpp = [&](auto ctrl_) {   // another lane of the row of 16
-            constexpr int c = decltype(ctrl_)::value;
-            const int ov = __builtin_amdgcn_update_dpp(0, __float_as_int(bv), c, 0xf, 0xf, true), oi = __builtin_amdgcn_update_dpp(0, bi, c, 0xf, 0xf, true);
-            merge(__int_as_float(ov), oi);
-        };
-        auto over_swap = [&](auto swap) {   // both lanes get both values and keep the better one
-            const auto v2 = swap(__float_as_int(bv)), i2 = swap(bi);
-            bv = __int_as_float((int)v2[0]);
-            bi = (int)i2[0];
-            merge(__int_as_float((int)v2[1]), (int)i2[1]);
-        };
-        over_dpp(std::integral_constant<int, 0xb1>());    // xor 1
-        over_dpp(std::integral_constant<int, 0x4e>());    // xor 2
-        over_dpp(std::integral_constant<int, 0x141>());   // the mirrored eight
-        over_dpp(std::integral_constant<int, 0x140>());   // the mirrored sixteen
-        over_swap([](int v) { return __builtin_amdgcn_permlane16_swap(v, v, false, false); });
-        over_swap([](int v) { return __builtin_amdgcn_permlane32_swap(v, v, false, false); });
-        // the winners of a position's waves meet in the exchange slot no row sum uses
-        int* const met = reinterpret_cast<int*>(xch + 2 * XS);
-        if (lane == 0) {
-            met[2 * wave] = __float_as_int(bv);
-            met[2 * wave + 1] = bi;
-        }
-        barrier();
-        if (q == 0 && (NP == 2 || sub == 0) && store) {
-#pragma unroll
-            for (int w = 1; w < 8 / NP; w++) {
-                const int o = NP == 2 ? 4 * sub + w : w;
-                merge(__int_as_float(met[2 * o]), met[2 * o + 1]);
-            }
-            if (lane == 0) a.best[b] = bi == NONE ? -1 : bi;
-        }
-    }
+    heads.store(xch + 2 * XS, barrier);   // the exchange slot no row sum uses
     // ---- pooled value heads (reference brokefish/nn/model.py:576-617) --------------------------------
     // The value row is the mean over the live tokens of the normalised stream ("pooled", mode 1) or
     // the final LayerNorm of the mean of the residual stream ("prenorm", mode 2); it goes through
@@ -1224,21 +1056,7 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
 #pragma unroll
         for (int p = 0; p < NP; p++) publish(p, hv[p]);
         barrier();
-        if (extra && xth == 0) {
-            // tile 2's rows once more, against the pooled row (every token column holds the same row), in the same order as above
-            v4f hd = {0, 0, 0, 0};
-            const uint8_t* const of = operands_of(xmine);
-            for (int f0 = 0; f0 < 8 * HB; f0 += RING_POOL) {
-#pragma unroll
-                for (int j = 0; j < RING_POOL; j++) load_head(tile2, from0, f0 + j, j);
-#pragma unroll
-                for (int j = 0; j < RING_POOL; j++) steps(frt[j], operand(of, 0, f0 + j), hd);
-            }
-            if (lane == 16 && xstore) {
-                const float v = value_of(hd);
-                a.value[xb] = xctrl > 0 ? v : -v;
-            }
-        }
+        heads.pooled();
     }
     if constexpr (PROF) {
         BF_PHASE(PH_STORE);
@@ -1258,7 +1076,8 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 
 // Both forms in one launch: a.pairs workgroups of two positions, and behind them those of one position that carry the last
 // round.  As a launch of its own the last round waited until every pair was done, and over a leaf list (whose count is on
-// the device, so that either may have nothing to do) it cost a launch: MEASURED.
+// the device, so that either may have nothing to do) it cost a launch: 600 positions 290.7 -> 288.3 us, 700 291.8 -> 289.9, 2200 823.5
+// -> 821.5, e4m3, 700 positions 380.6 -> 377.2, a list of 370 of 1000 with its expansion 184.0 -> 181.9.
 template <int MODE, bool FP8>
 __global__ __launch_bounds__(512, 1) void ragged_kernel(const KArgs a) {
     const int block = (int)blockIdx.x;

@@ -30,9 +30,7 @@
 // fp32) take act and hid.
 #pragma once
 
-#include "bf_board.hip.h"
-
-typedef float v2f __attribute__((ext_vector_type(2)));
+#include "bf_heads.hip.h"
 
 namespace bf {
 namespace wide {
@@ -733,116 +731,22 @@ __global__ __launch_bounds__(512, 1) void wide_kernel(const KArgs a) {
     }
 
     // ---- final norm and heads --------------------------------------------------------------------------
-    const int hblk0 = (a.n_layers - a.l0) * BPW;
-#pragma unroll
-    for (int f = 0; f < 8; f++) load_frag(hblk0, f);
+    constexpr int STREAM_P = NT * 4 * FRAG;   // a position's normalised stream, bytes: both take act and hid
+    Heads<NP, HB, 8> heads(a, BPW, lane, wave, bp, live, ctrl, C::ACT_OFF, STREAM_P);
+    heads.ask();
     float hn[NP][TWW][16];
     layernorm2(x, gp + C::G_NFG + 32 * tile0, gp + C::G_NFB + 32 * tile0, hn, nothing);   // its barriers: every wave is done with the hidden rows
-    float* const stream = reinterpret_cast<float*>(act);
-    constexpr int STREAM_P = NT * 4 * FRAG / 4;   // floats of a position's normalised stream
-    // publish as B-operand fragments (n, j): lane holds the four floats of register quad j
     auto publish = [&](const float (&v)[NP][TWW][16]) {
 #pragma unroll
         for (int p = 0; p < NP; p++)
 #pragma unroll
-            for (int i = 0; i < TWW; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    *reinterpret_cast<v4f*>(stream + p * STREAM_P + (((tile0 + i) * 4 + j) * 64 + lane) * 4) =
-                        v4f{v[p][i][4 * j], v[p][i][4 * j + 1], v[p][i][4 * j + 2], v[p][i][4 * j + 3]};
+            for (int i = 0; i < TWW; i++) heads.publish(p, tile0 + i, v[p][i]);
     };
     publish(hn);
     barrier();
-    // Wave (m, p) multiplies head tile m (rows 32m..32m+31 of [policy; promo; value; 0]) with the normalised stream of
-    // position p, one fused-multiply-add chain in (tile, quad, element) order; quarter 3's tile is zero.
-    const float* const hnb = stream + sub * STREAM_P;
-    v16f head = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (q < 3) {
-#pragma unroll 1
-        for (int hb = 0; hb < HB; hb++)
-#pragma unroll
-            for (int f = 0; f < 8; f++) {
-                const v4f w = __builtin_bit_cast(v4f, frt[f]);
-                const v4f hv = *reinterpret_cast<const v4f*>(hnb + ((8 * hb + f) * 64 + lane) * 4);
-#pragma unroll
-                for (int k = 0; k < 4; k++) head = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k], hv[k], head, 0, 0, 0);
-                load_frag(hblk0 + hb + 1, f);   // the stream is padded by one block
-            }
-    }
+    heads.products();
     BF_PHASE(PH_HEADS);
-    const int b = sub ? bp[1] : bp[0];
-    const bool store = sub ? live[1] : live[0];
-    const int ctrl_m = sub ? ctrl[1] : ctrl[0];
-    auto value_of = [&](const v16f& hd) -> float {
-        if (a.n_value == 1) return tanh_dev(hd[0]);
-        const float r0 = hd[0], r1 = hd[1], r2 = hd[2];   // classes loss, draw, win
-        const float mx = __builtin_fmaxf(__builtin_fmaxf(r0, r1), r2);
-        const float e0 = exp_neg(r0 - mx), e1 = exp_neg(r1 - mx), e2 = exp_neg(r2 - mx);
-        return (e2 - e0) / ((e0 + e1) + e2);
-    };
-    if (q == 2 && store) {   // value (king head): lane half 1 holds rows 68..70; promo: rows 64..67 are lane half 0's
-        const int king = ctrl_m < 0 ? 31 : 15;
-        if (a.vmode == 0 && lane == 32 + king) a.value[b] = value_of(head);
-        if (g == 0) {
-            if (a.out_fp32) {
-                *reinterpret_cast<v4f*>((float*)a.promo + ((size_t)b * T + t) * 4) = v4f{head[0], head[1], head[2], head[3]};
-            } else {
-                const v4h v = {(_Float16)head[0], (_Float16)head[1], (_Float16)head[2], (_Float16)head[3]};
-                *reinterpret_cast<v4h*>((_Float16*)a.promo + ((size_t)b * T + t) * 4) = v;
-            }
-        }
-    }
-    // policy (quarters 0 and 1: squares 0..31 and 32..63), optional legal-move AND and argmax
-    float bv = -__builtin_inff();
-    int bi = 0x7fffffff;
-    if (q < 2) {
-        unsigned long long mw = ~0ull;
-        if (a.mask) mw = a.mask[(size_t)b * T + t];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float v[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int sq = 32 * q + 8 * j + 4 * g + k;
-                const bool legal = (mw >> sq) & 1ull;
-                v[k] = legal ? head[4 * j + k] : -__builtin_inff();
-                // squares are visited in increasing order within a lane, so '>' keeps the lowest
-                if (legal && (bi == 0x7fffffff || v[k] > bv)) { bv = v[k]; bi = t * 64 + sq; }
-            }
-            const size_t at = ((size_t)b * T + t) * 64 + 32 * q + 8 * j + 4 * g;
-            if (store) {
-                if (a.out_fp32) {
-                    *reinterpret_cast<v4f*>((float*)a.policy + at) = v4f{v[0], v[1], v[2], v[3]};
-                } else {
-                    const v4h vv = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-                    *reinterpret_cast<v4h*>((_Float16*)a.policy + at) = vv;
-                }
-            }
-        }
-    }
-    if (a.mask && a.best) {
-        auto better = [&](float ov, int oi) { return (oi != 0x7fffffff) && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi)); };
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            const float ov = __shfl_xor(bv, d);
-            const int oi = __shfl_xor(bi, d);
-            const bool take = better(ov, oi);
-            bv = take ? ov : bv;
-            bi = take ? oi : bi;
-        }
-        // the two policy waves' winners of a position meet where the activation scales were
-        if (q < 2 && lane == 0) {
-            tok[sub * 4 + q * 2] = bv;
-            tok[sub * 4 + q * 2 + 1] = __int_as_float(bi);
-        }
-        barrier();
-        if (q == 0 && lane == 0 && store) {
-            const float ov = tok[sub * 4 + 2];
-            const int oi = __float_as_int(tok[sub * 4 + 3]);
-            if (better(ov, oi)) bi = oi;
-            a.best[b] = bi == 0x7fffffff ? -1 : bi;
-        }
-    }
+    heads.store(tok, barrier);   // where the activation scales were
     // ---- pooled value heads (see bf_duo.hip.h) ----------------------------------------------------------
     if (a.vmode != 0) {
         float pv[NP][TWW][16], hv[NP][TWW][16];
@@ -873,19 +777,7 @@ __global__ __launch_bounds__(512, 1) void wide_kernel(const KArgs a) {
         barrier();   // every wave has finished reading the normalised streams
         publish(hv);
         barrier();
-        if (q == 2) {
-            v16f hd = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            for (int f = 0; f < 8 * HB; f++) {
-                const v4f w = *reinterpret_cast<const v4f*>(wsrc + (size_t)hblk0 * BLOCK + (size_t)f * FRAG + lane16);
-                const v4f hvv = *reinterpret_cast<const v4f*>(hnb + (f * 64 + lane) * 4);
-#pragma unroll
-                for (int k = 0; k < 4; k++) hd = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k], hvv[k], hd, 0, 0, 0);
-            }
-            if (lane == 32 && store) {
-                const float v = value_of(hd);
-                a.value[b] = ctrl_m > 0 ? v : -v;
-            }
-        }
+        heads.pooled();
     }
     if constexpr (PROF) {
         BF_PHASE(PH_STORE);
