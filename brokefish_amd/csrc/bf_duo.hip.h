@@ -509,7 +509,8 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
         // between products (attention, the LayerNorms).
         // BETWEEN(s) runs after step s has been issued: an eighth of the previous product's epilogue,
         // which the vector ALU works through while the matrix pipe runs; nothing is scheduled across
-        // the end of a step.
+        // the end of a step.  One position per workgroup: the epilogue starts a step later, so that its first value is there
+        // when it is asked for (200 positions 112.5 -> 111.8 us; two positions, whose other wavefront has work meanwhile: no change).
         // The operand fragments come from LDS AHEAD steps early, also across the products of a phase: in its last
         // steps a product fetches the first operands of the next one (at NEXT, if there is one whose operands are
         // written already: MORE).  BF_DUO_OPERANDS opens a phase with the first product's.
@@ -524,7 +525,9 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
             if (s_ + AHEAD < 8) ops_[(s_ + AHEAD) % (AHEAD + 1)] = ldsfrag(b_ + (s_ + AHEAD) * FRAG); \
             else if (MORE) ops_[(s_ + AHEAD) % (AHEAD + 1)] = ldsfrag(n_ + (s_ + AHEAD - 8) * FRAG);   \
             (R) = frag_mma<SWAP>(frt[(8 * (k) + s_) % RING], ops_[s_ % (AHEAD + 1)], (R));           \
-            BETWEEN(s_);                                                                             \
+            if (NP == 2) BETWEEN(s_);                                                                \
+            else if (s_ > 0) BETWEEN(s_ - 1);                                                        \
+            if (NP == 1 && s_ == 7) BETWEEN(7);                                                      \
             __builtin_amdgcn_sched_barrier(0);                                                       \
             if ((p) == NP - 1) fetch_frag(8 * (k) + s_ + RING, lbase, lfollow);                      \
         }                                                                                            \
