@@ -235,20 +235,28 @@ std::array<torch::Tensor, N> fresh_together(const std::array<Want, N>& want, boo
     return t;
 }
 
-// hip_impl.movegen: (mask [n, 32] int64, in_check [n] bool)
-std::pair<torch::Tensor, torch::Tensor> movegen(const torch::Tensor& boards, const torch::Tensor& control,
-                                                const c10::optional<std::pair<torch::Tensor, torch::Tensor>>& out) {
-    const int64_t n = boards.dim() ? boards.size(0) : 0;
+void check_boards(const torch::Tensor& boards, const torch::Tensor& control, int64_t n) {
     BF_VALUE_CHECK(shape_is(boards, {n, BF_TOKENS}) && boards.scalar_type() == torch::kShort && shape_is(control, {n}) &&
                        control.scalar_type() == torch::kShort, "boards must be [n,32] int16 and control [n] int16");
     BF_VALUE_CHECK(boards.is_cuda() && control.is_cuda(), "boards and control must be on the GPU");
     BF_VALUE_CHECK(boards.is_contiguous() && control.is_contiguous(), "boards and control must be contiguous");
+}
+// legal-move words and check flags
+std::array<torch::Tensor, 2> fresh_moves(int64_t n, const c10::Device& dev) {
+    return fresh_together<2>({{{{n, BF_TOKENS}, torch::kLong}, {{n}, torch::kBool}}}, false, dev);
+}
+
+// hip_impl.movegen: (mask [n, 32] int64, in_check [n] bool)
+std::pair<torch::Tensor, torch::Tensor> movegen(const torch::Tensor& boards, const torch::Tensor& control,
+                                                const c10::optional<std::pair<torch::Tensor, torch::Tensor>>& out) {
+    const int64_t n = boards.dim() ? boards.size(0) : 0;
+    check_boards(boards, control, n);
     const c10::Device dev = boards.device();
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
     torch::Tensor mask, chk;
     if (out) std::tie(mask, chk) = *out;
     else {
-        auto made = fresh_together<2>({{{{n, BF_TOKENS}, torch::kLong}, {{n}, torch::kBool}}}, false, dev);
+        auto made = fresh_moves(n, dev);
         mask = std::move(made[0]);
         chk = std::move(made[1]);
     }
@@ -285,10 +293,11 @@ std::pair<torch::Tensor, torch::Tensor> compact_leaves(const torch::Tensor& flag
     return {index, count};
 }
 
-// hip_impl.expand_edges: the dict of edge tensors
+// hip_impl.expand_edges: the dict of edge tensors.  GENERATE: mask_ and in_check are generated first, in the same launch
+template <bool GENERATE = false>
 py::dict expand_edges(const torch::Tensor& policy_, const torch::Tensor& promo_, const torch::Tensor& value_, const torch::Tensor& mask_,
                       const torch::Tensor& boards_, const torch::Tensor& control_, int64_t max_edges, const OptTensor& active_,
-                      const c10::optional<py::dict>& out, const OptLeaves& leaves) {
+                      const c10::optional<py::dict>& out, const OptLeaves& leaves, const torch::Tensor* in_check = nullptr) {
     const int64_t n = policy_.dim() ? policy_.size(0) : 0;
     const auto lt = policy_.scalar_type();
     BF_VALUE_CHECK(shape_is(policy_, {n, BF_TOKENS, BF_POLICY}) && shape_is(promo_, {n, BF_TOKENS, BF_PROMO}) && lt == promo_.scalar_type() &&
@@ -322,15 +331,15 @@ py::dict expand_edges(const torch::Tensor& policy_, const torch::Tensor& promo_,
     }
     // temporaries made here were allocated on the current stream, where the launch is queued: their memory
     // is handed out again only to work that this stream runs after the kernel
-    const torch::Tensor policy = policy_.contiguous(), promo = promo_.contiguous(), value = value_.contiguous(),
-                        mask = mask_.contiguous(), boards = boards_.contiguous(), control = control_.contiguous();
+    const c10::MaybeOwned<torch::Tensor> policy = policy_.expect_contiguous(), promo = promo_.expect_contiguous(), value = value_.expect_contiguous(),
+                                         mask = mask_.expect_contiguous(), boards = boards_.expect_contiguous(), control = control_.expect_contiguous();
     bf_expand_args a{};
-    a.policy = policy.data_ptr();
-    a.promo = promo.data_ptr();
-    a.value = static_cast<const float*>(value.data_ptr());
-    a.mask = static_cast<const uint64_t*>(mask.data_ptr());
-    a.boards = static_cast<const uint16_t*>(boards.data_ptr());
-    a.control = static_cast<const int16_t*>(control.data_ptr());
+    a.policy = policy->data_ptr();
+    a.promo = promo->data_ptr();
+    a.value = static_cast<const float*>(value->data_ptr());
+    a.mask = static_cast<const uint64_t*>(mask->data_ptr());
+    a.boards = static_cast<const uint16_t*>(boards->data_ptr());
+    a.control = static_cast<const int16_t*>(control->data_ptr());
     torch::Tensor act;
     if (active_) {
         act = active_->scalar_type() == torch::kBool ? active_->contiguous() : active_->to(torch::kByte).contiguous();
@@ -352,8 +361,30 @@ py::dict expand_edges(const torch::Tensor& policy_, const torch::Tensor& promo_,
     a.count = static_cast<int32_t*>(made[3].data_ptr());
     a.dropped = static_cast<float*>(made[4].data_ptr());
     a.node_value = made[5].data_ptr();
-    const int rc = bf_expand(&a, stream_of(dev));
+    int rc;
+    if constexpr (GENERATE) {
+        a.mask = nullptr;
+        rc = bf_movegen_expand(&a, static_cast<uint64_t*>(mask->data_ptr()), static_cast<uint8_t*>(in_check->data_ptr()), stream_of(dev));
+    } else {
+        rc = bf_expand(&a, stream_of(dev));
+    }
     TORCH_CHECK(rc == BF_OK, "bf_expand failed (", rc, "): ", bf_last_error());
+    return res;
+}
+
+// movegen and expand_edges in one launch: the dict of edge tensors with mask and in_check
+py::dict movegen_expand(const torch::Tensor& policy, const torch::Tensor& promo, const torch::Tensor& value, const torch::Tensor& boards,
+                        const torch::Tensor& control, int64_t max_edges, const c10::optional<py::dict>& out) {
+    const int64_t n = policy.dim() ? policy.size(0) : 0;
+    check_boards(boards, control, n);
+    BF_VALUE_CHECK(policy.is_cuda() && policy.device() == boards.device() && control.device() == boards.device(), "all inputs must be on one GPU");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(boards.device());
+    const auto made = fresh_moves(n, boards.device());
+    py::dict res = expand_edges<true>(policy, promo, value, made[0], boards, control, max_edges, c10::nullopt, out, c10::nullopt, &made[1]);
+    for (const auto& kv : {std::make_pair("mask", &made[0]), std::make_pair("in_check", &made[1])}) {
+        const py::object t = py::reinterpret_steal<py::object>(THPVariable_Wrap(*kv.second));
+        if (!t || PyDict_SetItemString(res.ptr(), kv.first, t.ptr())) throw py::error_already_set();
+    }
     return res;
 }
 
@@ -668,10 +699,21 @@ PyObject* call_expand_edges(PyObject*, PyObject* const* a, Py_ssize_t n) {   // 
                             opt_tensor_arg(a[7]), out, opt_pair_arg(a[9])).release().ptr();
     });
 }
+PyObject* call_movegen_expand(PyObject*, PyObject* const* a, Py_ssize_t n) {   // as movegen_expand
+    return guarded(n, 7, [&]() -> PyObject* {
+        const long edges = PyLong_AsLong(a[5]);
+        if (edges == -1 && PyErr_Occurred()) throw py::error_already_set();
+        c10::optional<py::dict> out;
+        if (a[6] != Py_None) out = py::reinterpret_borrow<py::object>(a[6]).cast<py::dict>();
+        return movegen_expand(tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]), tensor_arg(a[3]), tensor_arg(a[4]), edges, out).release().ptr();
+    });
+}
 PyMethodDef vector_calls[] = {
     {"movegen", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&call_movegen)), METH_FASTCALL, "(boards, control, out) -> legal-move words and check flags"},
     {"expand_edges", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&call_expand_edges)), METH_FASTCALL,
      "(policy, promo, value, mask, boards, control, max_edges, active, out, leaves) -> edges of search nodes"},
+    {"movegen_expand", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&call_movegen_expand)), METH_FASTCALL,
+     "(policy, promo, value, boards, control, max_edges, out) -> edges of search nodes, legal-move words and check flags"},
     {nullptr, nullptr, 0, nullptr}};
 
 }  // namespace

@@ -438,6 +438,11 @@ typedef struct {
 
 int bf_expand(const bf_expand_args* args, void* stream);
 
+/* bf_movegen and bf_expand in one launch, for every position: args->mask, active and the leaf list are NULL, the legal-move
+ * words and check flags that bf_movegen would write go to mask ([n,32]) and in_check ([n]).  The fewer positions, the
+ * more a launch is worth: from a few thousand on the two are faster apart. */
+int bf_movegen_expand(const bf_expand_args* args, uint64_t* mask, uint8_t* in_check, void* stream);
+
 /* Compaction of the search's leaf flags into the list the evaluator and the expansion take: writes
  * the numbers of the positions whose flag is non-zero, in ascending order, to leaf_index[0 .. count)
  * and the count to leaf_count[0] (both DEVICE memory; leaf_index holds n entries, entries past the

@@ -1,0 +1,87 @@
+"""bf_movegen_expand, move generation and edge expansion in one launch, against the two calls: every output equal, at the edges of its
+workgroups of eight positions, for positions of ordinary and of very many moves; and what it refuses."""
+import ctypes
+
+import pytest
+import torch
+
+from brokefish_amd import encoder_impl, hip_impl, positions
+from brokefish_amd.hip_impl import expand_edges, movegen
+from brokefish_amd.net import BrokefishNet
+
+PAWN, QUEEN, KING, BLACK, CAPTURED = 0, 4 << 6, 5 << 6, 0x400, 0x800
+
+
+def crowded(n, seed):
+    """``n`` boards of eight white queens and seven pawns about to promote, most with more than 128 edges (a second build of the expansion)."""
+    g = torch.Generator().manual_seed(seed)
+    boards = torch.full((n, 32), CAPTURED, dtype=torch.int32)
+    for i in range(n):
+        pawns, victims, rest = (torch.randperm(k, generator=g) for k in (8, 8, 40))
+        for k in range(8):
+            boards[i, k] = int(rest[k]) | QUEEN
+        for k in range(7):
+            boards[i, 8 + k] = 48 + int(pawns[k]) | PAWN
+        boards[i, 15] = int(rest[8]) | KING
+        for k in range(4):
+            boards[i, 16 + k] = 56 + int(victims[k]) | PAWN | BLACK
+        boards[i, 31] = int(rest[9]) | KING | BLACK
+    return boards.to(torch.int16), torch.ones(n, dtype=torch.int16)
+
+
+def both(policy, promo, value, boards, control, edges):
+    mask, check = movegen(boards, control)
+    want = expand_edges(policy, promo, value, mask, boards, control, edges)
+    got = hip_impl._native().movegen_expand(policy, promo, value, boards, control, edges, None)
+    assert torch.equal(got["mask"], mask) and torch.equal(got["in_check"], check)
+    for k, v in want.items():
+        assert torch.equal(got[k], v), k
+    return want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("n,edges", [(1, 96), (2, 1), (7, 96), (8, 32), (9, 255), (250, 96), (1001, 40)])
+def test_one_launch_is_the_two_calls(n, edges, fp32):
+    boards, control, _, _ = [t.cuda() for t in positions.random_positions(n, plies=120, seed=n)]
+    g = torch.Generator("cuda").manual_seed(n)
+    dt = torch.float32 if fp32 else torch.float16
+    policy, promo = (torch.randn(n, 32, k, generator=g, device="cuda").to(dt) for k in (64, 4))
+    both(policy, promo, torch.tanh(torch.randn(n, generator=g, device="cuda")), boards, control, edges)
+
+
+@pytest.mark.gpu
+def test_positions_of_very_many_moves():
+    n = 61
+    boards, control = [t.cuda() for t in crowded(n, 3)]
+    g = torch.Generator("cuda").manual_seed(3)
+    policy, promo = (torch.randn(n, 32, k, generator=g, device="cuda") for k in (64, 4))
+    count = both(policy, promo, torch.zeros(n, device="cuda"), boards, control, 96)["count"]
+    assert int((count > 128).sum()) > 0 and int((count <= 128).sum()) > 0
+
+
+@pytest.mark.gpu
+def test_forward_expand_on_either_side_of_the_line(monkeypatch):
+    torch.manual_seed(0)
+    model = encoder_impl("hip")(BrokefishNet(n_layers=1).eval().randomise_layers_(seed=4), int8=True)
+    batch = [t.cuda() for t in positions.random_positions(70, plies=100, seed=4)][:3]
+    got = {k: v.clone() for k, v in model.forward_expand(*batch).items()}
+    monkeypatch.setattr(hip_impl, "MOVEGEN_EXPAND_MOST", 69)
+    want = model.forward_expand(*batch)
+    assert got.keys() == want.keys() and all(torch.equal(got[k], v) for k, v in want.items())
+
+
+def test_refused_arguments():
+    lib = hip_impl.load_library()
+    a = hip_impl._ExpandArgs()
+    a.n, a.max_edges = 4, 96
+    for name in ("policy", "promo", "value", "boards", "control", "edge_move", "edge_prior", "n_edges"):
+        setattr(a, name, 16)
+    call = lambda mask=16, check=16: lib.bf_movegen_expand(ctypes.byref(a), ctypes.c_void_p(mask), ctypes.c_void_p(check), None)
+    assert call(mask=None) == -1 and call(check=None) == -1
+    for name in ("mask", "active", "leaf_index"):
+        setattr(a, name, 16)
+        assert call() == -1
+        setattr(a, name, None)
+    a.max_edges = 256
+    assert call() == -1
