@@ -117,7 +117,7 @@ struct KArgs {
     const uint8_t* active;        // optional [n]: positions with 0 are skipped, their outputs untouched
     const int* leaf_index;        // optional compacted list: slot j of the launch evaluates position leaf_index[j] ...
     const int* leaf_count;        // ... for j < *leaf_count; slots past the count do nothing
-    // A leaf list shared by two launches, the two-position kernel in front and its one-position form behind:
+    // A leaf list shared by two forms (512 wide: two launches), the two-position kernel in front and its one-position form behind:
     // the former takes whole rounds, the latter what round_rest() leaves.
     int list_split;
     int grid;                     // workgroups of the one-position form, 0: one per position

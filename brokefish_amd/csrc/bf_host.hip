@@ -323,7 +323,7 @@ static int team_limit(const bf_eval_args* a, bool profile, bool enc) {
 struct Route {
     int form;       // enum bf_form
     bool enc;       // the encoder-only build
-    bool rounds;    // whole rounds of two positions per workgroup (form), the rest in a launch of its own
+    bool rounds;    // whole rounds of two positions per workgroup (form), the rest in other workgroups behind them
     int team;       // positions a team launch may hold, 0: none
     bool by_teams(const bf_eval_args* a, int64_t n) const {   // whether n of the launch's positions go to teams
         return team > 0 && !(a->leaf_index && n > team) && n <= (a->shape.d_model == 512 ? 2 : 1) * team;
@@ -371,10 +371,9 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
         e = launch_teams(k);
     } else if (to.rounds) {
         // Two positions per workgroup, in rounds of 512 positions that cost the same full or not: a last round of at most 256
-        // goes to the one-position form in a second launch on the same stream (640 positions: 0.33 ms instead of 0.39, e4m3
-        // 0.39 instead of 0.48).  With a leaf list the count is on the device: both forms are launched and each
-        // takes its share of the list (a launch that finds nothing to do costs 3 us; 200 live leaves of 1000 take a third
-        // less).  Not with other taps or the profile.
+        // goes to the one-position form (640 positions: 0.33 ms instead of 0.39, e4m3 0.39 instead of 0.48), 256 wide in the same launch
+        // (ragged_kernel).  With a leaf list the count is on the device: both forms run and each takes its share of the list (200 live
+        // leaves of 1000 take a third less).  Not with other taps or the profile.
         const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n), pairs = (k.leaf_index ? k.n + 1 : k.n - rest) / 2;
         const bool f8 = a->quant == BF_QUANT_E4M3, teams = rest && !k.leaf_index && to.by_teams(a, rest);
         bf::KArgs front = k, back = k;

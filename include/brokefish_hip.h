@@ -61,7 +61,7 @@ enum bf_quant {
  * carry a network and a format return bit-identical results for it (in the range given at bf_shape), so AUTO may pick by batch
  * size: OCTO up to 256 positions, above that two positions per workgroup: DUO, and a form of its own for the
  * 512-wide network (bf_launch_form tells).  They run in rounds of 512 positions; when AUTO has chosen them and the last round
- * would hold at most 256 positions, those are given to the one-position form in a second launch on the
+ * would hold at most 256 positions, those are given to the one-position form (512 wide, or at most 64: in a second launch) on the
  * same stream. */
 enum bf_kernel {
     BF_KERNEL_AUTO = 0,
