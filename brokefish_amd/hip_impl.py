@@ -987,8 +987,10 @@ class FusedEncoder:
         extra = {}
         ext = _native()
         # every position of a few thousand at most: moves and edges in one launch
-        if mask is None and active is None and leaves is None and ext is not None and boards.dim() == 2 and boards.shape[0] <= MOVEGEN_EXPAND_MOST and \
-                boards.dtype is control.dtype is torch.int16 and boards.is_cuda and control.is_cuda and boards.is_contiguous() and control.is_contiguous():
+        n = boards.shape[0] if boards.dim() else 0
+        if mask is None and active is None and leaves is None and ext is not None and 0 < n <= MOVEGEN_EXPAND_MOST and \
+                boards.shape == (n, T) and control.shape == (n,) and boards.dtype is torch.int16 and control.dtype is torch.int16 and \
+                boards.is_cuda and control.is_cuda and boards.is_contiguous() and control.is_contiguous():
             return ext.movegen_expand(*self.forward_full(boards, control, rep), boards, control, max_edges, out)
         if mask is None:
             mask, chk = movegen(boards, control)
