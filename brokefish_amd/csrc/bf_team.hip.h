@@ -15,7 +15,7 @@
 // So a layer has two exchanges (five members and more: B in two steps, each member summing the accumulators of its two
 // tiles and giving the sums to all, which is a fifth of the bytes at width 512), its weights are read once per team
 // except the output projection's, and a wavefront has one tile (width 512: two) in a matmul.  Measured, one position:
-// 120 -> 74.5 us, e4m3 155 -> 90, width 512 with 16 layers 738 -> 255; 64 positions 120 -> 80, e4m3 155 -> 94.5; 32 of the
+// 120 -> 73.8 us, e4m3 155 -> 88.7, width 512 with 16 layers 738 -> 255; 64 positions 120 -> 78.7, e4m3 155 -> 93.3; 32 of the
 // wide network 738 -> 314.  The arithmetic is that of the other kernels, operation for operation: the results are
 // bit-identical to theirs.
 //
@@ -37,7 +37,8 @@
 // loads stand matters as much as how many they are (one position, 82.3 us before):
 //   - a layer's parameters, asked for right before the Q, K, V products, made those wait for them (all loads return in order);
 //     the four wavefronts without attention ask for the next layer's in that time: 81.5, width 512 273 -> 265;
-//   - weights between the vector instructions of the LayerNorms and the softmax instead of all at once: 78.7;
+//   - weights between the vector instructions of the LayerNorms and the softmax instead of all at once: 78.7 (and, once the ends were shorter,
+//     six instructions apart in LayerNorm 1 and fifteen in 2, not five and ten: 74.7 -> 73.8, 64 positions 79.6 -> 78.7, e4m3 90.2 -> 88.7);
 //   - a member's own piece of exchange B through LDS (96 KB instead of 128), each copy of the sum in the order of the loads: 76.4.
 //
 // An exchange: a wavefront stores its piece, waits until the L2 has it (vmcnt), and stores a flag; the wavefronts that
@@ -468,7 +469,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             fetch_qkv(l);
             if constexpr (TWW == 1) fetch_out(SB, l, 0);
             layernorm(x, pr + C::A_LN1G, pr + C::A_LN1B, y);
-            spaced(std::integral_constant<int, TWW == 1 ? 5 : 12>(), std::integral_constant<int, 16>());
+            spaced(std::integral_constant<int, TWW == 1 ? 6 : 12>(), std::integral_constant<int, 16>());
             __builtin_amdgcn_sched_barrier(0);
             quantise(y);
         }
@@ -643,7 +644,7 @@ __global__ __launch_bounds__(512, 1) void team_kernel(const KArgs a) {
             float y[NP][16];
             if constexpr (TWW == 1) fetch_ff2(l);
             layernorm(x, pr + C::P_B + C::B_LN2G, pr + C::P_B + C::B_LN2B, y);
-            if constexpr (TWW == 1) spaced(std::integral_constant<int, 10>(), std::integral_constant<int, 8>());
+            if constexpr (TWW == 1) spaced(std::integral_constant<int, 15>(), std::integral_constant<int, 8>());
             __builtin_amdgcn_sched_barrier(0);
             quantise(y);
         }
