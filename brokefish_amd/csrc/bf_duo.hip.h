@@ -74,6 +74,18 @@ struct Cfg : Layout<256> {
     static constexpr int LDS_BYTES = NP == 1 && USED_BYTES < 81 * 1024 ? 81 * 1024 : USED_BYTES;
     static_assert(LDS_BYTES <= 160 * 1024, "LDS budget: one workgroup per compute unit");
     static_assert(NT * 4 * FRAG <= HID_P, "normalised stream overlay");
+
+    static constexpr int RING = NP == 2 ? 8 : 12;   // weight fragments (four registers each) in flight or in use
+    // L2 warm-up (see warm_l2 in the kernel): touches of a wavefront per layer; the line of the quarters' streams that touch j of a lane
+    // falls on, and whether there is one
+    static constexpr int WARM = NP == 1 ? 2 : 0, LAYER_LINES = Layout<256>::BPW * BLOCK / 128;   // lines of a layer, per quarter
+    static __host__ __device__ constexpr int warm_line(int j, int block, int blocks, int wave, int lane) {
+        return ((j * ((blocks + 7) >> 3) + (block >> 3)) * 8 + wave) * 64 + lane;
+    }
+    static __host__ __device__ constexpr bool warms(int line, int blocks) { return blocks > 24 && blocks <= 256 && line < 4 * LAYER_LINES; }
+    // Loads that every wavefront has under way behind the first layer's parameters, whatever the launch: the ring's first fill.  A touch is
+    // none of them, since a launch, or a wavefront of it, may have none.  (tests/test_duo_start.py goes through all of them.)
+    static constexpr int BEHIND_PARAMETERS = RING;
 };
 
 // one 16-deep step on operands already widened to fp16; int8 builds never call it
@@ -95,10 +107,10 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
     constexpr int STEPS = C::STEPS, BPW = C::BPW, HB = C::HB;
     constexpr int NB = BPW / 2;      // weight blocks a wave consumes per layer
     constexpr int HT = 2;            // hidden tiles a wave computes per feed-forward step
-    // Weight fragments (four registers each) in flight or in use, and steps between the LDS fetch of an operand fragment and its use
+    // Weight fragments in flight or in use, and steps between the LDS fetch of an operand fragment and its use
     // (4096 positions: 1496 us with one, 1498 with three, as a SIMD's other wavefront covers the latency; the one-position form at 100
     // positions: 118.3 and 116.7; encoder-only, two positions, 512 of them: 179.0, and 179.8 with a register spilled)
-    constexpr int RING = NP == 2 ? 8 : 12, AHEAD = NP == 2 && ENC ? 1 : 3;
+    constexpr int RING = C::RING, AHEAD = NP == 2 && ENC ? 1 : 3;
     constexpr bool SUBN = !FP8 && !TAPS;   // how accumulators are descaled, see descale() (tapped accumulators are stored as they are)
     constexpr int XS = C::XS, PS = C::NW * 64;   // floats of an exchange slot; of one position's part of it
     static_assert(C::KC == 1 && STEPS == TW && KCF == 2 * STEPS, "the 256-wide network");
@@ -256,16 +268,14 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
     // touches (workgroups that left early, another dispatch order) costs time, not correctness.
     // Below four workgroups per XCD the touches cover too little to pay for the loads they delay
     // (loads return in order), above one workgroup per compute unit the launch is not in step.
-    constexpr int WARM = NP == 1 ? 2 : 0;
-    constexpr int LAYER_LINES = BPW * BLOCK / 128;   // per quarter
+    constexpr int WARM = C::WARM, LAYER_LINES = C::LAYER_LINES;
     int warm[WARM > 0 ? WARM : 1] = {};
     auto warm_l2 = [&](int blk0) {
         if constexpr (WARM > 0) {
-            const int per = (blocks + 7) >> 3;
 #pragma unroll
             for (int j = 0; j < WARM; j++) {
-                const int line = ((j * per + (block >> 3)) * 8 + wave) * 64 + lane;
-                if (line < 4 * LAYER_LINES && blocks > 24 && blocks <= 256) {
+                const int line = C::warm_line(j, block, blocks, wave, lane);
+                if (C::warms(line, blocks)) {
                     const int qq = line / LAYER_LINES, off = line % LAYER_LINES;
                     warm[j] = *reinterpret_cast<const int*>(
                         a.wstream + ((size_t)qq * ((size_t)a.n_layers * BPW + HB + 1) + (size_t)blk0) * BLOCK + (size_t)off * 128);
@@ -491,7 +501,7 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
             for (int r = 0; r < 16; r++) a.taps.embed[((size_t)b * T + t) * D + 32 * tile + ch(r, g)] = x[p][r];
     }
 
-    wait_vm<RING + WARM>();   // the parameters have landed: what was asked for after them may not (published to the quarter's other wave by the next barrier)
+    wait_vm<C::BEHIND_PARAMETERS>();   // the parameters have landed: what was asked for after them may not (published to the quarter's other wave by the next barrier)
     warm_done();
     BF_PHASE(PH_EMBED);
 
