@@ -381,10 +381,14 @@ py::dict movegen_expand(const torch::Tensor& policy, const torch::Tensor& promo,
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(boards.device());
     const auto made = fresh_moves(n, boards.device());
     py::dict res = expand_edges<true>(policy, promo, value, made[0], boards, control, max_edges, c10::nullopt, out, c10::nullopt, &made[1]);
+    // a caller's subclass of dict may keep more than the dict (an OrderedDict its order): its own update() sees the two
+    const bool plain = PyDict_CheckExact(res.ptr());
+    const py::dict moves = plain ? res : py::dict();
     for (const auto& kv : {std::make_pair("mask", &made[0]), std::make_pair("in_check", &made[1])}) {
         const py::object t = py::reinterpret_steal<py::object>(THPVariable_Wrap(*kv.second));
-        if (!t || PyDict_SetItemString(res.ptr(), kv.first, t.ptr())) throw py::error_already_set();
+        if (!t || PyDict_SetItemString(moves.ptr(), kv.first, t.ptr())) throw py::error_already_set();
     }
+    if (!plain) res.attr("update")(moves);
     return res;
 }
 

@@ -1,5 +1,6 @@
 """bf_movegen_expand, move generation and edge expansion in one launch, against the two calls: every output equal, at the edges of its
 workgroups of eight positions, for positions of ordinary and of very many moves; and what it refuses."""
+import collections
 import ctypes
 
 import pytest
@@ -69,6 +70,19 @@ def test_forward_expand_on_either_side_of_the_line(monkeypatch):
     monkeypatch.setattr(hip_impl, "MOVEGEN_EXPAND_MOST", 69)
     want = model.forward_expand(*batch)
     assert got.keys() == want.keys() and all(torch.equal(got[k], v) for k, v in want.items())
+
+
+@pytest.mark.gpu
+def test_the_callers_dict_is_the_one_that_comes_back():
+    # an OrderedDict lists what was put into it by its own methods only
+    n = 9
+    torch.manual_seed(0)
+    model = encoder_impl("hip")(BrokefishNet(n_layers=1).eval().randomise_layers_(seed=4), int8=True)
+    batch = [t.cuda() for t in positions.random_positions(n, plies=100, seed=4)][:3]
+    for kind in (dict, collections.OrderedDict):
+        out = kind((k, v.clone()) for k, v in model.forward_expand(*batch).items() if k not in ("mask", "in_check"))
+        got = model.forward_expand(*batch, out=out)
+        assert got is out and list(got)[6:] == ["mask", "in_check"] and len(got.values()) == 8
 
 
 def test_refused_arguments():
