@@ -986,9 +986,11 @@ class FusedEncoder:
         available as ``policy_out`` / ``promo_out`` / ``value_out`` until the next call."""
         extra = {}
         ext = _native()
-        # every position of a few thousand at most: moves and edges in one launch
-        n = boards.shape[0] if boards.dim() else 0
-        if mask is None and active is None and leaves is None and ext is not None and 0 < n <= MOVEGEN_EXPAND_MOST and \
+        # every position of a few thousand at most: moves and edges in one launch (anything else than boards and control
+        # as they have to be goes on to movegen and its errors)
+        if mask is None and active is None and leaves is None and ext is not None and \
+                isinstance(boards, torch.Tensor) and isinstance(control, torch.Tensor) and boards.dim() == 2 and \
+                0 < (n := boards.shape[0]) <= MOVEGEN_EXPAND_MOST and \
                 boards.shape == (n, T) and control.shape == (n,) and boards.dtype is torch.int16 and control.dtype is torch.int16 and \
                 boards.is_cuda and control.is_cuda and boards.is_contiguous() and control.is_contiguous():
             return ext.movegen_expand(*self.forward_full(boards, control, rep), boards, control, max_edges, out)

@@ -85,6 +85,15 @@ def test_the_callers_dict_is_the_one_that_comes_back():
         assert got is out and list(got)[6:] == ["mask", "in_check"] and len(got.values()) == 8
 
 
+@pytest.mark.parametrize("boards,control", [([[0] * 32], torch.ones(1)), (None, torch.ones(1)), (torch.zeros(1, 32).numpy(), torch.ones(1)),
+                                            (torch.zeros(1, 32, dtype=torch.int16), None), (torch.zeros(1, 32, dtype=torch.int16), [1])])
+def test_what_is_no_tensor_is_refused_as_by_movegen(boards, control):
+    with pytest.raises(Exception) as want:
+        movegen(boards, control)
+    with pytest.raises(want.type, match=str(want.value)):
+        hip_impl.FusedEncoder.forward_expand(None, boards, control, None)
+
+
 def test_refused_arguments():
     lib = hip_impl.load_library()
     a = hip_impl._ExpandArgs()
