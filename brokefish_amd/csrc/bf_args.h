@@ -117,11 +117,11 @@ struct KArgs {
     const uint8_t* active;        // optional [n]: positions with 0 are skipped, their outputs untouched
     const int* leaf_index;        // optional compacted list: slot j of the launch evaluates position leaf_index[j] ...
     const int* leaf_count;        // ... for j < *leaf_count; slots past the count do nothing
-    // A leaf list shared by two forms (512 wide: two launches), the two-position kernel in front and its one-position form behind:
-    // the former takes whole rounds, the latter what round_rest() leaves.
-    int list_split;
-    int grid;                     // workgroups of the one-position form, 0: one per position
-    int pairs, single_from;       // both forms in one launch: workgroups of two positions in front; without a list, the first position behind theirs
+    // A launch in rounds: two positions to a workgroup, and behind them one to a workgroup for what round_rest() leaves.  256 wide both
+    // are one launch, 512 wide two.
+    int list_split;               // they share a leaf list, whose count is on the device
+    int grid;                     // workgroups of one position, of both in one launch or with list_split; else 0, one per position
+    int pairs, single_from;       // both in one launch: workgroups of two positions; without a list, the first position behind theirs
     int n;
     const uint8_t* wstream;
     const float* fparams;

@@ -1116,7 +1116,7 @@ inline hipError_t launch_kernel(void (*kernel)(KArgs), std::atomic<unsigned long
 template <int MODE, bool FP8 = false, bool PROF = false, int NPOS = 2>
 hipError_t launch_duo(const KArgs& k, hipStream_t stream) {
     static std::atomic<unsigned long long> lds_set{0};
-    return launch_kernel(&duo_kernel<MODE, FP8, PROF, NPOS>, lds_set, Cfg<FP8, NPOS>::LDS_BYTES, k.grid ? k.grid : (k.n + NPOS - 1) / NPOS, k, stream);
+    return launch_kernel(&duo_kernel<MODE, FP8, PROF, NPOS>, lds_set, Cfg<FP8, NPOS>::LDS_BYTES, (k.n + NPOS - 1) / NPOS, k, stream);
 }
 
 // k.pairs workgroups of two positions and k.grid of one

@@ -374,24 +374,24 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
         // goes to the one-position form (640 positions: 0.33 ms instead of 0.39, e4m3 0.39 instead of 0.48), 256 wide in the same launch
         // (ragged_kernel).  With a leaf list the count is on the device: both forms run and each takes its share of the list (200 live
         // leaves of 1000 take a third less).  Not with other taps or the profile.
-        const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n), pairs = (k.leaf_index ? k.n + 1 : k.n - rest) / 2;
+        const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n);
         const bool f8 = a->quant == BF_QUANT_E4M3, teams = rest && !k.leaf_index && to.by_teams(a, rest);
-        bf::KArgs front = k, back = k;
-        if (k.leaf_index) {
-            front.list_split = back.list_split = 1;
-            back.grid = rest;
-        } else if (rest) {
-            front = slice(k, a->shape.d_model, 0, k.n - rest);
-            back = slice(k, a->shape.d_model, k.n - rest, rest);
-        }
-        if (rest && !wide && !teams) {   // the 256-wide network has both forms in one launch
+        if (rest && !wide && !teams) {
             bf::KArgs both = k;
-            both.list_split = front.list_split;
-            both.pairs = pairs;
+            both.list_split = k.leaf_index != nullptr;
+            both.pairs = (k.leaf_index ? k.n + 1 : k.n - rest) / 2;
             both.single_from = k.leaf_index ? 0 : k.n - rest;
             both.grid = rest;
             e = (f8 ? (enc ? bf::launch_ragged256_fp8_enc : bf::launch_ragged256_fp8) : (enc ? bf::launch_ragged256_enc : bf::launch_ragged256))(both, stream);
-        } else {
+        } else {   // of the 256-wide network: no list, and no last round but the teams'
+            bf::KArgs front = k, back = k;
+            if (k.leaf_index) {
+                front.list_split = back.list_split = 1;
+                back.grid = rest;
+            } else if (rest) {
+                front = slice(k, a->shape.d_model, 0, k.n - rest);
+                back = slice(k, a->shape.d_model, k.n - rest, rest);
+            }
             e = (wide ? (enc ? bf::launch_wide512_enc : bf::launch_wide512)
                  : f8 ? (enc ? bf::launch_duo256_fp8_enc : bf::launch_duo256_fp8)
                       : (enc ? bf::launch_duo256_enc : bf::launch_duo256))(front, stream);
