@@ -94,6 +94,25 @@ def test_what_is_no_tensor_is_refused_as_by_movegen(boards, control):
         hip_impl.FusedEncoder.forward_expand(None, boards, control, None)
 
 
+@pytest.mark.gpu
+def test_into_the_callers_buffers():
+    # node storage that earlier steps have written: every row is this step's, in the caller's memory
+    n = 21
+    torch.manual_seed(0)
+    model = encoder_impl("hip")(BrokefishNet(n_layers=1).eval().randomise_layers_(seed=4), int8=True)
+    steps = [[t.cuda() for t in positions.random_positions(n, plies=100, seed=s)][:3] for s in (5, 6)]
+    want = [{k: v.clone() for k, v in model.forward_expand(*b).items()} for b in steps]
+    out = {k: torch.full_like(v, 7) for k, v in want[0].items() if k not in ("mask", "in_check")}
+    at = {k: v.data_ptr() for k, v in out.items()}
+    for batch, w in zip(steps, want):
+        got = model.forward_expand(*batch, out=out)
+        assert got is out and all(got[k].data_ptr() == p for k, p in at.items())
+        assert got.keys() == w.keys() and all(torch.equal(got[k], w[k]) for k in w)
+    for other, edges in (([t[:20] for t in steps[0]], 96), (steps[0], 40)):
+        with pytest.raises(ValueError, match="another n or max_edges"):
+            model.forward_expand(*other, max_edges=edges, out=out)
+
+
 def test_refused_arguments():
     lib = hip_impl.load_library()
     a = hip_impl._ExpandArgs()
@@ -102,9 +121,11 @@ def test_refused_arguments():
         setattr(a, name, 16)
     call = lambda mask=16, check=16: lib.bf_movegen_expand(ctypes.byref(a), ctypes.c_void_p(mask), ctypes.c_void_p(check), None)
     assert call(mask=None) == -1 and call(check=None) == -1
-    for name in ("mask", "active", "leaf_index"):
-        setattr(a, name, 16)
-        assert call() == -1
-        setattr(a, name, None)
+    for names in (("mask",), ("active",), ("leaf_index", "leaf_count"), ("leaf_index",), ("leaf_count",)):
+        for name in names:
+            setattr(a, name, 16)
+        assert call() == -1 and b"no mask, flags or leaf list" in lib.bf_last_error()
+        for name in names:
+            setattr(a, name, None)
     a.max_edges = 256
-    assert call() == -1
+    assert call() == -1 and b"max_edges" in lib.bf_last_error()

@@ -1,6 +1,6 @@
-"""Sizes whose last round of 512 positions goes to workgroups of one position, in the same launch as the pairs: outputs and the
-encoder alone against the kernel of one position per workgroup of four wavefronts, bit for bit.  (Leaf lists:
-test_leaf_split_gpu.py, test_rounds_gpu.py.)"""
+"""Sizes whose last round of 512 positions goes to workgroups of one position, in the same launch as the pairs: outputs (every value
+head, both formats of the logits) and the encoder alone against the kernel of one position per workgroup of four
+wavefronts, bit for bit.  (Leaf lists: test_leaf_split_gpu.py, test_rounds_gpu.py.)"""
 import pytest
 import torch
 
@@ -29,3 +29,18 @@ def test_a_last_round_in_the_same_launch(made, n):
     for g, w in zip(auto.forward_masked(*[t[:n] for t in batch]), want):
         assert torch.equal(g, w[:n])
     assert torch.equal(auto.forward(x[:n].contiguous(), alive[:n].contiguous()), stream[:n])
+
+
+@pytest.mark.parametrize("quant", ["int8", "fp8"])
+@pytest.mark.parametrize("head,n_value,dtype", [("king", 3, torch.float16), ("pooled", 1, torch.float16), ("pooled", 3, torch.float32),
+                                                ("prenorm", 1, torch.float32), ("prenorm", 3, torch.float16)])
+def test_value_heads_and_halves(quant, head, n_value, dtype):
+    torch.manual_seed(0)
+    net = BrokefishNet(n_layers=2, value_head=head, n_value=n_value).eval().randomise_layers_(seed=10)
+    auto, board = (encoder_impl("hip")(net, out_dtype=dtype, kernel=k, **{quant: True}) for k in ("auto", "board"))
+    batch = [t.cuda() for t in positions.random_positions(577, plies=100, seed=10)]      # a round of pairs and 65 alone
+    want = [t.clone() for t in board.forward_masked(*batch)]
+    got = auto.forward_masked(*batch)
+    assert got[0].dtype == dtype
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
