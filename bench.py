@@ -28,14 +28,14 @@ PEAK_INT8_OPS = 5.0e15                # MI355X dense int8 MFMA, ops/s
 PEAK_FP16_OPS = 2.5e15                # dense fp16 MFMA: the e4m3 format's products run on the fp16 instruction
 # HBM bytes per launch from the FETCH_SIZE / WRITE_SIZE counter runs summarised under profiles/
 # (calibrated on a copy of known size), by (network shape, kernel, batch).
-MEASURED_TRAFFIC_BYTES = {("base", "duo", 4096): 0.445e9, ("base", "twin", 4096): 0.77e9, ("base", "quad", 4096): 3.08e9,
+MEASURED_TRAFFIC_BYTES = {("base", "duo", 4096): 0.443e9, ("base", "twin", 4096): 0.77e9, ("base", "quad", 4096): 3.08e9,
                           ("base", "octo", 256): 5.5e7, ("stress", "octo", 16384): 2.87e10}
 MEASURED_TRAFFIC_BYTES_E4M3 = {("base", "twin", 4096): 0.97e9}
 # ... and of the forms with two positions per workgroup that AUTO runs above 256 positions, by format too
-MEASURED_TRAFFIC_BYTES_PAIRS = {("base", "duo", 4096, "e4m3"): 0.445e9, ("stress", "wide", 16384, "int8"): 1.33e10}
+MEASURED_TRAFFIC_BYTES_PAIRS = {("base", "duo", 4096, "e4m3"): 0.443e9, ("stress", "wide", 16384, "int8"): 1.33e10}
 # vector-ALU instructions per launch (SQ_INSTS_VALU of the same counter runs), by (network shape, kernel, batch):
 # with the matrix products hidden, the launch cannot be shorter than these instructions' issue time
-MEASURED_VALU_INSTS = {("base", "duo", 4096): 4.897e8, ("base", "twin", 4096): 5.131e8}
+MEASURED_VALU_INSTS = {("base", "duo", 4096): 4.896e8, ("base", "twin", 4096): 5.131e8}
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 PEAK_HBM_BPS = 8.0e12                 # MI355X HBM3E, bytes/s
 

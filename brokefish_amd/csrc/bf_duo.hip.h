@@ -415,7 +415,9 @@ __device__ __forceinline__ void evaluate(const KArgs& a, const int block, const 
     // Loads return in order, so what the first layer's weights would hold up is asked for in front of them: the words, then the rows they
     // name.  A unit takes a 16-byte load of 64 lanes in 16 clocks, and five rows for every token are 40 of them in each wave; so
     // the rows that a position's tokens share (clock and repetition, added; the two of colour) come once, four bytes a thread, by way of LDS.
-    // Phase 12.9 k -> 10.3 k ticks; 300 positions 169.6 -> 167.9 us, 200 114.2 -> 113.4, 4096 1425 -> 1415, e4m3 1904 -> 1901.
+    // Phase 12.9 k -> 10.1 k ticks; 300 positions 168.2 -> 167.0 us, 100 113.8 -> 113.0, 4096 1411 -> 1404, e4m3 1891 -> 1881.
+    // (Parameters, touches and the weights stand behind branches, where the compiler cannot count them, and it waits for all of them:
+    // the last position's rows are still used only once the first weights are there.)
     float x[NP][16];
     unsigned alive[NP], word[NP];
     int ctrl[NP], rp[NP];
@@ -1089,8 +1091,9 @@ __global__ __launch_bounds__(512, 1) void duo_kernel(const KArgs a) {
 
 // Both forms in one launch: a.pairs workgroups of two positions, and behind them those of one position that carry the last
 // round.  As a launch of its own the last round waited until every pair was done, and over a leaf list (whose count is on
-// the device, so that either may have nothing to do) it cost a launch: 600 positions 290.7 -> 288.3 us, 700 291.8 -> 289.9, 2200 823.5
-// -> 821.5, e4m3, 700 positions 380.6 -> 377.2, a list of 370 of 1000 with its expansion 184.0 -> 181.9.
+// the device, so that either may have nothing to do) it cost a launch: 577 positions 286.3 -> 283.6 us, 600 285.9 -> 283.0, e4m3, 600
+// positions 372.1 -> 368.9, a list of 370 of 1000 with its expansion 183.9 -> 182.5; 700 and 2200 positions as before.  Over a list
+// there is a workgroup for every pair of the buffer, and those without one only read the count (some 80 live of 4000, with compaction and expansion, 129.1 us, 120 of 12000 135.6).
 template <int MODE, bool FP8>
 __global__ __launch_bounds__(512, 1) void ragged_kernel(const KArgs a) {
     const int block = (int)blockIdx.x;

@@ -461,8 +461,9 @@ __device__ __forceinline__ void expand_pair(const KExpand& a, const Shared& sh, 
 
 // GENERATE: the legal-move words are made here, in a launch less.  Both rows of sixteen lanes of a half generate its position's moves, so that
 // each lane has the word of a slot; with two positions instead of four to a wavefront that costs twice the instructions, which
-// small launches, bound by the launch itself, do not notice: both 10.9 -> 7.2 us for 64 positions as calls of their own, 11.2 -> 7.8 for 4096, 12.0
-// -> 10.1 for 8192; behind an evaluation of 64 87.1 -> 85.2, of 4096 1406 -> 1403, of 8192 2797 -> 2801 and of 12000 4136 -> 4145.
+// small launches, bound by the launch itself, do not notice: both as calls of their own 11.1 -> 6.8 us for 64 positions, 11.7 -> 7.1 for 4096, 12.1
+// -> 9.6 for 8192, 13.7 -> 12.4 for 12000, but 17.0 -> 17.6 for 20000 and 40.4 -> 45.3 for 65536; behind an evaluation of 64 85.9 -> 84.0, and
+// from 1000 on less than runs differ by (4096: 1415 and 1421, 12000: 4162 and 4158).
 template <bool FP32, bool GENERATE>
 __global__ __launch_bounds__(64 * EXPAND_WAVES) void expand_kernel(const KExpand a) {
     __shared__ bf::moves::Table table;

@@ -7,7 +7,7 @@
 // tile 2, where promotion and value lie.  256 wide, two positions, that is 10.2 k clocks of every SIMD; as 32x32 products of
 // whole tiles (tile 2's 25 rows of zeros among them) it was 16.4 k of three SIMDs, and the fourth idled.  With the final norm's
 // parameters and the legal moves asked for ahead and the best move found without LDS permutations: phases heads + stores 29.9 k ->
-// 22.5 k ticks of 483 k; 300 positions 171.6 -> 168.4 us, 100 115.4 -> 113.4, 4096 1434 -> 1421, e4m3 1911 -> 1904.
+// 23.5 k ticks of 462 k; 300 positions 171.2 -> 168.2 us, 100 114.9 -> 113.8, 4096 1427 -> 1411, e4m3 300 230.6 -> 228.4, 4096 1901 -> 1891.
 #pragma once
 
 #include "bf_board.hip.h"
@@ -48,7 +48,8 @@ struct Heads {
           // 0 and 2 then.  (The last lanes' reads end four bytes behind the fragment, in the next one or the block of padding.)
           stream_p(stream_p_), from0((c16 + 32 * (G & 1)) * 16 + 4 * (G >> 1)), from(from0 + 256 * rh) {
         // A wave without a piece of tile 2 sees it empty, and its loads move nothing: with a branch around them the number of loads under way
-        // would not be known, and the chains behind would wait for all of them at every step (200 positions 113.4 -> 112.3 us).
+        // would not be known, and the chains behind would wait for all of them at every step (577 positions 283.5 -> 282.7 us; 100 and 200
+        // as before).
         const size_t stride = (size_t)a.n_layers * blocks_per_layer + HB + 1;
         auto tile = [&](int n, bool used) {
             return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.wstream + (n * stride + (size_t)a.n_layers * blocks_per_layer) * BLOCK), 0,

@@ -359,8 +359,8 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
     const Route to = route(a, kind, k.profile != nullptr);
     const bool enc = to.enc;
     // A launch whose teams have a compute unit for every member (64 positions, 512 wide: 32) goes to the team form (one
-    // position 120 -> 76 us, e4m3 155 -> 92; 512 wide 738 -> 265 us), and 512 wide so does one that two team launches hold
-    // (320 us each; the one-position form takes 738 for up to 256).
+    // position 117 -> 74 us, 64 112 -> 79, e4m3 138 -> 89 and 140 -> 94; 512 wide, one 755 -> 260, 32 728 -> 315), and 512 wide so does one
+    // that two team launches hold (33 positions 727 -> 572, 64 715 -> 620).
     auto launch_teams = [&](const bf::KArgs& s) {
         hipError_t r = hipSuccess;
         for (int at = 0; at < s.n && r == hipSuccess; at += to.team)
@@ -371,9 +371,9 @@ static int launch(const bf_eval_args* a, const bf::KArgs& k, int kind, hipStream
         e = launch_teams(k);
     } else if (to.rounds) {
         // Two positions per workgroup, in rounds of 512 positions that cost the same full or not: a last round of at most 256
-        // goes to the one-position form (640 positions: 0.33 ms instead of 0.39, e4m3 0.39 instead of 0.48), 256 wide in the same launch
-        // (ragged_kernel).  With a leaf list the count is on the device: both forms run and each takes its share of the list (200 live
-        // leaves of 1000 take a third less).  Not with other taps or the profile.
+        // goes to the one-position form (640 positions: 0.282 ms instead of 0.335, e4m3 0.368 instead of 0.452), 256 wide in the same
+        // launch (ragged_kernel).  With a leaf list the count is on the device: both forms run and each takes its share of the list (200
+        // live leaves of 1000 take 114 us instead of 166).  Not with other taps or the profile.
         const int rest = k.leaf_index ? bf::DUO_ROUND / 2 : bf::round_rest(k.n);
         const bool f8 = a->quant == BF_QUANT_E4M3, teams = rest && !k.leaf_index && to.by_teams(a, rest);
         if (rest && !wide && !teams) {

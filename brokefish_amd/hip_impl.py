@@ -247,8 +247,8 @@ def stream_rate(nbytes: int, workgroups: int = 4096, reps: int = 3, device="cuda
     return float(rate)
 
 
-# Positions up to which forward_expand generates moves in the expansion's launch: a step of 64 takes 85.2 us then, not 87.1, one of 4096
-# 1403 and 1406, one of 8192 2801 and 2797.
+# Positions up to which forward_expand generates moves in the expansion's launch: a step of 64 takes 84.0 us then, not 85.9; the two by
+# themselves 7.1 us, not 11.7, for 4096, which in a step is less than runs differ by, and 17.6, not 17.0, for 20000.
 MOVEGEN_EXPAND_MOST = 4096
 
 
