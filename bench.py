@@ -32,7 +32,7 @@ MEASURED_TRAFFIC_BYTES = {("base", "duo", 4096): 0.443e9, ("base", "twin", 4096)
                           ("base", "octo", 256): 5.5e7, ("stress", "octo", 16384): 2.87e10}
 MEASURED_TRAFFIC_BYTES_E4M3 = {("base", "twin", 4096): 0.97e9}
 # ... and of the forms with two positions per workgroup that AUTO runs above 256 positions, by format too
-MEASURED_TRAFFIC_BYTES_PAIRS = {("base", "duo", 4096, "e4m3"): 0.443e9, ("stress", "wide", 16384, "int8"): 1.33e10}
+MEASURED_TRAFFIC_BYTES_PAIRS = {("base", "duo", 4096, "e4m3"): 0.443e9, ("stress", "wide", 16384, "int8"): 1.32e10}
 # vector-ALU instructions per launch (SQ_INSTS_VALU of the same counter runs), by (network shape, kernel, batch):
 # with the matrix products hidden, the launch cannot be shorter than these instructions' issue time
 MEASURED_VALU_INSTS = {("base", "duo", 4096): 4.896e8, ("base", "twin", 4096): 5.131e8}

@@ -39,11 +39,13 @@ struct Heads {
     unsigned long long legal[HALVES];
     v4f head[HALVES], rest;
 
+    // by value: chosen as an element of the array, it was put into private memory (512 wide: 12 bytes a lane, 33 MiB written by 16384 positions)
+    static __device__ __forceinline__ int of(int p, int first, int second) { return p ? second : first; }
     __device__ __forceinline__ Heads(const KArgs& a_, int blocks_per_layer, int lane_, int wave, const int (&bp)[NP], const bool (&live_)[NP], const int (&ctrl)[NP],
                                      int stream_at_, int stream_p_)
         : a(a_), lane(lane_), q(wave & 3), sub(wave >> 2), G(lane_ >> 4), c16(lane_ & 15), ht(q & 1), rh(q >> 1), th0(NP == 2 ? 0 : sub), mine(NP == 2 ? sub : 0),
           extra(sub == 1 && (NP == 2 || q < 2)), xmine(NP == 2 ? q & 1 : 0), xth(NP == 2 ? q >> 1 : q), b(mine ? bp[NP - 1] : bp[0]), xb(xmine ? bp[NP - 1] : bp[0]),
-          xctrl(xmine ? ctrl[NP - 1] : ctrl[0]), live(mine ? live_[NP - 1] : live_[0]), xlive(xmine ? live_[NP - 1] : live_[0]), stream_at(stream_at_),
+          xctrl(of(xmine, ctrl[0], ctrl[NP - 1])), live(mine ? live_[NP - 1] : live_[0]), xlive(xmine ? live_[NP - 1] : live_[0]), stream_at(stream_at_),
           // Lane (row, k) reads, of a fragment, the lane of its row and of half k % 2, from element k / 2 on: what it multiplies lies in places
           // 0 and 2 then.  (The last lanes' reads end four bytes behind the fragment, in the next one or the block of padding.)
           stream_p(stream_p_), from0((c16 + 32 * (G & 1)) * 16 + 4 * (G >> 1)), from(from0 + 256 * rh) {
