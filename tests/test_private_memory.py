@@ -1,4 +1,4 @@
-"""The two-position kernels keep what they hold in registers and LDS: the compiler's own report of private memory (spills, arrays
+"""The int8 kernels with two positions per workgroup keep what they hold in registers and LDS: the compiler's own report of private memory (spills, arrays
 chosen from by a value that is not a constant) says none."""
 import os
 import re
