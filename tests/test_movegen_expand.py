@@ -62,6 +62,22 @@ def test_positions_of_very_many_moves():
 
 
 @pytest.mark.gpu
+def test_positions_of_more_moves_than_the_layout_holds():
+    # more than 256 edges (fifteen queens on one square): the words just generated are read back, beside positions of the ordinary kind
+    n = 21
+    boards, control = [t[:n].clone() for t in positions.random_positions(n, plies=80, seed=7)[:2]]
+    for i in (0, 3, 4, 8, 15, 20):
+        boards[i] = CAPTURED
+        boards[i, :15] = (27 + i) | QUEEN
+        boards[i, 15], boards[i, 31] = KING, 63 | KING | BLACK
+        control[i] = 1
+    g = torch.Generator("cuda").manual_seed(7)
+    policy, promo = (torch.randn(n, 32, k, generator=g, device="cuda").half() for k in (64, 4))
+    count = both(policy, promo, torch.zeros(n, device="cuda"), boards.cuda(), control.cuda(), 96)["count"]
+    assert int((count > 256).sum()) == 6 and int((count <= 128).sum()) == 15
+
+
+@pytest.mark.gpu
 def test_forward_expand_on_either_side_of_the_line(monkeypatch):
     torch.manual_seed(0)
     model = encoder_impl("hip")(BrokefishNet(n_layers=1).eval().randomise_layers_(seed=4), int8=True)

@@ -44,3 +44,23 @@ def test_value_heads_and_halves(quant, head, n_value, dtype):
     assert got[0].dtype == dtype
     for g, w in zip(got, want):
         assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("n,live", [(577, 0), (577, 1), (600, 200), (768, 700), (1281, 1281)])
+def test_flags_passed_to_the_library_as_they_are(n, live):
+    # FusedEncoder compacts flags above 256 positions; a C caller need not (e4m3 and 512 wide: test_rounds_gpu.py)
+    torch.manual_seed(0)
+    net = BrokefishNet(n_layers=2).eval().randomise_layers_(seed=9)
+    auto, board = (encoder_impl("hip")(net, int8=True, out_dtype=torch.float32, kernel=k) for k in ("auto", "board"))
+    batch = [t.cuda() for t in positions.random_positions(n, plies=100, seed=9)]
+    want = [t.clone() for t in board.forward_masked(*batch)]
+    flags = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    flags[torch.randperm(n, generator=torch.Generator().manual_seed(live))[:live].cuda()] = 1
+    on = flags != 0
+    auto.forward_masked(*batch)                                # the buffers exist
+    outs = (auto.policy_out, auto.promo_out, auto.value_out, auto.best_out)
+    for t in outs:
+        t.fill_(7)
+    auto._call(auto._args(*batch, *outs, active=flags))
+    for g, w in zip(outs, want):
+        assert torch.equal(g[on], w[on]) and bool((g[~on] == 7).all())
